@@ -58,7 +58,7 @@ extern "C" {
 #define MUON_HIP_K_BX_UPDATE 10 /* the a.X + B.X launch that carries the parameter update in its epilogue */
 #define MUON_HIP_K_COUNT 11
 
-/* GEMM kernel variants; MUON_HIP_CFG_AUTO picks per kernel and shape.  All feed LDS with direct
+/* GEMM kernel variants; MUON_HIP_CFG_AUTO picks per kernel, shape and number of tiles.  All feed LDS with direct
  * global->LDS loads (global_load_lds_dwordx4), software pipelined behind the MFMAs. */
 #define MUON_HIP_CFG_AUTO (-1)
 #define MUON_HIP_CFG_128_PIPE 0      /* 128x128 tile, 4 waves, 64-column k-tiles, two LDS stages */
@@ -69,7 +69,9 @@ extern "C" {
                                         the next tile's first loads land behind an epilogue that needs no LDS.  Taken by launches
                                         of more than one round of tiles: a.X + B.X, and the symmetric products with reductions
                                         of at most 2048; everything else runs MUON_HIP_CFG_256_PINGPONG */
-#define MUON_HIP_CFG_COUNT 5
+#define MUON_HIP_CFG_64_DEEP 5       /* 64x64 tile, 4 waves, eight stages of 64 columns: launches that leave most compute units
+                                        idle.  The a.X + B.X launch that carries the parameter update runs MUON_HIP_CFG_128_PINGPONG */
+#define MUON_HIP_CFG_COUNT 6
 
 int muon_hip_version(void);
 const char* muon_hip_last_error(void);

@@ -94,7 +94,7 @@ struct Timed {
 
 // ---- geometry / workspace ------------------------------------------------------------
 struct Plan {
-    int rows, cols, batch, M, K, Mp, Kp, tile, cfg, nparts;
+    int rows, cols, batch, M, K, Mp, Kp, tile, nparts;
     bool transposed;
     long n, strideU, strideX, strideA;  // elements per matrix: U dense, the others blocked
     size_t offX[2], offA, offB, offParts, offDenom, offPpx, total;
@@ -105,20 +105,26 @@ inline long round_up(long v, long m) { return (v + m - 1) / m * m; }
 // Tile edge for a matrix whose short side is M: 256 when M is a whole number of 256-tiles.
 bool use_tile256(int M) { return M % 256 == 0 && M >= 512; }
 
+// A configuration, and whether the launcher may replace it by one with smaller tiles where a launch has too few (it may not
+// when the caller has named it).
+struct Cfg {
+    int id;
+    bool adapt;
+};
+
 // Configuration per kernel, from a sweep of every variant over the benchmark shapes: the ping-pong kernel
 // everywhere, on 256-tiles where they fill the machine and on 128-tiles (two workgroups per compute unit) for
 // short sides that are no whole number of 256-tiles and for the symmetric products of matrices up to 512 rows.
-int pick_cfg(int M, int epi = EPI_BX, int kdim = 0) {
+Cfg pick_cfg(int M, int epi = EPI_BX) {
     const int forced = g_forced_cfg.load(std::memory_order_relaxed);
-    if (forced != MUON_HIP_CFG_AUTO) return forced;
-    (void)kdim;
-    if (!use_tile256(M)) return GEMM_CFG_128_PINGPONG;
-    if (epi != EPI_BX && M <= 512) return GEMM_CFG_128_PINGPONG;
+    if (forced != MUON_HIP_CFG_AUTO) return {forced, false};
+    if (!use_tile256(M)) return {GEMM_CFG_128_PINGPONG, true};
+    if (epi != EPI_BX && M <= 512) return {GEMM_CFG_128_PINGPONG, true};
     // The persistent kernel where the launcher takes it: a.X + B.X, and the symmetric products with reductions of at
     // most 2048 (past that a tile is long enough that what the persistent kernel removes around it no longer shows in
     // a step that runs at the power limit); launches of at most one round of tiles and those that carry the parameter
     // update run the one-tile ping-pong kernel.
-    return GEMM_CFG_256_PERSIST;
+    return {GEMM_CFG_256_PERSIST, true};
 }
 
 int make_plan(int rows, int cols, int batch, Plan& p) {
@@ -130,9 +136,9 @@ int make_plan(int rows, int cols, int batch, Plan& p) {
     p.transposed = rows > cols;
     p.M = rows < cols ? rows : cols;
     p.K = rows < cols ? cols : rows;
-    p.cfg = pick_cfg(p.M);
-    p.tile = gemm_cfg_tile(p.cfg);
-    if (p.tile == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration %d", p.cfg);
+    p.tile = gemm_cfg_tile(pick_cfg(p.M).id);
+    if (p.tile == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration");
+    if (p.tile < 128) p.tile = 128;  // the elementwise kernels move whole 128-tiles
     p.Mp = (int)round_up(p.M, p.tile);
     p.Kp = (int)round_up(p.K, p.tile);
     p.n = (long)rows * cols;
@@ -179,39 +185,36 @@ int check_gemm(int cfg, int Mp, int Kp, int batch, int& tile) {
     tile = gemm_cfg_tile(cfg);
     if (tile == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration %d", cfg);
     if (Mp <= 0 || Kp <= 0 || batch <= 0) return fail(MUON_HIP_EINVAL, "sizes must be positive");
-    if (Mp % tile || Kp % tile) return fail(MUON_HIP_ESHAPE, "Mp=%d, Kp=%d must be multiples of the %d tile", Mp, Kp, tile);
+    const int edge = tile < 128 ? 128 : tile;  // every kernel's reduction is a multiple of 128
+    if (Mp % edge || Kp % edge) return fail(MUON_HIP_ESHAPE, "Mp=%d, Kp=%d must be multiples of the %d tile", Mp, Kp, edge);
     const long T = Mp / tile, TN = Kp / tile;
     if (T * TN * batch > 0x7fffffffL) return fail(MUON_HIP_ESHAPE, "too many tiles for one launch");
     return 0;
 }
 
 // The three products on blocked buffers; matrix b of a batch starts at b * blocked_elems(rows, cols).
-int do_syrk(int cfg, const bf16_t* X, bf16_t* A, int Mp, int Kp, int batch, unsigned* ppx, hipStream_t s) {
+int do_syrk(const Cfg& cfg, const bf16_t* X, bf16_t* A, int Mp, int Kp, int batch, unsigned* ppx, hipStream_t s) {
     GemmArgs g = {};
-    const int tile = gemm_cfg_tile(cfg), T = Mp / tile;
     g.P = g.Q = X;
     g.strideP = g.strideQ = blocked_elems(Mp, Kp);
     g.kdim = Kp;
-    g.tiles_m = g.tiles_n = T;
-    g.tiles_per_mat = T * (T + 1) / 2;
+    g.rows = g.cols = Mp;
     g.batch = batch;
     g.C = g.Ct = A;
     g.strideC = g.strideCt = blocked_elems(Mp, Mp);
     g.cbC = g.cbCt = Mp / BLK_COLS;
     g.ppx = ppx;
     Timed t(MUON_HIP_K_SYRK, s);
-    hipError_t e = launch_gemm_nt(cfg, EPI_SYRK, g, s);
+    hipError_t e = launch_gemm_nt(cfg.id, EPI_SYRK, g, cfg.adapt, s);
     return e == hipSuccess ? 0 : hip_fail(e, "syrk launch");
 }
 
-int do_sympoly(int cfg, const bf16_t* A, bf16_t* B, int Mp, int batch, double b, double c, unsigned* ppx, hipStream_t s) {
+int do_sympoly(const Cfg& cfg, const bf16_t* A, bf16_t* B, int Mp, int batch, double b, double c, unsigned* ppx, hipStream_t s) {
     GemmArgs g = {};
-    const int tile = gemm_cfg_tile(cfg), T = Mp / tile;
     g.P = g.Q = A;
     g.strideP = g.strideQ = blocked_elems(Mp, Mp);
     g.kdim = Mp;
-    g.tiles_m = g.tiles_n = T;
-    g.tiles_per_mat = T * (T + 1) / 2;
+    g.rows = g.cols = Mp;
     g.batch = batch;
     g.C = g.Ct = B;
     g.strideC = g.strideCt = blocked_elems(Mp, Mp);
@@ -223,7 +226,7 @@ int do_sympoly(int cfg, const bf16_t* A, bf16_t* B, int Mp, int batch, double b,
     g.s1 = (float)c;
     g.ppx = ppx;
     Timed t(MUON_HIP_K_SYMPOLY, s);
-    hipError_t e = launch_gemm_nt(cfg, EPI_SYMPOLY, g, s);
+    hipError_t e = launch_gemm_nt(cfg.id, EPI_SYMPOLY, g, cfg.adapt, s);
     return e == hipSuccess ? 0 : hip_fail(e, "sympoly launch");
 }
 
@@ -234,19 +237,17 @@ struct FoldUpdate {
     double scale, lr, weight_decay;
 };
 
-int do_bx(int cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp, int Kp, int batch, double a, unsigned* ppx,
+int do_bx(const Cfg& cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp, int Kp, int batch, double a, unsigned* ppx,
           hipStream_t s, const FoldUpdate* fold = nullptr) {
     GemmArgs g = {};
-    const int tile = gemm_cfg_tile(cfg);
     g.P = B;
     g.strideP = blocked_elems(Mp, Mp);
     g.Q = X;
     g.strideQ = blocked_elems(Mp, Kp);
     g.cbQ = Kp / BLK_COLS;
     g.kdim = Mp;
-    g.tiles_m = Mp / tile;
-    g.tiles_n = Kp / tile;
-    g.tiles_per_mat = g.tiles_m * g.tiles_n;
+    g.rows = Mp;
+    g.cols = Kp;
     g.batch = batch;
     g.C = Xout;
     g.strideC = blocked_elems(Mp, Kp);
@@ -266,7 +267,7 @@ int do_bx(int cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp, int K
     }
     g.ppx = ppx;
     Timed t(fold ? MUON_HIP_K_BX_UPDATE : MUON_HIP_K_BX, s);
-    hipError_t e = launch_gemm_nt(cfg, !fold ? EPI_BX : fold->rows <= fold->cols ? EPI_BX_UPD : EPI_BX_UPD_T, g, s);
+    hipError_t e = launch_gemm_nt(cfg.id, !fold ? EPI_BX : fold->rows <= fold->cols ? EPI_BX_UPD : EPI_BX_UPD_T, g, cfg.adapt, s);
     return e == hipSuccess ? 0 : hip_fail(e, "bx launch");
 }
 
@@ -364,7 +365,7 @@ int ns_chain(void* workspace, int rows, int cols, int batch, int steps, double a
     unsigned* ppx = ws_ppx(workspace, p);  // zero: muon_hip_normalize has just cleared them
     int cur = 0;
     for (int it = 0; it < steps; ++it) {
-        if (int rc = do_syrk(pick_cfg(p.M, EPI_SYRK, p.Kp), X[cur], A, p.Mp, p.Kp, batch, ppx, s)) return rc;
+        if (int rc = do_syrk(pick_cfg(p.M, EPI_SYRK), X[cur], A, p.Mp, p.Kp, batch, ppx, s)) return rc;
         if (int rc = do_sympoly(pick_cfg(p.M, EPI_SYMPOLY), A, B, p.Mp, batch, b, c, ppx, s)) return rc;
         if (int rc = do_bx(pick_cfg(p.M, EPI_BX), B, X[cur], X[cur ^ 1], p.Mp, p.Kp, batch, a, ppx, s,
                            it == steps - 1 ? fold : nullptr))
@@ -455,33 +456,33 @@ int muon_hip_unpack_bf16(const void* src, int rows_p, int cols_p, void* dst, lon
 }
 
 int muon_hip_syrk_bf16(const void* X, void* A, int Mp, int Kp, int batch, int cfg, void* counters, void* stream) {
-    if (cfg == MUON_HIP_CFG_AUTO) cfg = pick_cfg(Mp, EPI_SYRK, Kp);
+    const Cfg use = cfg == MUON_HIP_CFG_AUTO ? pick_cfg(Mp, EPI_SYRK) : Cfg{cfg, false};
     int tile;
-    if (int rc = check_gemm(cfg, Mp, Kp, batch, tile)) return rc;
+    if (int rc = check_gemm(use.id, Mp, Kp, batch, tile)) return rc;
     if (!X || !A) return fail(MUON_HIP_EINVAL, "null operand");
     if (int rc = check_counters(counters)) return rc;
-    return do_syrk(cfg, (const bf16_t*)X, (bf16_t*)A, Mp, Kp, batch, (unsigned*)counters, (hipStream_t)stream);
+    return do_syrk(use, (const bf16_t*)X, (bf16_t*)A, Mp, Kp, batch, (unsigned*)counters, (hipStream_t)stream);
 }
 
 int muon_hip_sympoly_bf16(const void* A, void* B, int Mp, int batch, double b, double c, int cfg, void* counters,
                           void* stream) {
-    if (cfg == MUON_HIP_CFG_AUTO) cfg = pick_cfg(Mp, EPI_SYMPOLY);
+    const Cfg use = cfg == MUON_HIP_CFG_AUTO ? pick_cfg(Mp, EPI_SYMPOLY) : Cfg{cfg, false};
     int tile;
-    if (int rc = check_gemm(cfg, Mp, Mp, batch, tile)) return rc;
+    if (int rc = check_gemm(use.id, Mp, Mp, batch, tile)) return rc;
     if (!A || !B || A == B) return fail(MUON_HIP_EINVAL, "null or aliased operand");
     if (int rc = check_counters(counters)) return rc;
-    return do_sympoly(cfg, (const bf16_t*)A, (bf16_t*)B, Mp, batch, b, c, (unsigned*)counters, (hipStream_t)stream);
+    return do_sympoly(use, (const bf16_t*)A, (bf16_t*)B, Mp, batch, b, c, (unsigned*)counters, (hipStream_t)stream);
 }
 
 int muon_hip_bx_axpy_bf16(const void* B, const void* X, void* Xout, int Mp, int Kp, int batch, double a, int cfg,
                           void* counters, void* stream) {
-    if (cfg == MUON_HIP_CFG_AUTO) cfg = pick_cfg(Mp, EPI_BX);
+    const Cfg use = cfg == MUON_HIP_CFG_AUTO ? pick_cfg(Mp, EPI_BX) : Cfg{cfg, false};
     int tile;
-    if (int rc = check_gemm(cfg, Mp, Kp, batch, tile)) return rc;
+    if (int rc = check_gemm(use.id, Mp, Kp, batch, tile)) return rc;
     if (!B || !X || !Xout) return fail(MUON_HIP_EINVAL, "null operand");
     if (Xout == X) return fail(MUON_HIP_EINVAL, "Xout must not alias X");
     if (int rc = check_counters(counters)) return rc;
-    return do_bx(cfg, (const bf16_t*)B, (const bf16_t*)X, (bf16_t*)Xout, Mp, Kp, batch, a, (unsigned*)counters, (hipStream_t)stream);
+    return do_bx(use, (const bf16_t*)B, (const bf16_t*)X, (bf16_t*)Xout, Mp, Kp, batch, a, (unsigned*)counters, (hipStream_t)stream);
 }
 
 int muon_hip_adamw(void* p, const void* g, void* exp_avg, void* exp_avg_sq, int dtype, long n, int step, double lr,

@@ -67,7 +67,13 @@ __device__ __forceinline__ float wave_sum(float v) {
 __device__ __forceinline__ int xcd_remap(int pid, int nblocks, int xcd_shift) {
     const int span = XCD_CHUNK << xcd_shift;  // one run for every XCD
     const int full = nblocks / span * span;
-    if (pid >= full) return pid;
-    const int xcd = pid & ((1 << xcd_shift) - 1), local = pid >> xcd_shift;
+    const int xcds = 1 << xcd_shift, xcd = pid & (xcds - 1);
+    if (pid >= full) {
+        // Less than a run per XCD is left: equal runs, so that each XCD still works on neighbouring tiles and fetches the
+        // panels of its own run only (dealt one by one, every XCD fetched nearly every panel).
+        const int rest = nblocks - full, local = (pid - full) >> xcd_shift, each = rest >> xcd_shift, more = rest & (xcds - 1);
+        return full + xcd * each + (xcd < more ? xcd : more) + local;
+    }
+    const int local = pid >> xcd_shift;
     return (((local / XCD_CHUNK) << xcd_shift) + xcd) * XCD_CHUNK + local % XCD_CHUNK;
 }

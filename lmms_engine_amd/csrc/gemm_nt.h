@@ -18,7 +18,8 @@ enum {
                                 // tile's first loads land behind an epilogue without LDS): a.X + B.X, and the symmetric
                                 // products with reductions up to 2048; launches of at most one round and the launches that
                                 // carry the parameter update run GEMM_CFG_256_PINGPONG
-    GEMM_CFG_COUNT = 5
+    GEMM_CFG_64_DEEP = 5,       // 64x64 tile, 4 waves, eight stages of 64 columns: launches that leave most compute units idle
+    GEMM_CFG_COUNT = 6
 };
 
 struct GemmArgs {
@@ -27,8 +28,9 @@ struct GemmArgs {
     long strideP, strideQ;  // elements between matrices of the batch
     int cbQ;                // BX: column blocks of Q
     int kdim;               // reduction length, a multiple of 128
-    int tiles_m, tiles_n;   // tile grid of one matrix (triangular kernels: tiles_m == tiles_n)
-    int tiles_per_mat;      // tiles_m*(tiles_m+1)/2 for the symmetric kernels, tiles_m*tiles_n for BX
+    int rows, cols;         // of C, padded to whole 128-tiles (symmetric kernels: rows == cols)
+    int tiles_m, tiles_n;   // set by the launcher: tile grid of one matrix
+    int tiles_per_mat;      // set by the launcher: tiles_m*(tiles_m+1)/2 for the symmetric kernels, tiles_m*tiles_n for BX
     int batch;
     bf16_t* C;              // out[i][j], blocked with cbC column blocks
     long strideC;
@@ -67,4 +69,6 @@ struct MachineShape {
 hipError_t machine_shape(MachineShape& ms);
 
 int gemm_cfg_tile(int cfg);
-hipError_t launch_gemm_nt(int cfg, int epi, const GemmArgs& g, hipStream_t stream);
+// `adapt`: cfg is the choice by shape, and a launch whose tiles would not fill the machine may run on smaller ones (same
+// results bit for bit).  Without it the launch runs cfg as named.
+hipError_t launch_gemm_nt(int cfg, int epi, const GemmArgs& g, bool adapt, hipStream_t stream);

@@ -1032,6 +1032,153 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pp_kernel(const GemmArg
     pp_tile<BM, BN, WGM, WGN, EPI>(g, decode_tile<EPI>(g), smem);
 }
 
+// ---- kernel 2b: a deep pipeline on 64x64 tiles, for launches that leave compute units idle --------
+// One matrix makes few tiles: 896 x 4864 has 28 triangular 128-tiles for 256 compute units, and a lone workgroup is paced by
+// the latency of its three k-tiles in flight (157 ns per 32 columns).  64-tiles are four times the workgroups at half the
+// bytes each, and with at most one workgroup per compute unit all of its LDS can hold stages: eight of 64 columns, 112 KB in
+// flight.  Four waves of 2x2 fragments, one barrier per k-tile; the fragment reads of k-tile t+1 and the loads of k-tile t+7
+// issue between the MFMAs of k-tile t.  What bounds it then is the L2 (136 workgroups pull 12 TB/s).  Nothing is loaded past
+// the end (short reductions are the common case): the last eight k-tiles are a straight line of their own with the counts of
+// what is still in flight.  Measured against 128-tiles: X.Xt of 896 x 4864 30 -> 17.7 us, of 1024 x 1024 9.8 -> 6.5,
+// b.A + c.A.A of 896 rows 9.9 -> 6.4; the same structure on 128-tiles was no faster than the ping-pong kernel (34 against
+// 25 us for 1024 x 4096).  Stage layout, swizzle and transposing reads are those of kernel 1, the register epilogues those of
+// the persistent kernel, and every element sums its products in the same order: the results are the other kernels' bit for bit.
+template <int EPI>
+__global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmArgs g) {
+    static_assert(EPI == EPI_BX || EPI == EPI_SYRK || EPI == EPI_SYMPOLY, "the epilogues that need no LDS");
+    constexpr int BM = 64, BN = 64, WGM = 2, WGN = 2, NW = 4;
+    constexpr int WTM = BM / WGM, WTN = BN / WGN, FM = WTM / 16, FN = WTN / 16;
+    constexpr int A_BYTES = BM * ROW_BYTES, STAGE = A_BYTES + BN * ROW_BYTES, NST = 8;
+    constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW, NLD = LA + LB;  // 1 KB load instructions per wave and k-tile
+    constexpr int KS = 2, NRD = FM + FN;
+    constexpr bool QT = EPI == EPI_BX;
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WGN, wn = wave % WGN;
+    const TileCoord tc = decode_tile<EPI>(g);
+    const int kb = g.kdim / BLK_COLS;
+    const bf16_t* Pb = uniform_ptr(g.P + tc.bidx * g.strideP + panel_offset(tc.ti * BM, kb));
+    const bf16_t* Qb = uniform_ptr(g.Q + tc.bidx * g.strideQ +
+                                   (QT ? (long)(tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel_offset(tc.tj * BN, kb)));
+    const int drow = lane >> 3;
+    // byte offsets of this lane's 16 bytes of each load instruction, from the scalar base of the k-tile (ping-pong kernel: no
+    // vector ALU work per load)
+    auto chunk_off = [](int e) { return (e >> BLK_SHIFT) * BLK_ELEMS + (e & (BLK_COLS - 1)); };
+    unsigned offa[LA], offb[LB];
+#pragma unroll
+    for (int n = 0; n < LA; ++n)  // LA is even: instruction n of a wave covers an even or an odd group of eight rows
+        offa[n] = (unsigned)(((wave * LA + n) * 8 + drow) * BLK_COLS + chunk_off(((lane & 7) ^ (((n & 1) << 2) | (drow >> 1))) * 8)) * 2;
+#pragma unroll
+    for (int n = 0; n < LB; ++n) {
+        const int t = wave * LB + n;
+        offb[n] = QT ? (unsigned)((t >> 2) * BLK_ELEMS + ((t & 3) * 16 + (lane >> 2)) * BLK_COLS + ((lane & 3) ^ (((lane >> 5) & 1) << 1)) * 8) * 2
+                     : (unsigned)((t * 8 + drow) * BLK_COLS + chunk_off(((lane & 7) ^ (((n & 1) << 2) | (drow >> 1))) * 8)) * 2;
+    }
+    constexpr int KT_BLOCKS = 64 / BLK_COLS;
+    const unsigned lds_base = (unsigned)(uintptr_t)(lds_void_ptr)smem;
+    auto dma = [&](const char* base, unsigned voff, unsigned lds_byte) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :
+                     : "s"(lds_byte), "v"(voff), "s"(base)
+                     : "memory");
+    };
+    auto issue_one = [&](int n, int kt) {  // load instruction n of k-tile kt: rows of P first, then Q
+        const unsigned st = lds_base + (kt & (NST - 1)) * STAGE;
+        const long koff = (long)kt * KT_BLOCKS * BLK_ELEMS;
+        const int k0 = kt * 64;
+        if (n < LA) dma((const char*)(Pb + koff), offa[n], st + (wave * LA + n) * 8 * ROW_BYTES);
+        else
+            dma((const char*)(Qb + (QT ? (long)(k0 >> 8) * g.cbQ * BLK_ELEMS + (k0 & 255) * BLK_COLS : koff)), offb[n - LA],
+                st + A_BYTES + (wave * LB + n - LA) * 8 * ROW_BYTES);
+    };
+    const int sw = (lane >> 1) & 7, kq = lane >> 4;
+    const int a_off = (wm * WTM + (lane & 15)) * ROW_BYTES;
+    const int b_off = A_BYTES + (wn * WTN + (lane & 15)) * ROW_BYTES;
+    const int q_off[2] = {A_BYTES + wn * (WTN / 32) * 4096 + qt_lane_offset(lane, 0),
+                          A_BYTES + wn * (WTN / 32) * 4096 + qt_lane_offset(lane, 1)};
+    bf16x8 fr[2][KS * NRD];
+    auto read_one = [&](auto buf_c, int o, const unsigned char* st) {
+        constexpr int BUF = decltype(buf_c)::value;
+        const int ks = o / NRD, n = o % NRD, co = (((ks << 2) | kq) ^ sw) << 4;
+        if (n < FM) fr[BUF][o] = *(const bf16x8*)(st + a_off + n * 16 * ROW_BYTES + co);
+        else if (QT) fr[BUF][o] = lds_read_qt(st + q_off[(n - FM) & 1] + ((n - FM) >> 1) * 4096 + ks * 32 * 64);
+        else fr[BUF][o] = *(const bf16x8*)(st + b_off + (n - FM) * 16 * ROW_BYTES + co);
+    };
+    f32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // k-tile kt: its fragments are in flight from LDS.  WAIT: k-tiles after kt+1 whose loads may be outstanding (-1: there is
+    // no k-tile kt+1).  After the barrier every wave has read k-tile kt-1, so its stage takes k-tile kt+NST-1.  The fragment
+    // reads of k-tile kt+1 and the loads stand between the MFMAs and issue in their shadow (a lone wave per SIMD has nothing
+    // else to hide them behind); the fences pin that order.
+    auto body = [&](int kt, auto buf_c, auto issue_c, auto wait_c) {
+        constexpr int BUF = decltype(buf_c)::value, WAIT = decltype(wait_c)::value;
+        constexpr int NRD2 = WAIT >= 0 ? KS * NRD : 0, NOTH = NRD2 + (decltype(issue_c)::value ? NLD : 0);
+        constexpr int NMF = KS * FM * FN, PER = (KS * NRD + NLD + NMF - 1) / NMF;
+        WAIT_LGKM0();
+        if constexpr (WAIT >= 0) {
+            WAIT_VM(WAIT * NLD);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+        const unsigned char* stn = smem + ((kt + 1) & (NST - 1)) * STAGE;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < NMF; ++m) {
+            const int ks = m / (FM * FN), j = m % (FM * FN) / FM, ii = m % FM, i = (j & 1) ? FM - 1 - ii : ii;
+            const bf16x8 p = fr[BUF][ks * NRD + i], q = fr[BUF][ks * NRD + FM + j];
+            acc[i][j] = QT ? mfma16(q, p, acc[i][j]) : mfma16(p, q, acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int o = m * PER + u;
+                if (o < NRD2) read_one(std::integral_constant<int, BUF ^ 1>{}, o, stn);
+                else if (o < NOTH) issue_one(o - NRD2, kt + NST - 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    const int nk = g.kdim / 64;  // even: reductions are multiples of 128
+    // k-tiles nk-R and nk-R+1, the first of the last R
+    auto tail_pair = [&](auto r_c) {
+        constexpr int R = decltype(r_c)::value;
+        if (nk < R) return;
+        constexpr int W0 = R - 2 < NST - 3 ? R - 2 : NST - 3, W1 = R - 3 < NST - 3 ? R - 3 : NST - 3;
+        body(nk - R, I0{}, std::integral_constant<bool, R == NST>{}, std::integral_constant<int, W0>{});
+        body(nk - R + 1, I1{}, std::false_type{}, std::integral_constant<int, W1>{});
+    };
+    const int first = nk < NST - 1 ? nk : NST - 1;
+    for (int t = 0; t < first; ++t)
+#pragma unroll
+        for (int n = 0; n < NLD; ++n) issue_one(n, t);
+    if (nk >= NST) WAIT_VM((NST - 2) * NLD);
+    else if (nk == 6) WAIT_VM(5 * NLD);
+    else if (nk == 4) WAIT_VM(3 * NLD);
+    else WAIT_VM(NLD);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int o = 0; o < KS * NRD; ++o) read_one(I0{}, o, smem);
+    for (int kt = 0; kt + NST < nk; kt += 2) {
+        body(kt, I0{}, std::true_type{}, std::integral_constant<int, NST - 3>{});
+        body(kt + 1, I1{}, std::true_type{}, std::integral_constant<int, NST - 3>{});
+    }
+    tail_pair(std::integral_constant<int, 8>{});
+    tail_pair(std::integral_constant<int, 6>{});
+    tail_pair(std::integral_constant<int, 4>{});
+    tail_pair(std::integral_constant<int, 2>{});
+    if constexpr (QT) epilogue_nn_reg<BM, BN, WGM, WGN>(g, tc, acc);
+    else epilogue_sym_reg<BM, BN, WGM, WGN, EPI>(g, tc, acc);
+}
+
 // The same with a split tail: when the tile count leaves the last round of the compute units mostly empty,
 // the first g.big_blocks workgroups compute 256x256 tiles as above and every remaining tile is cut
 // into four 128x128 tiles, one workgroup each, which fill the CUs that would otherwise idle for a
@@ -1354,12 +1501,24 @@ hipError_t launch_one(const GemmArgs& g, int nblocks, hipStream_t stream) {
 }
 
 template <int EPI>
+hipError_t launch_deep(const GemmArgs& g, int nblocks, hipStream_t stream) {
+    constexpr int smem = 8 * (64 + 64) * ROW_BYTES;
+    static std::atomic<unsigned long long> configured{0};
+    if (hipError_t e = allow_dynamic_lds((const void*)gemm_nt_deep_kernel<EPI>, smem, configured); e != hipSuccess) return e;
+    hipLaunchKernelGGL(gemm_nt_deep_kernel<EPI>, dim3(nblocks), dim3(256), smem, stream, g);
+    return hipGetLastError();
+}
+
+template <int EPI>
 hipError_t launch_cfg(int cfg, const GemmArgs& g, int nblocks, hipStream_t stream) {
     switch (cfg) {
         case GEMM_CFG_128_PIPE: return launch_one<128, 128, 2, 2, EPI, 0>(g, nblocks, stream);
         case GEMM_CFG_256_PIPE: return launch_one<256, 256, 2, 4, EPI, 0>(g, nblocks, stream);
         case GEMM_CFG_256_PINGPONG: return launch_one<256, 256, 2, 4, EPI, 1>(g, nblocks, stream);
         case GEMM_CFG_128_PINGPONG: return launch_one<128, 128, 2, 4, EPI, 1>(g, nblocks, stream);
+        case GEMM_CFG_64_DEEP:
+            if constexpr (EPI == EPI_BX_UPD || EPI == EPI_BX_UPD_T) return hipErrorInvalidValue;  // the launcher takes 128-tiles
+            else return launch_deep<EPI>(g, nblocks, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1368,6 +1527,7 @@ hipError_t launch_cfg(int cfg, const GemmArgs& g, int nblocks, hipStream_t strea
 
 int gemm_cfg_tile(int cfg) {
     switch (cfg) {
+        case GEMM_CFG_64_DEEP: return 64;
         case GEMM_CFG_128_PIPE:
         case GEMM_CFG_128_PINGPONG: return 128;
         case GEMM_CFG_256_PIPE:
@@ -1414,14 +1574,39 @@ hipError_t machine_shape(MachineShape& ms) {
     return hipSuccess;
 }
 
-hipError_t launch_gemm_nt(int cfg, int epi, const GemmArgs& args, hipStream_t stream) {
+// Workgroups of one launch that cuts C into square tiles of `tile`.
+long count_tiles(const GemmArgs& g, int epi, int tile) {
+    const long tm = g.rows / tile, tn = g.cols / tile;
+    return (epi_is_bx(epi) ? tm * tn : tm * (tm + 1) / 2) * g.batch;
+}
+
+// Smaller tiles for a launch that would not fill the machine (every configuration sums in the same order, so the result does
+// not depend on the choice).  Measured on one to 48 matrices of 128 to 5120 rows, times per k-tile of 32 columns: a round of
+// 256-tiles (one workgroup per compute unit) 460 ns, of 128-tiles 157 ns alone on a compute unit and 336 ns for two.  So
+// 128-tiles win while they need no more than the two places per compute unit (X.Xt of 2048 x 5632: 84 -> 36 us, of
+// 3072 x 8192 with 300 tiles 119 -> 91) and lose beyond (4096 x 4096 with 528: 68 -> 76); 64-tiles win while each has a
+// compute unit of its own (896 x 4864: 30 -> 18) and lose with two (512 x 1408 x 8, 288 tiles: 11.7 -> 14.0).
+int fill_machine(int cfg, int epi, const GemmArgs& g, int cus) {
+    if (gemm_cfg_tile(cfg) == 256 && count_tiles(g, epi, 128) <= 2 * cus) cfg = GEMM_CFG_128_PINGPONG;
+    if (cfg == GEMM_CFG_128_PINGPONG && !epi_fold_mode(epi) && count_tiles(g, epi, 64) <= cus) cfg = GEMM_CFG_64_DEEP;
+    return cfg;
+}
+
+hipError_t launch_gemm_nt(int cfg, int epi, const GemmArgs& args, bool adapt, hipStream_t stream) {
     GemmArgs g = args;
     MachineShape ms;
     if (hipError_t e = machine_shape(ms); e != hipSuccess) return e;
     g.xcd_shift = ms.xcd_shift;
     const int cus = ms.cus;
-    const int nblocks = g.tiles_per_mat * g.batch;
+    if (adapt) cfg = fill_machine(cfg, epi, g, cus);
+    if (cfg == GEMM_CFG_64_DEEP && epi_fold_mode(epi)) cfg = GEMM_CFG_128_PINGPONG;
+    const int tile = gemm_cfg_tile(cfg);
+    if (tile == 0) return hipErrorInvalidValue;
+    const int nblocks = (int)count_tiles(g, epi, tile);  // the callers have checked that it fits
     if (nblocks <= 0) return hipSuccess;
+    g.tiles_m = g.rows / tile;
+    g.tiles_n = g.cols / tile;
+    g.tiles_per_mat = nblocks / g.batch;
     // Ping-pong kernel: split the tiles of a last round that would fill at most a quarter of the CUs (a 128x128
     // tile takes about 0.6 of the time of a 256x256 one, so one round of quarters beats a round of whole tiles).
     const int rest = nblocks % cus;
