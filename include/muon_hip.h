@@ -137,6 +137,22 @@ int muon_hip_step_grouped(const void* const* p_ptrs, const void* const* g_ptrs, 
                           double lr, double weight_decay, double beta, int nesterov, int ns_steps, double scale,
                           double a, double b, double c, int write_back_grad, void* stream);
 
+/* The same for the matrices of several shapes at once: every stage is one launch over all of them as far as their tile
+ * configurations allow, so that a set of a few matrices of each shape fills the machine and pays for one sequence of
+ * launches.  Equal to muon_hip_step_grouped per bucket bit for bit.  `workspace` holds the buckets' workspaces one after the
+ * other: the sum of muon_hip_workspace_bytes over them.  `scale` as in muon_hip_apply_update. */
+#define MUON_HIP_MAX_BUCKETS 16
+typedef struct {
+    const void* const* p_ptrs; /* device tables of `batch` pointers each */
+    const void* const* g_ptrs;
+    const void* const* m_ptrs;
+    int rows, cols, batch;
+    double scale;
+} muon_hip_bucket;
+int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int g_dtype, int m_dtype, void* workspace, double lr,
+                        double weight_decay, double beta, int nesterov, int ns_steps, double a, double b, double c,
+                        int write_back_grad, void* stream);
+
 /* ---- blocked matrices and single GEMM entry points ---------------------------------------
  * The Newton-Schulz operands are kept in blocks of 256 rows x 32 columns (16 KB, 64-byte
  * rows back to back): element (r, c) of a matrix with cb = cols / 32 column blocks is at

@@ -24,6 +24,16 @@ MULTI_CHUNK = 16384  # MUON_HIP_MULTI_CHUNK
 STATIC_MAX_CHUNKS = 1 << 20  # MUON_HIP_STATIC_MAX_CHUNKS
 PPX_COUNTER_BYTES = 576  # MUON_HIP_PPX_COUNTER_BYTES
 
+MAX_BUCKETS = 16  # MUON_HIP_MAX_BUCKETS
+
+
+class Bucket(ctypes.Structure):
+    """muon_hip_bucket"""
+
+    _fields_ = [("p_ptrs", c_void_p), ("g_ptrs", c_void_p), ("m_ptrs", c_void_p), ("rows", c_int), ("cols", c_int),
+                ("batch", c_int), ("scale", c_double)]
+
+
 # name -> (restype, argtypes); mirrors include/muon_hip.h one to one
 SIGNATURES = {
     "muon_hip_version": (c_int, []),
@@ -42,6 +52,8 @@ SIGNATURES = {
     "muon_hip_step_grouped": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int,
                                       c_double, c_double, c_double, c_int, c_int, c_double, c_double, c_double,
                                       c_double, c_int, c_void_p]),
+    "muon_hip_step_multi": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_double, c_double, c_double, c_int, c_int,
+                                    c_double, c_double, c_double, c_int, c_void_p]),
     "muon_hip_blocked_elems": (c_long, [c_int, c_int]),
     "muon_hip_pack_bf16": (c_int, [c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
     "muon_hip_unpack_bf16": (c_int, [c_void_p, c_int, c_int, c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p]),

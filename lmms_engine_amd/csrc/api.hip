@@ -168,7 +168,6 @@ int make_plan(int rows, int cols, int batch, Plan& p) {
 }
 
 inline bf16_t* wsp(void* ws, size_t off) { return (bf16_t*)((char*)ws + off); }
-inline unsigned* ws_ppx(void* ws, const Plan& p) { return (unsigned*)((char*)ws + p.offPpx); }
 
 int check_ws(const void* ws) {
     if (!ws) return fail(MUON_HIP_EINVAL, "workspace is null");
@@ -193,8 +192,11 @@ int check_gemm(int cfg, int Mp, int Kp, int batch, int& tile) {
 }
 
 // The three products on blocked buffers; matrix b of a batch starts at b * blocked_elems(rows, cols).
-int do_syrk(const Cfg& cfg, const bf16_t* X, bf16_t* A, int Mp, int Kp, int batch, unsigned* ppx, hipStream_t s) {
-    GemmArgs g = {};
+GemmItem syrk_item(int cfg, const bf16_t* X, bf16_t* A, int Mp, int Kp, int batch, unsigned* ppx) {
+    GemmItem it = {};
+    GemmArgs& g = it.g;
+    it.cfg = cfg;
+    it.epi = EPI_SYRK;
     g.P = g.Q = X;
     g.strideP = g.strideQ = blocked_elems(Mp, Kp);
     g.kdim = Kp;
@@ -204,13 +206,14 @@ int do_syrk(const Cfg& cfg, const bf16_t* X, bf16_t* A, int Mp, int Kp, int batc
     g.strideC = g.strideCt = blocked_elems(Mp, Mp);
     g.cbC = g.cbCt = Mp / BLK_COLS;
     g.ppx = ppx;
-    Timed t(MUON_HIP_K_SYRK, s);
-    hipError_t e = launch_gemm_nt(cfg.id, EPI_SYRK, g, cfg.adapt, s);
-    return e == hipSuccess ? 0 : hip_fail(e, "syrk launch");
+    return it;
 }
 
-int do_sympoly(const Cfg& cfg, const bf16_t* A, bf16_t* B, int Mp, int batch, double b, double c, unsigned* ppx, hipStream_t s) {
-    GemmArgs g = {};
+GemmItem sympoly_item(int cfg, const bf16_t* A, bf16_t* B, int Mp, int batch, double b, double c, unsigned* ppx) {
+    GemmItem it = {};
+    GemmArgs& g = it.g;
+    it.cfg = cfg;
+    it.epi = EPI_SYMPOLY;
     g.P = g.Q = A;
     g.strideP = g.strideQ = blocked_elems(Mp, Mp);
     g.kdim = Mp;
@@ -225,21 +228,20 @@ int do_sympoly(const Cfg& cfg, const bf16_t* A, bf16_t* B, int Mp, int batch, do
     g.s0 = (float)b;
     g.s1 = (float)c;
     g.ppx = ppx;
-    Timed t(MUON_HIP_K_SYMPOLY, s);
-    hipError_t e = launch_gemm_nt(cfg.id, EPI_SYMPOLY, g, cfg.adapt, s);
-    return e == hipSuccess ? 0 : hip_fail(e, "sympoly launch");
+    return it;
 }
 
-// Parameter update folded into the last B.X of a step (the parameter is X's image when rows <= cols, its transpose otherwise).
-struct FoldUpdate {
-    const void* const* p_ptrs;
-    int p_dtype, rows, cols;
-    double scale, lr, weight_decay;
+// What the last B.X of a step does to the parameters (which are X's image when rows <= cols, its transpose otherwise).
+struct UpdateArgs {
+    int p_dtype;
+    double lr, weight_decay;
 };
 
-int do_bx(const Cfg& cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp, int Kp, int batch, double a, unsigned* ppx,
-          hipStream_t s, const FoldUpdate* fold = nullptr) {
-    GemmArgs g = {};
+GemmItem bx_item(int cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp, int Kp, int batch, double a, unsigned* ppx) {
+    GemmItem it = {};
+    GemmArgs& g = it.g;
+    it.cfg = cfg;
+    it.epi = EPI_BX;
     g.P = B;
     g.strideP = blocked_elems(Mp, Mp);
     g.Q = X;
@@ -256,22 +258,125 @@ int do_bx(const Cfg& cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp
     g.strideEt = blocked_elems(Mp, Kp);
     g.cbEt = Kp / BLK_COLS;
     g.s0 = (float)a;
-    if (fold) {
-        g.upd_ptrs = fold->p_ptrs;
-        g.upd_dtype = fold->p_dtype;
-        g.upd_rows = fold->rows;
-        g.upd_cols = fold->cols;
-        g.upd_scale = (float)fold->scale;
-        g.upd_decay = (float)(1.0 - fold->lr * fold->weight_decay);
-        g.upd_alpha = (float)(-fold->lr);
-    }
     g.ppx = ppx;
-    Timed t(fold ? MUON_HIP_K_BX_UPDATE : MUON_HIP_K_BX, s);
-    hipError_t e = launch_gemm_nt(cfg.id, !fold ? EPI_BX : fold->rows <= fold->cols ? EPI_BX_UPD : EPI_BX_UPD_T, g, cfg.adapt, s);
-    return e == hipSuccess ? 0 : hip_fail(e, "bx launch");
+    return it;
+}
+
+void fold_update(GemmItem& it, const void* const* p_ptrs, int rows, int cols, double scale, const UpdateArgs& u) {
+    it.epi = rows <= cols ? EPI_BX_UPD : EPI_BX_UPD_T;
+    it.g.upd_ptrs = p_ptrs;
+    it.g.upd_dtype = u.p_dtype;
+    it.g.upd_rows = rows;
+    it.g.upd_cols = cols;
+    it.g.upd_scale = (float)scale;
+    it.g.upd_decay = (float)(1.0 - u.lr * u.weight_decay);
+    it.g.upd_alpha = (float)(-u.lr);
+}
+
+int launch_items(int kernel_id, const char* what, const GemmItem* items, int n, bool adapt, hipStream_t s) {
+    Timed t(kernel_id, s);
+    hipError_t e = launch_gemm_nt(items, n, adapt, s);
+    return e == hipSuccess ? 0 : hip_fail(e, what);
 }
 
 int dtype_ok(int d) { return d == MUON_HIP_F32 || d == MUON_HIP_BF16; }
+
+// The same-shape matrices of one call, each shape with its own part of the workspace.  Every stage is one launch over all of
+// them as far as the kernels' configurations allow: a set of a few matrices of several shapes would otherwise leave most of
+// the machine idle in every launch, and pay 3 to 5 us of host and device time for each.
+struct Bucket {
+    Plan p;
+    char* ws;
+    const void* const* p_ptrs = nullptr;
+    const void* const* g_ptrs = nullptr;
+    const void* const* m_ptrs = nullptr;
+    double scale = 1.0;
+    int init(int rows, int cols, int batch, void* workspace) {
+        ws = (char*)workspace;
+        return make_plan(rows, cols, batch, p);
+    }
+    bf16_t* at(size_t off) const { return (bf16_t*)(ws + off); }
+    EwBucket ew() const {
+        return EwBucket{g_ptrs, m_ptrs, at(p.offX[1]), p.strideU, (float*)(ws + p.offParts), (float*)(ws + p.offDenom), at(p.offX[0]),
+                        p.strideX, p.rows, p.cols, p.Mp, p.Kp, p.nparts, p.batch};
+    }
+};
+struct Work {
+    int n = 0;
+    Bucket b[MUON_HIP_MAX_BUCKETS];
+};
+static_assert(MUON_HIP_MAX_BUCKETS <= GEMM_MAX_LIST && MUON_HIP_MAX_BUCKETS <= EW_MAX_LIST, "a launch takes every bucket of a call");
+
+int one_bucket(int rows, int cols, int batch, void* workspace, Work& w) {
+    w.n = 1;
+    if (int rc = w.b[0].init(rows, cols, batch, workspace)) return rc;
+    return check_ws(workspace);
+}
+
+void ew_list(const Work& w, EwList& l) {
+    l.n = w.n;
+    for (int i = 0; i < w.n; ++i) l.b[i] = w.b[i].ew();
+}
+
+int do_momentum(const Work& w, int g_dtype, int m_dtype, double beta, int nesterov, int write_back_grad, hipStream_t s) {
+    for (int i = 0; i < w.n; ++i)
+        if (!w.b[i].g_ptrs || !w.b[i].m_ptrs) return fail(MUON_HIP_EINVAL, "pointer table is null");
+    const bool combo = (g_dtype == MUON_HIP_F32 && m_dtype == MUON_HIP_F32) ||
+                       (g_dtype == MUON_HIP_BF16 && (m_dtype == MUON_HIP_F32 || m_dtype == MUON_HIP_BF16));
+    if (!combo) return fail(MUON_HIP_EINVAL, "unsupported (grad, momentum) dtypes (%d, %d)", g_dtype, m_dtype);
+    EwList l;
+    ew_list(w, l);
+    Timed t(MUON_HIP_K_MOMENTUM, s);
+    hipError_t e = launch_momentum_norm(l, g_dtype, m_dtype, beta, nesterov, write_back_grad, s);
+    return e == hipSuccess ? 0 : hip_fail(e, "momentum_norm launch");
+}
+
+// The tile counters of the persistent kernels are those of the first bucket; the normalisation clears them.
+unsigned* ppx_counters(const Work& w) { return (unsigned*)(w.b[0].ws + w.b[0].p.offPpx); }
+
+int do_normalize(const Work& w, hipStream_t s) {
+    EwList l;
+    ew_list(w, l);
+    Timed t(MUON_HIP_K_NORMALIZE, s);
+    hipError_t e = launch_normalize(l, ppx_counters(w), (int)(GEMM_PPX_COUNTER_BYTES / sizeof(unsigned)), s);
+    return e == hipSuccess ? 0 : hip_fail(e, "normalize launch");
+}
+
+// Normalise, then `steps` iterations; with `upd` the last B.X applies the parameter update instead of writing X'.
+int ns_chain(const Work& w, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s) {
+    if (steps < 0) return fail(MUON_HIP_EINVAL, "steps must be >= 0");
+    if (int rc = do_normalize(w, s)) return rc;
+    unsigned* ppx = ppx_counters(w);
+    GemmItem items[MUON_HIP_MAX_BUCKETS];
+    for (int it = 0; it < steps; ++it) {
+        const int cur = it & 1;
+        bool adapt = true;
+        auto each = [&](int epi, auto make) {
+            for (int i = 0; i < w.n; ++i) {
+                const Bucket& k = w.b[i];
+                const Cfg cfg = pick_cfg(k.p.M, epi);
+                adapt = cfg.adapt;  // the same for all: a forced configuration is forced for every launch
+                items[i] = make(k, cfg.id);
+            }
+        };
+        each(EPI_SYRK, [&](const Bucket& k, int cfg) {
+            return syrk_item(cfg, k.at(k.p.offX[cur]), k.at(k.p.offA), k.p.Mp, k.p.Kp, k.p.batch, ppx);
+        });
+        if (int rc = launch_items(MUON_HIP_K_SYRK, "syrk launch", items, w.n, adapt, s)) return rc;
+        each(EPI_SYMPOLY, [&](const Bucket& k, int cfg) {
+            return sympoly_item(cfg, k.at(k.p.offA), k.at(k.p.offB), k.p.Mp, k.p.batch, b, c, ppx);
+        });
+        if (int rc = launch_items(MUON_HIP_K_SYMPOLY, "sympoly launch", items, w.n, adapt, s)) return rc;
+        const bool last = upd && it == steps - 1;
+        each(EPI_BX, [&](const Bucket& k, int cfg) {
+            GemmItem g = bx_item(cfg, k.at(k.p.offB), k.at(k.p.offX[cur]), k.at(k.p.offX[cur ^ 1]), k.p.Mp, k.p.Kp, k.p.batch, a, ppx);
+            if (last) fold_update(g, k.p_ptrs, k.p.rows, k.p.cols, k.scale, *upd);
+            return g;
+        });
+        if (int rc = launch_items(last ? MUON_HIP_K_BX_UPDATE : MUON_HIP_K_BX, "bx launch", items, w.n, adapt, s)) return rc;
+    }
+    return 0;
+}
 
 }  // namespace
 
@@ -307,19 +412,11 @@ size_t muon_hip_workspace_bytes(int rows, int cols, int batch) {
 int muon_hip_momentum_norm(const void* const* g_ptrs, const void* const* m_ptrs, int g_dtype, int m_dtype,
                            void* workspace, int rows, int cols, int batch, double beta, int nesterov,
                            int write_back_grad, void* stream) {
-    Plan p;
-    if (int rc = make_plan(rows, cols, batch, p)) return rc;
-    if (int rc = check_ws(workspace)) return rc;
-    if (!g_ptrs || !m_ptrs) return fail(MUON_HIP_EINVAL, "pointer table is null");
-    const bool combo = (g_dtype == MUON_HIP_F32 && m_dtype == MUON_HIP_F32) ||
-                       (g_dtype == MUON_HIP_BF16 && (m_dtype == MUON_HIP_F32 || m_dtype == MUON_HIP_BF16));
-    if (!combo) return fail(MUON_HIP_EINVAL, "unsupported (grad, momentum) dtypes (%d, %d)", g_dtype, m_dtype);
-    hipStream_t s = (hipStream_t)stream;
-    Timed t(MUON_HIP_K_MOMENTUM, s);
-    hipError_t e = launch_momentum_norm(g_ptrs, m_ptrs, g_dtype, m_dtype, wsp(workspace, p.offX[1]), p.strideU,
-                                        (float*)((char*)workspace + p.offParts), p.nparts, p.n, batch, beta, nesterov,
-                                        write_back_grad, s);
-    return e == hipSuccess ? 0 : hip_fail(e, "momentum_norm launch");
+    Work w;
+    if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
+    w.b[0].g_ptrs = g_ptrs;
+    w.b[0].m_ptrs = m_ptrs;
+    return do_momentum(w, g_dtype, m_dtype, beta, nesterov, write_back_grad, (hipStream_t)stream);
 }
 
 int muon_hip_cast_norm(const void* G, int g_dtype, void* workspace, int rows, int cols, int batch, void* stream) {
@@ -335,52 +432,16 @@ int muon_hip_cast_norm(const void* G, int g_dtype, void* workspace, int rows, in
 }
 
 int muon_hip_normalize(void* workspace, int rows, int cols, int batch, void* stream) {
-    Plan p;
-    if (int rc = make_plan(rows, cols, batch, p)) return rc;
-    if (int rc = check_ws(workspace)) return rc;
-    hipStream_t s = (hipStream_t)stream;
-    Timed t(MUON_HIP_K_NORMALIZE, s);
-    hipError_t e = launch_normalize(wsp(workspace, p.offX[1]), p.strideU, (const float*)((char*)workspace + p.offParts),
-                                    p.nparts, (float*)((char*)workspace + p.offDenom), wsp(workspace, p.offX[0]),
-                                    p.strideX, rows, cols, p.Mp, p.Kp, batch, ws_ppx(workspace, p),
-                                    (int)(GEMM_PPX_COUNTER_BYTES / sizeof(unsigned)), s);
-    return e == hipSuccess ? 0 : hip_fail(e, "normalize launch");
+    Work w;
+    if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
+    return do_normalize(w, (hipStream_t)stream);
 }
-
-}  // extern "C"
-
-namespace {
-// normalise, then `steps` iterations; with `fold` the last B.X applies the parameter update instead of writing X'
-int ns_chain(void* workspace, int rows, int cols, int batch, int steps, double a, double b, double c, void* stream,
-             const FoldUpdate* fold) {
-    Plan p;
-    if (int rc = make_plan(rows, cols, batch, p)) return rc;
-    if (int rc = check_ws(workspace)) return rc;
-    if (steps < 0) return fail(MUON_HIP_EINVAL, "steps must be >= 0");
-    if (int rc = muon_hip_normalize(workspace, rows, cols, batch, stream)) return rc;
-    hipStream_t s = (hipStream_t)stream;
-    bf16_t* X[2] = {wsp(workspace, p.offX[0]), wsp(workspace, p.offX[1])};
-    bf16_t* A = wsp(workspace, p.offA);
-    bf16_t* B = wsp(workspace, p.offB);
-    unsigned* ppx = ws_ppx(workspace, p);  // zero: muon_hip_normalize has just cleared them
-    int cur = 0;
-    for (int it = 0; it < steps; ++it) {
-        if (int rc = do_syrk(pick_cfg(p.M, EPI_SYRK), X[cur], A, p.Mp, p.Kp, batch, ppx, s)) return rc;
-        if (int rc = do_sympoly(pick_cfg(p.M, EPI_SYMPOLY), A, B, p.Mp, batch, b, c, ppx, s)) return rc;
-        if (int rc = do_bx(pick_cfg(p.M, EPI_BX), B, X[cur], X[cur ^ 1], p.Mp, p.Kp, batch, a, ppx, s,
-                           it == steps - 1 ? fold : nullptr))
-            return rc;
-        cur ^= 1;
-    }
-    return 0;
-}
-}  // namespace
-
-extern "C" {
 
 int muon_hip_ns_grouped(void* workspace, int rows, int cols, int batch, int steps, double a, double b, double c,
                         void* stream) {
-    return ns_chain(workspace, rows, cols, batch, steps, a, b, c, stream, nullptr);
+    Work w;
+    if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
+    return ns_chain(w, steps, a, b, c, nullptr, (hipStream_t)stream);
 }
 
 int muon_hip_apply_update(const void* const* p_ptrs, int p_dtype, void* workspace, int rows, int cols, int batch,
@@ -408,23 +469,47 @@ int muon_hip_ns_output(void* workspace, int rows, int cols, int batch, int steps
     return e == hipSuccess ? 0 : hip_fail(e, "ns_output launch");
 }
 
+int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int g_dtype, int m_dtype, void* workspace, double lr,
+                        double weight_decay, double beta, int nesterov, int ns_steps, double a, double b, double c,
+                        int write_back_grad, void* stream) {
+    if (!buckets || n < 1 || n > MUON_HIP_MAX_BUCKETS)
+        return fail(MUON_HIP_EINVAL, "1 to %d buckets per call", MUON_HIP_MAX_BUCKETS);
+    if (int rc = check_ws(workspace)) return rc;
+    if (!dtype_ok(p_dtype) || ns_steps < 0) return fail(MUON_HIP_EINVAL, "bad dtype or steps");
+    Work w;
+    w.n = n;
+    char* base = (char*)workspace;
+    for (int i = 0; i < n; ++i) {
+        const muon_hip_bucket& in = buckets[i];
+        if (!in.p_ptrs) return fail(MUON_HIP_EINVAL, "pointer table is null");
+        if (int rc = w.b[i].init(in.rows, in.cols, in.batch, base)) return rc;
+        w.b[i].p_ptrs = in.p_ptrs;
+        w.b[i].g_ptrs = in.g_ptrs;
+        w.b[i].m_ptrs = in.m_ptrs;
+        w.b[i].scale = in.scale;
+        base += w.b[i].p.total;
+    }
+    hipStream_t s = (hipStream_t)stream;
+    if (int rc = do_momentum(w, g_dtype, m_dtype, beta, nesterov, write_back_grad, s)) return rc;
+    // The parameter is updated by the epilogue of the last B.X (for rows > cols through a transposing gather out of
+    // LDS): the final X' is then neither written nor read back.  Without an iteration there is no such product.
+    const UpdateArgs u{p_dtype, lr, weight_decay};
+    if (int rc = ns_chain(w, ns_steps, a, b, c, &u, s)) return rc;
+    if (ns_steps == 0)
+        for (int i = 0; i < n; ++i)
+            if (int rc = muon_hip_apply_update(w.b[i].p_ptrs, p_dtype, w.b[i].ws, w.b[i].p.rows, w.b[i].p.cols, w.b[i].p.batch, 0,
+                                               w.b[i].scale, lr, weight_decay, stream))
+                return rc;
+    return 0;
+}
+
 int muon_hip_step_grouped(const void* const* p_ptrs, const void* const* g_ptrs, const void* const* m_ptrs,
                           int p_dtype, int g_dtype, int m_dtype, void* workspace, int rows, int cols, int batch,
                           double lr, double weight_decay, double beta, int nesterov, int ns_steps, double scale,
                           double a, double b, double c, int write_back_grad, void* stream) {
-    if (int rc = muon_hip_momentum_norm(g_ptrs, m_ptrs, g_dtype, m_dtype, workspace, rows, cols, batch, beta, nesterov,
-                                        write_back_grad, stream))
-        return rc;
-    // The parameter is updated by the epilogue of the last B.X (for rows > cols through a transposing gather out of
-    // LDS): the final X' is then neither written nor read back.  Without an iteration there is no such product.
-    if (ns_steps >= 1) {
-        if (!p_ptrs || !dtype_ok(p_dtype)) return fail(MUON_HIP_EINVAL, "bad pointer table, dtype or steps");
-        const FoldUpdate fold{p_ptrs, p_dtype, rows, cols, scale, lr, weight_decay};
-        return ns_chain(workspace, rows, cols, batch, ns_steps, a, b, c, stream, &fold);
-    }
-    if (int rc = muon_hip_ns_grouped(workspace, rows, cols, batch, ns_steps, a, b, c, stream)) return rc;
-    return muon_hip_apply_update(p_ptrs, p_dtype, workspace, rows, cols, batch, ns_steps, scale, lr, weight_decay,
-                                 stream);
+    const muon_hip_bucket one{p_ptrs, g_ptrs, m_ptrs, rows, cols, batch, scale};
+    return muon_hip_step_multi(&one, 1, p_dtype, g_dtype, m_dtype, workspace, lr, weight_decay, beta, nesterov, ns_steps, a, b, c,
+                               write_back_grad, stream);
 }
 
 long muon_hip_blocked_elems(int rows, int cols) {
@@ -461,7 +546,8 @@ int muon_hip_syrk_bf16(const void* X, void* A, int Mp, int Kp, int batch, int cf
     if (int rc = check_gemm(use.id, Mp, Kp, batch, tile)) return rc;
     if (!X || !A) return fail(MUON_HIP_EINVAL, "null operand");
     if (int rc = check_counters(counters)) return rc;
-    return do_syrk(use, (const bf16_t*)X, (bf16_t*)A, Mp, Kp, batch, (unsigned*)counters, (hipStream_t)stream);
+    const GemmItem it = syrk_item(use.id, (const bf16_t*)X, (bf16_t*)A, Mp, Kp, batch, (unsigned*)counters);
+    return launch_items(MUON_HIP_K_SYRK, "syrk launch", &it, 1, use.adapt, (hipStream_t)stream);
 }
 
 int muon_hip_sympoly_bf16(const void* A, void* B, int Mp, int batch, double b, double c, int cfg, void* counters,
@@ -471,7 +557,8 @@ int muon_hip_sympoly_bf16(const void* A, void* B, int Mp, int batch, double b, d
     if (int rc = check_gemm(use.id, Mp, Mp, batch, tile)) return rc;
     if (!A || !B || A == B) return fail(MUON_HIP_EINVAL, "null or aliased operand");
     if (int rc = check_counters(counters)) return rc;
-    return do_sympoly(use, (const bf16_t*)A, (bf16_t*)B, Mp, batch, b, c, (unsigned*)counters, (hipStream_t)stream);
+    const GemmItem it = sympoly_item(use.id, (const bf16_t*)A, (bf16_t*)B, Mp, batch, b, c, (unsigned*)counters);
+    return launch_items(MUON_HIP_K_SYMPOLY, "sympoly launch", &it, 1, use.adapt, (hipStream_t)stream);
 }
 
 int muon_hip_bx_axpy_bf16(const void* B, const void* X, void* Xout, int Mp, int Kp, int batch, double a, int cfg,
@@ -482,7 +569,8 @@ int muon_hip_bx_axpy_bf16(const void* B, const void* X, void* Xout, int Mp, int 
     if (!B || !X || !Xout) return fail(MUON_HIP_EINVAL, "null operand");
     if (Xout == X) return fail(MUON_HIP_EINVAL, "Xout must not alias X");
     if (int rc = check_counters(counters)) return rc;
-    return do_bx(use, (const bf16_t*)B, (const bf16_t*)X, (bf16_t*)Xout, Mp, Kp, batch, a, (unsigned*)counters, (hipStream_t)stream);
+    const GemmItem it = bx_item(use.id, (const bf16_t*)B, (const bf16_t*)X, (bf16_t*)Xout, Mp, Kp, batch, a, (unsigned*)counters);
+    return launch_items(MUON_HIP_K_BX, "bx launch", &it, 1, use.adapt, (hipStream_t)stream);
 }
 
 int muon_hip_adamw(void* p, const void* g, void* exp_avg, void* exp_avg_sq, int dtype, long n, int step, double lr,

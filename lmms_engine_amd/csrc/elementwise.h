@@ -7,14 +7,31 @@
 #define MUON_MAX_PARTS 65536   // partial sums per matrix, at most (larger matrices put more elements into each)
 
 int momentum_parts(long n);
-hipError_t launch_momentum_norm(const void* const* g_ptrs, const void* const* m_ptrs, int g_dtype, int m_dtype,
-                                bf16_t* U, long strideU, float* partials, int nparts, long n, int batch,
-                                double beta, int nesterov, int write_back, hipStream_t stream);
+
+// The matrices of one shape as the momentum and normalisation kernels see them, and a list of such buckets: one launch works
+// on all of them (workgroup t of a launch belongs to the bucket with start[i] <= t < start[i + 1]).
+struct EwBucket {
+    const void* const* g_ptrs;  // device tables, `batch` entries each
+    const void* const* m_ptrs;
+    bf16_t* U;                  // the blend, dense in the parameter's layout, strideU elements per matrix
+    long strideU;
+    float* partials;            // nparts sums of squares per matrix
+    float* denom;
+    bf16_t* X;                  // the normalised operand, blocked, Mp x Kp
+    long strideX;
+    int rows, cols, Mp, Kp, nparts, batch;
+};
+constexpr int EW_MAX_LIST = 16;
+struct EwList {
+    int n;
+    int start[EW_MAX_LIST + 1];
+    EwBucket b[EW_MAX_LIST];
+};
+hipError_t launch_momentum_norm(EwList& l, int g_dtype, int m_dtype, double beta, int nesterov, int write_back, hipStream_t stream);
 hipError_t launch_cast_norm(const void* G, long strideG, int g_dtype, bf16_t* U, long strideU, float* partials,
                             int nparts, long n, int batch, hipStream_t stream);
-hipError_t launch_normalize(const bf16_t* U, long strideU, const float* partials, int nparts, float* denom, bf16_t* X,
-                            long strideX, int rows, int cols, int Mp, int Kp, int batch, unsigned* clear, int clear_words,
-                            hipStream_t stream);
+// Also clears `clear_words` words at `clear` (the tile counters of the persistent GEMM kernels that follow on the stream).
+hipError_t launch_normalize(EwList& l, unsigned* clear, int clear_words, hipStream_t stream);
 hipError_t launch_apply_update(const void* const* p_ptrs, int p_dtype, const bf16_t* O, long strideO, int cbo,
                                int rows, int cols, int batch, double scale, double lr, double wd,
                                hipStream_t stream);

@@ -90,15 +90,24 @@ __device__ __forceinline__ float momentum_one(float g, float m, const MomentumMa
     return mm.nesterov ? lerp_aten(g, mn, mm.w2, mm.w2m1, mm.small2) : mn;
 }
 
+// The bucket of workgroup `block` of a list.
+__device__ __forceinline__ int list_bucket(const EwList& l, int block) {
+    int i = 0;
+    while (i + 1 < l.n && block >= l.start[i + 1]) ++i;
+    return __builtin_amdgcn_readfirstlane(i);
+}
+
 template <typename GT, typename MT>
 __global__ void __launch_bounds__(256)
-momentum_norm_kernel(const void* const* g_ptrs, const void* const* m_ptrs, bf16_t* U, long strideU,
-                     float* partials, long n, MomentumMath mm, int write_back) {
+momentum_norm_kernel(const EwList l, MomentumMath mm, int write_back) {
     __shared__ float red[4];
-    const int b = blockIdx.y;
-    GT* g = (GT*)g_ptrs[b];
-    MT* m = (MT*)m_ptrs[b];
-    bf16_t* u = U + b * strideU;
+    const int bucket = list_bucket(l, blockIdx.x);
+    const EwBucket& e = l.b[bucket];
+    const int local = blockIdx.x - l.start[bucket], b = local / e.nparts, part = local - b * e.nparts;
+    GT* g = (GT*)e.g_ptrs[b];
+    MT* m = (MT*)e.m_ptrs[b];
+    bf16_t* u = e.U + b * e.strideU;
+    const long n = (long)e.rows * e.cols;
     float ss = 0.f;
     const bool vec = ((((uintptr_t)g) | ((uintptr_t)m)) & 15) == 0;
     const long n8 = vec ? n / 8 : 0;
@@ -109,8 +118,8 @@ momentum_norm_kernel(const void* const* g_ptrs, const void* const* m_ptrs, bf16_
     // times, and 11 % faster than the fourteen trips a single 28672 x 8192 matrix used to take under the old cap of
     // 4096 blocks per matrix (a plain in-place kernel shows the same: 5.98 TB/s at one 16-byte access per thread, 5.52 at
     // four, 4.27 at eight).
-    const long per_block = ((n8 + gridDim.x - 1) / gridDim.x + 511) / 512 * 512;
-    const long lo8 = (long)blockIdx.x * per_block, hi8 = lo8 + per_block < n8 ? lo8 + per_block : n8;
+    const long per_block = ((n8 + e.nparts - 1) / e.nparts + 511) / 512 * 512;
+    const long lo8 = (long)part * per_block, hi8 = lo8 + per_block < n8 ? lo8 + per_block : n8;
     for (long i8 = lo8 + threadIdx.x; i8 < hi8; i8 += 512) {
         const long j8 = i8 + 256;
         const bool two = j8 < hi8;
@@ -146,7 +155,7 @@ momentum_norm_kernel(const void* const* g_ptrs, const void* const* m_ptrs, bf16_
         }
     }
     // scalar tail (or everything when the pointers are not 16-byte aligned)
-    for (long i = n8 * 8 + (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
+    for (long i = n8 * 8 + (long)part * 256 + threadIdx.x; i < n; i += (long)e.nparts * 256) {
         float mo;
         float uu = momentum_one<GT, MT>(Ld<GT>::load(g + i), Ld<MT>::load(m + i), mm, mo);
         Ld<MT>::store(m + i, mo);
@@ -156,7 +165,7 @@ momentum_norm_kernel(const void* const* g_ptrs, const void* const* m_ptrs, bf16_
         ss = fmaf(uu, uu, ss);
     }
     ss = block_sum_256(ss, red);
-    if (threadIdx.x == 0) partials[(long)b * gridDim.x + blockIdx.x] = ss;
+    if (threadIdx.x == 0) e.partials[(long)b * e.nparts + part] = ss;
 }
 
 // Sum of squares of an existing bf16 (or fp32, rounded to bf16 first) matrix: the
@@ -193,16 +202,9 @@ cast_norm_kernel(const GT* G, long strideG, bf16_t* U, long strideU, float* part
     if (threadIdx.x == 0) partials[(long)b * gridDim.x + blockIdx.x] = ss;
 }
 
-// d = bf(bf(sqrt(sum)) + 1e-7) per matrix, from its partial sums in a fixed order.  The first workgroup also clears
-// `clear_words` words at `clear` (the tile counters of the persistent GEMM kernels that follow on the stream).
-__global__ void __launch_bounds__(256) frob_finalize_kernel(const float* partials, int nparts, float* denom,
-                                                            unsigned* clear, int clear_words) {
-    __shared__ float red[4];
-    const int b = blockIdx.x;
-    if (b == 0 && clear)
-        for (int i = threadIdx.x; i < clear_words; i += 256) clear[i] = 0u;
-    // eight partial sums in flight per thread (a matrix of 2^28 elements has 65536 of them), added in a fixed order
-    const float* p = partials + (long)b * nparts;
+// d = bf(bf(sqrt(sum)) + 1e-7) of one matrix from its partial sums, added in a fixed order by the 256 threads of a workgroup
+// (eight in flight per thread: a matrix of 2^28 elements has 65536 of them).
+__device__ __forceinline__ float frob_denom(const float* p, int nparts, float* red) {
     float s = 0.f;
     int i = threadIdx.x;
     for (; i + 7 * 256 < nparts; i += 8 * 256) {
@@ -213,65 +215,53 @@ __global__ void __launch_bounds__(256) frob_finalize_kernel(const float* partial
     }
     for (; i < nparts; i += 256) s += p[i];
     s = block_sum_256(s, red);
-    if (threadIdx.x == 0) {
-        const float nrm = rbf(sqrtf(s));
-        denom[b] = rbf(nrm + 1e-7f);
-    }
+    const float nrm = rbf(sqrtf(s));
+    return rbf(nrm + 1e-7f);
+}
+
+// Matrices of up to this many partial sums (a million elements) have no finalising launch: every workgroup of the
+// normalisation adds the sums itself, one per thread, behind its own load of u.  It costs 1 KB from L2 per workgroup of 4 KB
+// and saves 2 to 5 us per launch sequence; larger matrices would read as much in sums as in data.
+constexpr int kInlineParts = 256;
+
+__global__ void __launch_bounds__(256) frob_finalize_kernel(const EwList l) {
+    __shared__ float red[4];
+    const int bucket = list_bucket(l, blockIdx.x);
+    const EwBucket& e = l.b[bucket];
+    const int b = blockIdx.x - l.start[bucket];
+    const float d = frob_denom(e.partials + (long)b * e.nparts, e.nparts, red);
+    if (threadIdx.x == 0) e.denom[b] = d;
 }
 
 // The bf16 blend u (parameter layout, rows x cols) divided by d, written into the blocked X (M x K, zero padded to
-// Mp x Kp).  Both kernels give a thread as little as one 16-byte load and one 16-byte store: measured on every bucket of
+// Mp x Kp).  A thread has as little as one 16-byte load and one 16-byte store: measured on every bucket of
 // the benchmark sets, tiles of 16 x 128 stream 8 % faster than the 64 x 128 tiles (four accesses each way per thread)
 // they replace (5.7 to 5.8 against 5.3 TB/s), the same way a plain in-place kernel loses 8 % from one to four accesses.
 //
 // A parameter in X's orientation (rows <= cols): one tile of 16 rows x 128 columns per workgroup, straight through
 // registers; in X, 16 rows of a column block lie back to back (1 KB runs).
-__global__ void __launch_bounds__(256)
-normalize_kernel(const bf16_t* U, long strideU, const float* denom, bf16_t* X, long strideX, int rows, int cols, int Kp) {
-    constexpr int TR = 16, TC = 128;
-    const int b = blockIdx.y;
-    const float d = denom[b];
-    const bf16_t* u = U + b * strideU;
-    bf16_t* x = X + b * strideX;
-    const int cbx = Kp / BLK_COLS;
-    const int tiles_c = Kp / TC;
-    const int r = (blockIdx.x / tiles_c) * TR + (threadIdx.x >> 4), c = (blockIdx.x % tiles_c) * TC + (threadIdx.x & 15) * 8;
-    bf16x8 v;
-    if (r < rows && (cols % 8) == 0 && c + 8 <= cols) {
-        v = *(const bf16x8*)(u + (long)r * cols + c);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = (r < rows && c + i < cols) ? u[(long)r * cols + c + i] : (bf16_t)0.f;
-    }
-    bf16x8 o;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = f2bf(__fdiv_rn(bf2f(v[i]), d));
-    *(bf16x8*)(x + blocked_offset(r, c, cbx)) = o;
-}
-
-// A parameter with rows > cols (X = u^T): a tile of TR rows x TC columns of u goes through an LDS transpose and leaves
-// as TC rows of X, TR elements each (TR = 32: the 64-byte rows of one column block, TC of them back to back).
-template <int TR, int TC>
-__global__ void __launch_bounds__(256)
-normalize_t_kernel(const bf16_t* U, long strideU, const float* denom, bf16_t* X, long strideX, int rows, int cols,
-                   int Mp, int Kp) {
-    constexpr int PITCH = TC + 8;
-    constexpr int LCH = TC / 8, LROWS = 256 / LCH, LPASS = TR / LROWS;  // load: chunks per tile row, rows and passes
-    constexpr int SCH = TR / 8, SROWS = 256 / SCH, SPASS = TC / SROWS;  // store: chunks per X row, X rows and passes
-    static_assert(LPASS >= 1 && SPASS >= 1 && TR % 8 == 0 && TC % 8 == 0, "a whole number of passes");
+//
+// A parameter with rows > cols (X = u^T): a tile of 32 rows x 128 columns of u goes through an LDS transpose and leaves
+// as 128 rows of X, 32 elements each (the 64-byte rows of one column block, back to back).  32 x 128 measured best of
+// {32, 64} x {64, 128}: 5.5 to 5.7 TB/s against 5.2 to 5.5 for 64 x 128.
+constexpr int NORM_TR = 16, NORM_T_TR = 32, NORM_TC = 128;
+__global__ void __launch_bounds__(256) normalize_kernel(const EwList l, unsigned* clear, int clear_words) {
+    constexpr int TC = NORM_TC, TR = NORM_T_TR, PITCH = TC + 8;
     __shared__ __align__(16) bf16_t tile[TR][PITCH];
-    const int b = blockIdx.y;
-    const float d = denom[b];
-    const bf16_t* u = U + b * strideU;
-    bf16_t* x = X + b * strideX;
-    const int cbx = Kp / BLK_COLS;
-    const int tiles_c = Mp / TC;  // u's padded image is Kp rows x Mp columns
-    const int r0 = (blockIdx.x / tiles_c) * TR, c0 = (blockIdx.x % tiles_c) * TC;
-    const int tr = threadIdx.x / LCH, tc = (threadIdx.x % LCH) * 8;
-    const bool vec = (cols % 8) == 0;
-#pragma unroll
-    for (int h = 0; h < LPASS; ++h) {
-        const int r = r0 + tr + h * LROWS, c = c0 + tc;
+    __shared__ float red[4];
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < clear_words; i += 256) clear[i] = 0u;
+    const int bucket = list_bucket(l, blockIdx.x);
+    const EwBucket& e = l.b[bucket];
+    const int rows = e.rows, cols = e.cols, cbx = e.Kp / BLK_COLS;
+    const bool vec = (cols % 8) == 0, turn = rows > cols;
+    // u's padded image is Mp x Kp, or Kp x Mp when it is turned; both are whole 128-tiles
+    const int tiles_c = (turn ? e.Mp : e.Kp) / TC, per_mat = turn ? (e.Kp / TR) * tiles_c : (e.Mp / NORM_TR) * tiles_c;
+    const int local = blockIdx.x - l.start[bucket], b = local / per_mat, t = local - b * per_mat;
+    const bf16_t* u = e.U + b * e.strideU;
+    bf16_t* x = e.X + b * e.strideX;
+    const int r0 = (t / tiles_c) * (turn ? TR : NORM_TR), c0 = (t % tiles_c) * TC;
+    auto load8 = [&](int r, int c) {
         bf16x8 v;
         if (r < rows && vec && c + 8 <= cols) {
             v = *(const bf16x8*)(u + (long)r * cols + c);
@@ -279,17 +269,31 @@ normalize_t_kernel(const bf16_t* U, long strideU, const float* denom, bf16_t* X,
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = (r < rows && c + i < cols) ? u[(long)r * cols + c + i] : (bf16_t)0.f;
         }
+        return v;
+    };
+    const int tr = threadIdx.x >> 4, tc = (threadIdx.x & 15) * 8;
+    bf16x8 v[2];
+    v[0] = load8(r0 + tr, c0 + tc);
+    if (turn) v[1] = load8(r0 + tr + 16, c0 + tc);
+    const float d = e.nparts <= kInlineParts ? frob_denom(e.partials + (long)b * e.nparts, e.nparts, red) : e.denom[b];
+    auto divide = [&](const bf16x8& a) {
         bf16x8 o;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = f2bf(__fdiv_rn(bf2f(v[i]), d));
-        *(bf16x8*)(&tile[tr + h * LROWS][tc]) = o;
+        for (int i = 0; i < 8; ++i) o[i] = f2bf(__fdiv_rn(bf2f(a[i]), d));
+        return o;
+    };
+    if (!turn) {
+        *(bf16x8*)(x + blocked_offset(r0 + tr, c0 + tc, cbx)) = divide(v[0]);
+        return;
     }
+    *(bf16x8*)(&tile[tr][tc]) = divide(v[0]);
+    *(bf16x8*)(&tile[tr + 16][tc]) = divide(v[1]);
     __syncthreads();
     // X[c][r]: a thread gathers 8 consecutive r of one column of the tile
-    const int fr = (threadIdx.x % SCH) * 8, fc0 = threadIdx.x / SCH;
+    const int fr = (threadIdx.x & 3) * 8, fc0 = threadIdx.x >> 2;
 #pragma unroll
-    for (int h = 0; h < SPASS; ++h) {
-        const int fc = fc0 + h * SROWS;
+    for (int h = 0; h < 2; ++h) {
+        const int fc = fc0 + h * 64;
         bf16x8 o;
 #pragma unroll
         for (int i = 0; i < 8; ++i) o[i] = tile[fr + i][fc];
@@ -575,6 +579,13 @@ inline int blocks_for(long n, int per_block, int cap) {
     return (int)b;
 }
 
+// Bucket i of a list takes the next `blocks` workgroups; false when a launch cannot have that many.
+inline bool append_blocks(EwList& l, int i, long blocks) {
+    if (l.start[i] + blocks > 0x7fffffffL) return false;
+    l.start[i + 1] = l.start[i] + (int)blocks;
+    return true;
+}
+
 inline void lerp_consts(double weight, float& w, float& wm1, bool& small) {
     w = (float)weight;
     wm1 = w - 1.0f;
@@ -585,24 +596,22 @@ inline void lerp_consts(double weight, float& w, float& wm1, bool& small) {
 
 int momentum_parts(long n) { return blocks_for(n, MUON_PART_ELEMS, MUON_MAX_PARTS); }
 
-hipError_t launch_momentum_norm(const void* const* g_ptrs, const void* const* m_ptrs, int g_dtype, int m_dtype,
-                                bf16_t* U, long strideU, float* partials, int nparts, long n, int batch,
-                                double beta, int nesterov, int write_back, hipStream_t stream) {
+hipError_t launch_momentum_norm(EwList& l, int g_dtype, int m_dtype, double beta, int nesterov, int write_back, hipStream_t stream) {
     MomentumMath mm;
     lerp_consts(1.0 - beta, mm.w1, mm.w1m1, mm.small1);
     lerp_consts(beta, mm.w2, mm.w2m1, mm.small2);
     mm.nesterov = nesterov != 0;
     if (!mm.nesterov) write_back = 0;  // without Nesterov the update is the momentum buffer and the gradient stays as it is
-    dim3 grid(nparts, batch), block(256);
+    l.start[0] = 0;
+    for (int i = 0; i < l.n; ++i)
+        if (!append_blocks(l, i, (long)l.b[i].nparts * l.b[i].batch)) return hipErrorInvalidValue;
+    dim3 grid(l.start[l.n]), block(256);
     if (g_dtype == MUON_HIP_F32 && m_dtype == MUON_HIP_F32)
-        hipLaunchKernelGGL((momentum_norm_kernel<float, float>), grid, block, 0, stream, g_ptrs, m_ptrs, U, strideU,
-                           partials, n, mm, write_back);
+        hipLaunchKernelGGL((momentum_norm_kernel<float, float>), grid, block, 0, stream, l, mm, write_back);
     else if (g_dtype == MUON_HIP_BF16 && m_dtype == MUON_HIP_F32)
-        hipLaunchKernelGGL((momentum_norm_kernel<bf16_t, float>), grid, block, 0, stream, g_ptrs, m_ptrs, U, strideU,
-                           partials, n, mm, write_back);
+        hipLaunchKernelGGL((momentum_norm_kernel<bf16_t, float>), grid, block, 0, stream, l, mm, write_back);
     else if (g_dtype == MUON_HIP_BF16 && m_dtype == MUON_HIP_BF16)
-        hipLaunchKernelGGL((momentum_norm_kernel<bf16_t, bf16_t>), grid, block, 0, stream, g_ptrs, m_ptrs, U, strideU,
-                           partials, n, mm, write_back);
+        hipLaunchKernelGGL((momentum_norm_kernel<bf16_t, bf16_t>), grid, block, 0, stream, l, mm, write_back);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
@@ -622,20 +631,23 @@ hipError_t launch_cast_norm(const void* G, long strideG, int g_dtype, bf16_t* U,
     return hipGetLastError();
 }
 
-hipError_t launch_normalize(const bf16_t* U, long strideU, const float* partials, int nparts, float* denom, bf16_t* X,
-                            long strideX, int rows, int cols, int Mp, int Kp, int batch, unsigned* clear, int clear_words,
-                            hipStream_t stream) {
-    hipLaunchKernelGGL(frob_finalize_kernel, dim3(batch), dim3(256), 0, stream, partials, nparts, denom, clear, clear_words);
-    // u's padded image has whole 128-tiles in both directions (Mp and Kp are multiples of the GEMM tile edge)
-    if (rows > cols) {
-        // 32 x 128 measured best of {32, 64} x {64, 128}: 5.5 to 5.7 TB/s against 5.2 to 5.5 for 64 x 128
-        constexpr int TR = 32, TC = 128;
-        dim3 grid((Kp / TR) * (Mp / TC), batch), block(256);
-        hipLaunchKernelGGL((normalize_t_kernel<TR, TC>), grid, block, 0, stream, U, strideU, denom, X, strideX, rows, cols, Mp, Kp);
-    } else {
-        dim3 grid((Mp / 16) * (Kp / 128), batch), block(256);
-        hipLaunchKernelGGL(normalize_kernel, grid, block, 0, stream, U, strideU, denom, X, strideX, rows, cols, Kp);
+hipError_t launch_normalize(EwList& l, unsigned* clear, int clear_words, hipStream_t stream) {
+    EwList f;  // the matrices with too many partial sums for every workgroup to add
+    f.n = 0;
+    f.start[0] = 0;
+    l.start[0] = 0;
+    for (int i = 0; i < l.n; ++i) {
+        const EwBucket& e = l.b[i];
+        const long per_mat = e.rows > e.cols ? (long)(e.Kp / NORM_T_TR) * (e.Mp / NORM_TC) : (long)(e.Mp / NORM_TR) * (e.Kp / NORM_TC);
+        if (!append_blocks(l, i, per_mat * e.batch)) return hipErrorInvalidValue;
+        if (e.nparts > kInlineParts) {
+            f.b[f.n] = e;
+            f.start[f.n + 1] = f.start[f.n] + e.batch;
+            ++f.n;
+        }
     }
+    if (f.n) hipLaunchKernelGGL(frob_finalize_kernel, dim3(f.start[f.n]), dim3(256), 0, stream, f);
+    hipLaunchKernelGGL(normalize_kernel, dim3(l.start[l.n]), dim3(256), 0, stream, l, clear, clear_words);
     return hipGetLastError();
 }
 

@@ -48,11 +48,22 @@ struct GemmArgs {
     int upd_dtype;                // MUON_HIP_F32 or MUON_HIP_BF16
     int upd_rows, upd_cols;       // the parameter's own (unpadded) shape
     float upd_scale, upd_decay, upd_alpha;  // python-double scale, 1 - lr*wd and -lr, as fp32
-    int big_blocks;         // set by the launcher: workgroups that compute whole 256x256 tiles (split-tail kernel)
     unsigned* ppx;          // tile counters of the persistent kernel (GEMM_PPX_COUNTER_BYTES, zero between launches);
                             // null: the launcher takes the one-tile kernels instead
-    int xcd_shift;          // set by the launcher: log2 of the XCD count of the device
 };
+
+// One launch works on up to GEMM_MAX_LIST products of different sizes, each a batch of its own (matrices of several shapes in
+// one optimizer step): tile t of the launch belongs to the entry with start[i] <= t < start[i + 1].  Passed by value, in the
+// 4 KB that a kernel's arguments may take.
+constexpr int GEMM_MAX_LIST = 16;
+struct GemmList {
+    int n;
+    int xcd_shift;   // log2 of the XCD count of the device
+    int big_blocks;  // split-tail kernel: workgroups that compute whole 256x256 tiles
+    int start[GEMM_MAX_LIST + 1];
+    GemmArgs g[GEMM_MAX_LIST];
+};
+static_assert(sizeof(GemmList) <= 4096, "kernel arguments");
 
 // Tile counters of one persistent launch: a 64-byte line per XCD (tiles handed out beyond the two static rounds) and one
 // for the workgroups that have left.  A launch finds them zero and leaves them zero (the last workgroup out resets them),
@@ -69,6 +80,11 @@ struct MachineShape {
 hipError_t machine_shape(MachineShape& ms);
 
 int gemm_cfg_tile(int cfg);
-// `adapt`: cfg is the choice by shape, and a launch whose tiles would not fill the machine may run on smaller ones (same
-// results bit for bit).  Without it the launch runs cfg as named.
-hipError_t launch_gemm_nt(int cfg, int epi, const GemmArgs& g, bool adapt, hipStream_t stream);
+// The products args[0..n) of one kind, each with the configuration that its shape asks for, in as few launches as their
+// configurations allow.  `adapt`: launches whose tiles would not fill the machine may run on smaller ones (same results bit
+// for bit); without it every product runs its configuration as named.
+struct GemmItem {
+    GemmArgs g;
+    int cfg, epi;
+};
+hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t stream);

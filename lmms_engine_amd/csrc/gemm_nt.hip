@@ -86,9 +86,11 @@ __device__ __forceinline__ TileCoord tile_of(const GemmArgs& g, int logical) {
     return TileCoord{bidx, ti, tj};
 }
 
-template <int EPI>
-__device__ __forceinline__ TileCoord decode_tile(const GemmArgs& g) {
-    return tile_of<EPI>(g, xcd_remap(blockIdx.x, gridDim.x, g.xcd_shift));
+// Tile `logical` of a list: its entry, and its place in that entry.
+__device__ __forceinline__ int list_entry(const GemmList& l, int logical) {
+    int i = 0;
+    while (i + 1 < l.n && logical >= l.start[i + 1]) ++i;
+    return __builtin_amdgcn_readfirstlane(i);
 }
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
@@ -643,7 +645,7 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
 constexpr int ROW_BYTES = 128;
 
 template <int BM, int BN, int WGM, int WGN, int EPI>
-__global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pipe_kernel(const GemmArgs g) {
+__global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pipe_kernel(const GemmList l) {
     constexpr int NW = WGM * WGN;
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
     constexpr int FM = WTM / 16, FN = WTN / 16;
@@ -659,7 +661,9 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pipe_kernel(const GemmA
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    const TileCoord tc = decode_tile<EPI>(g);
+    const int logical = xcd_remap(blockIdx.x, gridDim.x, l.xcd_shift), entry = list_entry(l, logical);
+    const GemmArgs& g = l.g[entry];
+    const TileCoord tc = tile_of<EPI>(g, logical - l.start[entry]);
     constexpr bool QT = epi_is_bx(EPI);  // Q is X itself, rows = reduction index
     const int kb = g.kdim / BLK_COLS;
     const bf16_t* Pb = g.P + tc.bidx * g.strideP + panel_offset(tc.ti * BM, kb);
@@ -1027,9 +1031,10 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
 }
 
 template <int BM, int BN, int WGM, int WGN, int EPI>
-__global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pp_kernel(const GemmArgs g) {
+__global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pp_kernel(const GemmList l) {
     extern __shared__ __align__(16) unsigned char smem[];
-    pp_tile<BM, BN, WGM, WGN, EPI>(g, decode_tile<EPI>(g), smem);
+    const int logical = xcd_remap(blockIdx.x, gridDim.x, l.xcd_shift), entry = list_entry(l, logical);
+    pp_tile<BM, BN, WGM, WGN, EPI>(l.g[entry], tile_of<EPI>(l.g[entry], logical - l.start[entry]), smem);
 }
 
 // ---- kernel 2b: a deep pipeline on 64x64 tiles, for launches that leave compute units idle --------
@@ -1044,7 +1049,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pp_kernel(const GemmArg
 // 25 us for 1024 x 4096).  Stage layout, swizzle and transposing reads are those of kernel 1, the register epilogues those of
 // the persistent kernel, and every element sums its products in the same order: the results are the other kernels' bit for bit.
 template <int EPI>
-__global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmArgs g) {
+__global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmList l) {
     static_assert(EPI == EPI_BX || EPI == EPI_SYRK || EPI == EPI_SYMPOLY, "the epilogues that need no LDS");
     constexpr int BM = 64, BN = 64, WGM = 2, WGN = 2, NW = 4;
     constexpr int WTM = BM / WGM, WTN = BN / WGN, FM = WTM / 16, FN = WTN / 16;
@@ -1056,7 +1061,9 @@ __global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmArgs g) {
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    const TileCoord tc = decode_tile<EPI>(g);
+    const int logical = xcd_remap(blockIdx.x, gridDim.x, l.xcd_shift), entry = list_entry(l, logical);
+    const GemmArgs& g = l.g[entry];
+    const TileCoord tc = tile_of<EPI>(g, logical - l.start[entry]);
     const int kb = g.kdim / BLK_COLS;
     const bf16_t* Pb = uniform_ptr(g.P + tc.bidx * g.strideP + panel_offset(tc.ti * BM, kb));
     const bf16_t* Qb = uniform_ptr(g.Q + tc.bidx * g.strideQ +
@@ -1180,18 +1187,22 @@ __global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmArgs g) {
 }
 
 // The same with a split tail: when the tile count leaves the last round of the compute units mostly empty,
-// the first g.big_blocks workgroups compute 256x256 tiles as above and every remaining tile is cut
+// the first big_blocks workgroups compute 256x256 tiles as above and every remaining tile is cut
 // into four 128x128 tiles, one workgroup each, which fill the CUs that would otherwise idle for a
 // whole tile time.  The lower-left quarter of a diagonal tile of the symmetric kernels is the mirror
 // of the upper-right one and is skipped.
 template <int EPI>
-__global__ void __launch_bounds__(512) gemm_nt_pp_tail_kernel(const GemmArgs g) {
+__global__ void __launch_bounds__(512) gemm_nt_pp_tail_kernel(const GemmList l) {
     extern __shared__ __align__(16) unsigned char smem[];
-    if ((int)blockIdx.x < g.big_blocks) {
-        pp_tile<256, 256, 2, 4, EPI>(g, tile_of<EPI>(g, xcd_remap(blockIdx.x, g.big_blocks, g.xcd_shift)), smem);
+    const bool big = (int)blockIdx.x < l.big_blocks;
+    const int s = blockIdx.x - l.big_blocks, quarter = s & 3;
+    const int logical = big ? xcd_remap(blockIdx.x, l.big_blocks, l.xcd_shift) : l.big_blocks + (s >> 2);
+    const int entry = list_entry(l, logical);
+    const GemmArgs& g = l.g[entry];
+    TileCoord tc = tile_of<EPI>(g, logical - l.start[entry]);
+    if (big) {
+        pp_tile<256, 256, 2, 4, EPI>(g, tc, smem);
     } else {
-        const int s = blockIdx.x - g.big_blocks, quarter = s & 3;
-        TileCoord tc = tile_of<EPI>(g, g.big_blocks + (s >> 2));
         if (!epi_is_bx(EPI) && tc.ti == tc.tj && quarter == 2) return;
         tc.ti = tc.ti * 2 + (quarter >> 1);
         tc.tj = tc.tj * 2 + (quarter & 1);
@@ -1220,7 +1231,7 @@ struct PpxCounters {
 static_assert(sizeof(PpxCounters) == GEMM_PPX_COUNTER_BYTES, "the size the header promises");
 
 template <int EPI>
-__global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g) {
+__global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, const int xcd_shift) {
     static_assert(EPI == EPI_BX || EPI == EPI_SYRK || EPI == EPI_SYMPOLY, "the epilogues that need no LDS");
     constexpr bool QT = EPI == EPI_BX;  // Q is X itself, rows = reduction index
     constexpr int BM = 256, BN = 256, WGM = 2, WGN = 4, NW = 8;
@@ -1239,7 +1250,7 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g) {
     const int wm = wave / WGN, wn = wave % WGN;
     const int kb = g.kdim / BLK_COLS;
     const int total = g.tiles_per_mat * g.batch;
-    const int grid = gridDim.x, xcds = 1 << g.xcd_shift, xcd = blockIdx.x & (xcds - 1);
+    const int grid = gridDim.x, xcds = 1 << xcd_shift, xcd = blockIdx.x & (xcds - 1);
     PpxCounters& ctr = *(PpxCounters*)g.ppx;
 
     auto panel_p = [&](const TileCoord& t) { return uniform_ptr(g.P + t.bidx * g.strideP + panel_offset(t.ti * BM, kb)); };
@@ -1302,7 +1313,7 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g) {
 
     // this workgroup's tiles: the current one, the one after it (virtual ids; >= total means none)
     int pid_cur = blockIdx.x, pid_nxt = blockIdx.x + grid;
-    TileCoord tc = tile_of<EPI>(g, xcd_remap(pid_cur, total, g.xcd_shift));
+    TileCoord tc = tile_of<EPI>(g, xcd_remap(pid_cur, total, xcd_shift));
     const bf16_t* Pb = panel_p(tc);
     const bf16_t* Qb = panel_q(tc);
 
@@ -1317,7 +1328,7 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g) {
     for (;;) {
         const bool has_next = pid_nxt < total;
         // without a next tile the last phases load this tile's first k-tiles again, into stages nobody reads any more
-        const TileCoord ntc = has_next ? tile_of<EPI>(g, xcd_remap(pid_nxt, total, g.xcd_shift)) : tc;
+        const TileCoord ntc = has_next ? tile_of<EPI>(g, xcd_remap(pid_nxt, total, xcd_shift)) : tc;
         const bf16_t* Pn = panel_p(ntc);
         const bf16_t* Qn = panel_q(ntc);
 
@@ -1441,7 +1452,7 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g) {
         // (the answer stays untouched until here: any arithmetic on it would be scheduled next to the atomic, with a
         // wait for it)
         asm volatile("" : "+v"(fetched));
-        if (tid == 0) *(int*)(smem + SLOT_OFF) = has_next ? (((2 * (grid >> g.xcd_shift) + (int)fetched)) << g.xcd_shift) + xcd : total;
+        if (tid == 0) *(int*)(smem + SLOT_OFF) = has_next ? (((2 * (grid >> xcd_shift) + (int)fetched)) << xcd_shift) + xcd : total;
         // The loads of the epilogue are behind those of the next tile's first k-tiles in the queue and have been
         // consumed, so every wave's share of those k-tiles has landed: publish them, and the id.
         __syncthreads();
@@ -1477,50 +1488,86 @@ hipError_t allow_dynamic_lds(const void* kern, int bytes, std::atomic<unsigned l
 }
 
 template <int EPI>
-hipError_t launch_ppx(const GemmArgs& g, int nblocks, int cus, hipStream_t stream) {
+hipError_t launch_ppx(const GemmArgs& g, int nblocks, const MachineShape& ms, hipStream_t stream) {
     constexpr int smem = 4 * (256 + 256) * 64 + 64;
     static std::atomic<unsigned long long> configured{0};  // per instantiation
     if (hipError_t e = allow_dynamic_lds((const void*)gemm_nt_ppx_kernel<EPI>, smem, configured); e != hipSuccess) return e;
-    const int grid = nblocks < cus ? nblocks : cus;  // a whole number of XCDs: the caller launches more tiles than CUs
-    hipLaunchKernelGGL(gemm_nt_ppx_kernel<EPI>, dim3(grid), dim3(512), smem, stream, g);
+    const int grid = nblocks < ms.cus ? nblocks : ms.cus;  // a whole number of XCDs: the caller launches more tiles than CUs
+    hipLaunchKernelGGL(gemm_nt_ppx_kernel<EPI>, dim3(grid), dim3(512), smem, stream, g, ms.xcd_shift);
     return hipGetLastError();
 }
 
 template <int BM, int BN, int WGM, int WGN, int EPI, int FEED>
-hipError_t launch_one(const GemmArgs& g, int nblocks, hipStream_t stream) {
+hipError_t launch_one(const GemmList& l, int nblocks, hipStream_t stream) {
     constexpr int stages = 2 * (BM + BN) * ROW_BYTES;
     constexpr int epi = epi_is_bx(EPI) ? epilogue_nn_bytes<BM, BN>() : epilogue_bytes<BM, BN>();
     constexpr int smem = stages > epi ? stages : epi;
     static std::atomic<unsigned long long> configured{0};  // per instantiation; setting the attribute twice is harmless
-    void (*kern)(const GemmArgs);
+    void (*kern)(const GemmList);
     if constexpr (FEED == 1) kern = gemm_nt_pp_kernel<BM, BN, WGM, WGN, EPI>;
     else kern = gemm_nt_pipe_kernel<BM, BN, WGM, WGN, EPI>;
     if (hipError_t e = allow_dynamic_lds((const void*)kern, smem, configured); e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(nblocks), dim3(WGM * WGN * 64), smem, stream, g);
+    hipLaunchKernelGGL(kern, dim3(nblocks), dim3(WGM * WGN * 64), smem, stream, l);
     return hipGetLastError();
 }
 
 template <int EPI>
-hipError_t launch_deep(const GemmArgs& g, int nblocks, hipStream_t stream) {
+hipError_t launch_deep(const GemmList& l, int nblocks, hipStream_t stream) {
     constexpr int smem = 8 * (64 + 64) * ROW_BYTES;
     static std::atomic<unsigned long long> configured{0};
     if (hipError_t e = allow_dynamic_lds((const void*)gemm_nt_deep_kernel<EPI>, smem, configured); e != hipSuccess) return e;
-    hipLaunchKernelGGL(gemm_nt_deep_kernel<EPI>, dim3(nblocks), dim3(256), smem, stream, g);
+    hipLaunchKernelGGL(gemm_nt_deep_kernel<EPI>, dim3(nblocks), dim3(256), smem, stream, l);
     return hipGetLastError();
 }
 
 template <int EPI>
-hipError_t launch_cfg(int cfg, const GemmArgs& g, int nblocks, hipStream_t stream) {
+hipError_t launch_pp_tail(GemmList& l, int nblocks, int rest, hipStream_t stream) {
+    constexpr int stages = 2 * (256 + 256) * ROW_BYTES;
+    constexpr int epi = epi_is_bx(EPI) ? epilogue_nn_bytes<256, 256>() : epilogue_bytes<256, 256>();
+    constexpr int smem = stages > epi ? stages : epi;  // the 128-tiles need less of both
+    static std::atomic<unsigned long long> configured{0};
+    auto kern = gemm_nt_pp_tail_kernel<EPI>;
+    if (hipError_t e = allow_dynamic_lds((const void*)kern, smem, configured); e != hipSuccess) return e;
+    l.big_blocks = nblocks - rest;
+    hipLaunchKernelGGL(kern, dim3(l.big_blocks + 4 * rest), dim3(512), smem, stream, l);
+    return hipGetLastError();
+}
+
+template <int EPI>
+hipError_t launch_cfg(int cfg, GemmList& l, int nblocks, int cus, hipStream_t stream) {
     switch (cfg) {
-        case GEMM_CFG_128_PIPE: return launch_one<128, 128, 2, 2, EPI, 0>(g, nblocks, stream);
-        case GEMM_CFG_256_PIPE: return launch_one<256, 256, 2, 4, EPI, 0>(g, nblocks, stream);
-        case GEMM_CFG_256_PINGPONG: return launch_one<256, 256, 2, 4, EPI, 1>(g, nblocks, stream);
-        case GEMM_CFG_128_PINGPONG: return launch_one<128, 128, 2, 4, EPI, 1>(g, nblocks, stream);
+        case GEMM_CFG_128_PIPE: return launch_one<128, 128, 2, 2, EPI, 0>(l, nblocks, stream);
+        case GEMM_CFG_256_PIPE: return launch_one<256, 256, 2, 4, EPI, 0>(l, nblocks, stream);
+        case GEMM_CFG_256_PINGPONG: {
+            // Split the tiles of a last round that would fill at most a quarter of the CUs (a 128x128 tile takes about 0.6 of
+            // the time of a 256x256 one, so one round of quarters beats a round of whole tiles).
+            const int rest = nblocks % cus;
+            if (nblocks > cus && rest > 0 && rest <= cus / 4) return launch_pp_tail<EPI>(l, nblocks, rest, stream);
+            return launch_one<256, 256, 2, 4, EPI, 1>(l, nblocks, stream);
+        }
+        case GEMM_CFG_128_PINGPONG: return launch_one<128, 128, 2, 4, EPI, 1>(l, nblocks, stream);
         case GEMM_CFG_64_DEEP:
             if constexpr (EPI == EPI_BX_UPD || EPI == EPI_BX_UPD_T) return hipErrorInvalidValue;  // the launcher takes 128-tiles
-            else return launch_deep<EPI>(g, nblocks, stream);
+            else return launch_deep<EPI>(l, nblocks, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_epi(int epi, int cfg, GemmList& l, int nblocks, int cus, hipStream_t stream) {
+    switch (epi) {
+        case EPI_SYRK: return launch_cfg<EPI_SYRK>(cfg, l, nblocks, cus, stream);
+        case EPI_SYMPOLY: return launch_cfg<EPI_SYMPOLY>(cfg, l, nblocks, cus, stream);
+        case EPI_BX: return launch_cfg<EPI_BX>(cfg, l, nblocks, cus, stream);
+        case EPI_BX_UPD: return launch_cfg<EPI_BX_UPD>(cfg, l, nblocks, cus, stream);
+        case EPI_BX_UPD_T: return launch_cfg<EPI_BX_UPD_T>(cfg, l, nblocks, cus, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+// Workgroups of one launch that cuts C into square tiles of `tile`.
+long count_tiles(const GemmItem& it, int tile) {
+    const long tm = it.g.rows / tile, tn = it.g.cols / tile;
+    return (epi_is_bx(it.epi) ? tm * tn : tm * (tm + 1) / 2) * it.g.batch;
 }
 
 }  // namespace
@@ -1535,19 +1582,6 @@ int gemm_cfg_tile(int cfg) {
         case GEMM_CFG_256_PERSIST: return 256;
         default: return 0;
     }
-}
-
-template <int EPI>
-hipError_t launch_pp_tail(GemmArgs g, int nblocks, int rest, hipStream_t stream) {
-    constexpr int stages = 2 * (256 + 256) * ROW_BYTES;
-    constexpr int epi = epi_is_bx(EPI) ? epilogue_nn_bytes<256, 256>() : epilogue_bytes<256, 256>();
-    constexpr int smem = stages > epi ? stages : epi;  // the 128-tiles need less of both
-    static std::atomic<unsigned long long> configured{0};
-    auto kern = gemm_nt_pp_tail_kernel<EPI>;
-    if (hipError_t e = allow_dynamic_lds((const void*)kern, smem, configured); e != hipSuccess) return e;
-    g.big_blocks = nblocks - rest;
-    hipLaunchKernelGGL(kern, dim3(g.big_blocks + 4 * rest), dim3(512), smem, stream, g);
-    return hipGetLastError();
 }
 
 #ifndef PPX_SYRK_MAXK
@@ -1574,67 +1608,78 @@ hipError_t machine_shape(MachineShape& ms) {
     return hipSuccess;
 }
 
-// Workgroups of one launch that cuts C into square tiles of `tile`.
-long count_tiles(const GemmArgs& g, int epi, int tile) {
-    const long tm = g.rows / tile, tn = g.cols / tile;
-    return (epi_is_bx(epi) ? tm * tn : tm * (tm + 1) / 2) * g.batch;
-}
-
-// Smaller tiles for a launch that would not fill the machine (every configuration sums in the same order, so the result does
-// not depend on the choice).  Measured on one to 48 matrices of 128 to 5120 rows, times per k-tile of 32 columns: a round of
-// 256-tiles (one workgroup per compute unit) 460 ns, of 128-tiles 157 ns alone on a compute unit and 336 ns for two.  So
-// 128-tiles win while they need no more than the two places per compute unit (X.Xt of 2048 x 5632: 84 -> 36 us, of
-// 3072 x 8192 with 300 tiles 119 -> 91) and lose beyond (4096 x 4096 with 528: 68 -> 76); 64-tiles win while each has a
-// compute unit of its own (896 x 4864: 30 -> 18) and lose with two (512 x 1408 x 8, 288 tiles: 11.7 -> 14.0).
-int fill_machine(int cfg, int epi, const GemmArgs& g, int cus) {
-    if (gemm_cfg_tile(cfg) == 256 && count_tiles(g, epi, 128) <= 2 * cus) cfg = GEMM_CFG_128_PINGPONG;
-    if (cfg == GEMM_CFG_128_PINGPONG && !epi_fold_mode(epi) && count_tiles(g, epi, 64) <= cus) cfg = GEMM_CFG_64_DEEP;
-    return cfg;
-}
-
-hipError_t launch_gemm_nt(int cfg, int epi, const GemmArgs& args, bool adapt, hipStream_t stream) {
-    GemmArgs g = args;
+hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t stream) {
+    if (n < 1 || n > GEMM_MAX_LIST) return hipErrorInvalidValue;
     MachineShape ms;
     if (hipError_t e = machine_shape(ms); e != hipSuccess) return e;
-    g.xcd_shift = ms.xcd_shift;
     const int cus = ms.cus;
-    if (adapt) cfg = fill_machine(cfg, epi, g, cus);
-    if (cfg == GEMM_CFG_64_DEEP && epi_fold_mode(epi)) cfg = GEMM_CFG_128_PINGPONG;
-    const int tile = gemm_cfg_tile(cfg);
-    if (tile == 0) return hipErrorInvalidValue;
-    const int nblocks = (int)count_tiles(g, epi, tile);  // the callers have checked that it fits
-    if (nblocks <= 0) return hipSuccess;
-    g.tiles_m = g.rows / tile;
-    g.tiles_n = g.cols / tile;
-    g.tiles_per_mat = nblocks / g.batch;
-    // Ping-pong kernel: split the tiles of a last round that would fill at most a quarter of the CUs (a 128x128
-    // tile takes about 0.6 of the time of a 256x256 one, so one round of quarters beats a round of whole tiles).
-    const int rest = nblocks % cus;
-    if (cfg == GEMM_CFG_256_PERSIST) {
-        // at least 8 k-tiles, more tiles than compute units and a counter buffer; everything else takes the one-tile kernel
-        if (g.kdim >= 256 && nblocks > cus && g.ppx) {
-            if (epi == EPI_BX) return launch_ppx<EPI_BX>(g, nblocks, cus, stream);
-            if (epi == EPI_SYRK && g.kdim <= PPX_SYRK_MAXK) return launch_ppx<EPI_SYRK>(g, nblocks, cus, stream);
-            if (epi == EPI_SYMPOLY && g.kdim <= PPX_SYMPOLY_MAXK) return launch_ppx<EPI_SYMPOLY>(g, nblocks, cus, stream);
-        }
-        cfg = GEMM_CFG_256_PINGPONG;
+    int cfg[GEMM_MAX_LIST];
+    bool done[GEMM_MAX_LIST] = {};
+    long all128 = 0, own128 = 0, all64 = 0;
+    bool fold = false;
+    for (int i = 0; i < n; ++i) {
+        cfg[i] = items[i].cfg;
+        if (gemm_cfg_tile(cfg[i]) == 0) return hipErrorInvalidValue;
+        all128 += count_tiles(items[i], 128);
+        if (gemm_cfg_tile(cfg[i]) == 256) own128 += count_tiles(items[i], 128);
+        all64 += count_tiles(items[i], 64);
+        fold |= epi_fold_mode(items[i].epi) != 0;
     }
-    if (cfg == GEMM_CFG_256_PINGPONG && nblocks > cus && rest > 0 && rest <= cus / 4) {
-        switch (epi) {
-            case EPI_SYRK: return launch_pp_tail<EPI_SYRK>(g, nblocks, rest, stream);
-            case EPI_SYMPOLY: return launch_pp_tail<EPI_SYMPOLY>(g, nblocks, rest, stream);
-            case EPI_BX: return launch_pp_tail<EPI_BX>(g, nblocks, rest, stream);
-            case EPI_BX_UPD: return launch_pp_tail<EPI_BX_UPD>(g, nblocks, rest, stream);
-            case EPI_BX_UPD_T: return launch_pp_tail<EPI_BX_UPD_T>(g, nblocks, rest, stream);
-            default: return hipErrorInvalidValue;
+    // Smaller tiles for launches that would not fill the machine (every configuration sums in the same order, so the result
+    // does not depend on the choice).  Measured on one to 48 matrices of 128 to 5120 rows, times per k-tile of 32 columns: a
+    // round of 256-tiles (one workgroup per compute unit) 460 ns, of 128-tiles 157 ns alone on a compute unit and 336 ns for
+    // two.  So 128-tiles win while they need no more than the two places per compute unit (X.Xt of 2048 x 5632: 84 -> 36 us,
+    // of 3072 x 8192 with 300 tiles 119 -> 91) and lose beyond (4096 x 4096 with 528: 68 -> 76); 64-tiles win while each has
+    // a compute unit of its own (896 x 4864: 30 -> 18) and lose with two (512 x 1408 x 8, 288 tiles: 11.7 -> 14.0).
+    if (adapt) {
+        for (int i = 0; i < n; ++i) {
+            if (gemm_cfg_tile(cfg[i]) == 256 && own128 <= 2 * cus) cfg[i] = GEMM_CFG_128_PINGPONG;
+            if (all128 <= 2 * cus && all64 <= cus && !fold) cfg[i] = GEMM_CFG_64_DEEP;
         }
     }
-    switch (epi) {
-        case EPI_SYRK: return launch_cfg<EPI_SYRK>(cfg, g, nblocks, stream);
-        case EPI_SYMPOLY: return launch_cfg<EPI_SYMPOLY>(cfg, g, nblocks, stream);
-        case EPI_BX: return launch_cfg<EPI_BX>(cfg, g, nblocks, stream);
-        case EPI_BX_UPD: return launch_cfg<EPI_BX_UPD>(cfg, g, nblocks, stream);
-        case EPI_BX_UPD_T: return launch_cfg<EPI_BX_UPD_T>(cfg, g, nblocks, stream);
-        default: return hipErrorInvalidValue;
+    for (int i = 0; i < n; ++i) {
+        const GemmItem& it = items[i];
+        if (cfg[i] == GEMM_CFG_64_DEEP && epi_fold_mode(it.epi)) cfg[i] = GEMM_CFG_128_PINGPONG;
+        if (cfg[i] != GEMM_CFG_256_PERSIST) continue;
+        // The persistent kernel: at least 8 k-tiles, more tiles than compute units and a counter buffer; one product per
+        // launch (its tile counters and registers have no room for more).  Everything else takes the one-tile kernel.
+        const long nblocks = count_tiles(it, 256);
+        cfg[i] = GEMM_CFG_256_PINGPONG;
+        if (it.g.kdim < 256 || nblocks <= cus || !it.g.ppx) continue;
+        GemmArgs g = it.g;
+        g.tiles_m = g.rows / 256;
+        g.tiles_n = g.cols / 256;
+        g.tiles_per_mat = (int)(nblocks / g.batch);
+        hipError_t e = hipErrorNotReady;
+        if (it.epi == EPI_BX) e = launch_ppx<EPI_BX>(g, (int)nblocks, ms, stream);
+        else if (it.epi == EPI_SYRK && g.kdim <= PPX_SYRK_MAXK) e = launch_ppx<EPI_SYRK>(g, (int)nblocks, ms, stream);
+        else if (it.epi == EPI_SYMPOLY && g.kdim <= PPX_SYMPOLY_MAXK) e = launch_ppx<EPI_SYMPOLY>(g, (int)nblocks, ms, stream);
+        if (e == hipErrorNotReady) continue;
+        if (e != hipSuccess) return e;
+        done[i] = true;
     }
+    for (int i = 0; i < n; ++i) {  // one launch per kind and configuration
+        if (done[i]) continue;
+        GemmList l;
+        l.n = 0;
+        l.xcd_shift = ms.xcd_shift;
+        l.big_blocks = 0;
+        l.start[0] = 0;
+        const int tile = gemm_cfg_tile(cfg[i]);
+        for (int k = i; k < n; ++k) {
+            if (done[k] || cfg[k] != cfg[i] || items[k].epi != items[i].epi) continue;
+            const long blocks = count_tiles(items[k], tile);
+            if (l.n > 0 && l.start[l.n] + blocks > 0x7fffffffL) continue;  // goes with a later launch
+            GemmArgs& g = l.g[l.n];
+            g = items[k].g;
+            g.tiles_m = g.rows / tile;
+            g.tiles_n = g.cols / tile;
+            g.tiles_per_mat = (int)(blocks / g.batch);
+            l.start[l.n + 1] = l.start[l.n] + (int)blocks;
+            ++l.n;
+            done[k] = true;
+        }
+        if (hipError_t e = launch_epi(items[i].epi, cfg[i], l, l.start[l.n], cus, stream); e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }

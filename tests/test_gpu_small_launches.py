@@ -41,3 +41,32 @@ def test_the_choice_by_tile_count_does_not_change_the_result(env, M, K, batch):
     ref = _products(env, M, K, batch, env["abi"].CFG_128_PIPE)
     for name, r, got in zip(("syrk", "sympoly", "bx"), ref, _products(env, M, K, batch, env["abi"].CFG_AUTO)):
         assert torch.equal(r, got), name
+
+
+# one call over many shapes: more shapes than a call takes, a bucket that runs the persistent kernel beside small ones, both
+# orientations, ragged edges, the norms of matrices above and below the limit of the inline sums, bf16 momentum
+@pytest.mark.parametrize("name,shapes,dtype,mdtype", [
+    ("17 shapes", [(64 + 8 * i, 100 + 16 * i) for i in range(17)], torch.float32, None),
+    ("persistent beside small", [(512, 1024)] * 36 + [(256, 384)] * 3 + [(300, 100)] * 2 + [(33, 47), (1024, 1100)], torch.bfloat16,
+     torch.float32),
+    ("tall and wide", [(1408, 256), (256, 1408), (1, 9), (200, 200)], torch.bfloat16, None),
+])
+def test_one_call_over_many_shapes_equals_one_call_per_matrix(env, name, shapes, dtype, mdtype):
+    print(f"many shapes: {name}", flush=True)
+    mu, dev = env["mu"], env["dev"]
+    g = torch.Generator().manual_seed(len(shapes))
+    ws = [(0.02 * torch.randn(*s, generator=g)).to(dtype) for s in shapes]
+    gs = [(1e-3 * torch.randn(*s, generator=g)).to(dtype) for s in shapes]
+    hp = dict(lr=0.02, momentum=0.95, nesterov=True, weight_decay=0.01, ns_steps=5, rms_scale=True)
+    pa, pb = ([torch.nn.Parameter(w.clone().to(dev)) for w in ws] for _ in range(2))
+    for p, q, gr in zip(pa, pb, gs):
+        p.grad, q.grad = gr.to(dev), gr.to(dev)
+    opt = mu.Muon([dict(params=list(pa), use_muon=True, **hp)], momentum_dtype=mdtype)
+    opt.step()
+    for q in pb:
+        st = {"momentum_buffer": torch.zeros_like(q, dtype=mdtype or dtype)}
+        mu.SingelDeviceWork(q, st, dict(opt.param_groups[0]), 0).start()
+    torch.cuda.synchronize()
+    for s, p, q, w in zip(shapes, pa, pb, ws):
+        assert torch.equal(p.detach(), q.detach()), s
+        assert not torch.equal(p.detach().cpu(), w), s
