@@ -95,6 +95,7 @@ struct Timed {
 // ---- geometry / workspace ------------------------------------------------------------
 struct Plan {
     int rows, cols, batch, M, K, Mp, Kp, tile, nparts;
+    int Kr;  // K in whole 128-tiles: the extent that the products work on; Kp, the extent of the storage, may be larger
     bool transposed;
     long n, strideU, strideX, strideA;  // elements per matrix: U dense, the others blocked
     size_t offX[2], offA, offB, offParts, offDenom, offPpx, total;
@@ -102,8 +103,8 @@ struct Plan {
 
 inline long round_up(long v, long m) { return (v + m - 1) / m * m; }
 
-// Tile edge for a matrix whose short side is M: 256 when M is a whole number of 256-tiles.
-bool use_tile256(int M) { return M % 256 == 0 && M >= 512; }
+// Tile edge for a matrix whose short side is M: 256 when M, padded to 128-tiles, is a whole number of 256-tiles.
+bool use_tile256(int M) { return M >= 512 - 127 && round_up(M, 128) % 256 == 0; }
 
 // A configuration, and whether the launcher may replace it by one with smaller tiles where a launch has too few (it may not
 // when the caller has named it).
@@ -114,7 +115,8 @@ struct Cfg {
 
 // Configuration per kernel, from a sweep of every variant over the benchmark shapes: the ping-pong kernel
 // everywhere, on 256-tiles where they fill the machine and on 128-tiles (two workgroups per compute unit) for
-// short sides that are no whole number of 256-tiles and for the symmetric products of matrices up to 512 rows.
+// short sides that, in whole 128-tiles, are no whole number of 256-tiles (for a.X + B.X the launcher has tiles of other heights
+// for those) and for the symmetric products of matrices up to 512 rows.
 Cfg pick_cfg(int M, int epi = EPI_BX) {
     const int forced = g_forced_cfg.load(std::memory_order_relaxed);
     if (forced != MUON_HIP_CFG_AUTO) return {forced, false};
@@ -140,13 +142,15 @@ int make_plan(int rows, int cols, int batch, Plan& p) {
     if (p.tile == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration");
     if (p.tile < 128) p.tile = 128;  // the elementwise kernels move whole 128-tiles
     p.Mp = (int)round_up(p.M, p.tile);
-    p.Kp = (int)round_up(p.K, p.tile);
+    p.Kr = (int)round_up(p.K, 128);
+    // the tiles of a.X + B.X may be 256 wide whatever their height
+    p.Kp = (int)round_up(p.K, p.Mp >= 384 ? 256 : 128);
     p.n = (long)rows * cols;
     p.strideU = round_up(p.n, 8);
     p.strideX = blocked_elems(p.Mp, p.Kp);
     p.strideA = blocked_elems(p.Mp, p.Mp);
     p.nparts = momentum_parts(p.n);
-    const long T = p.Mp / p.tile, TN = p.Kp / p.tile;
+    const long T = p.Mp / 128, TN = p.Kp / 128;
     if (T * TN * batch > 0x7fffffffL) return fail(MUON_HIP_ESHAPE, "too many tiles for one launch");
     size_t off = 0;
     auto seg = [&](size_t bytes) {
@@ -192,14 +196,16 @@ int check_gemm(int cfg, int Mp, int Kp, int batch, int& tile) {
 }
 
 // The three products on blocked buffers; matrix b of a batch starts at b * blocked_elems(rows, cols).
-GemmItem syrk_item(int cfg, const bf16_t* X, bf16_t* A, int Mp, int Kp, int batch, unsigned* ppx) {
+// Kr: the columns of X that hold the matrix, in whole 128-tiles; Kp: the columns of its storage.
+GemmItem syrk_item(int cfg, const bf16_t* X, bf16_t* A, int Mp, int Kr, int Kp, int batch, unsigned* ppx) {
     GemmItem it = {};
     GemmArgs& g = it.g;
     it.cfg = cfg;
     it.epi = EPI_SYRK;
     g.P = g.Q = X;
     g.strideP = g.strideQ = blocked_elems(Mp, Kp);
-    g.kdim = Kp;
+    g.cbP = Kp / BLK_COLS;
+    g.kdim = Kr;
     g.rows = g.cols = Mp;
     g.batch = batch;
     g.C = g.Ct = A;
@@ -216,6 +222,7 @@ GemmItem sympoly_item(int cfg, const bf16_t* A, bf16_t* B, int Mp, int batch, do
     it.epi = EPI_SYMPOLY;
     g.P = g.Q = A;
     g.strideP = g.strideQ = blocked_elems(Mp, Mp);
+    g.cbP = Mp / BLK_COLS;
     g.kdim = Mp;
     g.rows = g.cols = Mp;
     g.batch = batch;
@@ -237,7 +244,7 @@ struct UpdateArgs {
     double lr, weight_decay;
 };
 
-GemmItem bx_item(int cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp, int Kp, int batch, double a, unsigned* ppx) {
+GemmItem bx_item(int cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp, int Kr, int Kp, int batch, double a, unsigned* ppx) {
     GemmItem it = {};
     GemmArgs& g = it.g;
     it.cfg = cfg;
@@ -247,9 +254,10 @@ GemmItem bx_item(int cfg, const bf16_t* B, const bf16_t* X, bf16_t* Xout, int Mp
     g.Q = X;
     g.strideQ = blocked_elems(Mp, Kp);
     g.cbQ = Kp / BLK_COLS;
+    g.cbP = Mp / BLK_COLS;
     g.kdim = Mp;
     g.rows = Mp;
-    g.cols = Kp;
+    g.cols = Kr;
     g.batch = batch;
     g.C = Xout;
     g.strideC = blocked_elems(Mp, Kp);
@@ -360,7 +368,7 @@ int ns_chain(const Work& w, int steps, double a, double b, double c, const Updat
             }
         };
         each(EPI_SYRK, [&](const Bucket& k, int cfg) {
-            return syrk_item(cfg, k.at(k.p.offX[cur]), k.at(k.p.offA), k.p.Mp, k.p.Kp, k.p.batch, ppx);
+            return syrk_item(cfg, k.at(k.p.offX[cur]), k.at(k.p.offA), k.p.Mp, k.p.Kr, k.p.Kp, k.p.batch, ppx);
         });
         if (int rc = launch_items(MUON_HIP_K_SYRK, "syrk launch", items, w.n, adapt, s)) return rc;
         each(EPI_SYMPOLY, [&](const Bucket& k, int cfg) {
@@ -369,7 +377,7 @@ int ns_chain(const Work& w, int steps, double a, double b, double c, const Updat
         if (int rc = launch_items(MUON_HIP_K_SYMPOLY, "sympoly launch", items, w.n, adapt, s)) return rc;
         const bool last = upd && it == steps - 1;
         each(EPI_BX, [&](const Bucket& k, int cfg) {
-            GemmItem g = bx_item(cfg, k.at(k.p.offB), k.at(k.p.offX[cur]), k.at(k.p.offX[cur ^ 1]), k.p.Mp, k.p.Kp, k.p.batch, a, ppx);
+            GemmItem g = bx_item(cfg, k.at(k.p.offB), k.at(k.p.offX[cur]), k.at(k.p.offX[cur ^ 1]), k.p.Mp, k.p.Kr, k.p.Kp, k.p.batch, a, ppx);
             if (last) fold_update(g, k.p_ptrs, k.p.rows, k.p.cols, k.scale, *upd);
             return g;
         });
@@ -546,7 +554,7 @@ int muon_hip_syrk_bf16(const void* X, void* A, int Mp, int Kp, int batch, int cf
     if (int rc = check_gemm(use.id, Mp, Kp, batch, tile)) return rc;
     if (!X || !A) return fail(MUON_HIP_EINVAL, "null operand");
     if (int rc = check_counters(counters)) return rc;
-    const GemmItem it = syrk_item(use.id, (const bf16_t*)X, (bf16_t*)A, Mp, Kp, batch, (unsigned*)counters);
+    const GemmItem it = syrk_item(use.id, (const bf16_t*)X, (bf16_t*)A, Mp, Kp, Kp, batch, (unsigned*)counters);
     return launch_items(MUON_HIP_K_SYRK, "syrk launch", &it, 1, use.adapt, (hipStream_t)stream);
 }
 
@@ -569,7 +577,7 @@ int muon_hip_bx_axpy_bf16(const void* B, const void* X, void* Xout, int Mp, int 
     if (!B || !X || !Xout) return fail(MUON_HIP_EINVAL, "null operand");
     if (Xout == X) return fail(MUON_HIP_EINVAL, "Xout must not alias X");
     if (int rc = check_counters(counters)) return rc;
-    const GemmItem it = bx_item(use.id, (const bf16_t*)B, (const bf16_t*)X, (bf16_t*)Xout, Mp, Kp, batch, a, (unsigned*)counters);
+    const GemmItem it = bx_item(use.id, (const bf16_t*)B, (const bf16_t*)X, (bf16_t*)Xout, Mp, Kp, Kp, batch, a, (unsigned*)counters);
     return launch_items(MUON_HIP_K_BX, "bx launch", &it, 1, use.adapt, (hipStream_t)stream);
 }
 

@@ -14,10 +14,11 @@ enum {
     GEMM_CFG_256_PIPE = 1,      // 256x256 tile, 8 waves, the same pipeline
     GEMM_CFG_256_PINGPONG = 2,  // 256x256 tile, 8 waves in two alternating groups, four stages of 32 columns
     GEMM_CFG_128_PINGPONG = 3,  // 128x128 tile, the same eight-wave kernel, two workgroups per compute unit
-    GEMM_CFG_256_PERSIST = 4,   // the ping-pong loop as a persistent kernel (a workgroup per compute unit walks tiles, the next
-                                // tile's first loads land behind an epilogue without LDS): a.X + B.X, and the symmetric
-                                // products with reductions up to 2048; launches of at most one round and the launches that
-                                // carry the parameter update run GEMM_CFG_256_PINGPONG
+    GEMM_CFG_256_PERSIST = 4,   // the ping-pong loop as a persistent kernel (a workgroup per compute unit walks tiles of one or
+                                // several products, the next tile's first loads land behind an epilogue without LDS): a.X + B.X,
+                                // and the symmetric products with reductions up to 2048; launches of at most one round, a few
+                                // rounds with a nearly empty last one, and launches that carry the parameter update run
+                                // GEMM_CFG_256_PINGPONG
     GEMM_CFG_64_DEEP = 5,       // 64x64 tile, 4 waves, eight stages of 64 columns: launches that leave most compute units idle
     GEMM_CFG_COUNT = 6
 };
@@ -26,9 +27,10 @@ struct GemmArgs {
     const bf16_t* P;        // left operand: rows x kdim, blocked
     const bf16_t* Q;        // right operand, blocked: rows x kdim (SYRK, SYMPOLY) or kdim x columns (BX)
     long strideP, strideQ;  // elements between matrices of the batch
+    int cbP;                // column blocks of P (and of Q in the symmetric kernels): its storage may be wider than the reduction
     int cbQ;                // BX: column blocks of Q
     int kdim;               // reduction length, a multiple of 128
-    int rows, cols;         // of C, padded to whole 128-tiles (symmetric kernels: rows == cols)
+    int rows, cols;         // of C, whole 128-tiles (symmetric kernels: rows == cols); larger tiles may overhang into the storage
     int tiles_m, tiles_n;   // set by the launcher: tile grid of one matrix
     int tiles_per_mat;      // set by the launcher: tiles_m*(tiles_m+1)/2 for the symmetric kernels, tiles_m*tiles_n for BX
     int batch;

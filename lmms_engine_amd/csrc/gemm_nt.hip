@@ -467,27 +467,30 @@ __device__ __forceinline__ unsigned pack_bf16x2(float a, float b) {
     const bf16x2 p = {f2bf(a), f2bf(b)};
     return *(const unsigned*)&p;
 }
-template <int BM, int BN, int WGM, int WGN>
-__device__ __forceinline__ void epilogue_nn_reg(const GemmArgs& g, const TileCoord& tc,
-                                                f32x4 (&acc)[BM / WGM / 16][BN / WGN / 16]) {
-    constexpr int WTM = BM / WGM, WTN = BN / WGN;
-    constexpr int FM = WTM / 16, FN = WTN / 16;
-    static_assert(FN % 2 == 0 && BLK_COLS == 32, "a pair of fragments is one column block");
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+//
+// SPLIT: rows of the tile that the first of its two wave rows holds.  The wave rows may differ (variable-height tiles of the
+// persistent kernel).  FMU: fragment rows this wave holds.  IN_BLOCK: the tile lies inside one row block, so that fragment rows
+// are instruction offsets apart; otherwise each is addressed on its own, with scalar arithmetic.
+template <int BN, int WGN, int SPLIT, int FMU, bool IN_BLOCK, int FM, int FN>
+__device__ __forceinline__ void epilogue_nn_reg(const GemmArgs& g, int bidx, int m0, int n0, f32x4 (&acc)[FM][FN]) {
+    constexpr int WTN = BN / WGN;
+    static_assert(FN % 2 == 0 && FN * 16 == WTN && BLK_COLS == 32, "a pair of fragments is one column block");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / WGN, wn = wave % WGN, row = lane >> 4;
-    const int m0 = tc.ti * BM, n0 = tc.tj * BN;
-    // piece (i, t): row m0 + wm*WTM + 16 i + lane%16, columns n0 + wn*WTN + 32 t + 16 (row & 1) + 8 (row >> 1) .. + 7
-    const long lane_off = (long)((n0 >> BLK_SHIFT) + wn * (WTN / 32)) * BLK_ELEMS + (wm * WTM + (lane & 15)) * BLK_COLS +
-                          (row & 1) * 16 + (row >> 1) * 8;
-    const bf16_t* Et = g.Et + tc.bidx * g.strideEt + panel_offset(m0, g.cbEt) + lane_off;
-    bf16_t* C = g.C + tc.bidx * g.strideC + panel_offset(m0, g.cbC) + lane_off;
-    bf16x8 ev[FM][FN / 2];
+    // piece (i, t): row m0 + wm*SPLIT + 16 i + lane%16, columns n0 + wn*WTN + 32 t + 16 (row & 1) + 8 (row >> 1) .. + 7
+    const int lane_off = (lane & 15) * BLK_COLS + (row & 1) * 16 + (row >> 1) * 8;
+    const int m = m0 + wm * SPLIT;
+    auto at = [&](int i, int cb) { return IN_BLOCK ? panel_offset(m, cb) + i * 16 * BLK_COLS : panel_offset(m + i * 16, cb); };
+    const bf16_t* Et = g.Et + bidx * g.strideEt + (long)((n0 >> BLK_SHIFT) + wn * (WTN / 32)) * BLK_ELEMS + lane_off;
+    bf16_t* C = g.C + bidx * g.strideC + (long)((n0 >> BLK_SHIFT) + wn * (WTN / 32)) * BLK_ELEMS + lane_off;
+    bf16x8 ev[FMU][FN / 2];
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FMU; ++i)
 #pragma unroll
-        for (int t = 0; t < FN / 2; ++t) ev[i][t] = *(const bf16x8*)(Et + i * 16 * BLK_COLS + (long)t * BLK_ELEMS);
+        for (int t = 0; t < FN / 2; ++t) ev[i][t] = *(const bf16x8*)(Et + at(i, g.cbEt) + (long)t * BLK_ELEMS);
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < FMU; ++i)
 #pragma unroll
         for (int t = 0; t < FN / 2; ++t) {
             const f32x4 a = acc[i][2 * t], b = acc[i][2 * t + 1];
@@ -498,7 +501,7 @@ __device__ __forceinline__ void epilogue_nn_reg(const GemmArgs& g, const TileCoo
             bf16x8 o;
 #pragma unroll
             for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[i][t][k])) + bf2f(tv[k]));
-            *(bf16x8*)(C + i * 16 * BLK_COLS + (long)t * BLK_ELEMS) = o;
+            *(bf16x8*)(C + at(i, g.cbC) + (long)t * BLK_ELEMS) = o;
         }
 }
 
@@ -665,7 +668,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pipe_kernel(const GemmL
     const GemmArgs& g = l.g[entry];
     const TileCoord tc = tile_of<EPI>(g, logical - l.start[entry]);
     constexpr bool QT = epi_is_bx(EPI);  // Q is X itself, rows = reduction index
-    const int kb = g.kdim / BLK_COLS;
+    const int kb = g.cbP;
     const bf16_t* Pb = g.P + tc.bidx * g.strideP + panel_offset(tc.ti * BM, kb);
     const bf16_t* Qb = g.Q + tc.bidx * g.strideQ +
                        (QT ? (long)(tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel_offset(tc.tj * BN, kb));
@@ -847,7 +850,7 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     const int grp = wave >> 2;
     const int wm = wave / WGN, wn = wave % WGN;
     constexpr bool QT = epi_is_bx(EPI);  // Q is X itself, rows = reduction index
-    const int kb = g.kdim / BLK_COLS;
+    const int kb = g.cbP;
     const bf16_t* Pb = uniform_ptr(g.P + tc.bidx * g.strideP + panel_offset(tc.ti * BM, kb));
     const bf16_t* Qb = uniform_ptr(g.Q + tc.bidx * g.strideQ +
                                    (QT ? (long)(tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel_offset(tc.tj * BN, kb)));
@@ -1017,7 +1020,7 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     if constexpr (EPI == EPI_BX) {
         // no LDS in this epilogue: the loads issued past the end may land while it runs (its own loads are behind
         // them in the queue, so they have landed before the wave ends)
-        epilogue_nn_reg<BM, BN, WGM, WGN>(g, tc, acc);
+        epilogue_nn_reg<BN, WGN, WTM, FM, true>(g, tc.bidx, tc.ti * BM, tc.tj * BN, acc);
         return;
     }
     if constexpr (EPI == EPI_SYMPOLY && BM == 256) {
@@ -1064,7 +1067,7 @@ __global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmList l) {
     const int logical = xcd_remap(blockIdx.x, gridDim.x, l.xcd_shift), entry = list_entry(l, logical);
     const GemmArgs& g = l.g[entry];
     const TileCoord tc = tile_of<EPI>(g, logical - l.start[entry]);
-    const int kb = g.kdim / BLK_COLS;
+    const int kb = g.cbP;
     const bf16_t* Pb = uniform_ptr(g.P + tc.bidx * g.strideP + panel_offset(tc.ti * BM, kb));
     const bf16_t* Qb = uniform_ptr(g.Q + tc.bidx * g.strideQ +
                                    (QT ? (long)(tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel_offset(tc.tj * BN, kb)));
@@ -1182,7 +1185,7 @@ __global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmList l) {
     tail_pair(std::integral_constant<int, 6>{});
     tail_pair(std::integral_constant<int, 4>{});
     tail_pair(std::integral_constant<int, 2>{});
-    if constexpr (QT) epilogue_nn_reg<BM, BN, WGM, WGN>(g, tc, acc);
+    if constexpr (QT) epilogue_nn_reg<BN, WGN, WTM, FM, true>(g, tc.bidx, tc.ti * BM, tc.tj * BN, acc);
     else epilogue_sym_reg<BM, BN, WGM, WGN, EPI>(g, tc, acc);
 }
 
@@ -1230,16 +1233,25 @@ struct PpxCounters {
 };
 static_assert(sizeof(PpxCounters) == GEMM_PPX_COUNTER_BYTES, "the size the header promises");
 
-template <int EPI>
-__global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, const int xcd_shift) {
+// The products of a launch share one walk over the tiles of all of them (12 of 2731 x 1000, 6 of 1000 x 2731 and 12 of
+// 1000 x 1000, 3.8 rounds: 172 us in launches of their own, 123 in one).
+//
+// F0, F1: fragment rows (16 rows each) of the two wave rows of a tile, 8 + 8 for the 256x256 tile.  a.X + B.X also has tiles
+// of 8 + 6 (224 rows) and 6 + 6 (192 rows), for short sides that leave half of a last 256-tile empty (896 = 4 x 224, 1152 =
+// 6 x 192).  Waves w and w + 4 share a SIMD and belong to different wave rows, so every SIMD has the same work.
+// LIST: the launch holds several products (one: its extents stay out of the per-tile state).
+template <int EPI, int F0, int F1, bool LIST>
+__global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmList l) {
     static_assert(EPI == EPI_BX || EPI == EPI_SYRK || EPI == EPI_SYMPOLY, "the epilogues that need no LDS");
     constexpr bool QT = EPI == EPI_BX;  // Q is X itself, rows = reduction index
-    constexpr int BM = 256, BN = 256, WGM = 2, WGN = 4, NW = 8;
+    static_assert(F0 >= F1 && F0 <= 8 && (QT || (F0 == 8 && F1 == 8)), "tile heights");
+    constexpr int BM = 16 * (F0 + F1), BN = 256, WGM = 2, WGN = 4, NW = 8;
     constexpr int BK4 = 32, ROWB = 64;
-    constexpr int WTM = BM / WGM, WTN = BN / WGN;
-    constexpr int FM = WTM / 16, FN = WTN / 16;
-    constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB, STAGE = A_BYTES + B_BYTES;
-    constexpr int LA = BM / 16 / NW, LB = BN / 16 / NW;
+    constexpr int WTM = 16 * F0, WTN = BN / WGN;
+    constexpr int FM = F0, FN = WTN / 16;
+    constexpr bool WHOLE = BM == 256;  // a tile is a row block; otherwise its panels may cross from one to the next
+    constexpr int A_BYTES = 256 * ROWB, B_BYTES = BN * ROWB, STAGE = A_BYTES + B_BYTES;
+    constexpr int LA = 256 / 16 / NW, LB = BN / 16 / NW;
     constexpr int NLD = LA + LB;
     constexpr int SLOT_OFF = 4 * STAGE;  // behind the four stages: where lane 0 leaves the next tile's id for the others
 
@@ -1248,15 +1260,40 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2;
     const int wm = wave / WGN, wn = wave % WGN;
-    const int kb = g.kdim / BLK_COLS;
-    const int total = g.tiles_per_mat * g.batch;
-    const int grid = gridDim.x, xcds = 1 << xcd_shift, xcd = blockIdx.x & (xcds - 1);
-    PpxCounters& ctr = *(PpxCounters*)g.ppx;
+    const int total = l.start[l.n];
+    const int grid = gridDim.x, xcd_shift = l.xcd_shift, xcds = 1 << xcd_shift, xcd = blockIdx.x & (xcds - 1);
+    PpxCounters& ctr = *(PpxCounters*)l.g[0].ppx;
 
-    auto panel_p = [&](const TileCoord& t) { return uniform_ptr(g.P + t.bidx * g.strideP + panel_offset(t.ti * BM, kb)); };
-    auto panel_q = [&](const TileCoord& t) {
-        return uniform_ptr(g.Q + t.bidx * g.strideQ +
-                           (QT ? (long)(t.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel_offset(t.tj * BN, kb)));
+    // A tile: its product, its place there, and where its operands start.  p: this wave's load instructions of P, 16 rows each.
+    // A tile that is a row block needs one pointer; in the others every instruction has its own, and the last waves, past the
+    // end of the tile, fetch rows of it once more into a part of the stage that nobody reads.
+    struct Tile {
+        int entry, nk, cbQ;  // nk: k-tiles, a multiple of 4, at least 8 (the launcher checks)
+        TileCoord tc;
+        const bf16_t* p[WHOLE ? 1 : LA];
+        const bf16_t* q;
+    };
+    auto tile_at = [&](int pid) {
+        Tile t;
+        const int logical = xcd_remap(pid, total, xcd_shift);
+        t.entry = LIST ? list_entry(l, logical) : 0;
+        const GemmArgs& g = l.g[LIST ? t.entry : 0];
+        t.tc = tile_of<EPI>(g, LIST ? logical - l.start[t.entry] : logical);
+        t.nk = g.kdim / BK4;
+        t.cbQ = g.cbQ;
+        const bf16_t* P = g.P + t.tc.bidx * g.strideP;
+        if constexpr (WHOLE) {
+            t.p[0] = uniform_ptr(P + panel_offset(t.tc.ti * BM, g.cbP));
+        } else {
+#pragma unroll
+            for (int n = 0; n < LA; ++n) {
+                const int grp16 = wave * LA + n < BM / 16 ? wave * LA + n : BM / 16 - 1;
+                t.p[n] = uniform_ptr(P + panel_offset(t.tc.ti * BM + grp16 * 16, g.cbP));
+            }
+        }
+        t.q = uniform_ptr(g.Q + t.tc.bidx * g.strideQ +
+                          (QT ? (long)(t.tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel_offset(t.tc.tj * BN, g.cbP)));
+        return t;
     };
 
     // per-lane load offsets and LDS addresses: as in pp_tile
@@ -1264,7 +1301,7 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
     const int dch = ((lane & 3) ^ pp_swizzle((lane >> 4) & 3)) * 8;
     unsigned offa[LA], offb[LB];
 #pragma unroll
-    for (int n = 0; n < LA; ++n) offa[n] = (unsigned)(((wave * 16 * LA + n * 16 + drow) * BLK_COLS + dch) * 2);
+    for (int n = 0; n < LA; ++n) offa[n] = (unsigned)((((WHOLE ? wave * 16 * LA + n * 16 : 0) + drow) * BLK_COLS + dch) * 2);
     const int qch = ((lane & 3) ^ (((drow >> 3) & 1) << 1)) * 8;
 #pragma unroll
     for (int n = 0; n < LB; ++n) {
@@ -1274,7 +1311,6 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
     }
     const int lds_a = wave * 16 * LA * ROWB;
     const int lds_b = A_BYTES + wave * 16 * LB * ROWB;
-    const int nk = g.kdim / BK4;  // a multiple of 4, at least 8 (the launcher checks)
 
     auto dma = [&](const char* base, unsigned voff, unsigned lds_byte) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -1283,15 +1319,14 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
                      : "memory");
     };
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_void_ptr)smem;
-    // k-tile kt of the tile whose panels are (P, Q), into stage kt & 3
-    auto issue_tile = [&](const bf16_t* P, const bf16_t* Q, int kt) {
+    // k-tile kt of tile t, into stage kt & 3
+    auto issue_tile = [&](const Tile& t, int kt) {
         const int k0 = kt * BK4;
         const long koff = (long)(k0 >> BLK_SHIFT) * BLK_ELEMS + (k0 & (BLK_COLS - 1));
-        const char* ba = (const char*)(P + koff);
-        const char* bb = (const char*)(Q + (QT ? (long)(k0 >> 8) * g.cbQ * BLK_ELEMS + (k0 & 255) * BLK_COLS : koff));
+        const char* bb = (const char*)(t.q + (QT ? (long)(k0 >> 8) * (LIST ? t.cbQ : l.g[0].cbQ) * BLK_ELEMS + (k0 & 255) * BLK_COLS : koff));
         const unsigned st = lds_base + (kt & 3) * STAGE;
 #pragma unroll
-        for (int n = 0; n < LA; ++n) dma(ba, offa[n], st + lds_a + n * 16 * ROWB);
+        for (int n = 0; n < LA; ++n) dma((const char*)(t.p[WHOLE ? 0 : n] + koff), offa[n], st + lds_a + n * 16 * ROWB);
 #pragma unroll
         for (int n = 0; n < LB; ++n) dma(bb, offb[n], st + lds_b + n * 16 * ROWB);
     };
@@ -1313,13 +1348,11 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
 
     // this workgroup's tiles: the current one, the one after it (virtual ids; >= total means none)
     int pid_cur = blockIdx.x, pid_nxt = blockIdx.x + grid;
-    TileCoord tc = tile_of<EPI>(g, xcd_remap(pid_cur, total, xcd_shift));
-    const bf16_t* Pb = panel_p(tc);
-    const bf16_t* Qb = panel_q(tc);
+    Tile cur = tile_at(pid_cur);
 
-    issue_tile(Pb, Qb, 0);
-    issue_tile(Pb, Qb, 1);
-    issue_tile(Pb, Qb, 2);
+    issue_tile(cur, 0);
+    issue_tile(cur, 1);
+    issue_tile(cur, 2);
     WAIT_VM(0);  // a tile starts with its k-tiles 0, 1 and 2 in LDS
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -1328,11 +1361,10 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
     for (;;) {
         const bool has_next = pid_nxt < total;
         // without a next tile the last phases load this tile's first k-tiles again, into stages nobody reads any more
-        const TileCoord ntc = has_next ? tile_of<EPI>(g, xcd_remap(pid_nxt, total, xcd_shift)) : tc;
-        const bf16_t* Pn = panel_p(ntc);
-        const bf16_t* Qn = panel_q(ntc);
-
-        const bool diag = !QT && tc.ti == tc.tj;
+        const Tile next = tile_at(has_next ? pid_nxt : pid_cur);
+        const GemmArgs& g = l.g[LIST ? cur.entry : 0];
+        const int nk = LIST ? cur.nk : l.g[0].kdim / BK4;
+        const bool diag = !QT && cur.tc.ti == cur.tc.tj;
         unsigned fetched = 0;
         // One tile, k loop and epilogue, for the waves whose skip mask in a diagonal tile is `mask_c` (pp_tile): a copy of
         // its own per mask, each with its own accumulators from the first MFMA to the last store.
@@ -1366,8 +1398,8 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
                     if (QT) fb[j] = lds_read_qt(rb[SIDX >> 1][j & 1] + (SIDX & 1) * STAGE + (j >> 1) * 2048);
                     else fb[j] = *(const bf16x8*)(rb[SIDX >> 1][0] + (SIDX & 1) * STAGE + j * 16 * ROWB);
                 }
-                if constexpr (NEXT) issue_tile(Pn, Qn, kt + 3 - nk);
-                else issue_tile(Pb, Qb, kt + 3);
+                if constexpr (NEXT) issue_tile(next, kt + 3 - nk);
+                else issue_tile(cur, kt + 3);
                 WAIT_LGKM0();
                 if constexpr (!NOWAIT) WAIT_VM(2 * NLD);  // own loads of k-tile kt+1 have landed
                 __builtin_amdgcn_sched_barrier(0);
@@ -1381,8 +1413,8 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
                     for (int ii = 0; ii < FM; ++ii) {
                         const int i = (j & 1) ? FM - 1 - ii : ii;  // back and forth: consecutive MFMAs share an operand
                         const f32x4 c = FIRST ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[i][j];
-                        if (QT) acc[i][j] = mfma16(fb[j], fa[i], c);
-                        else if (kept(i, j)) acc[i][j] = mfma16(fa[i], fb[j], c);
+                        if (!kept(i, j)) continue;
+                        acc[i][j] = QT ? mfma16(fb[j], fa[i], c) : mfma16(fa[i], fb[j], c);
                     }
                 __builtin_amdgcn_sched_barrier(0);
                 asm volatile("" ::: "memory");
@@ -1417,9 +1449,9 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
             // reduction by the compiler, which then waits for the answer on the spot); the answer is needed at the end.
             if (has_next && tid == 0) fetched = atomicInc(&ctr.next[xcd][0], 0xffffffffu);
             if constexpr (QT) {
-                epilogue_nn_reg<BM, BN, WGM, WGN>(g, tc, acc);
+                epilogue_nn_reg<BN, WGN, WTM, MASK == 0 ? F0 : F1, WHOLE>(g, cur.tc.bidx, cur.tc.ti * BM, cur.tc.tj * BN, acc);
             } else {
-                epilogue_sym_reg<BM, BN, WGM, WGN, EPI, MASK>(g, tc, acc);
+                epilogue_sym_reg<BM, BN, WGM, WGN, EPI, MASK>(g, cur.tc, acc);
                 // What says that this wave's share of the next tile's first k-tiles has landed: B.X and b.A + c.A.A consume
                 // loads that were issued after them (the queue returns in order).  X.Xt loads nothing, and in a diagonal
                 // tile a wave may have nothing to finish at all: there the count is explicit (48 stores went out after the
@@ -1430,7 +1462,10 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
                 asm volatile("" ::: "memory");
             }
         };  // run_tile
-        if (!diag) {
+        if constexpr (F1 < F0) {
+            if (wm == 0) run_tile(std::integral_constant<unsigned, 0>{});
+            else run_tile(std::integral_constant<unsigned, (unsigned)((1ull << (F0 * FN)) - (1ull << (F1 * FN)))>{});
+        } else if (!diag) {
             run_tile(std::integral_constant<unsigned, 0>{});
         } else {
             auto run_if_mine = [&](auto wave_c) {
@@ -1459,9 +1494,7 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmArgs g, cons
         if (!has_next) break;
         pid_cur = pid_nxt;
         pid_nxt = __builtin_amdgcn_readfirstlane(*(const int*)(smem + SLOT_OFF));
-        tc = ntc;
-        Pb = Pn;
-        Qb = Qn;
+        cur = next;
         if (grp) __builtin_amdgcn_s_barrier();  // and enter the next tile a phase apart again
     }
     if (tid == 0) {
@@ -1487,14 +1520,19 @@ hipError_t allow_dynamic_lds(const void* kern, int bytes, std::atomic<unsigned l
     return hipSuccess;
 }
 
-template <int EPI>
-hipError_t launch_ppx(const GemmArgs& g, int nblocks, const MachineShape& ms, hipStream_t stream) {
+template <int EPI, int F0, int F1, bool LIST>
+hipError_t launch_ppx_as(const GemmList& l, int nblocks, int cus, hipStream_t stream) {
     constexpr int smem = 4 * (256 + 256) * 64 + 64;
     static std::atomic<unsigned long long> configured{0};  // per instantiation
-    if (hipError_t e = allow_dynamic_lds((const void*)gemm_nt_ppx_kernel<EPI>, smem, configured); e != hipSuccess) return e;
-    const int grid = nblocks < ms.cus ? nblocks : ms.cus;  // a whole number of XCDs: the caller launches more tiles than CUs
-    hipLaunchKernelGGL(gemm_nt_ppx_kernel<EPI>, dim3(grid), dim3(512), smem, stream, g, ms.xcd_shift);
+    const auto kern = gemm_nt_ppx_kernel<EPI, F0, F1, LIST>;
+    if (hipError_t e = allow_dynamic_lds((const void*)kern, smem, configured); e != hipSuccess) return e;
+    const int grid = nblocks < cus ? nblocks : cus;  // a whole number of XCDs: the caller launches more tiles than CUs
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), smem, stream, l);
     return hipGetLastError();
+}
+template <int EPI, int F0 = 8, int F1 = 8>
+hipError_t launch_ppx(const GemmList& l, int nblocks, int cus, hipStream_t stream) {
+    return l.n > 1 ? launch_ppx_as<EPI, F0, F1, true>(l, nblocks, cus, stream) : launch_ppx_as<EPI, F0, F1, false>(l, nblocks, cus, stream);
 }
 
 template <int BM, int BN, int WGM, int WGN, int EPI, int FEED>
@@ -1564,10 +1602,24 @@ hipError_t launch_epi(int epi, int cfg, GemmList& l, int nblocks, int cus, hipSt
     }
 }
 
-// Workgroups of one launch that cuts C into square tiles of `tile`.
-long count_tiles(const GemmItem& it, int tile) {
-    const long tm = it.g.rows / tile, tn = it.g.cols / tile;
+// Workgroups of one launch that cuts C into square tiles of `tile`, or (a.X + B.X) into tiles of `height` x `tile`.
+long count_tiles(const GemmItem& it, int tile, int height = 0) {
+    const long tm = (it.g.rows + (height ? height : tile) - 1) / (height ? height : tile), tn = (it.g.cols + tile - 1) / tile;
     return (epi_is_bx(it.epi) ? tm * tn : tm * (tm + 1) / 2) * it.g.batch;
+}
+
+// Tile height of the persistent a.X + B.X for a matrix of `rows` rows: the one that covers the fewest, the tallest among equals.
+// The storage of a matrix is whole row blocks of 256; a tile may overhang into it, but not past it.  The overhang reads and
+// writes storage that no other product takes for anything: its values never meet a row of the matrix, because every reduction
+// ends at the matrix's own extent in whole 128-tiles.
+int ppx_height(int rows) {
+    const int storage = (rows + 255) / 256 * 256;
+    int best = 256, cover = storage;
+    for (int h : {224, 192}) {
+        const int c = (rows + h - 1) / h * h;
+        if (c < cover) best = h, cover = c;
+    }
+    return best;
 }
 
 }  // namespace
@@ -1637,27 +1689,64 @@ hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t 
             if (all128 <= 2 * cus && all64 <= cus && !fold) cfg[i] = GEMM_CFG_64_DEEP;
         }
     }
-    for (int i = 0; i < n; ++i) {
-        const GemmItem& it = items[i];
-        if (cfg[i] == GEMM_CFG_64_DEEP && epi_fold_mode(it.epi)) cfg[i] = GEMM_CFG_128_PINGPONG;
-        if (cfg[i] != GEMM_CFG_256_PERSIST) continue;
-        // The persistent kernel: at least 8 k-tiles, more tiles than compute units and a counter buffer; one product per
-        // launch (its tile counters and registers have no room for more).  Everything else takes the one-tile kernel.
-        const long nblocks = count_tiles(it, 256);
-        cfg[i] = GEMM_CFG_256_PINGPONG;
-        if (it.g.kdim < 256 || nblocks <= cus || !it.g.ppx) continue;
-        GemmArgs g = it.g;
-        g.tiles_m = g.rows / 256;
-        g.tiles_n = g.cols / 256;
-        g.tiles_per_mat = (int)(nblocks / g.batch);
-        hipError_t e = hipErrorNotReady;
-        if (it.epi == EPI_BX) e = launch_ppx<EPI_BX>(g, (int)nblocks, ms, stream);
-        else if (it.epi == EPI_SYRK && g.kdim <= PPX_SYRK_MAXK) e = launch_ppx<EPI_SYRK>(g, (int)nblocks, ms, stream);
-        else if (it.epi == EPI_SYMPOLY && g.kdim <= PPX_SYMPOLY_MAXK) e = launch_ppx<EPI_SYMPOLY>(g, (int)nblocks, ms, stream);
-        if (e == hipErrorNotReady) continue;
-        if (e != hipSuccess) return e;
-        done[i] = true;
+    for (int i = 0; i < n; ++i)
+        if (cfg[i] == GEMM_CFG_64_DEEP && epi_fold_mode(items[i].epi)) cfg[i] = GEMM_CFG_128_PINGPONG;
+    // The persistent kernel: more tiles than compute units, and products with at least 8 k-tiles and a counter buffer; one launch
+    // per tile height.  Short sides that are an odd number of 128-tiles take it for a.X + B.X, with tiles of their own height:
+    // the loops of 128-tiles are bound by the LDS (six fragment reads per eight MFMAs against twelve per 32).  Measured, us per
+    // product, 128-tiles | this: 72 of 896 x 4864 713 | 525 (224 rows; 570 with 256), 60 of 640 x 2560 190 | 155 (224), 27 of
+    // 1152 x 4304 362 | 289 (192; 304 with 224), 150 of 384 x 1536 128 | 104 (192); a single row of tiles (200 of 256 x 1024)
+    // 57 | 60.
+    for (int epi : {EPI_SYRK, EPI_SYMPOLY, EPI_BX}) {
+        for (int h : {256, 224, 192}) {
+            GemmList l;
+            l.n = 0;
+            l.xcd_shift = ms.xcd_shift;
+            l.big_blocks = 0;
+            l.start[0] = 0;
+            int from[GEMM_MAX_LIST];
+            long blocks = 0;
+            bool odd = false;
+            for (int i = 0; i < n; ++i) {
+                const GemmArgs& g = items[i].g;
+                if (done[i] || items[i].epi != epi || g.kdim < 256 || !g.ppx) continue;
+                if (cfg[i] == GEMM_CFG_256_PERSIST) {
+                    if (h != 256 || (epi != EPI_BX && g.kdim > (epi == EPI_SYRK ? PPX_SYRK_MAXK : PPX_SYMPOLY_MAXK))) continue;
+                } else {
+                    if (!adapt || cfg[i] != GEMM_CFG_128_PINGPONG || epi != EPI_BX || g.rows < 384 || h != ppx_height(g.rows)) continue;
+                    if (g.cbC * BLK_COLS < (g.cols + 255) / 256 * 256) continue;  // a tile would leave the storage
+                    odd = true;
+                }
+                const long t = count_tiles(items[i], 256, h);
+                if (blocks + t > 0x7fffffffL) continue;
+                GemmArgs& e = l.g[l.n];
+                e = g;
+                e.tiles_m = (g.rows + h - 1) / h;
+                e.tiles_n = (g.cols + 255) / 256;
+                e.tiles_per_mat = (int)(t / g.batch);
+                from[l.n++] = i;
+                blocks += t;
+                l.start[l.n] = (int)blocks;
+            }
+            if (blocks <= cus) continue;
+            // A few rounds with a nearly empty last one: the one-tile kernel cuts that round's tiles into quarters (264 tiles of
+            // 1000 x 2731 43 us against 52, 792 tiles 102 against 107; 1200 tiles of 512 x 1408 111 against 105).  Tiles of odd
+            // heights have no quarters: 128-tiles unless three quarters of the rounds are full (608 tiles of 896 x 4864, 2.4
+            // rounds: 74 us on 128-tiles, 70 here).
+            const long rest = blocks % cus, rounds = (blocks + cus - 1) / cus;
+            if (odd ? 4 * blocks < 3 * rounds * cus : adapt && rest > 0 && rest <= cus / 4 && blocks <= 4L * cus) continue;
+            hipError_t e;
+            if (epi == EPI_SYRK) e = launch_ppx<EPI_SYRK>(l, (int)blocks, cus, stream);
+            else if (epi == EPI_SYMPOLY) e = launch_ppx<EPI_SYMPOLY>(l, (int)blocks, cus, stream);
+            else if (h == 256) e = launch_ppx<EPI_BX>(l, (int)blocks, cus, stream);
+            else if (h == 224) e = launch_ppx<EPI_BX, 8, 6>(l, (int)blocks, cus, stream);
+            else e = launch_ppx<EPI_BX, 6, 6>(l, (int)blocks, cus, stream);
+            if (e != hipSuccess) return e;
+            for (int i = 0; i < l.n; ++i) done[from[i]] = true;
+        }
     }
+    for (int i = 0; i < n; ++i)
+        if (!done[i] && cfg[i] == GEMM_CFG_256_PERSIST) cfg[i] = GEMM_CFG_256_PINGPONG;
     for (int i = 0; i < n; ++i) {  // one launch per kind and configuration
         if (done[i]) continue;
         GemmList l;
@@ -1673,7 +1762,7 @@ hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t 
             GemmArgs& g = l.g[l.n];
             g = items[k].g;
             g.tiles_m = g.rows / tile;
-            g.tiles_n = g.cols / tile;
+            g.tiles_n = (g.cols + tile - 1) / tile;
             g.tiles_per_mat = (int)(blocks / g.batch);
             l.start[l.n + 1] = l.start[l.n] + (int)blocks;
             ++l.n;

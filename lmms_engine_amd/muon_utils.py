@@ -145,7 +145,7 @@ def matmul_transpose_assign(d_in: Tensor, d_out: Tensor) -> None:
     if d_in.dtype != torch.bfloat16:
         raise TypeError(f"the MI355X kernel multiplies bfloat16 operands, got {d_in.dtype}")
     M, K = d_in.shape
-    tile = 256 if (M % 256 == 0 and M >= 512) else 128
+    tile = 256 if (-(-M // 128) % 2 == 0 and M > 384) else 128
     cfg = _abi.CFG_AUTO  # the library picks the kernel for the padded size
     Mp, Kp = -(-M // tile) * tile, -(-K // tile) * tile
     lib = _abi.lib()
@@ -331,9 +331,9 @@ def _pick_chunk(n: int, cap: int, rows: int, cols: int, cus: int = 256) -> int:
     if cap >= n or cap <= 2:
         return max(1, min(n, cap))
     M, K = min(rows, cols), max(rows, cols)
-    if M % 256 or M < 512:
+    if -(-M // 128) % 2 or M <= 384:
         return cap  # 128-tiles: many small tiles, rounds hardly matter
-    T, TN = M // 256, -(-K // 256)
+    T, TN = -(-M // 256), -(-K // 256)
     tri, rect = T * (T + 1) // 2, T * TN
 
     def rounds(t):

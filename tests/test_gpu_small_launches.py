@@ -49,6 +49,8 @@ def test_the_choice_by_tile_count_does_not_change_the_result(env, M, K, batch):
     ("17 shapes", [(64 + 8 * i, 100 + 16 * i) for i in range(17)], torch.float32, None),
     ("persistent beside small", [(512, 1024)] * 36 + [(256, 384)] * 3 + [(300, 100)] * 2 + [(33, 47), (1024, 1100)], torch.bfloat16,
      torch.float32),
+    ("persistent lists of every tile height", [(896, 1000)] * 20 + [(1100, 900)] * 20 + [(650, 640)] * 60 + [(1000, 1024)] * 9 + [(1030, 990)] * 9,
+     torch.float32, None),
     ("tall and wide", [(1408, 256), (256, 1408), (1, 9), (200, 200)], torch.bfloat16, None),
 ])
 def test_one_call_over_many_shapes_equals_one_call_per_matrix(env, name, shapes, dtype, mdtype):
@@ -70,3 +72,33 @@ def test_one_call_over_many_shapes_equals_one_call_per_matrix(env, name, shapes,
     for s, p, q, w in zip(shapes, pa, pb, ws):
         assert torch.equal(p.detach(), q.detach()), s
         assert not torch.equal(p.detach().cpu(), w), s
+
+
+# a.X + B.X on tiles of the matrix's own height: 224, 192 and 256 rows, short sides that end inside the last 128 rows, long
+# sides whose last 256-tile overhangs, more than one row block, and rounds that are filled enough and not
+@pytest.mark.parametrize("rows,cols,batch", [(896, 1000, 40), (900, 640, 90), (384, 520, 100), (1160, 1152, 24), (1290, 1408, 12),
+                                             (1000, 1100, 30), (1000, 1000, 17), (896, 1000, 20), (2700, 1930, 8)])
+def test_odd_short_sides_do_not_change_the_result(env, rows, cols, batch):
+    print(f"odd short side {batch} x {rows} x {cols}", flush=True)
+    lib, abi, mu = env["lib"], env["abi"], env["mu"]
+    g = torch.randn(batch, rows, cols, generator=torch.Generator().manual_seed(rows + cols)).bfloat16().to(env["dev"])
+    got = mu.fast_newtonschulz(g, 5)
+    abi.check(lib.muon_hip_set_gemm_config(abi.CFG_128_PIPE))
+    try:
+        ref = mu.fast_newtonschulz(g, 5)
+    finally:
+        abi.check(lib.muon_hip_set_gemm_config(abi.CFG_AUTO))
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(ref.float()).all())
+    assert torch.equal(got, ref)
+
+
+# the single product where the short side is padded to whole 256-tiles and the long one is not
+@pytest.mark.parametrize("M,K", [(1000, 640), (400, 130), (1930, 1000)])
+def test_matmul_transpose_of_padded_short_sides(env, M, K):
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).bfloat16()
+    got = env["mu"].matmul_transpose(x.to(env["dev"])).cpu().double()
+    ref = x.double() @ x.double().T
+    # one rounding to bf16 and an fp32 sum of K products
+    assert ((got - ref).abs() <= ref.abs() * 2.0**-8 + K * 2.0**-24 * (x.double().abs() @ x.double().abs().T)).all()
+    assert torch.equal(got, got.T)
