@@ -56,7 +56,8 @@ extern "C" {
 #define MUON_HIP_K_GRAD_NORM 8
 #define MUON_HIP_K_CLIP_SCALE 9
 #define MUON_HIP_K_BX_UPDATE 10 /* the a.X + B.X launch that carries the parameter update in its epilogue */
-#define MUON_HIP_K_COUNT 11
+#define MUON_HIP_K_SMALL_CHAIN 11 /* normalisation, iterations and update of matrices with a short side of at most 64 */
+#define MUON_HIP_K_COUNT 12
 
 /* GEMM kernel variants; MUON_HIP_CFG_AUTO picks per kernel, shape and number of tiles.  All feed LDS with direct
  * global->LDS loads (global_load_lds_dwordx4), software pipelined behind the MFMAs. */

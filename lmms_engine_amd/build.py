@@ -13,7 +13,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmuon_hip.so")
-SOURCES = ["gemm_nt.hip", "elementwise.hip", "multi_tensor.hip", "api.hip"]
+SOURCES = ["gemm_nt.hip", "elementwise.hip", "small_chain.hip", "multi_tensor.hip", "api.hip"]
 # Measurement kernels (MFMA-only loops) for the benchmark's operand-power legs: a library of their own, no part of the product.
 PROBE_LIB = os.path.join(HERE, "libmuon_probe.so")
 PROBE_SOURCES = ["probe.hip"]

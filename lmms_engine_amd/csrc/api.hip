@@ -15,6 +15,7 @@
 #include "elementwise.h"
 #include "gemm_nt.h"
 #include "multi_tensor.h"
+#include "small_chain.h"
 
 namespace {
 
@@ -97,6 +98,7 @@ struct Plan {
     int rows, cols, batch, M, K, Mp, Kp, tile, nparts;
     int Kr;  // K in whole 128-tiles: the extent that the products work on; Kp, the extent of the storage, may be larger
     bool transposed;
+    bool small;  // the whole chain runs in one workgroup per matrix (small_chain.hip) instead of as tiled products
     long n, strideU, strideX, strideA;  // elements per matrix: U dense, the others blocked
     size_t offX[2], offA, offB, offParts, offDenom, offPpx, total;
 };
@@ -138,7 +140,9 @@ int make_plan(int rows, int cols, int batch, Plan& p) {
     p.transposed = rows > cols;
     p.M = rows < cols ? rows : cols;
     p.K = rows < cols ? cols : rows;
-    p.tile = gemm_cfg_tile(pick_cfg(p.M).id);
+    const Cfg cfg = pick_cfg(p.M);
+    p.small = cfg.adapt && chain_fits(p.M, p.K);  // a configuration that the caller has named is one of the tiled kernels
+    p.tile = gemm_cfg_tile(cfg.id);
     if (p.tile == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration");
     if (p.tile < 128) p.tile = 128;  // the elementwise kernels move whole 128-tiles
     p.Mp = (int)round_up(p.M, p.tile);
@@ -170,6 +174,10 @@ int make_plan(int rows, int cols, int batch, Plan& p) {
     p.total = off;
     return 0;
 }
+
+// Where `steps` iterations leave X.  The one-workgroup chain leaves it in the first buffer whatever their number: the other
+// holds the blend that workgroups of other matrices may still have to read.
+size_t result_offset(const Plan& p, int steps) { return p.small && steps > 0 ? p.offX[0] : p.offX[steps & 1]; }
 
 inline bf16_t* wsp(void* ws, size_t off) { return (bf16_t*)((char*)ws + off); }
 
@@ -313,7 +321,7 @@ struct Work {
     int n = 0;
     Bucket b[MUON_HIP_MAX_BUCKETS];
 };
-static_assert(MUON_HIP_MAX_BUCKETS <= GEMM_MAX_LIST && MUON_HIP_MAX_BUCKETS <= EW_MAX_LIST, "a launch takes every bucket of a call");
+static_assert(MUON_HIP_MAX_BUCKETS <= GEMM_MAX_LIST && MUON_HIP_MAX_BUCKETS <= EW_MAX_LIST && MUON_HIP_MAX_BUCKETS <= CHAIN_MAX_LIST, "a launch takes every bucket of a call");
 
 int one_bucket(int rows, int cols, int batch, void* workspace, Work& w) {
     w.n = 1;
@@ -351,8 +359,35 @@ int do_normalize(const Work& w, hipStream_t s) {
 }
 
 // Normalise, then `steps` iterations; with `upd` the last B.X applies the parameter update instead of writing X'.
-int ns_chain(const Work& w, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s) {
+int ns_chain(const Work& all, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s) {
     if (steps < 0) return fail(MUON_HIP_EINVAL, "steps must be >= 0");
+    Work w;  // the matrices that go through the tiled products
+    if (steps > 0) {
+        ChainBucket small[MUON_HIP_MAX_BUCKETS];
+        int n = 0;
+        for (int i = 0; i < all.n; ++i) {
+            const Bucket& k = all.b[i];
+            if (!k.p.small) {
+                w.b[w.n++] = k;
+                continue;
+            }
+            small[n++] = ChainBucket{k.at(k.p.offX[1]), k.p.strideU, (const float*)(k.ws + k.p.offParts), k.at(k.p.offX[0]), k.p.strideX,
+                                     upd ? k.p_ptrs : nullptr, (float)k.scale, k.p.Kp / BLK_COLS, k.p.nparts, k.p.rows, k.p.cols, k.p.batch};
+        }
+        if (n) {
+            ChainMath cm{steps, (float)a, (float)b, (float)c, 0, 1.f, 0.f};
+            if (upd) {
+                cm.p_dtype = upd->p_dtype;
+                cm.decay = (float)(1.0 - upd->lr * upd->weight_decay);
+                cm.alpha = (float)(-upd->lr);
+            }
+            Timed t(MUON_HIP_K_SMALL_CHAIN, s);
+            if (hipError_t e = launch_ns_chain(small, n, cm, s); e != hipSuccess) return hip_fail(e, "ns_chain launch");
+        }
+        if (!w.n) return 0;
+    } else {
+        w = all;
+    }
     if (int rc = do_normalize(w, s)) return rc;
     unsigned* ppx = ppx_counters(w);
     GemmItem items[MUON_HIP_MAX_BUCKETS];
@@ -459,7 +494,7 @@ int muon_hip_apply_update(const void* const* p_ptrs, int p_dtype, void* workspac
     if (int rc = check_ws(workspace)) return rc;
     if (!p_ptrs || !dtype_ok(p_dtype) || steps < 0) return fail(MUON_HIP_EINVAL, "bad pointer table, dtype or steps");
     hipStream_t s = (hipStream_t)stream;
-    const bf16_t* O = wsp(workspace, p.offX[steps & 1]);  // X (M x K): the parameter's image, or its transpose when rows > cols
+    const bf16_t* O = wsp(workspace, result_offset(p, steps));  // X (M x K): the parameter's image, or its transpose when rows > cols
     Timed t(MUON_HIP_K_UPDATE, s);
     hipError_t e = launch_apply_update(p_ptrs, p_dtype, O, p.strideX, p.Kp / BLK_COLS, rows, cols, batch, scale, lr,
                                        weight_decay, s);
@@ -472,7 +507,7 @@ int muon_hip_ns_output(void* workspace, int rows, int cols, int batch, int steps
     if (int rc = check_ws(workspace)) return rc;
     if (!out || steps < 0) return fail(MUON_HIP_EINVAL, "bad output pointer or steps");
     hipStream_t s = (hipStream_t)stream;
-    const bf16_t* O = wsp(workspace, p.offX[steps & 1]);
+    const bf16_t* O = wsp(workspace, result_offset(p, steps));
     hipError_t e = launch_unpack((bf16_t*)out, p.n, cols, O, p.strideX, p.Kp / BLK_COLS, rows, cols, p.transposed, batch, s);
     return e == hipSuccess ? 0 : hip_fail(e, "ns_output launch");
 }

@@ -1,0 +1,33 @@
+// The whole Newton-Schulz chain of a matrix with a short side of at most 64 in one workgroup (see small_chain.hip).
+#pragma once
+#include <hip/hip_runtime.h>
+#include "common.h"
+
+// The matrices of one shape, and a list of such buckets as one launch takes them.
+struct ChainBucket {
+    const bf16_t* U;             // the blend, dense in the parameter's layout, strideU elements per matrix
+    long strideU;
+    const float* partials;       // nparts sums of squares per matrix
+    bf16_t* X;                   // work area of strideX elements per matrix; without p_ptrs the result, blocked with cbx column blocks
+    long strideX;
+    const void* const* p_ptrs;   // device table of the parameters to update; null: the result goes to X
+    float scale;
+    int cbx, nparts, rows, cols, batch;
+};
+constexpr int CHAIN_MAX_LIST = 16;
+struct ChainList {
+    int n;
+    int start[CHAIN_MAX_LIST + 1];
+    ChainBucket b[CHAIN_MAX_LIST];
+};
+struct ChainMath {
+    int steps;
+    float a, b, c;
+    int p_dtype;
+    float decay, alpha;  // 1 - lr*wd and -lr
+};
+
+// A short side of M, a long side of K: whether the registers of one workgroup hold the matrix.
+bool chain_fits(int M, int K);
+// Every bucket must fit; steps >= 1.
+hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, hipStream_t stream);

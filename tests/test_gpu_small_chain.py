@@ -1,0 +1,65 @@
+"""Matrices with a short side of at most 64, whose whole Newton-Schulz chain runs in one workgroup each (small_chain.hip): edges
+of the 16-row blocks and 32-column chunks, one chunk per wave and less, the longest long side of every kernel and one past it
+(which the tiled products take), both orientations, ragged sizes."""
+import pytest
+import torch
+
+from tests.helpers import rel_fro
+from tests.test_gpu_parity import NS_TOL, env  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1), (1, 9), (3, 33), (15, 16), (16, 31), (16, 256), (16, 257), (13, 2048), (16, 2049), (16, 4097), (16, 8192), (7, 8185),
+          (17, 17), (32, 96), (24, 1024), (32, 1025), (31, 4095), (33, 64), (64, 64), (64, 512), (48, 513), (50, 1025), (64, 2048),
+          (16, 8193), (32, 4097), (64, 2049), (65, 128)]
+
+
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_small_chain_against_the_oracle(env, rows, cols):
+    """One iteration differs by the order of its fp32 sums, which a bf16 rounding shows as one unit in the last place (2^-8) of
+    the few values next to a rounding point: below 2e-3 in norm, plus 2^-8 where the norm itself, a bf16 value, comes out as its
+    neighbour.  More iterations are held to the bound of every shape."""
+    print(f"small chain {rows}x{cols}", flush=True)
+    mu, O = env["mu"], env["O"]
+    G = torch.randn(2, rows, cols, generator=torch.Generator().manual_seed(rows * 7 + cols)) * 1e-3
+    for g in (G, G.mT.contiguous()):
+        for steps, tol in ((1, 2e-3 + 2**-8), (2, NS_TOL), (5, NS_TOL)):
+            got = mu.fast_newtonschulz(g.to(env["dev"]), steps)
+            assert got.shape == g.shape
+            for i in range(2):
+                assert rel_fro(got[i], O.newton_schulz(g[i], steps)) <= tol, (steps, i)
+
+
+@pytest.mark.parametrize("pdtype", [torch.float32, torch.bfloat16])
+def test_small_chain_in_a_step_equals_the_stages_bitwise(env, pdtype):
+    """One call over all the shapes (several kernels and the tiled products in one launch sequence, parameters updated by the
+    chain) against momentum, iterations and update as calls of their own, for parameters on a 16-byte boundary and off it."""
+    print(f"small chain step {pdtype}", flush=True)
+    lib, abi, mu, O, dev = (env[k] for k in ("lib", "abi", "mu", "O", "dev"))
+    gen = torch.Generator().manual_seed(5)
+    shapes = SHAPES + [(c, r) for r, c in SHAPES if r != c]
+    hp = dict(lr=0.02, momentum=0.95, nesterov=True, weight_decay=0.01, ns_steps=5, rms_scale=True)
+
+    def off(t, by):  # the same values, `by` elements past an aligned address
+        buf = torch.zeros(t.numel() + 8, dtype=t.dtype, device=dev)
+        buf[by:by + t.numel()] = t.reshape(-1).to(dev)
+        return buf[by:by + t.numel()].view(t.shape)
+
+    ws = [(0.02 * torch.randn(*s, generator=gen)).to(pdtype) for s in shapes]
+    gs = [(1e-3 * torch.randn(*s, generator=gen)).to(pdtype) for s in shapes]
+    params = [torch.nn.Parameter(off(w, i % 2)) for i, w in enumerate(ws)]
+    for p, g in zip(params, gs):
+        p.grad = g.to(dev)
+    mu.Muon([dict(params=list(params), use_muon=True, **hp)]).step()
+    a, b, c = O.NS_COEFFS
+    code = abi.dtype_code(pdtype)
+    for s, p, w, g in zip(shapes, params, ws, gs):
+        q, gd, m = w.to(dev), g.to(dev), torch.zeros(s, dtype=pdtype, device=dev)
+        area = torch.empty(abi.workspace_bytes(*s, 1), dtype=torch.uint8, device=dev)
+        table = torch.tensor([t.data_ptr() for t in (q, gd, m)], dtype=torch.int64, device=dev)
+        tp, tg, tm = (table.data_ptr() + 8 * i for i in range(3))
+        abi.check(lib.muon_hip_momentum_norm(tg, tm, code, code, area.data_ptr(), *s, 1, hp["momentum"], 1, 0, 0))
+        abi.check(lib.muon_hip_ns_grouped(area.data_ptr(), *s, 1, 5, a, b, c, 0))
+        abi.check(lib.muon_hip_apply_update(tp, code, area.data_ptr(), *s, 1, 5, mu.scale_factor(*s, True), hp["lr"], hp["weight_decay"], 0))
+        torch.cuda.synchronize()
+        assert torch.equal(p.detach(), q), s
