@@ -29,22 +29,26 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
     norm_type = float(norm_type)
     if norm_type != norm_type:
         raise ValueError("norm_type is NaN")
-    grads = [p.grad for p in parameters if p.grad is not None]
+    grads = [g for g in [p.grad for p in parameters] if g is not None]
     if len(grads) == 0:
         return torch.tensor(0.0)  # what _get_total_norm returns for an empty list
     for g in grads:
         if not g.is_cuda:
             raise _abi.MuonHipError(f"gradients must live on a GPU: this build has no CPU path (got {g.device})")
-    dev = grads[0].device
+    dev, index = grads[0].device, grads[0].get_device()
     groups: "OrderedDict[torch.dtype, list]" = OrderedDict()
     strided = []  # gradients with other than row-major strides are scaled through a row-major copy that is written back
     for g in grads:
-        if g.device != dev:
+        if g.get_device() != index:
             raise NotImplementedError("gradients on several devices")
-        c = g if g.is_contiguous() else g.contiguous()
-        if c is not g:
+        c = g
+        if not g.is_contiguous():
+            c = g.contiguous()
             strided.append((g, c))
-        groups.setdefault(g.dtype, []).append(c)
+        same = groups.get(g.dtype)
+        if same is None:
+            same = groups[g.dtype] = []
+        same.append(c)
     lib = _abi.lib()
     # torch stacks the per-tensor norms of all dtype groups; stacking promotes, so the total has the widest dtype
     out_dtype = torch.float32 if torch.float32 in groups else torch.bfloat16

@@ -8,7 +8,7 @@ muon_hip_grad_norms and muon_hip_clip_scale.
 """
 from __future__ import annotations
 
-import struct
+from array import array
 from typing import Sequence
 
 import torch
@@ -17,35 +17,43 @@ from torch import Tensor
 from . import _abi
 
 
+def _reject(t: Tensor, first: Tensor, numel: int) -> None:
+    if not t.is_cuda:
+        raise _abi.MuonHipError(f"tensors must live on a GPU: this build has no CPU path (got {t.device})")
+    if t.device != first.device or t.dtype != first.dtype or t.numel() != numel:
+        raise ValueError("a tensor list holds tensors of one device and dtype; roles must match in size")
+    raise NotImplementedError("multi-tensor kernels need contiguous tensors")
+
+
 class TensorListTable:
     def __init__(self, roles: Sequence[Sequence[Tensor]], doubles: Sequence[Sequence[float]] = ()):
         n = len(roles[0])
         assert n > 0 and all(len(r) == n for r in roles) and all(len(d) == n for d in doubles)
         first = roles[0][0]
+        index, dtype = first.get_device(), first.dtype  # -1 for a tensor that is not on a GPU
+        numel = [t.numel() for t in roles[0]]
         for r in roles:
-            for t, ref in zip(r, roles[0]):
-                if not t.is_cuda:
-                    raise _abi.MuonHipError(f"tensors must live on a GPU: this build has no CPU path (got {t.device})")
-                if t.device != first.device or t.dtype != first.dtype or t.numel() != ref.numel():
-                    raise ValueError("a tensor list holds tensors of one device and dtype; roles must match in size")
-                if not t.is_contiguous():
-                    raise NotImplementedError("multi-tensor kernels need contiguous tensors")
+            for t, ne in zip(r, numel):
+                if index < 0 or t.get_device() != index or t.dtype != dtype or t.numel() != ne or not t.is_contiguous():
+                    _reject(t, first, ne)
         self.n = n
         self.device = first.device
-        self.dtype = first.dtype
-        numel = [t.numel() for t in roles[0]]
+        self.dtype = dtype
         starts = [0]
+        at = 0
         for ne in numel:
-            starts.append(starts[-1] + (ne + _abi.MULTI_CHUNK - 1) // _abi.MULTI_CHUNK)
-        self.chunks = starts[-1]
-        words = []
+            at += (ne + _abi.MULTI_CHUNK - 1) // _abi.MULTI_CHUNK
+            starts.append(at)
+        self.chunks = at
+        words = array("q")
         for r in roles:
-            words.extend(t.data_ptr() for t in r)
+            words.extend([t.data_ptr() for t in r])
         words.extend(numel)
         words.extend(starts)
         for d in doubles:
-            words.extend(struct.unpack("<q", struct.pack("<d", float(v)))[0] for v in d)
-        host = torch.tensor(words, dtype=torch.int64, pin_memory=True)
+            words.frombytes(array("d", d).tobytes())
+        host = torch.empty(len(words), dtype=torch.int64, pin_memory=True)
+        host.copy_(torch.frombuffer(words, dtype=torch.int64))
         self.table = host.to(self.device, non_blocking=True)
         self._keep = (host, [list(r) for r in roles])  # the tensors stay alive while kernels may read them
         base, k = self.table.data_ptr(), len(roles)

@@ -638,8 +638,9 @@ class Muon(torch.optim.Optimizer):
                 strided = []
                 for i, p in enumerate(group["params"]):
                     assert p.ndim == 2, p.shape
-                    if p.grad is None:
-                        p.grad = torch.zeros_like(p)
+                    g = p.grad
+                    if g is None:
+                        g = p.grad = torch.zeros_like(p)
                     state = self._init_muon_state(p)
                     class_work, prefetch_factor = self._get_work_class(p)
                     if class_work is not SingelDeviceWork:
@@ -649,17 +650,23 @@ class Muon(torch.optim.Optimizer):
                         if len(dq) > prefetch_factor:
                             dq.popleft().finish()
                         continue
-                    _require_cuda(p, "a Muon parameter")
+                    if not p.is_cuda:
+                        _require_cuda(p, "a Muon parameter")
                     # The kernels read row-major tensors.  A parameter, gradient or momentum buffer with other strides
                     # (the reference's torch expressions take any) steps through row-major copies that are written back.
-                    g = p.grad if p.grad.is_contiguous() else p.grad.contiguous()
                     m = state["momentum_buffer"]
-                    pc = p if p.is_contiguous() else p.detach().contiguous()
-                    mc = m if m.is_contiguous() else m.contiguous()
-                    if pc is not p or mc is not m or (g is not p.grad and self.write_back_grad):
-                        strided.append((p, pc, m, mc, g))
-                    key = (p.device, tuple(p.shape), p.dtype, g.dtype, m.dtype)
-                    buckets.setdefault(key, []).append((pc, g, mc))
+                    pc, mc = p, m
+                    if not (g.is_contiguous() and p.is_contiguous() and m.is_contiguous()):
+                        g = g.contiguous()
+                        pc = p if p.is_contiguous() else p.detach().contiguous()
+                        mc = m.contiguous()
+                        if pc is not p or mc is not m or (g is not p.grad and self.write_back_grad):
+                            strided.append((p, pc, m, mc, g))
+                    key = (p.get_device(), p.shape, p.dtype, g.dtype, m.dtype)
+                    same = buckets.get(key)
+                    if same is None:
+                        same = buckets[key] = []
+                    same.append((pc, g, mc))
                 ns_steps, nesterov = group["ns_steps"], group["nesterov"]
                 if self.reference_bug_compat:
                     ns_steps, nesterov = int(bool(group["nesterov"])), bool(group["ns_steps"])

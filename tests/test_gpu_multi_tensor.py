@@ -252,9 +252,9 @@ def test_clip_grad_norm_full_size(env):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("max_norm,moves", [(1e6, False), (99.0, True)])
+@pytest.mark.parametrize("max_norm,moves", [(1.5, False), (0.5, True)])
 def test_clip_within_the_limit_leaves_every_bit(env, dtype, max_norm, moves):
-    """The zero-norm counts elements, so the limit can lie above it with infinities, signed zeros and denormals among them."""
+    """The zero-norm of one gradient is one, so the limit can lie above it with infinities, signed zeros and denormals among them."""
     g = torch.randn(20000, generator=torch.Generator().manual_seed(9)).to(dtype)
     g[:6] = torch.tensor([float("inf"), -float("inf"), 0.0, -0.0, 1e-39, 3e38]).to(dtype)
     p = torch.nn.Parameter(torch.zeros_like(g, device=env["dev"]))
