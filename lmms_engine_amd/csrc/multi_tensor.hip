@@ -11,7 +11,7 @@
 //
 // A tensor list is cut into chunks of MUON_MULTI_CHUNK elements; chunk_start[t] is the index of
 // tensor t's first chunk (chunk_start[n] = number of chunks = grid size).  A block finds its
-// tensor by bisection and handles one chunk: 16-byte vectors when every base pointer of the
+// tensor in its chunk table and handles one chunk or a part of one: 16-byte vectors when every base pointer of the
 // tensor is 16-byte aligned, scalars otherwise and for the last few elements.
 #include "multi_tensor.h"
 #include <type_traits>
@@ -55,15 +55,19 @@ template <> struct Mt<bf16_t> {
 
 __device__ __forceinline__ float rnd_dtype(float x, int dtype) { return dtype == MUON_HIP_BF16 ? rbf(x) : x; }
 
-// tensor index t with chunk_start[t] <= chunk < chunk_start[t + 1]
+// Tensor index t with chunk_start[t] <= chunk < chunk_start[t + 1].  The lanes of a wave look at 64 entries at once: one load
+// for every factor of 64 in n, where a bisection makes one after the other for every factor of two.
 __device__ __forceinline__ int find_tensor(const long* chunk_start, int n, long chunk) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (chunk_start[mid] <= chunk) lo = mid;
-        else hi = mid - 1;
+    const int lane = threadIdx.x & 63;
+    int lo = 0, len = n;  // the answer lies in [lo, lo + len)
+    while (len > 1) {
+        const int step = (len + 63) >> 6, at = lane * step;
+        const bool before = at < len && chunk_start[lo + at] <= chunk;  // true up to some lane, of which the first is one
+        const int skip = (__popcll(__ballot(before)) - 1) * step;
+        lo += skip;
+        len = len - skip < step ? len - skip : step;
     }
-    return lo;
+    return __builtin_amdgcn_readfirstlane(lo);
 }
 
 struct ChunkRange {
@@ -72,9 +76,11 @@ struct ChunkRange {
 };
 
 // The range of workgroup blockIdx.x when every chunk is shared by SUB workgroups (a power of two): chunk blockIdx.x / SUB,
-// piece blockIdx.x % SUB of it.  The kernels that read and write (AdamW, the clip scaling) run four workgroups per chunk, one
-// trip of 4096 elements each: measured, short-lived workgroups stream 3 to 6 % faster there than one workgroup making four
-// trips; the read-only norm kernel is faster with one workgroup per chunk (fewer partial sums).
+// piece blockIdx.x % SUB of it.  The kernels that read and write run several workgroups per chunk, because short-lived ones
+// stream better there: the clip scaling four (3 to 6 % over one workgroup making four trips), AdamW eight, one group of eight
+// elements per thread (1.24 G bf16 elements, 17.4 GB: 3357 us with four, 3225 with eight and the search above), or four for lists
+// so long that eight would pass the 2^32 threads of a launch; the read-only norm kernel is faster with one workgroup per chunk
+// (fewer partial sums).
 template <int SUB = 1>
 __device__ __forceinline__ ChunkRange my_chunk(const long* numel, const long* chunk_start, int n) {
     constexpr long PIECE = MUON_MULTI_CHUNK / SUB;
@@ -86,7 +92,8 @@ __device__ __forceinline__ ChunkRange my_chunk(const long* numel, const long* ch
     r.len = left < 0 ? 0 : left < PIECE ? left : PIECE;
     return r;
 }
-constexpr int RW_SUB = 4;  // workgroups per chunk of the read-and-write kernels
+constexpr int RW_SUB = 4, ADAM_SUB = 8;
+constexpr long MOST_GROUPS = 0xffffffffL / 256;  // workgroups of a launch
 
 __device__ __forceinline__ float lerp_aten(float s, float e, float w, float wm1, bool small) {
     const float d = e - s;
@@ -114,12 +121,12 @@ __device__ __forceinline__ void adam_one(float& p, float g, float& e1, float& e2
     p = fmaf(am.alpha, upd, pd);  // stored through Mt<T>::store*, which rounds
 }
 
-template <typename T>
+template <typename T, int SUB>
 __global__ void __launch_bounds__(256)
 adamw_multi_kernel(const void* const* p_ptrs, const void* const* g_ptrs, const void* const* e1_ptrs,
                    const void* const* e2_ptrs, const long* numel, const long* chunk_start, const double* bias1,
                    const double* bias2, int n, AdamConst am) {
-    const ChunkRange r = my_chunk<RW_SUB>(numel, chunk_start, n);
+    const ChunkRange r = my_chunk<SUB>(numel, chunk_start, n);
     T* p = (T*)p_ptrs[r.t] + r.begin;
     const T* g = (const T*)g_ptrs[r.t] + r.begin;
     T* e1 = (T*)e1_ptrs[r.t] + r.begin;
@@ -302,15 +309,19 @@ hipError_t launch_adamw_multi(const MultiTensorList& l, const void* const* g_ptr
     am.eps = (float)eps;
     am.decay = (float)(1.0 - lr * wd);
     am.alpha = (float)(-lr);
-    dim3 grid((unsigned)(l.chunks * RW_SUB)), block(256);
-    if (dtype == MUON_HIP_F32)
-        hipLaunchKernelGGL((adamw_multi_kernel<float>), grid, block, 0, stream, l.ptrs, g_ptrs, e1_ptrs, e2_ptrs, l.numel,
-                           l.chunk_start, bias1, bias2, l.n, am);
-    else if (dtype == MUON_HIP_BF16)
-        hipLaunchKernelGGL((adamw_multi_kernel<bf16_t>), grid, block, 0, stream, l.ptrs, g_ptrs, e1_ptrs, e2_ptrs, l.numel,
-                           l.chunk_start, bias1, bias2, l.n, am);
-    else
-        return hipErrorInvalidValue;
+    const auto launch = [&](auto t, auto sub_c) {
+        using T = decltype(t);
+        constexpr int SUB = decltype(sub_c)::value;
+        hipLaunchKernelGGL((adamw_multi_kernel<T, SUB>), dim3((unsigned)(l.chunks * SUB)), dim3(256), 0, stream, l.ptrs, g_ptrs, e1_ptrs,
+                           e2_ptrs, l.numel, l.chunk_start, bias1, bias2, l.n, am);
+    };
+    const auto launch_dtype = [&](auto sub_c) {
+        if (dtype == MUON_HIP_F32) launch(float{}, sub_c);
+        else launch(bf16_t{}, sub_c);
+    };
+    if (dtype != MUON_HIP_F32 && dtype != MUON_HIP_BF16) return hipErrorInvalidValue;
+    if (l.chunks <= MOST_GROUPS / ADAM_SUB) launch_dtype(std::integral_constant<int, ADAM_SUB>{});
+    else launch_dtype(std::integral_constant<int, RW_SUB>{});
     return hipGetLastError();
 }
 

@@ -262,3 +262,21 @@ def test_clip_within_the_limit_leaves_every_bit(env, dtype, max_norm, moves):
     env["clip"].clip_grad_norm_([p], max_norm, norm_type=0)
     same = torch.equal(p.grad.cpu().view(torch.uint8), g.view(torch.uint8))
     assert same != moves
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 128, 129, 4096, 4097])
+def test_every_chunk_finds_its_tensor(env, n):
+    """Lists around the widths of the search: 64 entries a round.  Each tensor is scaled by a power of two of its own bits, so a
+    chunk that took another tensor's place would leave its own untouched; empty tensors and tensors of two chunks among them."""
+    print(f"{n} tensors", flush=True)
+    sizes = [(3, 0, 16385, 2048, 2049)[i % 5] if n <= 129 else (3, 0, 9)[i % 3] for i in range(n)]
+    g = [torch.randn(s, generator=torch.Generator().manual_seed(i)) for i, s in enumerate(sizes)]
+    ps = [torch.nn.Parameter(torch.zeros_like(t, device=env["dev"])) for t in g]
+    for p, t in zip(ps, g):
+        p.grad = t.to(env["dev"])
+    total = env["clip"].clip_grad_norm_(ps, 0.25, norm_type=float("inf"))
+    top = max(t.abs().max().item() for t in g if t.numel())
+    assert total.item() == top
+    coef = min(1.0, (torch.tensor(0.25) * (torch.tensor(top) + 1e-6).reciprocal()).item())
+    for p, t in zip(ps, g):
+        assert torch.equal(p.grad.cpu(), t * torch.tensor(coef))
