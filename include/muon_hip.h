@@ -85,7 +85,9 @@ int muon_hip_geometry(int rows, int cols, int* M, int* K, int* Mp, int* Kp, int*
 size_t muon_hip_workspace_bytes(int rows, int cols, int batch);
 
 /* Force one tile configuration for every later call (MUON_HIP_CFG_AUTO restores the default).
- * Affects geometry and workspace size; meant for benchmarking sweeps. */
+ * Affects geometry, workspace size and where the iterations leave their result (short sides of at most 64 run in one workgroup
+ * each under MUON_HIP_CFG_AUTO only), so it stays as it is from muon_hip_workspace_bytes to the call that reads the result; meant
+ * for benchmarking sweeps. */
 int muon_hip_set_gemm_config(int cfg);
 
 /* ---- stage entry points (workspace based) ------------------------------------------- */
