@@ -3,28 +3,34 @@
 //
 // The tiled products of gemm_nt.hip pad a short side to 128 rows and stream X from memory three times an iteration: for 16 rows
 // that is 64 times the multiplications, eight times the bytes and 17 launches.  Here the matrix is read once and the result (or
-// the parameter) written once; what bounds it is the chain of dependent steps inside a workgroup (five iterations of a walk over
-// the wave's chunks and four barriers) times the rounds of workgroups, not memory.  fast_newtonschulz, us, tiles | this:
-//      16 x  512, 1 | 256 | 1024 matrices   97 |  191 |  609    22 |  22 |  42
-//      16 x 5632                           217 | 1414 | 5461    58 |  95 | 416
-//      32 x 4096                           181 | 1087 | 4229    78 | 149 | 586
-//      64 x 2048                           137 |  556 | 2322    87 | 159 | 623
-//    2048 x   64                           139 |  567 | 2363   100 | 182 | 705
+// the parameter) written once; what bounds it is the chain of dependent steps inside a workgroup (five iterations of the sums of
+// X Xt handed from wave to wave, a walk over the wave's chunks, and three barriers) times the rounds of workgroups, not memory.
+// fast_newtonschulz, us, tiles | this:
+//      16 x  512, 1 | 256 | 1024 matrices   97 |  191 |  609    20 |  25 |  50
+//      16 x 5632                           217 | 1414 | 5461    82 | 118 | 511
+//      32 x 4096                           181 | 1087 | 4229    90 | 160 | 635
+//      64 x 2048                           137 |  556 | 2322    97 | 165 | 660
+//    2048 x   64                           139 |  567 | 2363   109 | 191 | 747
 // It wins wherever the registers hold the matrix, so that is the rule (chain_fits); larger ones take the tiled products.
 //
-// Eight waves share the columns of X in chunks of 32.  Lane (i = l%16, q = l/16) of a wave holds X[16 t + i][8q .. 8q+7] of a
-// chunk for every block t of 16 rows: an operand fragment of v_mfma_f32_16x16x32_bf16 as it stands, so
-//   A = X Xt      contracts such fragments with one another; the eight partial sums meet in LDS;
+// Eight waves share the columns of X in chunks of 32, a run of consecutive chunks each.  Lane (i = l%16, q = l/16) of a wave holds
+// X[r][8q .. 8q+7] of a chunk for one row r of every block of 16 rows (chain_row): an operand fragment of
+// v_mfma_f32_16x16x32_bf16 as it stands, so
+//   A = X Xt      contracts such fragments with one another; the sum of a 16x16 block goes from wave to wave through LDS;
 //   B = bA + cAA  is a handful of MFMAs on A in LDS;
 //   X' = aX + BX  contracts rows, for which a chunk is turned by multiplying it with selected columns of the identity (exact:
 //                 one product is the element, the others are zero): the result's four registers are four rows of one column,
-//                 the fragment that B's rows meet, and what comes out lies as X lay.
-// Rounding points are those of the tiled kernels (bf(X Xt); bf(bf(bA) + bf(c bf(AA))); bf(bf(aX) + bf(BX))), sums are fp32.
+//                 and the rows are dealt to the lanes so that two blocks make eight consecutive rows, the fragment that B's rows
+//                 meet; what comes out lies as X lay.
+// Results are those of the tiled kernels bit for bit: the same rounding points (bf(X Xt); bf(bf(bA) + bf(c bf(AA)));
+// bf(bf(aX) + bf(BX))), and every fp32 sum in their order, ascending in 32-deep MFMAs with the reduction index in its natural
+// place.  That order is why a block of X Xt is one chain through the waves and not eight partial sums, which take 3 to 30 % less
+// time (16 x 5632: 57 | 95 | 415, 64 x 2048: 87 | 160 | 621): a bf16 value that rounds the other way moves through the remaining
+// iterations, up to 1e-3 of the result in norm.
 #include "small_chain.h"
+#include <type_traits>
 
 namespace {
-
-typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ f32x4 mfma(const bf16x8& p, const bf16x8& q, const f32x4& c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(p, q, c, 0, 0, 0);
@@ -70,6 +76,28 @@ __device__ __forceinline__ void update8(PT* p, const bf16x8& x, int row, int col
     for (int e = 0; e < 8 && col + e < K; ++e) d[e] = (PT)update_one<PT>((float)d[e], x[e], scale, decay, alpha);
 }
 
+// The row that lane i of 16 holds in block t of 16 rows.  The turned fragment of a block has rows i = 4q .. 4q+3 of it in lane group
+// q; in this order blocks 2p and 2p + 1 put rows 32p + 8q .. 32p + 8q + 7 there, which is where an MFMA has them.  A single block
+// (MT = 1) is in natural order: its fragment is put together by lane swaps instead.
+template <int MT>
+__device__ __forceinline__ int chain_row(int t, int i) {
+    return MT == 1 ? i : 32 * (t >> 1) + 8 * (i >> 2) + 4 * (t & 1) + (i & 3);
+}
+
+// Rows 4q .. 4q+3 of a column in lane group q = l/16 become rows 8q .. 8q+7 in groups 0 and 1, and zeros in 2 and 3.
+__device__ __forceinline__ bf16x8 gather_rows16(const bf16x4& v) {
+    u32x2 r = __builtin_bit_cast(u32x2, v);
+    u32x4 o;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const auto half = __builtin_amdgcn_permlane32_swap(r[e], 0u, false, false);      // groups 0, 1 and 2, 3, each before zeros
+        const auto part = __builtin_amdgcn_permlane16_swap(half[0], half[1], false, false);  // groups 0, 2 and 1, 3
+        o[e] = part[0];
+        o[2 + e] = part[1];
+    }
+    return __builtin_bit_cast(bf16x8, o);
+}
+
 constexpr int CHAIN_WAVES = 8;
 constexpr int CHAIN_FRAGS = 32;  // fragments of X a lane can hold: 128 of the 256 registers of a wave
 
@@ -79,8 +107,8 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
     constexpr int NP = (MT + 1) / 2;         // 32-deep reductions over the rows
     constexpr int PITCH = 32 * NP + 8;       // of A and B in LDS; with MT = 1 columns 16 to 31 stay zero
     constexpr int NF = MT * (MT + 1) / 2;    // 16 x 16 blocks of A on or above the diagonal
-    constexpr int HALF = CHAIN_WAVES / 2;
-    __shared__ __align__(16) f32x4 part[HALF][NF][64];
+    constexpr int LEG = MT == 4 ? 2 : 1, NLEG = NF / LEG;  // blocks that a wave adds its chunks to at a time
+    __shared__ __align__(16) f32x4 sum[NF][64];
     __shared__ __align__(16) bf16_t As[MT * 16][PITCH], Bs[MT * 16][PITCH];
     __shared__ float red[4];
 
@@ -117,7 +145,7 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
     for (int j = 0; j < per; ++j) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            const int row = t * 16 + i, col = col0 + j * 32;
+            const int row = chain_row<MT>(t, i), col = col0 + j * 32;
             bf16x8 v;
             if (vec && row < M && col < K) {
                 v = *(const bf16x8*)(u + (long)row * K + col);
@@ -139,45 +167,52 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         for (int h = 0; h < 2; ++h) unit[h][e] = (bf16_t)((q == i >> 2 && e == 4 * h + (i & 3)) ? 1.f : 0.f);
     }
     bf16x8 x[NCH][MT];
-    f32x4 acc[NF];
-#pragma unroll
-    for (int f = 0; f < NF; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto gram = [&](const bf16x8 (&xc)[MT]) {
-        int f = 0;
-#pragma unroll
-        for (int ti = 0; ti < MT; ++ti)
-#pragma unroll
-            for (int tj = ti; tj < MT; ++tj, ++f) acc[f] = mfma(xc[ti], xc[tj], acc[f]);
-    };
 #pragma unroll
     for (int j = 0; j < NCH; ++j)
 #pragma unroll
         for (int t = 0; t < MT; ++t) x[j][t] = j < per ? mine[(j * MT + t) * 64] : zero8;
+    // The sum of leg `leg` (LEG blocks of A) over this wave's chunks, on top of the waves' before it.
+    auto add_leg = [&](auto leg_c) {
+        constexpr int F0 = decltype(leg_c)::value * LEG;
+        f32x4 acc[LEG];
 #pragma unroll
-    for (int j = 0; j < NCH; ++j) gram(x[j]);
+        for (int f = 0; f < LEG; ++f) acc[f] = wave == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum[F0 + f][lane];
+#pragma unroll
+        for (int j = 0; j < NCH; ++j)
+            if (j < per) {
+                int f = 0;
+#pragma unroll
+                for (int ti = 0; ti < MT; ++ti)
+#pragma unroll
+                    for (int tj = ti; tj < MT; ++tj, ++f)
+                        if (f >= F0 && f < F0 + LEG) acc[f - F0] = mfma(x[j][ti], x[j][tj], acc[f - F0]);
+            }
+#pragma unroll
+        for (int f = 0; f < LEG; ++f) sum[F0 + f][lane] = acc[f];
+    };
 
     for (int it = 0; it < cm.steps; ++it) {
-        // the eight partial sums, in a fixed order
-        if (wave >= HALF) {
-#pragma unroll
-            for (int f = 0; f < NF; ++f) part[wave - HALF][f][lane] = acc[f];
+        // A wave starts a leg when the wave before it has left it, so the legs follow one another through the waves.
+        for (int slot = 0; slot < NLEG + CHAIN_WAVES - 1; ++slot) {
+            const int leg = slot - wave;
+            if (leg == 0) add_leg(std::integral_constant<int, 0>{});
+            if constexpr (NLEG > 1) if (leg == 1) add_leg(std::integral_constant<int, 1>{});
+            if constexpr (NLEG > 2) if (leg == 2) add_leg(std::integral_constant<int, 2>{});
+            if constexpr (NLEG > 3) if (leg == 3) add_leg(std::integral_constant<int, 3>{});
+            if constexpr (NLEG > 4) if (leg == 4) add_leg(std::integral_constant<int, 4>{});
+            static_assert(NLEG <= 5 && NLEG * LEG == NF, "every leg has its branch");
+            __syncthreads();
         }
-        __syncthreads();
-        if (wave < HALF) {
-#pragma unroll
-            for (int f = 0; f < NF; ++f) part[wave][f][lane] = part[wave][f][lane] + acc[f];
-        }
-        __syncthreads();
         for (int t = tid; t < NF * 64; t += 64 * CHAIN_WAVES) {
             const int ln = t & 63;
             int f = t >> 6, ti = 0;
-            const f32x4 sum = (part[0][f][ln] + part[1][f][ln]) + (part[2][f][ln] + part[3][f][ln]);
+            const f32x4 v = sum[f][ln];
             while (f >= MT - ti) f -= MT - ti++;
-            const int tj = ti + f, r = ti * 16 + (ln >> 4) * 4, c = tj * 16 + (ln & 15);
-            bf16x4_t o;
+            const int tj = ti + f, r = chain_row<MT>(ti, (ln >> 4) * 4), c = chain_row<MT>(tj, ln & 15);
+            bf16x4 o;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) o[e] = f2bf(sum[e]);
-            *(bf16x4_t*)&As[c][r] = o;  // A is symmetric: the mirrored block in one piece, this one element by element
+            for (int e = 0; e < 4; ++e) o[e] = f2bf(v[e]);
+            *(bf16x4*)&As[c][r] = o;  // A is symmetric: the mirrored block in one piece, this one element by element
             if (ti != tj) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) As[r + e][c] = o[e];
@@ -190,36 +225,31 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
 #pragma unroll
             for (int p = 0; p < NP; ++p)
                 aa = mfma(*(const bf16x8*)&As[ti * 16 + i][p * 32 + 8 * q], *(const bf16x8*)&As[tj * 16 + i][p * 32 + 8 * q], aa);
-            const bf16x4_t av = *(const bf16x4_t*)&As[tj * 16 + i][ti * 16 + 4 * q];
-            bf16x4_t o;
+            const bf16x4 av = *(const bf16x4*)&As[tj * 16 + i][ti * 16 + 4 * q];
+            bf16x4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = f2bf(rbf(cm.b * bf2f(av[e])) + rbf(cm.c * rbf(aa[e])));
-            *(bf16x4_t*)&Bs[tj * 16 + i][ti * 16 + 4 * q] = o;
+            *(bf16x4*)&Bs[tj * 16 + i][ti * 16 + 4 * q] = o;
         }
         __syncthreads();
-        bf16x8 bfr[MT][NP];  // B's rows, in the order that the turned chunks have their rows in
+        bf16x8 bfr[MT][NP];  // B's rows, in the order of X's
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                const bf16x4_t lo = *(const bf16x4_t*)&Bs[t * 16 + i][p * 32 + 4 * q], hi = *(const bf16x4_t*)&Bs[t * 16 + i][p * 32 + 16 + 4 * q];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    bfr[t][p][e] = lo[e];
-                    bfr[t][p][4 + e] = hi[e];
-                }
-            }
-#pragma unroll
-        for (int f = 0; f < NF; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int p = 0; p < NP; ++p) bfr[t][p] = *(const bf16x8*)&Bs[chain_row<MT>(t, i)][p * 32 + 8 * q];
         auto next_chunk = [&](bf16x8 (&xc)[MT]) {
             bf16x8 xt[2][NP];
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int t = 0; t < 2 * NP; ++t) {
-                    const f32x4 v = t < MT ? mfma(xc[t < MT ? t : 0], unit[h], f32x4{0.f, 0.f, 0.f, 0.f}) : f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int t = 0; t < MT; ++t) {
+                    const f32x4 v = mfma(xc[t], unit[h], f32x4{0.f, 0.f, 0.f, 0.f});
+                    if constexpr (MT == 1) {
+                        xt[h][0] = gather_rows16(bf16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])});
+                    } else {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) xt[h][t / 2][4 * (t & 1) + e] = f2bf(v[e]);
+                        for (int e = 0; e < 4; ++e) xt[h][t / 2][4 * (t & 1) + e] = f2bf(v[e]);
+                    }
                 }
 #pragma unroll
             for (int t = 0; t < MT; ++t)
@@ -231,7 +261,6 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
 #pragma unroll
                     for (int e = 0; e < 4; ++e) xc[t][4 * h + e] = f2bf(rbf(cm.a * bf2f(xc[t][4 * h + e])) + rbf(v[e]));
                 }
-            gram(xc);
         };
 #pragma unroll
         for (int j = 0; j < NCH; ++j)
@@ -243,7 +272,7 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         for (int j = 0; j < NCH; ++j)
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                const int row = t * 16 + i, col = col0 + j * 32;
+                const int row = chain_row<MT>(t, i), col = col0 + j * 32;
                 if (j < per && row < M && col < K) *(bf16x8*)(area + blocked_offset(row, col, k.cbx)) = x[j][t];
             }
         return;
@@ -257,7 +286,7 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
     for (int j = 0; j < per; ++j)
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            const int row = t * 16 + i, col = col0 + j * 32;
+            const int row = chain_row<MT>(t, i), col = col0 + j * 32;
             if (row >= M || col >= K) continue;
             const bf16x8 v = mine[(j * MT + t) * 64];
             if (cm.p_dtype == MUON_HIP_BF16) update8((bf16_t*)p, v, row, col, k.cols, M, K, turn, k.scale, cm.decay, cm.alpha);

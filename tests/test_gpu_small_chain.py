@@ -16,8 +16,8 @@ SHAPES = [(1, 1), (1, 9), (3, 33), (15, 16), (16, 31), (16, 256), (16, 257), (13
 
 @pytest.mark.parametrize("rows,cols", SHAPES)
 def test_small_chain_against_the_oracle(env, rows, cols):
-    """One iteration differs by the order of its fp32 sums, which a bf16 rounding shows as one unit in the last place (2^-8) of
-    the few values next to a rounding point: below 2e-3 in norm, plus 2^-8 where the norm itself, a bf16 value, comes out as its
+    """One iteration differs from the oracle by the order of its fp32 sums, which a bf16 rounding shows as one unit in the last place
+    (2^-8) of the few values next to a rounding point: below 2e-3 in norm, plus 2^-8 where the norm itself, a bf16 value, comes out as its
     neighbour.  More iterations are held to the bound of every shape."""
     print(f"small chain {rows}x{cols}", flush=True)
     mu, O = env["mu"], env["O"]
@@ -28,6 +28,53 @@ def test_small_chain_against_the_oracle(env, rows, cols):
             assert got.shape == g.shape
             for i in range(2):
                 assert rel_fro(got[i], O.newton_schulz(g[i], steps)) <= tol, (steps, i)
+
+
+@pytest.mark.parametrize("rows,cols", SHAPES)
+def test_small_chain_is_bitwise_the_tiled_products(env, rows, cols):
+    """Every fp32 sum of the chain runs in the order of the tiled kernels (ascending k in 32-deep MFMAs), so a configuration named
+    for the tiled products gives the same bits."""
+    print(f"small chain against tiles {rows}x{cols}", flush=True)
+    lib, abi, mu = env["lib"], env["abi"], env["mu"]
+    G = torch.randn(3, rows, cols, generator=torch.Generator().manual_seed(rows * 11 + cols))
+    G *= torch.logspace(-3, 1, rows).view(1, rows, 1)  # rows of different sizes, as gradients have: small singular values too
+    for g in (G.to(env["dev"]), G.mT.contiguous().to(env["dev"])):
+        for steps in (1, 2, 5):
+            got = mu.fast_newtonschulz(g, steps)
+            abi.check(lib.muon_hip_set_gemm_config(abi.CFG_128_PIPE))
+            try:
+                ref = mu.fast_newtonschulz(g, steps)
+            finally:
+                abi.check(lib.muon_hip_set_gemm_config(abi.CFG_AUTO))
+            torch.cuda.synchronize()
+            assert bool(torch.isfinite(ref.float()).all())
+            assert torch.equal(got, ref), steps
+
+
+@pytest.mark.parametrize("pdtype", [torch.float32, torch.bfloat16])
+def test_small_chain_in_a_step_is_bitwise_the_tiled_products(env, pdtype):
+    """The same through Muon.step, where the chain applies the parameter update itself."""
+    print(f"small chain step against tiles {pdtype}", flush=True)
+    lib, abi, mu, dev = (env[k] for k in ("lib", "abi", "mu", "dev"))
+    gen = torch.Generator().manual_seed(6)
+    shapes = SHAPES + [(c, r) for r, c in SHAPES if r != c]
+    ws = [(0.02 * torch.randn(*s, generator=gen)).to(pdtype) for s in shapes]
+    gs = [(1e-3 * torch.randn(*s, generator=gen)).to(pdtype) for s in shapes]
+    out = []
+    for cfg in (abi.CFG_AUTO, abi.CFG_128_PIPE):
+        params = [torch.nn.Parameter(w.to(dev)) for w in ws]
+        for p, g in zip(params, gs):
+            p.grad = g.to(dev)
+        abi.check(lib.muon_hip_set_gemm_config(cfg))
+        try:
+            mu.Muon([dict(params=list(params), use_muon=True, lr=0.02, momentum=0.95, nesterov=True, weight_decay=0.01, ns_steps=5,
+                          rms_scale=True)]).step()
+        finally:
+            abi.check(lib.muon_hip_set_gemm_config(abi.CFG_AUTO))
+        torch.cuda.synchronize()
+        out.append([p.detach() for p in params])
+    for s, p, q in zip(shapes, *out):
+        assert torch.equal(p, q), s
 
 
 @pytest.mark.parametrize("pdtype", [torch.float32, torch.bfloat16])
