@@ -147,8 +147,8 @@ int make_plan(int rows, int cols, int batch, Plan& p) {
     if (p.tile < 128) p.tile = 128;  // the elementwise kernels move whole 128-tiles
     p.Mp = (int)round_up(p.M, p.tile);
     p.Kr = (int)round_up(p.K, 128);
-    // the tiles of a.X + B.X may be 256 wide whatever their height
-    p.Kp = (int)round_up(p.K, p.Mp >= 384 ? 256 : 128);
+    // whole tiles of the configuration, and the persistent a.X + B.X has tiles 256 wide whatever their height
+    p.Kp = (int)round_up(p.K, p.Mp >= 384 ? 256 : p.tile);
     p.n = (long)rows * cols;
     p.strideU = round_up(p.n, 8);
     p.strideX = blocked_elems(p.Mp, p.Kp);

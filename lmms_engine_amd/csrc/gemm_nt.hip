@@ -1608,6 +1608,17 @@ long count_tiles(const GemmItem& it, int tile, int height = 0) {
     return (epi_is_bx(it.epi) ? tm * tn : tm * (tm + 1) / 2) * it.g.batch;
 }
 
+// Whether whole tiles of height x width cover C without leaving the storage of an operand: row blocks of 256 and, along a row,
+// whole column blocks.
+bool tiles_fit(const GemmItem& it, int height, int width) {
+    const GemmArgs& g = it.g;
+    auto up = [](int v, int m) { return (v + m - 1) / m * m; };
+    if (up(g.rows, height) > up(g.rows, BLK_ROWS)) return false;
+    if (!epi_is_bx(it.epi)) return g.rows % height == 0 && g.rows <= g.cbC * BLK_COLS;
+    const int cols = up(g.cols, width);
+    return cols <= g.cbC * BLK_COLS && cols <= g.cbQ * BLK_COLS && cols <= g.cbEt * BLK_COLS;
+}
+
 // Tile height of the persistent a.X + B.X for a matrix of `rows` rows: the one that covers the fewest, the tallest among equals.
 // The storage of a matrix is whole row blocks of 256; a tile may overhang into it, but not past it.  The overhang reads and
 // writes storage that no other product takes for anything: its values never meet a row of the matrix, because every reduction
@@ -1709,12 +1720,11 @@ hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t 
             bool odd = false;
             for (int i = 0; i < n; ++i) {
                 const GemmArgs& g = items[i].g;
-                if (done[i] || items[i].epi != epi || g.kdim < 256 || !g.ppx) continue;
+                if (done[i] || items[i].epi != epi || g.kdim < 256 || !g.ppx || !tiles_fit(items[i], h, 256)) continue;
                 if (cfg[i] == GEMM_CFG_256_PERSIST) {
                     if (h != 256 || (epi != EPI_BX && g.kdim > (epi == EPI_SYRK ? PPX_SYRK_MAXK : PPX_SYMPOLY_MAXK))) continue;
                 } else {
                     if (!adapt || cfg[i] != GEMM_CFG_128_PINGPONG || epi != EPI_BX || g.rows < 384 || h != ppx_height(g.rows)) continue;
-                    if (g.cbC * BLK_COLS < (g.cols + 255) / 256 * 256) continue;  // a tile would leave the storage
                     odd = true;
                 }
                 const long t = count_tiles(items[i], 256, h);
@@ -1757,6 +1767,7 @@ hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t 
         const int tile = gemm_cfg_tile(cfg[i]);
         for (int k = i; k < n; ++k) {
             if (done[k] || cfg[k] != cfg[i] || items[k].epi != items[i].epi) continue;
+            if (items[k].g.rows % tile || !tiles_fit(items[k], tile, tile)) return hipErrorInvalidValue;
             const long blocks = count_tiles(items[k], tile);
             if (l.n > 0 && l.start[l.n] + blocks > 0x7fffffffL) continue;  // goes with a later launch
             GemmArgs& g = l.g[l.n];

@@ -102,3 +102,23 @@ def test_matmul_transpose_of_padded_short_sides(env, M, K):
     # one rounding to bf16 and an fp32 sum of K products
     assert ((got - ref).abs() <= ref.abs() * 2.0**-8 + K * 2.0**-24 * (x.double().abs() @ x.double().abs().T)).all()
     assert torch.equal(got, got.T)
+
+
+# configurations that the caller names, on short sides of one 256-tile and long sides that end inside a 256-tile, in batches: a
+# tile past the end of a matrix would write the next one
+@pytest.mark.parametrize("rows,cols,batch", [(100, 300, 5), (256, 640, 3), (640, 200, 4), (300, 700, 3)])
+def test_named_configurations_agree_bitwise(env, rows, cols, batch):
+    lib, abi, mu = env["lib"], env["abi"], env["mu"]
+    g = torch.randn(batch, rows, cols, generator=torch.Generator().manual_seed(rows + cols)).bfloat16().to(env["dev"])
+    out = []
+    for cfg in (abi.CFG_128_PIPE, abi.CFG_256_PIPE, abi.CFG_256_PINGPONG, abi.CFG_128_PINGPONG, abi.CFG_256_PERSIST, abi.CFG_64_DEEP):
+        print(f"named configuration {cfg}: {batch} x {rows} x {cols}", flush=True)
+        abi.check(lib.muon_hip_set_gemm_config(cfg))
+        try:
+            out.append(mu.fast_newtonschulz(g, 5))
+        finally:
+            abi.check(lib.muon_hip_set_gemm_config(abi.CFG_AUTO))
+        torch.cuda.synchronize()
+    assert bool(torch.isfinite(out[0].float()).all())
+    for i, o in enumerate(out[1:], 1):
+        assert torch.equal(o, out[0]), i

@@ -219,6 +219,20 @@ def test_host_only_entry_points():
         _abi.dtype_code(torch.float16)
 
 
+@pytest.mark.parametrize("rows,cols", [(100, 300), (256, 640), (640, 256), (1, 1), (300, 700), (896, 1000), (1000, 2731)])
+def test_geometry_is_whole_tiles_of_a_named_configuration(rows, cols):
+    """A kernel whose last tile passed the end of a matrix would read and write the next one."""
+    lib = _abi.lib()
+    for cfg in range(6):
+        assert lib.muon_hip_set_gemm_config(cfg) == 0
+        try:
+            geo = _abi.geometry(rows, cols)
+        finally:
+            assert lib.muon_hip_set_gemm_config(_abi.CFG_AUTO) == 0
+        assert geo["Mp"] >= min(rows, cols) and geo["Kp"] >= max(rows, cols)
+        assert geo["Mp"] % geo["tile"] == 0 and geo["Kp"] % geo["tile"] == 0, (cfg, geo)
+
+
 def test_clip_grad_norm_host_behaviour():
     """What clip_grad_norm_ decides before any kernel runs: the empty cases return what torch's
     _get_total_norm returns, a NaN order and CPU gradients are refused (no fallback path)."""
