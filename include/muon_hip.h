@@ -156,6 +156,15 @@ int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int 
                         double weight_decay, double beta, int nesterov, int ns_steps, double a, double b, double c,
                         int write_back_grad, void* stream);
 
+/* Which kernels such a call takes on a device of `cus` compute units, one entry per bucket, for the product named by its
+ * MUON_HIP_K_ id (syrk, sympoly, bx, bx_update); touches no device.  For tests and measurements. */
+typedef struct {
+    int cfg;    /* MUON_HIP_CFG_256_PERSIST: the persistent kernel; otherwise the configuration of the one-tile kernel */
+    int height; /* rows of a tile */
+    int launch; /* which launch of the stage it goes with; -1: no product, the whole chain runs in one workgroup per matrix */
+} muon_hip_route;
+int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cus, muon_hip_route* out);
+
 /* ---- blocked matrices and single GEMM entry points ---------------------------------------
  * The Newton-Schulz operands are kept in blocks of 256 rows x 32 columns (16 KB, 64-byte
  * rows back to back): element (r, c) of a matrix with cb = cols / 32 column blocks is at

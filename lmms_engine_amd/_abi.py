@@ -34,6 +34,12 @@ class Bucket(ctypes.Structure):
                 ("batch", c_int), ("scale", c_double)]
 
 
+class Route(ctypes.Structure):
+    """muon_hip_route"""
+
+    _fields_ = [("cfg", c_int), ("height", c_int), ("launch", c_int)]
+
+
 # name -> (restype, argtypes); mirrors include/muon_hip.h one to one
 SIGNATURES = {
     "muon_hip_version": (c_int, []),
@@ -54,6 +60,7 @@ SIGNATURES = {
                                       c_double, c_int, c_void_p]),
     "muon_hip_step_multi": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_double, c_double, c_double, c_int, c_int,
                                     c_double, c_double, c_double, c_int, c_void_p]),
+    "muon_hip_routes": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p]),
     "muon_hip_blocked_elems": (c_long, [c_int, c_int]),
     "muon_hip_pack_bf16": (c_int, [c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
     "muon_hip_unpack_bf16": (c_int, [c_void_p, c_int, c_int, c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p]),
@@ -134,6 +141,14 @@ def workspace_bytes(rows: int, cols: int, batch: int) -> int:
     if n == 0:
         raise MuonHipError(f"workspace_bytes({rows}, {cols}, {batch}): " + lib().muon_hip_last_error().decode())
     return n
+
+
+def routes(shapes, kernel: str, cus: int = 256):
+    """[(configuration, tile height, launch)] of the (rows, cols, matrices) of one call, for a product by its KERNEL_NAMES name."""
+    buckets = (Bucket * len(shapes))(*[Bucket(rows=r, cols=c, batch=n) for r, c, n in shapes])
+    out = (Route * len(shapes))()
+    check(lib().muon_hip_routes(buckets, len(shapes), KERNEL_NAMES.index(kernel), cus, out), "routes")
+    return [(r.cfg, r.height, r.launch) for r in out]
 
 
 def device_shape():

@@ -358,6 +358,22 @@ int do_normalize(const Work& w, hipStream_t s) {
     return e == hipSuccess ? 0 : hip_fail(e, "normalize launch");
 }
 
+// The products of one stage of an iteration that reads X from buffer `cur`; whether the launcher may choose smaller tiles for
+// them (the same for all: a configuration that the caller has named is named for every launch).
+bool stage_items(const Work& w, int epi, int cur, double a, double b, double c, unsigned* ppx, GemmItem* items) {
+    bool adapt = true;
+    for (int i = 0; i < w.n; ++i) {
+        const Bucket& k = w.b[i];
+        const Plan& p = k.p;
+        const Cfg cfg = pick_cfg(p.M, epi);
+        adapt = cfg.adapt;
+        if (epi == EPI_SYRK) items[i] = syrk_item(cfg.id, k.at(p.offX[cur]), k.at(p.offA), p.Mp, p.Kr, p.Kp, p.batch, ppx);
+        else if (epi == EPI_SYMPOLY) items[i] = sympoly_item(cfg.id, k.at(p.offA), k.at(p.offB), p.Mp, p.batch, b, c, ppx);
+        else items[i] = bx_item(cfg.id, k.at(p.offB), k.at(p.offX[cur]), k.at(p.offX[cur ^ 1]), p.Mp, p.Kr, p.Kp, p.batch, a, ppx);
+    }
+    return adapt;
+}
+
 // Normalise, then `steps` iterations; with `upd` the last B.X applies the parameter update instead of writing X'.
 int ns_chain(const Work& all, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s) {
     if (steps < 0) return fail(MUON_HIP_EINVAL, "steps must be >= 0");
@@ -393,29 +409,14 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
     GemmItem items[MUON_HIP_MAX_BUCKETS];
     for (int it = 0; it < steps; ++it) {
         const int cur = it & 1;
-        bool adapt = true;
-        auto each = [&](int epi, auto make) {
-            for (int i = 0; i < w.n; ++i) {
-                const Bucket& k = w.b[i];
-                const Cfg cfg = pick_cfg(k.p.M, epi);
-                adapt = cfg.adapt;  // the same for all: a forced configuration is forced for every launch
-                items[i] = make(k, cfg.id);
-            }
-        };
-        each(EPI_SYRK, [&](const Bucket& k, int cfg) {
-            return syrk_item(cfg, k.at(k.p.offX[cur]), k.at(k.p.offA), k.p.Mp, k.p.Kr, k.p.Kp, k.p.batch, ppx);
-        });
+        bool adapt = stage_items(w, EPI_SYRK, cur, a, b, c, ppx, items);
         if (int rc = launch_items(MUON_HIP_K_SYRK, "syrk launch", items, w.n, adapt, s)) return rc;
-        each(EPI_SYMPOLY, [&](const Bucket& k, int cfg) {
-            return sympoly_item(cfg, k.at(k.p.offA), k.at(k.p.offB), k.p.Mp, k.p.batch, b, c, ppx);
-        });
+        adapt = stage_items(w, EPI_SYMPOLY, cur, a, b, c, ppx, items);
         if (int rc = launch_items(MUON_HIP_K_SYMPOLY, "sympoly launch", items, w.n, adapt, s)) return rc;
+        adapt = stage_items(w, EPI_BX, cur, a, b, c, ppx, items);
         const bool last = upd && it == steps - 1;
-        each(EPI_BX, [&](const Bucket& k, int cfg) {
-            GemmItem g = bx_item(cfg, k.at(k.p.offB), k.at(k.p.offX[cur]), k.at(k.p.offX[cur ^ 1]), k.p.Mp, k.p.Kr, k.p.Kp, k.p.batch, a, ppx);
-            if (last) fold_update(g, k.p_ptrs, k.p.rows, k.p.cols, k.scale, *upd);
-            return g;
-        });
+        if (last)
+            for (int i = 0; i < w.n; ++i) fold_update(items[i], w.b[i].p_ptrs, w.b[i].p.rows, w.b[i].p.cols, w.b[i].scale, *upd);
         if (int rc = launch_items(last ? MUON_HIP_K_BX_UPDATE : MUON_HIP_K_BX, "bx launch", items, w.n, adapt, s)) return rc;
     }
     return 0;
@@ -543,6 +544,30 @@ int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int 
             if (int rc = muon_hip_apply_update(w.b[i].p_ptrs, p_dtype, w.b[i].ws, w.b[i].p.rows, w.b[i].p.cols, w.b[i].p.batch, 0,
                                                w.b[i].scale, lr, weight_decay, stream))
                 return rc;
+    return 0;
+}
+
+int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cus, muon_hip_route* out) {
+    if (!buckets || !out || n < 1 || n > MUON_HIP_MAX_BUCKETS || cus < 1) return fail(MUON_HIP_EINVAL, "bad bucket list or device");
+    const int epi = kernel_id == MUON_HIP_K_SYRK ? EPI_SYRK : kernel_id == MUON_HIP_K_SYMPOLY ? EPI_SYMPOLY : EPI_BX;
+    if (epi == EPI_BX && kernel_id != MUON_HIP_K_BX && kernel_id != MUON_HIP_K_BX_UPDATE) return fail(MUON_HIP_EINVAL, "not a product");
+    Work w;
+    int from[MUON_HIP_MAX_BUCKETS];
+    alignas(256) static char nowhere[256];  // stands for a workspace: plans hold addresses, nothing is read through them
+    for (int i = 0; i < n; ++i) {
+        out[i] = muon_hip_route{MUON_HIP_CFG_AUTO, 0, -1};
+        Bucket& k = w.b[w.n];
+        if (int rc = k.init(buckets[i].rows, buckets[i].cols, buckets[i].batch, nowhere)) return rc;
+        if (!k.p.small) from[w.n++] = i;
+    }
+    if (!w.n) return 0;
+    GemmItem items[MUON_HIP_MAX_BUCKETS];
+    GemmRoute route[MUON_HIP_MAX_BUCKETS];
+    const bool adapt = stage_items(w, epi, 0, 1.0, 1.0, 1.0, ppx_counters(w), items);
+    if (kernel_id == MUON_HIP_K_BX_UPDATE)
+        for (int i = 0; i < w.n; ++i) fold_update(items[i], nullptr, w.b[i].p.rows, w.b[i].p.cols, 1.0, UpdateArgs{});
+    if (plan_gemm_nt(items, w.n, adapt, cus, route) < 0) return fail(MUON_HIP_EINVAL, "no kernel takes these products");
+    for (int i = 0; i < w.n; ++i) out[from[i]] = muon_hip_route{route[i].cfg, route[i].height, route[i].launch};
     return 0;
 }
 

@@ -90,3 +90,10 @@ struct GemmItem {
     int cfg, epi;
 };
 hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t stream);
+
+// What launch_gemm_nt does with each of them on a device of `cus` compute units: the kernel, the rows of its tiles, and the
+// launch of the call (from 0) that it goes with.  The number of launches, or -1 when it refuses them; touches no device.
+struct GemmRoute {
+    int cfg, height, launch;
+};
+int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* route);

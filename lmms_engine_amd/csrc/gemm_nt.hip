@@ -1671,18 +1671,16 @@ hipError_t machine_shape(MachineShape& ms) {
     return hipSuccess;
 }
 
-hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t stream) {
-    if (n < 1 || n > GEMM_MAX_LIST) return hipErrorInvalidValue;
-    MachineShape ms;
-    if (hipError_t e = machine_shape(ms); e != hipSuccess) return e;
-    const int cus = ms.cus;
+int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* route) {
+    if (n < 1 || n > GEMM_MAX_LIST) return -1;
     int cfg[GEMM_MAX_LIST];
     bool done[GEMM_MAX_LIST] = {};
+    int launches = 0;
     long all128 = 0, own128 = 0, all64 = 0;
     bool fold = false;
     for (int i = 0; i < n; ++i) {
         cfg[i] = items[i].cfg;
-        if (gemm_cfg_tile(cfg[i]) == 0) return hipErrorInvalidValue;
+        if (gemm_cfg_tile(cfg[i]) == 0) return -1;
         all128 += count_tiles(items[i], 128);
         if (gemm_cfg_tile(cfg[i]) == 256) own128 += count_tiles(items[i], 128);
         all64 += count_tiles(items[i], 64);
@@ -1710,12 +1708,7 @@ hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t 
     // 57 | 60.
     for (int epi : {EPI_SYRK, EPI_SYMPOLY, EPI_BX}) {
         for (int h : {256, 224, 192}) {
-            GemmList l;
-            l.n = 0;
-            l.xcd_shift = ms.xcd_shift;
-            l.big_blocks = 0;
-            l.start[0] = 0;
-            int from[GEMM_MAX_LIST];
+            int from[GEMM_MAX_LIST], m = 0;
             long blocks = 0;
             bool odd = false;
             for (int i = 0; i < n; ++i) {
@@ -1729,14 +1722,8 @@ hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t 
                 }
                 const long t = count_tiles(items[i], 256, h);
                 if (blocks + t > 0x7fffffffL) continue;
-                GemmArgs& e = l.g[l.n];
-                e = g;
-                e.tiles_m = (g.rows + h - 1) / h;
-                e.tiles_n = (g.cols + 255) / 256;
-                e.tiles_per_mat = (int)(t / g.batch);
-                from[l.n++] = i;
+                from[m++] = i;
                 blocks += t;
-                l.start[l.n] = (int)blocks;
             }
             if (blocks <= cus) continue;
             // A few rounds with a nearly empty last one: the one-tile kernel cuts that round's tiles into quarters (264 tiles of
@@ -1745,41 +1732,70 @@ hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t 
             // rounds: 74 us on 128-tiles, 70 here).
             const long rest = blocks % cus, rounds = (blocks + cus - 1) / cus;
             if (odd ? 4 * blocks < 3 * rounds * cus : adapt && rest > 0 && rest <= cus / 4 && blocks <= 4L * cus) continue;
-            hipError_t e;
-            if (epi == EPI_SYRK) e = launch_ppx<EPI_SYRK>(l, (int)blocks, cus, stream);
-            else if (epi == EPI_SYMPOLY) e = launch_ppx<EPI_SYMPOLY>(l, (int)blocks, cus, stream);
-            else if (h == 256) e = launch_ppx<EPI_BX>(l, (int)blocks, cus, stream);
-            else if (h == 224) e = launch_ppx<EPI_BX, 8, 6>(l, (int)blocks, cus, stream);
-            else e = launch_ppx<EPI_BX, 6, 6>(l, (int)blocks, cus, stream);
-            if (e != hipSuccess) return e;
-            for (int i = 0; i < l.n; ++i) done[from[i]] = true;
+            for (int k = 0; k < m; ++k) {
+                route[from[k]] = GemmRoute{GEMM_CFG_256_PERSIST, h, launches};
+                done[from[k]] = true;
+            }
+            ++launches;
         }
     }
     for (int i = 0; i < n; ++i)
-        if (!done[i] && cfg[i] == GEMM_CFG_256_PERSIST) cfg[i] = GEMM_CFG_256_PINGPONG;
+        if (cfg[i] == GEMM_CFG_256_PERSIST) cfg[i] = GEMM_CFG_256_PINGPONG;
     for (int i = 0; i < n; ++i) {  // one launch per kind and configuration
         if (done[i]) continue;
+        const int tile = gemm_cfg_tile(cfg[i]);
+        long blocks = 0;
+        for (int k = i; k < n; ++k) {
+            if (done[k] || cfg[k] != cfg[i] || items[k].epi != items[i].epi) continue;
+            if (items[k].g.rows % tile || !tiles_fit(items[k], tile, tile)) return -1;
+            const long t = count_tiles(items[k], tile);
+            if (blocks > 0 && blocks + t > 0x7fffffffL) continue;  // goes with a later launch
+            blocks += t;
+            route[k] = GemmRoute{cfg[k], tile, launches};
+            done[k] = true;
+        }
+        ++launches;
+    }
+    return launches;
+}
+
+hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t stream) {
+    MachineShape ms;
+    if (hipError_t e = machine_shape(ms); e != hipSuccess) return e;
+    GemmRoute route[GEMM_MAX_LIST];
+    const int launches = plan_gemm_nt(items, n, adapt, ms.cus, route);
+    if (launches < 0) return hipErrorInvalidValue;
+    for (int k = 0; k < launches; ++k) {
         GemmList l;
         l.n = 0;
         l.xcd_shift = ms.xcd_shift;
         l.big_blocks = 0;
         l.start[0] = 0;
-        const int tile = gemm_cfg_tile(cfg[i]);
-        for (int k = i; k < n; ++k) {
-            if (done[k] || cfg[k] != cfg[i] || items[k].epi != items[i].epi) continue;
-            if (items[k].g.rows % tile || !tiles_fit(items[k], tile, tile)) return hipErrorInvalidValue;
-            const long blocks = count_tiles(items[k], tile);
-            if (l.n > 0 && l.start[l.n] + blocks > 0x7fffffffL) continue;  // goes with a later launch
+        int epi = 0, cfg = 0, height = 0;
+        for (int i = 0; i < n; ++i) {
+            if (route[i].launch != k) continue;
+            epi = items[i].epi;
+            cfg = route[i].cfg;
+            height = route[i].height;
+            const int width = gemm_cfg_tile(cfg);
+            const long t = count_tiles(items[i], width, height);
             GemmArgs& g = l.g[l.n];
-            g = items[k].g;
-            g.tiles_m = g.rows / tile;
-            g.tiles_n = (g.cols + tile - 1) / tile;
-            g.tiles_per_mat = (int)(blocks / g.batch);
-            l.start[l.n + 1] = l.start[l.n] + (int)blocks;
+            g = items[i].g;
+            g.tiles_m = (g.rows + height - 1) / height;
+            g.tiles_n = (g.cols + width - 1) / width;
+            g.tiles_per_mat = (int)(t / g.batch);
+            l.start[l.n + 1] = l.start[l.n] + (int)t;
             ++l.n;
-            done[k] = true;
         }
-        if (hipError_t e = launch_epi(items[i].epi, cfg[i], l, l.start[l.n], cus, stream); e != hipSuccess) return e;
+        const int blocks = l.start[l.n];
+        hipError_t e;
+        if (cfg != GEMM_CFG_256_PERSIST) e = launch_epi(epi, cfg, l, blocks, ms.cus, stream);
+        else if (epi == EPI_SYRK) e = launch_ppx<EPI_SYRK>(l, blocks, ms.cus, stream);
+        else if (epi == EPI_SYMPOLY) e = launch_ppx<EPI_SYMPOLY>(l, blocks, ms.cus, stream);
+        else if (height == 256) e = launch_ppx<EPI_BX>(l, blocks, ms.cus, stream);
+        else if (height == 224) e = launch_ppx<EPI_BX, 8, 6>(l, blocks, ms.cus, stream);
+        else e = launch_ppx<EPI_BX, 6, 6>(l, blocks, ms.cus, stream);
+        if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }

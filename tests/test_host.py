@@ -233,6 +233,22 @@ def test_geometry_is_whole_tiles_of_a_named_configuration(rows, cols):
         assert geo["Mp"] % geo["tile"] == 0 and geo["Kp"] % geo["tile"] == 0, (cfg, geo)
 
 
+def test_routes_name_the_kernels_of_a_call():
+    """The launcher's choice, on a device of 256 compute units: one case for each kernel it chooses between."""
+    r = _abi.routes
+    assert r([(16, 512, 4)], "bx_axpy") == [(_abi.CFG_AUTO, 0, -1)]  # one workgroup per matrix
+    assert r([(896, 4864, 1)], "syrk") == [(_abi.CFG_64_DEEP, 64, 0)]
+    assert r([(2048, 5632, 1)], "syrk") == [(_abi.CFG_128_PINGPONG, 128, 0)]
+    assert r([(768, 2048, 256)], "syrk") == [(_abi.CFG_256_PERSIST, 256, 0)]
+    assert r([(4096, 12288, 15)], "syrk") == [(_abi.CFG_256_PINGPONG, 256, 0)]  # a reduction past the persistent kernel's limit
+    assert r([(896, 4864, 72)], "bx_axpy") == [(_abi.CFG_256_PERSIST, 224, 0)]
+    assert r([(1152, 4304, 27)], "bx_axpy") == [(_abi.CFG_256_PERSIST, 192, 0)]
+    assert r([(4096, 4096, 72)], "bx_axpy_update") == [(_abi.CFG_256_PINGPONG, 256, 0)]
+    # products of one kernel share a launch
+    assert r([(768, 2048, 256), (640, 2560, 60), (16, 64, 1), (2048, 768, 128)], "bx_axpy") == [
+        (_abi.CFG_256_PERSIST, 256, 0), (_abi.CFG_256_PERSIST, 224, 1), (_abi.CFG_AUTO, 0, -1), (_abi.CFG_256_PERSIST, 256, 0)]
+
+
 def test_clip_grad_norm_host_behaviour():
     """What clip_grad_norm_ decides before any kernel runs: the empty cases return what torch's
     _get_total_norm returns, a NaN order and CPU gradients are refused (no fallback path)."""
