@@ -1709,7 +1709,7 @@ int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* r
     for (int epi : {EPI_SYRK, EPI_SYMPOLY, EPI_BX}) {
         for (int h : {256, 224, 192}) {
             int from[GEMM_MAX_LIST], m = 0;
-            long blocks = 0;
+            long blocks = 0, area = 0, shortest = 0x7fffffff;  // tiles, elements of C that they cover, the shortest reduction
             bool odd = false;
             for (int i = 0; i < n; ++i) {
                 const GemmArgs& g = items[i].g;
@@ -1724,14 +1724,21 @@ int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* r
                 if (blocks + t > 0x7fffffffL) continue;
                 from[m++] = i;
                 blocks += t;
+                area += (long)g.rows * g.cols * g.batch;
+                if (g.kdim < shortest) shortest = g.kdim;
             }
             if (blocks <= cus) continue;
             // A few rounds with a nearly empty last one: the one-tile kernel cuts that round's tiles into quarters (264 tiles of
-            // 1000 x 2731 43 us against 52, 792 tiles 102 against 107; 1200 tiles of 512 x 1408 111 against 105).  Tiles of odd
-            // heights have no quarters: 128-tiles unless three quarters of the rounds are full (608 tiles of 896 x 4864, 2.4
-            // rounds: 74 us on 128-tiles, 70 here).
+            // 1000 x 2731 43 us against 52, 792 tiles 102 against 107; 1200 tiles of 512 x 1408 111 against 105).
             const long rest = blocks % cus, rounds = (blocks + cus - 1) / cus;
-            if (odd ? 4 * blocks < 3 * rounds * cus : adapt && rest > 0 && rest <= cus / 4 && blocks <= 4L * cus) continue;
+            if (!odd && adapt && rest > 0 && rest <= cus / 4 && blocks <= 4L * cus) continue;
+            // Tiles of odd heights have no quarters, and their overhang is computed for nothing: 128-tiles unless the elements of
+            // the matrices fill 70 % of the rounds, and a k-tile's share more for the epilogue, which short reductions show.
+            // Measured on 785 batches of 384 to 2688 rows: 28 of the 590 that come here are slower than on 128-tiles, by 9 % at
+            // most, and 24 of the others would have been faster here, by as much (three quarters of the tiles instead of the
+            // elements took 72 that were slower, by up to 20 %: 16 of 1408 x 1408, 63 % full, 94 us on 128-tiles and 106 here; 20
+            // of 1152 x 1152, 70 %, 69 and 75; 608 tiles of 896 x 4864, 79 %, 74 and 70).
+            if (odd && area < (0.7 + 32.0 / shortest) * (256.0 * h) * rounds * cus) continue;
             for (int k = 0; k < m; ++k) {
                 route[from[k]] = GemmRoute{GEMM_CFG_256_PERSIST, h, launches};
                 done[from[k]] = true;

@@ -76,11 +76,13 @@ def test_one_call_over_many_shapes_equals_one_call_per_matrix(env, name, shapes,
 
 # a.X + B.X on tiles of the matrix's own height: 224, 192 and 256 rows, short sides that end inside the last 128 rows, long
 # sides whose last 256-tile overhangs, more than one row block, and rounds that are filled enough and not
-@pytest.mark.parametrize("rows,cols,batch", [(896, 1000, 40), (900, 640, 90), (384, 520, 100), (1160, 1152, 24), (1290, 1408, 12),
-                                             (1000, 1100, 30), (1000, 1000, 17), (896, 1000, 20), (2700, 1930, 8)])
-def test_odd_short_sides_do_not_change_the_result(env, rows, cols, batch):
+@pytest.mark.parametrize("rows,cols,batch,height", [
+    (896, 1000, 40, 224), (900, 640, 90, 224), (384, 520, 100, 128), (384, 520, 255, 192), (1160, 1152, 24, 192), (1290, 1408, 12, 128),
+    (1290, 1408, 14, 256), (1000, 1100, 30, 256), (1000, 1000, 17, 256), (896, 1000, 20, 128), (2700, 1930, 8, 256)])
+def test_odd_short_sides_do_not_change_the_result(env, rows, cols, batch, height):
     print(f"odd short side {batch} x {rows} x {cols}", flush=True)
     lib, abi, mu = env["lib"], env["abi"], env["mu"]
+    assert abi.routes([(rows, cols, batch)], "bx_axpy")[0][1] == height
     g = torch.randn(batch, rows, cols, generator=torch.Generator().manual_seed(rows + cols)).bfloat16().to(env["dev"])
     got = mu.fast_newtonschulz(g, 5)
     abi.check(lib.muon_hip_set_gemm_config(abi.CFG_128_PIPE))

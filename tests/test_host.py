@@ -249,6 +249,16 @@ def test_routes_name_the_kernels_of_a_call():
         (_abi.CFG_256_PERSIST, 256, 0), (_abi.CFG_256_PERSIST, 224, 1), (_abi.CFG_AUTO, 0, -1), (_abi.CFG_256_PERSIST, 256, 0)]
 
 
+@pytest.mark.parametrize("shape,height", [
+    # slower on tiles of their own height (94 -> 106 us, 69 -> 75, 58 -> 62, 68 -> 73, 109 -> 123): rounds filled by overhang
+    ((1408, 1408, 16), 128), ((1152, 1152, 20), 128), ((640, 2560, 20), 128), ((896, 896, 40), 128), ((384, 384, 448), 128),
+    # faster (713 -> 525 us, 190 -> 155, 362 -> 289, 128 -> 104)
+    ((896, 4864, 72), 224), ((640, 2560, 60), 224), ((1152, 4304, 27), 192), ((384, 1536, 150), 192), ((1408, 1408, 14), 256),
+    ((896, 4864, 8), 224)])
+def test_tiles_of_odd_heights_where_the_matrices_fill_their_rounds(shape, height):
+    assert _abi.routes([shape], "bx_axpy")[0][1] == height
+
+
 def test_clip_grad_norm_host_behaviour():
     """What clip_grad_norm_ decides before any kernel runs: the empty cases return what torch's
     _get_total_norm returns, a NaN order and CPU gradients are refused (no fallback path)."""
