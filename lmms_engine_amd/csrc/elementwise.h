@@ -20,6 +20,7 @@ struct EwBucket {
     bf16_t* X;                  // the normalised operand, blocked, Mp x Kp
     long strideX;
     int rows, cols, Mp, Kp, nparts, batch;
+    bool inline_norm;           // set by the launcher: the normalisation adds the partial sums itself, denom stays unset
 };
 constexpr int EW_MAX_LIST = 16;
 struct EwList {

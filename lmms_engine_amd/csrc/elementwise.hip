@@ -219,10 +219,13 @@ __device__ __forceinline__ float frob_denom(const float* p, int nparts, float* r
     return rbf(nrm + 1e-7f);
 }
 
-// Matrices of up to this many partial sums (a million elements) have no finalising launch: every workgroup of the
-// normalisation adds the sums itself, one per thread, behind its own load of u.  It costs 1 KB from L2 per workgroup of 4 KB
-// and saves 2 to 5 us per launch sequence; larger matrices would read as much in sums as in data.
+// Matrices of up to kInlineParts partial sums (a million elements) have no finalising launch: every workgroup of the
+// normalisation adds the sums itself, one per thread, behind its own load of u.  That saves a launch, 3.4 us, and costs every
+// workgroup a reduction between its load and its store, 0.15 to 0.2 ns each: measured on 128 to 1024 columns, 16384 workgroups of
+// straight tiles break even (32 of 1024 x 1024 29.6 us with the launch and 29.3 without, 64 of them 48.4 and 51.9, 256 185 and 200),
+// while the turned tiles, twice the size and with a barrier of their own, gain at every size (128 of 1024 x 768 76.9 and 74.2).
 constexpr int kInlineParts = 256;
+constexpr long kInlineGroups = 16384;
 
 __global__ void __launch_bounds__(256) frob_finalize_kernel(const EwList l) {
     __shared__ float red[4];
@@ -275,7 +278,7 @@ __global__ void __launch_bounds__(256) normalize_kernel(const EwList l, unsigned
     bf16x8 v[2];
     v[0] = load8(r0 + tr, c0 + tc);
     if (turn) v[1] = load8(r0 + tr + 16, c0 + tc);
-    const float d = e.nparts <= kInlineParts ? frob_denom(e.partials + (long)b * e.nparts, e.nparts, red) : e.denom[b];
+    const float d = e.inline_norm ? frob_denom(e.partials + (long)b * e.nparts, e.nparts, red) : e.denom[b];
     auto divide = [&](const bf16x8& a) {
         bf16x8 o;
 #pragma unroll
@@ -640,7 +643,8 @@ hipError_t launch_normalize(EwList& l, unsigned* clear, int clear_words, hipStre
         const EwBucket& e = l.b[i];
         const long per_mat = e.rows > e.cols ? (long)(e.Kp / NORM_T_TR) * (e.Mp / NORM_TC) : (long)(e.Mp / NORM_TR) * (e.Kp / NORM_TC);
         if (!append_blocks(l, i, per_mat * e.batch)) return hipErrorInvalidValue;
-        if (e.nparts > kInlineParts) {
+        l.b[i].inline_norm = e.nparts <= kInlineParts && (e.rows > e.cols || per_mat * e.batch <= kInlineGroups);
+        if (!e.inline_norm) {
             f.b[f.n] = e;
             f.start[f.n + 1] = f.start[f.n] + e.batch;
             ++f.n;

@@ -124,3 +124,14 @@ def test_named_configurations_agree_bitwise(env, rows, cols, batch):
     assert bool(torch.isfinite(out[0].float()).all())
     for i, o in enumerate(out[1:], 1):
         assert torch.equal(o, out[0]), i
+
+
+# 32 workgroups of the normalisation per 128 x 512 matrix: 512 matrices are the most whose workgroups add the norm's partial sums
+# themselves, one more takes the launch that adds them; turned matrices have no such limit
+@pytest.mark.parametrize("rows,cols,batch", [(128, 512, 512), (128, 512, 513), (512, 128, 1100)])
+def test_norms_of_large_and_small_batches_agree_bitwise(env, rows, cols, batch):
+    print(f"norms {batch} x {rows} x {cols}", flush=True)
+    g = torch.randn(batch, rows, cols, generator=torch.Generator().manual_seed(batch)).bfloat16().to(env["dev"])
+    got = env["mu"].fast_newtonschulz(g, 1)
+    for lo in (0, batch // 2, batch - 3):
+        assert torch.equal(got[lo:lo + 3], env["mu"].fast_newtonschulz(g[lo:lo + 3], 1)), lo
