@@ -600,7 +600,7 @@ def test_grouped_equals_per_matrix_bitwise(env):
 @pytest.mark.parametrize("pdtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("rows,cols,batch", [(256, 384, 3), (37, 53, 2), (100, 300, 2), (512, 1024, 2), (768, 2048, 3), (64, 64, 1),
                                              (384, 256, 3), (53, 37, 2), (300, 100, 2), (1024, 512, 2), (2048, 768, 3), (1000, 520, 2),
-                                             # more tiles than compute units: the persistent kernel carries the update
+                                             # more tiles than compute units: persistent products, and an update that is not
                                              (512, 1024, 40), (768, 2048, 24), (700, 1000, 30)])
 def test_folded_update_equals_the_staged_sequence_bitwise(env, pdtype, rows, cols, batch):
     """muon_hip_step_grouped lets the epilogue of the last B.X apply the scaled update to the parameter without writing
@@ -673,7 +673,7 @@ def _chunk_plan(env, rows, cols, n, cap):
 
 
 @pytest.mark.parametrize("rows,cols,n,cap,kernel", [
-    (2048, 2048, 23, 8, "persistent"),   # 36 + 36 + 64 tiles a matrix: all three products of a chunk of 8 walk tiles
+    (2048, 2048, 28, 12, "persistent"),  # 36 + 36 + 64 tiles a matrix: all three products of a chunk of 12 walk tiles
     (2048, 1024, 7, 3, "transposed"),    # rows > cols on 256-tiles: the update goes through the transposing gather
     (640, 384, 10, 4, "128-tiles"),      # short side no whole number of 256-tiles, transposed and ragged
 ])
@@ -690,8 +690,9 @@ def test_chunked_bucket_equals_the_unchunked_twin_bitwise(env, rows, cols, n, ca
     nchunks = -(-n // chunk)
     assert nchunks >= 3 and n % chunk != 0, (chunk, nchunks)
     if kernel == "persistent":
-        T = rows // 256
-        assert chunk * T * (T + 1) // 2 > 256 and chunk * T * (cols // 256) > 256  # more tiles than compute units
+        for product in ("syrk", "sympoly", "bx_axpy"):
+            for batch in (chunk, n):
+                assert env["abi"].routes([(rows, cols, batch)], product)[0][0] == env["abi"].CFG_256_PERSIST, (product, batch)
     gen = torch.Generator().manual_seed(rows + 3 * cols + n)
     w0 = [(0.02 * torch.randn(rows, cols, generator=gen)).bfloat16() for _ in range(n)]
     hp = dict(MUON_HP)

@@ -1,6 +1,8 @@
 """Launches that do not fill the machine: the 64-tile kernel and the choice of smaller tiles.  Every configuration sums the
 products of an element in ascending k, so all of them agree bit for bit; the two-stage 128-tile kernel, which
 tests/test_gpu_parity.py holds to the fp64 product, is the reference."""
+from collections import Counter
+
 import pytest
 import torch
 
@@ -45,17 +47,22 @@ def test_the_choice_by_tile_count_does_not_change_the_result(env, M, K, batch):
 
 # one call over many shapes: more shapes than a call takes, a bucket that runs the persistent kernel beside small ones, both
 # orientations, ragged edges, the norms of matrices above and below the limit of the inline sums, bf16 momentum
-@pytest.mark.parametrize("name,shapes,dtype,mdtype", [
-    ("17 shapes", [(64 + 8 * i, 100 + 16 * i) for i in range(17)], torch.float32, None),
-    ("persistent beside small", [(512, 1024)] * 36 + [(256, 384)] * 3 + [(300, 100)] * 2 + [(33, 47), (1024, 1100)], torch.bfloat16,
-     torch.float32),
-    ("persistent lists of every tile height", [(896, 1000)] * 20 + [(1100, 900)] * 20 + [(650, 640)] * 60 + [(1000, 1024)] * 9 + [(1030, 990)] * 9,
-     torch.float32, None),
-    ("tall and wide", [(1408, 256), (256, 1408), (1, 9), (200, 200)], torch.bfloat16, None),
+# lists: for a.X + B.X, how many shapes share one persistent launch, by tile height
+@pytest.mark.parametrize("name,shapes,dtype,mdtype,lists", [
+    ("17 shapes", [(64 + 8 * i, 100 + 16 * i) for i in range(17)], torch.float32, None, {}),
+    ("persistent beside small", [(512, 1024)] * 40 + [(256, 384)] * 3 + [(300, 100)] * 2 + [(33, 47), (1024, 1100)], torch.bfloat16,
+     torch.float32, {256: 2}),
+    ("persistent lists of every tile height", [(896, 1000)] * 20 + [(1100, 900)] * 20 + [(650, 640)] * 60 + [(1000, 1024)] * 9 +
+     [(1030, 990)] * 9 + [(1160, 1152)] * 24 + [(384, 700)] * 32, torch.float32, None, {256: 3, 224: 2, 192: 2}),
+    ("tall and wide", [(1408, 256), (256, 1408), (1, 9), (200, 200)], torch.bfloat16, None, {}),
 ])
-def test_one_call_over_many_shapes_equals_one_call_per_matrix(env, name, shapes, dtype, mdtype):
+def test_one_call_over_many_shapes_equals_one_call_per_matrix(env, name, shapes, dtype, mdtype, lists):
     print(f"many shapes: {name}", flush=True)
-    mu, dev = env["mu"], env["dev"]
+    mu, dev, abi = env["mu"], env["dev"], env["abi"]
+    if len(set(shapes)) <= abi.MAX_BUCKETS:
+        routes = abi.routes([(*s, shapes.count(s)) for s in sorted(set(shapes), reverse=True)], "bx_axpy")
+        persistent = Counter((launch, height) for cfg, height, launch in routes if cfg == abi.CFG_256_PERSIST)
+        assert {height: n for (_, height), n in persistent.items()} == lists
     g = torch.Generator().manual_seed(len(shapes))
     ws = [(0.02 * torch.randn(*s, generator=g)).to(dtype) for s in shapes]
     gs = [(1e-3 * torch.randn(*s, generator=g)).to(dtype) for s in shapes]
