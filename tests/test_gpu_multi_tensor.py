@@ -266,8 +266,9 @@ def test_clip_within_the_limit_leaves_every_bit(env, dtype, max_norm, moves):
 
 @pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 128, 129, 4096, 4097])
 def test_every_chunk_finds_its_tensor(env, n):
-    """Lists around the widths of the search: 64 entries a round.  Each tensor is scaled by a power of two of its own bits, so a
-    chunk that took another tensor's place would leave its own untouched; empty tensors and tensors of two chunks among them."""
+    """Lists around the widths of the search: 64 entries a round.  All tensors are scaled by one coefficient below one, so a chunk
+    that took another tensor's place would leave its own elements unscaled (and scale the other's twice); empty tensors and tensors
+    of two chunks among them."""
     print(f"{n} tensors", flush=True)
     sizes = [(3, 0, 16385, 2048, 2049)[i % 5] if n <= 129 else (3, 0, 9)[i % 3] for i in range(n)]
     g = [torch.randn(s, generator=torch.Generator().manual_seed(i)) for i, s in enumerate(sizes)]

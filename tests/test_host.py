@@ -381,9 +381,13 @@ def test_persistent_tile_handout_model():
     def xcd_remap(pid, nblocks, shift):
         span = XCD_CHUNK << shift
         full = nblocks // span * span
-        if pid >= full:
-            return pid
-        xcd, local = pid & ((1 << shift) - 1), pid >> shift
+        xcds = 1 << shift
+        xcd = pid & (xcds - 1)
+        if pid >= full:  # less than a run per XCD is left: equal runs
+            rest, local = nblocks - full, (pid - full) >> shift
+            each, more = rest >> shift, rest & (xcds - 1)
+            return full + xcd * each + min(xcd, more) + local
+        local = pid >> shift
         return (((local // XCD_CHUNK) << shift) + xcd) * XCD_CHUNK + local % XCD_CHUNK
 
     rng = random.Random(7)
