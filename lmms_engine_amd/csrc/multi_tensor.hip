@@ -78,7 +78,7 @@ struct ChunkRange {
 // The range of workgroup blockIdx.x when every chunk is shared by SUB workgroups (a power of two): chunk blockIdx.x / SUB,
 // piece blockIdx.x % SUB of it.  The kernels that read and write run several workgroups per chunk, because short-lived ones
 // stream better there: the clip scaling four (3 to 6 % over one workgroup making four trips), AdamW eight, one group of eight
-// elements per thread (1.24 G bf16 elements, 17.4 GB: 3357 us with four, 3225 with eight and the search above), or four for lists
+// elements per thread (1.24 G bf16 elements, 17.4 GB: 3304 to 3356 us with four, 3160 to 3291 with eight), or four for lists
 // so long that eight would pass the 2^32 threads of a launch; the read-only norm kernel is faster with one workgroup per chunk
 // (fewer partial sums).
 template <int SUB = 1>
@@ -274,8 +274,8 @@ __global__ void __launch_bounds__(256)
 clip_scale_multi_kernel(const void* const* g_ptrs, const long* numel, const long* chunk_start, int n,
                         const float* total_f32, int norm_dtype, float max_norm) {
     // A norm within the limit leaves every element as it is (x * 1 = x, infinities and NaN included): nothing is read or written.
-    // The coefficient is known on the device only, so the launch stays; without the pass it takes a twentieth of the time (494 M
-    // fp32 elements: a step of 9302 us to 8592; 2.4 G bf16 elements: 46.9 ms to 45.7).
+    // The coefficient is known on the device only, so the launch stays; without the pass it takes 31 us for 494 M fp32 elements
+    // (685 with it) and 131 us for 2.4 G bf16 elements (1705).
     const float coef = clip_coef(*total_f32, norm_dtype, max_norm);
     if (coef == 1.0f) return;
     const ChunkRange r = my_chunk<RW_SUB>(numel, chunk_start, n);
