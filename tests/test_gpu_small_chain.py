@@ -51,6 +51,31 @@ def test_small_chain_is_bitwise_the_tiled_products(env, rows, cols):
             assert torch.equal(got, ref), steps
 
 
+@pytest.mark.parametrize("rows,cols", [(16, 96), (5, 40), (32, 300), (64, 128)])
+def test_small_chain_on_infinities_zeros_and_nan(env, rows, cols):
+    """Zero matrices, an infinity, a NaN, sums of squares past fp32 and values near its smallest: the same values and the same NaN."""
+    print(f"small chain, special values {rows}x{cols}", flush=True)
+    lib, abi, mu = env["lib"], env["abi"], env["mu"]
+    G = torch.randn(7, rows, cols, generator=torch.Generator().manual_seed(rows))
+    G[0] = 0.0
+    G[1, rows // 2, cols // 3] = float("inf")
+    G[2, 0, cols - 1] = float("nan")
+    G[3] *= 1e30
+    G[4] *= 1e-36
+    G[5, :, 1:] = 0.0
+    for g in (G.to(env["dev"]), G.mT.contiguous().to(env["dev"])):
+        for steps in (1, 5):
+            got = mu.fast_newtonschulz(g, steps)
+            abi.check(lib.muon_hip_set_gemm_config(abi.CFG_128_PIPE))
+            try:
+                ref = mu.fast_newtonschulz(g, steps)
+            finally:
+                abi.check(lib.muon_hip_set_gemm_config(abi.CFG_AUTO))
+            torch.cuda.synchronize()
+            assert torch.equal(got.isnan(), ref.isnan()), steps
+            assert torch.equal(got.nan_to_num(nan=0.0).view(torch.int16), ref.nan_to_num(nan=0.0).view(torch.int16)), steps
+
+
 @pytest.mark.parametrize("pdtype", [torch.float32, torch.bfloat16])
 def test_small_chain_in_a_step_is_bitwise_the_tiled_products(env, pdtype):
     """The same through Muon.step, where the chain applies the parameter update itself."""

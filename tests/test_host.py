@@ -233,6 +233,39 @@ def test_geometry_is_whole_tiles_of_a_named_configuration(rows, cols):
         assert geo["Mp"] % geo["tile"] == 0 and geo["Kp"] % geo["tile"] == 0, (cfg, geo)
 
 
+def test_every_tile_lies_in_the_storage_of_its_matrix():
+    """Calls over drawn shapes, under every configuration and on devices of several sizes: none is refused, and no tile of a.X + B.X
+    passes the padded columns or the last block of 256 rows."""
+    import random
+
+    lib, rng = _abi.lib(), random.Random(3)
+
+    def size():
+        return rng.choice([rng.randint(1, 300), rng.randint(1, 9000), 128 * rng.randint(1, 40), 256 * rng.randint(1, 20)])
+
+    for _ in range(1500):
+        shapes = [(size(), size(), rng.choice([1, 2, 7, 20, 200])) for _ in range(rng.choice([1, 2, 8, 16]))]
+        cfg = rng.choice([_abi.CFG_AUTO, _abi.CFG_AUTO, 0, 1, 2, 3, 4, 5])
+        assert lib.muon_hip_set_gemm_config(cfg) == 0
+        try:
+            geo = [_abi.geometry(r, c) for r, c, _ in shapes]
+            for product in ("syrk", "sympoly", "bx_axpy", "bx_axpy_update"):
+                for g, (kernel, height, launch) in zip(geo, _abi.routes(shapes, product, rng.choice([256, 128, 32]))):
+                    if launch < 0:
+                        continue
+                    rows = -(-g["Mp"] // height) * height
+                    width = {_abi.CFG_128_PIPE: 128, _abi.CFG_128_PINGPONG: 128, _abi.CFG_64_DEEP: 64}.get(kernel, 256)
+                    cols = -(-(-(-g["K"] // 128) * 128) // width) * width
+                    if product.startswith("bx"):
+                        assert cols <= g["Kp"], (shapes, cfg, product)
+                    if kernel == _abi.CFG_256_PERSIST and product == "bx_axpy":
+                        assert rows <= -(-g["Mp"] // 256) * 256, (shapes, cfg, product)
+                    else:
+                        assert rows == g["Mp"], (shapes, cfg, product)
+        finally:
+            assert lib.muon_hip_set_gemm_config(_abi.CFG_AUTO) == 0
+
+
 def test_routes_name_the_kernels_of_a_call():
     """The launcher's choice, on a device of 256 compute units: one case for each kernel it chooses between."""
     r = _abi.routes
