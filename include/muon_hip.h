@@ -57,11 +57,14 @@ extern "C" {
 #define MUON_HIP_K_CLIP_SCALE 9
 #define MUON_HIP_K_BX_UPDATE 10 /* the a.X + B.X launch that carries the parameter update in its epilogue */
 #define MUON_HIP_K_SMALL_CHAIN 11 /* normalisation, iterations and update of matrices with a short side of at most 64 */
-#define MUON_HIP_K_COUNT 12
+#define MUON_HIP_K_FLOW_CHAIN 12  /* the iterations and the update of many small matrices in one launch */
+#define MUON_HIP_K_COUNT 13
 
 /* GEMM kernel variants; MUON_HIP_CFG_AUTO picks per kernel, shape and number of tiles.  All feed LDS with direct
  * global->LDS loads (global_load_lds_dwordx4), software pipelined behind the MFMAs. */
 #define MUON_HIP_CFG_AUTO (-1)
+#define MUON_HIP_CFG_STAGED (-2)     /* MUON_HIP_CFG_AUTO with a launch for every product: never the iterations of many small matrices
+                                        in one launch (muon_hip_flow_tiles); for muon_hip_set_gemm_config only */
 #define MUON_HIP_CFG_128_PIPE 0      /* 128x128 tile, 4 waves, 64-column k-tiles, two LDS stages */
 #define MUON_HIP_CFG_256_PIPE 1      /* 256x256 tile, 8 waves, the same pipeline */
 #define MUON_HIP_CFG_256_PINGPONG 2  /* 256x256 tile, two groups of 4 waves alternating memory / MFMA phases */
@@ -156,14 +159,27 @@ int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int 
                         double weight_decay, double beta, int nesterov, int ns_steps, double a, double b, double c,
                         int write_back_grad, void* stream);
 
-/* Which kernels such a call takes on a device of `cus` compute units, one entry per bucket, for the product named by its
- * MUON_HIP_K_ id (syrk, sympoly, bx, bx_update); touches no device.  For tests and measurements. */
+/* Which kernels the products of such a call take on a device of `cus` compute units where they are launched one by one, one entry per
+ * bucket, for the product named by its MUON_HIP_K_ id (syrk, sympoly, bx, bx_update); touches no device.  For tests and
+ * measurements. */
 typedef struct {
     int cfg;    /* MUON_HIP_CFG_256_PERSIST: the persistent kernel; otherwise the configuration of the one-tile kernel */
     int height; /* rows of a tile */
     int launch; /* which launch of the stage it goes with; -1: no product, the whole chain runs in one workgroup per matrix */
 } muon_hip_route;
 int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cus, muon_hip_route* out);
+
+/* The tiles of a call whose `steps` iterations run as one launch on a device of `xcds` XCDs, group after group (the matrices of a
+ * group belong to one XCD) in the order in which the workgroups of an XCD take them; update: the call updates parameters.  Writes at
+ * most `capacity` of them; *count is how many there are, 0 for a call whose products are launched one by one.  A tile starts when
+ * `before` tiles of its matrix are finished.  Touches no device; for tests and measurements. */
+typedef struct {
+    int group, bucket, matrix, iteration;
+    int product; /* MUON_HIP_K_SYRK, MUON_HIP_K_SYMPOLY or MUON_HIP_K_BX */
+    int tile, before;
+} muon_hip_flow_tile;
+int muon_hip_flow_tiles(const muon_hip_bucket* buckets, int n, int steps, int update, int xcds, muon_hip_flow_tile* out, long capacity,
+                        long* count);
 
 /* ---- blocked matrices and single GEMM entry points ---------------------------------------
  * The Newton-Schulz operands are kept in blocks of 256 rows x 32 columns (16 KB, 64-byte

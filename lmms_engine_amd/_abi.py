@@ -15,11 +15,12 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmuon_hip.so")
 
 F32, BF16 = 0, 1
+CFG_STAGED = -2
 CFG_AUTO, CFG_128_PIPE, CFG_256_PIPE, CFG_256_PINGPONG, CFG_128_PINGPONG, CFG_256_PERSIST, CFG_64_DEEP = -1, 0, 1, 2, 3, 4, 5
 GEMM_CONFIGS = list(range(4))
 K_MOMENTUM, K_NORMALIZE, K_SYRK, K_SYMPOLY, K_BX, K_UPDATE, K_ADAMW, K_ADAMW_MULTI, K_GRAD_NORM, K_CLIP_SCALE = range(10)
 KERNEL_NAMES = ["momentum_norm", "normalize", "syrk", "sympoly", "bx_axpy", "apply_update", "adamw", "adamw_multi",
-                "grad_norm", "clip_scale", "bx_axpy_update", "small_chain"]
+                "grad_norm", "clip_scale", "bx_axpy_update", "small_chain", "flow_chain"]
 MULTI_CHUNK = 16384  # MUON_HIP_MULTI_CHUNK
 STATIC_MAX_CHUNKS = 1 << 20  # MUON_HIP_STATIC_MAX_CHUNKS
 PPX_COUNTER_BYTES = 576  # MUON_HIP_PPX_COUNTER_BYTES
@@ -38,6 +39,12 @@ class Route(ctypes.Structure):
     """muon_hip_route"""
 
     _fields_ = [("cfg", c_int), ("height", c_int), ("launch", c_int)]
+
+
+class FlowTile(ctypes.Structure):
+    """muon_hip_flow_tile"""
+
+    _fields_ = [(f, c_int) for f in ("group", "bucket", "matrix", "iteration", "product", "tile", "before")]
 
 
 # name -> (restype, argtypes); mirrors include/muon_hip.h one to one
@@ -61,6 +68,7 @@ SIGNATURES = {
     "muon_hip_step_multi": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_double, c_double, c_double, c_int, c_int,
                                     c_double, c_double, c_double, c_int, c_void_p]),
     "muon_hip_routes": (c_int, [c_void_p, c_int, c_int, c_int, c_void_p]),
+    "muon_hip_flow_tiles": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_long, POINTER(c_long)]),
     "muon_hip_blocked_elems": (c_long, [c_int, c_int]),
     "muon_hip_pack_bf16": (c_int, [c_void_p, c_long, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int, c_void_p]),
     "muon_hip_unpack_bf16": (c_int, [c_void_p, c_int, c_int, c_void_p, c_long, c_int, c_int, c_int, c_int, c_void_p]),
@@ -149,6 +157,17 @@ def routes(shapes, kernel: str, cus: int = 256):
     out = (Route * len(shapes))()
     check(lib().muon_hip_routes(buckets, len(shapes), KERNEL_NAMES.index(kernel), cus, out), "routes")
     return [(r.cfg, r.height, r.launch) for r in out]
+
+
+def flow_tiles(shapes, steps: int, update: bool, xcds: int = 8):
+    """The tiles of the (rows, cols, matrices) of one call whose iterations run as one launch, as FlowTile; empty where they do not."""
+    buckets = (Bucket * len(shapes))(*[Bucket(rows=r, cols=c, batch=n) for r, c, n in shapes])
+    count = c_long()
+    args = (buckets, len(shapes), int(steps), int(update), int(xcds))
+    check(lib().muon_hip_flow_tiles(*args, None, 0, ctypes.byref(count)), "flow_tiles")
+    out = (FlowTile * count.value)()
+    check(lib().muon_hip_flow_tiles(*args, out, count.value, ctypes.byref(count)), "flow_tiles")
+    return list(out)
 
 
 def device_shape():

@@ -100,7 +100,7 @@ struct Plan {
     bool transposed;
     bool small;  // the whole chain runs in one workgroup per matrix (small_chain.hip) instead of as tiled products
     long n, strideU, strideX, strideA;  // elements per matrix: U dense, the others blocked
-    size_t offX[2], offA, offB, offParts, offDenom, offPpx, total;
+    size_t offX[2], offA, offB, offParts, offDenom, offCtr, ctrBytes, total;
 };
 
 inline long round_up(long v, long m) { return (v + m - 1) / m * m; }
@@ -121,7 +121,7 @@ struct Cfg {
 // for those) and for the symmetric products of matrices up to 512 rows.
 Cfg pick_cfg(int M, int epi = EPI_BX) {
     const int forced = g_forced_cfg.load(std::memory_order_relaxed);
-    if (forced != MUON_HIP_CFG_AUTO) return {forced, false};
+    if (forced >= 0) return {forced, false};
     if (!use_tile256(M)) return {GEMM_CFG_128_PINGPONG, true};
     if (epi != EPI_BX && M <= 512) return {GEMM_CFG_128_PINGPONG, true};
     // The persistent kernel where the launcher takes it: a.X + B.X, and the symmetric products with reductions of at
@@ -130,6 +130,9 @@ Cfg pick_cfg(int M, int epi = EPI_BX) {
     // update run the one-tile ping-pong kernel.
     return {GEMM_CFG_256_PERSIST, true};
 }
+
+// Where the counters of a bucket lie in their segment of its workspace.
+constexpr size_t kCtrFlow = GEMM_PPX_COUNTER_BYTES, kCtrMatrix = kCtrFlow + GEMM_FLOW_CONTROL_BYTES;
 
 int make_plan(int rows, int cols, int batch, Plan& p) {
     if (rows <= 0 || cols <= 0 || batch <= 0) return fail(MUON_HIP_EINVAL, "rows, cols and batch must be positive");
@@ -170,7 +173,9 @@ int make_plan(int rows, int cols, int batch, Plan& p) {
     p.offB = seg(ab);
     p.offParts = seg((size_t)batch * p.nparts * sizeof(float));
     p.offDenom = seg((size_t)batch * sizeof(float));
-    p.offPpx = seg(GEMM_PPX_COUNTER_BYTES);  // tile counters of the persistent kernels: cleared by the normalisation stage
+    // counters, cleared by the normalisation stage: of the persistent kernels, of the chain in one launch, one line per matrix
+    p.ctrBytes = kCtrMatrix + (size_t)batch * GEMM_FLOW_LINE * sizeof(unsigned);
+    p.offCtr = seg(p.ctrBytes);
     p.total = off;
     return 0;
 }
@@ -311,10 +316,12 @@ struct Bucket {
         ws = (char*)workspace;
         return make_plan(rows, cols, batch, p);
     }
+    size_t clear_bytes = 0;  // counters that the normalisation clears
     bf16_t* at(size_t off) const { return (bf16_t*)(ws + off); }
+    unsigned* counters(size_t off) const { return (unsigned*)(ws + p.offCtr + off); }
     EwBucket ew() const {
         return EwBucket{g_ptrs, m_ptrs, at(p.offX[1]), p.strideU, (float*)(ws + p.offParts), (float*)(ws + p.offDenom), at(p.offX[0]),
-                        p.strideX, p.rows, p.cols, p.Mp, p.Kp, p.nparts, p.batch};
+                        p.strideX, p.rows, p.cols, p.Mp, p.Kp, p.nparts, p.batch, counters(0), (int)(clear_bytes / sizeof(unsigned))};
     }
 };
 struct Work {
@@ -348,13 +355,14 @@ int do_momentum(const Work& w, int g_dtype, int m_dtype, double beta, int nester
 }
 
 // The tile counters of the persistent kernels are those of the first bucket; the normalisation clears them.
-unsigned* ppx_counters(const Work& w) { return (unsigned*)(w.b[0].ws + w.b[0].p.offPpx); }
+unsigned* ppx_counters(const Work& w) { return w.b[0].counters(0); }
 
-int do_normalize(const Work& w, hipStream_t s) {
+int do_normalize(Work& w, bool flow, hipStream_t s) {
+    for (int i = 0; i < w.n; ++i) w.b[i].clear_bytes = flow ? w.b[i].p.ctrBytes : i == 0 ? kCtrFlow : 0;
     EwList l;
     ew_list(w, l);
     Timed t(MUON_HIP_K_NORMALIZE, s);
-    hipError_t e = launch_normalize(l, ppx_counters(w), (int)(GEMM_PPX_COUNTER_BYTES / sizeof(unsigned)), s);
+    hipError_t e = launch_normalize(l, s);
     return e == hipSuccess ? 0 : hip_fail(e, "normalize launch");
 }
 
@@ -372,6 +380,40 @@ bool stage_items(const Work& w, int epi, int cur, double a, double b, double c, 
         else items[i] = bx_item(cfg.id, k.at(p.offB), k.at(p.offX[cur]), k.at(p.offX[cur ^ 1]), p.Mp, p.Kr, p.Kp, p.batch, a, ppx);
     }
     return adapt;
+}
+
+// The iterations as one launch (gemm_nt.h), where that is the faster way and nobody has named a configuration.
+bool flow_of(const Work& w, int steps, double a, double b, double c, const UpdateArgs* upd, int xcds, FlowList& l) {
+    if (g_forced_cfg.load(std::memory_order_relaxed) != MUON_HIP_CFG_AUTO) return false;
+    l.n = w.n;
+    l.steps = steps;
+    l.a = (float)a;
+    l.b = (float)b;
+    l.c = (float)c;
+    l.p_dtype = upd ? upd->p_dtype : 0;
+    l.decay = upd ? (float)(1.0 - upd->lr * upd->weight_decay) : 0.f;
+    l.alpha = upd ? (float)(-upd->lr) : 0.f;
+    l.control = w.b[0].counters(kCtrFlow);
+    for (int i = 0; i < w.n; ++i) {
+        const Bucket& k = w.b[i];
+        const Plan& p = k.p;
+        FlowEntry& e = l.e[i];
+        for (int x : {0, 1}) e.X[x] = k.at(p.offX[x]);
+        e.A = k.at(p.offA);
+        e.B = k.at(p.offB);
+        e.strideX = p.strideX;
+        e.strideA = p.strideA;
+        e.Mp = p.Mp;
+        e.Kr = p.Kr;
+        e.Kp = p.Kp;
+        e.batch = p.batch;
+        e.done = k.counters(kCtrMatrix);
+        e.p_ptrs = upd ? k.p_ptrs : nullptr;
+        e.rows = p.rows;
+        e.cols = p.cols;
+        e.scale = (float)k.scale;
+    }
+    return plan_flow(l, xcds);
 }
 
 // Normalise, then `steps` iterations; with `upd` the last B.X applies the parameter update instead of writing X'.
@@ -404,7 +446,16 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
     } else {
         w = all;
     }
-    if (int rc = do_normalize(w, s)) return rc;
+    FlowList fl;
+    MachineShape ms;
+    if (hipError_t e = machine_shape(ms); e != hipSuccess) return hip_fail(e, "device shape");
+    const bool flow = steps > 0 && flow_of(w, steps, a, b, c, upd, 1 << ms.xcd_shift, fl);
+    if (int rc = do_normalize(w, flow, s)) return rc;
+    if (flow) {
+        Timed t(MUON_HIP_K_FLOW_CHAIN, s);
+        hipError_t e = launch_flow(fl, s);
+        return e == hipSuccess ? 0 : hip_fail(e, "ns_flow launch");
+    }
     unsigned* ppx = ppx_counters(w);
     GemmItem items[MUON_HIP_MAX_BUCKETS];
     for (int it = 0; it < steps; ++it) {
@@ -431,7 +482,7 @@ int muon_hip_version(void) { return 100; }
 const char* muon_hip_last_error(void) { return g_err; }
 
 int muon_hip_set_gemm_config(int cfg) {
-    if (cfg != MUON_HIP_CFG_AUTO && gemm_cfg_tile(cfg) == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration %d", cfg);
+    if (cfg != MUON_HIP_CFG_AUTO && cfg != MUON_HIP_CFG_STAGED && gemm_cfg_tile(cfg) == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration %d", cfg);
     g_forced_cfg.store(cfg, std::memory_order_relaxed);
     return 0;
 }
@@ -478,7 +529,7 @@ int muon_hip_cast_norm(const void* G, int g_dtype, void* workspace, int rows, in
 int muon_hip_normalize(void* workspace, int rows, int cols, int batch, void* stream) {
     Work w;
     if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
-    return do_normalize(w, (hipStream_t)stream);
+    return do_normalize(w, false, (hipStream_t)stream);
 }
 
 int muon_hip_ns_grouped(void* workspace, int rows, int cols, int batch, int steps, double a, double b, double c,
@@ -568,6 +619,33 @@ int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cu
         for (int i = 0; i < w.n; ++i) fold_update(items[i], nullptr, w.b[i].p.rows, w.b[i].p.cols, 1.0, UpdateArgs{});
     if (plan_gemm_nt(items, w.n, adapt, cus, route) < 0) return fail(MUON_HIP_EINVAL, "no kernel takes these products");
     for (int i = 0; i < w.n; ++i) out[from[i]] = muon_hip_route{route[i].cfg, route[i].height, route[i].launch};
+    return 0;
+}
+
+int muon_hip_flow_tiles(const muon_hip_bucket* buckets, int n, int steps, int update, int xcds, muon_hip_flow_tile* out, long capacity,
+                        long* count) {
+    if (!buckets || !count || n < 1 || n > MUON_HIP_MAX_BUCKETS || capacity < 0 || (capacity && !out) || steps < 0 || xcds < 1 || xcds > GEMM_MAX_XCDS)
+        return fail(MUON_HIP_EINVAL, "bad bucket list, steps, XCDs or output");
+    *count = 0;
+    Work w;
+    int from[MUON_HIP_MAX_BUCKETS];
+    alignas(256) static char nowhere[256];  // as in muon_hip_routes
+    for (int i = 0; i < n; ++i) {
+        Bucket& k = w.b[w.n];
+        if (int rc = k.init(buckets[i].rows, buckets[i].cols, buckets[i].batch, nowhere)) return rc;
+        k.p_ptrs = (const void* const*)nowhere;
+        if (!k.p.small) from[w.n++] = i;
+    }
+    FlowList l;
+    const UpdateArgs u{};
+    if (!w.n || steps == 0 || !flow_of(w, steps, 1.0, 1.0, 1.0, update ? &u : nullptr, xcds, l)) return 0;
+    for (int g = 0; g < l.groups; ++g)
+        for (int t = 0; t < flow_tiles(l, g); ++t, ++*count) {
+            if (*count >= capacity) continue;
+            const FlowPlace p = flow_place(l, g, t);
+            const int product = p.stage == 0 ? MUON_HIP_K_SYRK : p.stage == 1 ? MUON_HIP_K_SYMPOLY : MUON_HIP_K_BX;
+            out[*count] = muon_hip_flow_tile{g, from[p.entry], p.matrix, p.it, product, p.tile, p.before};
+        }
     return 0;
 }
 

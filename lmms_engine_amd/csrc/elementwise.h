@@ -20,6 +20,8 @@ struct EwBucket {
     bf16_t* X;                  // the normalised operand, blocked, Mp x Kp
     long strideX;
     int rows, cols, Mp, Kp, nparts, batch;
+    unsigned* clear;            // clear_words words that the normalisation clears: counters of the products that follow on the stream
+    int clear_words;
     bool inline_norm;           // set by the launcher: the normalisation adds the partial sums itself, denom stays unset
 };
 constexpr int EW_MAX_LIST = 16;
@@ -31,8 +33,7 @@ struct EwList {
 hipError_t launch_momentum_norm(EwList& l, int g_dtype, int m_dtype, double beta, int nesterov, int write_back, hipStream_t stream);
 hipError_t launch_cast_norm(const void* G, long strideG, int g_dtype, bf16_t* U, long strideU, float* partials,
                             int nparts, long n, int batch, hipStream_t stream);
-// Also clears `clear_words` words at `clear` (the tile counters of the persistent GEMM kernels that follow on the stream).
-hipError_t launch_normalize(EwList& l, unsigned* clear, int clear_words, hipStream_t stream);
+hipError_t launch_normalize(EwList& l, hipStream_t stream);
 hipError_t launch_apply_update(const void* const* p_ptrs, int p_dtype, const bf16_t* O, long strideO, int cbo,
                                int rows, int cols, int batch, double scale, double lr, double wd,
                                hipStream_t stream);

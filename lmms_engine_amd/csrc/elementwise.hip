@@ -248,14 +248,14 @@ __global__ void __launch_bounds__(256) frob_finalize_kernel(const EwList l) {
 // as 128 rows of X, 32 elements each (the 64-byte rows of one column block, back to back).  32 x 128 measured best of
 // {32, 64} x {64, 128}: 5.5 to 5.7 TB/s against 5.2 to 5.5 for 64 x 128.
 constexpr int NORM_TR = 16, NORM_T_TR = 32, NORM_TC = 128;
-__global__ void __launch_bounds__(256) normalize_kernel(const EwList l, unsigned* clear, int clear_words) {
+__global__ void __launch_bounds__(256) normalize_kernel(const EwList l) {
     constexpr int TC = NORM_TC, TR = NORM_T_TR, PITCH = TC + 8;
     __shared__ __align__(16) bf16_t tile[TR][PITCH];
     __shared__ float red[4];
-    if (blockIdx.x == 0)
-        for (int i = threadIdx.x; i < clear_words; i += 256) clear[i] = 0u;
     const int bucket = list_bucket(l, blockIdx.x);
     const EwBucket& e = l.b[bucket];
+    if ((int)blockIdx.x == l.start[bucket])
+        for (int i = threadIdx.x; i < e.clear_words; i += 256) e.clear[i] = 0u;
     const int rows = e.rows, cols = e.cols, cbx = e.Kp / BLK_COLS;
     const bool vec = (cols % 8) == 0, turn = rows > cols;
     // u's padded image is Mp x Kp, or Kp x Mp when it is turned; both are whole 128-tiles
@@ -634,7 +634,7 @@ hipError_t launch_cast_norm(const void* G, long strideG, int g_dtype, bf16_t* U,
     return hipGetLastError();
 }
 
-hipError_t launch_normalize(EwList& l, unsigned* clear, int clear_words, hipStream_t stream) {
+hipError_t launch_normalize(EwList& l, hipStream_t stream) {
     EwList f;  // the matrices with too many partial sums for every workgroup to add
     f.n = 0;
     f.start[0] = 0;
@@ -651,7 +651,7 @@ hipError_t launch_normalize(EwList& l, unsigned* clear, int clear_words, hipStre
         }
     }
     if (f.n) hipLaunchKernelGGL(frob_finalize_kernel, dim3(f.start[f.n]), dim3(256), 0, stream, f);
-    hipLaunchKernelGGL(normalize_kernel, dim3(l.start[l.n]), dim3(256), 0, stream, l, clear, clear_words);
+    hipLaunchKernelGGL(normalize_kernel, dim3(l.start[l.n]), dim3(256), 0, stream, l);
     return hipGetLastError();
 }
 

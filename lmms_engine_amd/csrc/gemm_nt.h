@@ -97,3 +97,63 @@ struct GemmRoute {
     int cfg, height, launch;
 };
 int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* route);
+
+// The chain of many small matrices as one launch (gemm_nt_flow_kernel): every matrix belongs to one of `groups` groups, each of
+// which runs on one XCD.  Matrices first[g] .. first[g + 1] - 1 of an entry are those of group g.
+constexpr int GEMM_MAX_XCC_IDS = 16;                                       // values the hardware's XCD number can take
+constexpr int GEMM_FLOW_LINE = 16;                                         // words between the counters of two matrices
+constexpr size_t GEMM_FLOW_CONTROL_BYTES = (GEMM_MAX_XCDS + GEMM_MAX_XCC_IDS + 2) * 16 * sizeof(unsigned);
+struct FlowEntry {
+    bf16_t* X[2];              // iteration i reads X[i & 1] and writes the other; blocked, Mp x Kp
+    bf16_t *A, *B;             // Mp x Mp
+    long strideX, strideA;
+    int Mp, Kr, Kp, batch;     // as GemmArgs: Kr columns in whole 128-tiles of storage for Kp
+    unsigned* done;            // a counter per matrix, GEMM_FLOW_LINE words apart, zero before the launch
+    const void* const* p_ptrs; // device table of the parameters to update; null: the last iteration writes X'
+    int rows, cols;            // of the parameter
+    float scale;
+    int sym, rect;             // 128-tiles of a matrix: of a symmetric product, of a.X + B.X
+    int first[GEMM_MAX_XCDS + 1];
+};
+struct FlowList {
+    int n, groups, steps, p_dtype;
+    float a, b, c, decay, alpha;
+    unsigned* control;         // GEMM_FLOW_CONTROL_BYTES, zero before the launch
+    int sym[GEMM_MAX_XCDS], rect[GEMM_MAX_XCDS];  // per group: tiles of each symmetric product, of a.X + B.X
+    FlowEntry e[GEMM_MAX_LIST];
+};
+static_assert(sizeof(FlowList) <= 4096, "kernel arguments");
+
+// Tiles of a group are numbered by iteration, product (0 X.Xt, 1 b.A + c.A.A, 2 a.X + B.X), entry, matrix and place in the product.
+// Tile t of group g, and how many tiles of its matrix come before its product: all of them have to be finished first.
+struct FlowPlace {
+    int entry, matrix, tile, stage, it, before;
+};
+__host__ __device__ inline int flow_tiles(const FlowList& l, int g) { return l.steps * (2 * l.sym[g] + l.rect[g]); }
+__host__ __device__ inline FlowPlace flow_place(const FlowList& l, int g, int t) {
+    FlowPlace p;
+    const int sym = l.sym[g], each_it = 2 * sym + l.rect[g];
+    p.it = t / each_it;
+    t -= p.it * each_it;
+    p.stage = t < sym ? 0 : t < 2 * sym ? 1 : 2;
+    t -= p.stage * sym;
+    int each = 1;
+    for (p.entry = 0;; ++p.entry) {
+        const FlowEntry& e = l.e[p.entry];
+        each = p.stage == 2 ? e.rect : e.sym;
+        const int here = (e.first[g + 1] - e.first[g]) * each;
+        if (t < here || p.entry == l.n - 1) break;
+        t -= here;
+    }
+    const FlowEntry& e = l.e[p.entry];
+    const int m = t / each;
+    p.matrix = e.first[g] + m;
+    p.tile = t - m * each;
+    p.before = p.it * (2 * e.sym + e.rect) + p.stage * e.sym;
+    return p;
+}
+
+// Deals the matrices of l.e[0 .. l.n) to the XCDs (fills groups, sym and rect, here and in the entries, and every first); false where
+// launches of their own are the faster way.  Touches no device.
+bool plan_flow(FlowList& l, int xcds);
+hipError_t launch_flow(const FlowList& l, hipStream_t stream);

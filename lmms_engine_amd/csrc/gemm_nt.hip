@@ -22,6 +22,7 @@
 // Operands and results live in the blocked layout of common.h (256 x 32 blocks), zero padded
 // by the producers to whole tiles, so there is no masking here; the host launcher checks that
 // the shapes it is given are whole tiles before launching.
+#include <algorithm>
 #include <atomic>
 #include <type_traits>
 
@@ -96,6 +97,30 @@ __device__ __forceinline__ int list_entry(const GemmList& l, int logical) {
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
 typedef const __attribute__((address_space(1))) void* glb_void_ptr;
 
+// The thread's number.  COH: in a form that the compiler cannot take out of the loop over tiles, with everything that each kind of
+// tile computes from it (which it did, and spilled).
+template <bool COH>
+__device__ __forceinline__ int thread_number() {
+    int t = threadIdx.x;
+    if constexpr (COH) asm volatile("" : "+v"(t));
+    return t;
+}
+
+// 16 bytes at base + off elements.  COH: read at device scope, past this compute unit's vector cache, which may still hold what
+// the address contained before another compute unit of the same launch wrote it (gemm_nt_flow_kernel).
+typedef unsigned u32x4a __attribute__((ext_vector_type(4)));
+template <bool COH>
+__device__ __forceinline__ bf16x8 load16(const bf16_t* base, long off) {
+    if constexpr (COH) {
+        constexpr int kDeviceScope = 16;  // sc1
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, 0xffffffffu, 0x00027000);
+        const u32x4a v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)(off * 2), 0, kDeviceScope);
+        return *(const bf16x8*)&v;
+    } else {
+        return *(const bf16x8*)(base + off);
+    }
+}
+
 #define WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(0xC07F)
 // s_waitcnt with only vmcnt set: vmcnt is split over bits [3:0] and [15:14] (N < 64)
 #define WAIT_VM(N) __builtin_amdgcn_s_waitcnt(0x0F70 | ((N) & 15) | (((N) >> 4) << 14))
@@ -129,16 +154,24 @@ __device__ __forceinline__ s16x4 lds_read_tr16(const unsigned char* p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(lds_void_ptr)p);
 }
 
-template <int BM, int BN, int WGM, int WGN, int EPI, bool MASKED>
+//
+// The epilogues come in two parts: EPI_LOADS fetches the elementwise term into `ev` (16-byte pieces, tile_pieces of them for a
+// thread), EPI_REST does everything else.  On 128-tiles the registers have room for the term beside the accumulators: it is
+// fetched in front of the k loop and its latency passes behind the first k-tiles'.
+enum { EPI_LOADS = 1, EPI_REST = 2, EPI_ALL = 3 };
+template <int BM, int BN, int WGM, int WGN>
+constexpr int tile_pieces() { return BM * BN / 8 / (WGM * WGN * 64); }
+
+template <int BM, int BN, int WGM, int WGN, int EPI, bool MASKED, bool COH, int PART, int NEV>
 __device__ __forceinline__ void epilogue(const GemmArgs& g, const TileCoord& tc,
-                                         f32x4 (&acc)[BM / WGM / 16][BN / WGN / 16], unsigned char* smem) {
+                                         f32x4 (&acc)[BM / WGM / 16][BN / WGN / 16], unsigned char* smem, bf16x8 (&ev)[NEV]) {
     constexpr int NT = WGM * WGN * 64;
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
     constexpr int FM = WTM / 16, FN = WTN / 16;
     constexpr int S = BM * 2 + 16;      // Tt row pitch (bytes): conflict-free for the 8-byte pieces
     constexpr int NLE = BN * (BM / 8) / NT;  // 16-byte chunks per thread for a whole tile
     static_assert((BN * (BM / 8)) % NT == 0 && BM % 64 == 0, "even split");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = thread_number<COH>(), lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WGN, wn = wave % WGN, quad = lane >> 4;
     const int m0 = tc.ti * BM, n0 = tc.tj * BN;
     const bool diag = (!epi_is_bx(EPI)) && (tc.ti == tc.tj);
@@ -158,17 +191,18 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const TileCoord& tc,
     };
     // SYMPOLY: this thread's 16-byte pieces of the b.A term, in the layout of the Ct pass, go to registers
     // first, so that the loads are in flight while the accumulators are rounded into LDS
-    bf16x8 ev[EPI == EPI_SYMPOLY ? NLE : 1];
-    if (EPI == EPI_SYMPOLY) {
+    static_assert(NEV >= (EPI == EPI_SYMPOLY ? NLE : 1), "pieces of the b.A term");
+    if constexpr (EPI == EPI_SYMPOLY && (PART & EPI_LOADS)) {
         const bf16_t* Et = g.Et + tc.bidx * g.strideEt;
 #pragma unroll
         for (int u = 0; u < NLE; ++u) {
             long goff;
             int loff;
             tile_chunk(tid + u * NT, g.cbEt, goff, loff);
-            ev[u] = *(const bf16x8*)(Et + goff);
+            ev[u] = load16<COH>(Et, goff);
         }
     }
+    if constexpr (!(PART & EPI_REST)) return;
     __syncthreads();  // the operand stages are no longer read
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -242,19 +276,20 @@ constexpr int epilogue_nn_bytes() { return BM * (BN * 2 + 16); }
 // Folded parameter update: eight consecutive elements of one parameter row, o = bf16(X' * scale);
 // p <- rnd(p * decay); p <- rnd(p + alpha * o), the arithmetic of the stand-alone update kernel (elementwise.hip).
 // The parameter piece is fetched into registers early (fold_load) and applied after the tile has been through LDS.
+template <bool WHOLE>
 struct FoldPiece {
-    f32x4 lo;  // bf16 parameter: the eight values; fp32 parameter: the first four (the other four are fetched
-               // when the piece is applied, from the cache line that this fetch brought in)
+    f32x4 lo;                 // bf16 parameter: the eight values; fp32 parameter: the first four
+    f32x4 hi[WHOLE ? 1 : 0];  // the other four; without them they are fetched when the piece is applied, from the cache line that
+                              // the fetch of `lo` brought in
 };
-template <typename PT>
-__device__ __forceinline__ FoldPiece fold_load(const PT* p, bool vec, int left) {
-    FoldPiece f;
-    f.lo = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (vec && left >= 8) f.lo = __builtin_nontemporal_load((const f32x4*)p);
-    return f;
+template <typename PT, bool WHOLE>
+__device__ __forceinline__ void fold_load(FoldPiece<WHOLE>& f, const PT* p, bool vec, int left) {
+    if (!vec || left < 8) return;
+    f.lo = __builtin_nontemporal_load((const f32x4*)p);
+    if constexpr (WHOLE && sizeof(PT) == 4) f.hi[0] = __builtin_nontemporal_load((const f32x4*)(p + 4));
 }
-template <typename PT>
-__device__ __forceinline__ void fold_apply(PT* p, const FoldPiece& f, const bf16x8& x, bool vec, int left, const GemmArgs& g) {
+template <typename PT, bool WHOLE>
+__device__ __forceinline__ void fold_apply(PT* p, const FoldPiece<WHOLE>& f, const bf16x8& x, bool vec, int left, const GemmArgs& g) {
     constexpr bool PBF = std::is_same<PT, bf16_t>::value;
     auto one = [&](float pv, bf16_t xv) {
         const float os = rbf(bf2f(xv) * g.upd_scale);
@@ -268,7 +303,9 @@ __device__ __forceinline__ void fold_apply(PT* p, const FoldPiece& f, const bf16
             for (int k = 0; k < 8; ++k) pv[k] = f2bf(one(bf2f(pv[k]), x[k]));
             __builtin_nontemporal_store(pv, (bf16x8*)p);
         } else {
-            f32x4 a = f.lo, b = __builtin_nontemporal_load((const f32x4*)(p + 4));
+            f32x4 a = f.lo, b;
+            if constexpr (WHOLE) b = f.hi[0];
+            else b = __builtin_nontemporal_load((const f32x4*)(p + 4));
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 a[k] = one(a[k], x[k]);
@@ -285,9 +322,11 @@ __device__ __forceinline__ void fold_apply(PT* p, const FoldPiece& f, const bf16
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int FOLD>
-__device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& tc,
-                                            f32x4 (&acc)[BM / WGM / 16][BN / WGN / 16], unsigned char* smem) {
+// pv: the parameter's pieces, fetched with the a.X term.  PRELOAD: they are, with EPI_LOADS; otherwise this part comes later, with
+// the accumulators in LDS.
+template <int BM, int BN, int WGM, int WGN, int FOLD, bool COH, int PART, int NEV, bool PRELOAD, int NPV>
+__device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& tc, f32x4 (&acc)[BM / WGM / 16][BN / WGN / 16],
+                                            unsigned char* smem, bf16x8 (&ev)[NEV], FoldPiece<PRELOAD> (&pv)[NPV]) {
     constexpr int NT = WGM * WGN * 64;
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
     constexpr int FM = WTM / 16, FN = WTN / 16;
@@ -295,7 +334,7 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
     constexpr int CPB = BLK_COLS / 8;        // 16-byte chunks per row of a block
     constexpr int NLE = BM * (BN / 8) / NT;  // 16-byte chunks per thread for a whole tile
     static_assert((BM * (BN / 8)) % NT == 0 && BN % BLK_COLS == 0, "even split");
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = thread_number<COH>(), lane = tid & 63, wave = tid >> 6;
     const int wm = wave / WGN, wn = wave % WGN, quad = lane >> 4;
     const int m0 = tc.ti * BM, n0 = tc.tj * BN;
     // Last iteration of a step, parameter in the orientation of X: the scaled update goes straight into the
@@ -323,14 +362,48 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
         loff = m * S + (cbk * CPB + j) * 16;
     };
     const bf16_t* Et = g.Et + tc.bidx * g.strideEt;
-    bf16x8 ev[NLE];
+    static_assert(NEV == NLE && NPV >= (FOLD ? NLE : 1), "pieces of the tile");
+    if constexpr (PART & EPI_LOADS) {
 #pragma unroll
-    for (int u = 0; u < NLE; ++u) {
-        long goff;
-        int loff;
-        tile_chunk(tid + u * NT, g.cbEt, goff, loff);
-        ev[u] = *(const bf16x8*)(Et + goff);
+        for (int u = 0; u < NLE; ++u) {
+            long goff;
+            int loff;
+            tile_chunk(tid + u * NT, g.cbEt, goff, loff);
+            ev[u] = load16<COH>(Et, goff);
+        }
     }
+    // FOLD: the parameter, and this thread's piece u of the tile in it
+    void* pbase = FOLD ? const_cast<void*>(g.upd_ptrs[tc.bidx]) : nullptr;
+    const bool pvec = (g.upd_cols % 8 == 0) && ((((uintptr_t)pbase) & 15) == 0);
+    const bool pbf = g.upd_dtype == MUON_HIP_BF16;
+    constexpr int NSTRIP = BM / 128, NWV = NT / 64;
+    const int grp = lane >> 4, i16 = lane & 15;
+    auto piece = [&](int u, long& poff, int& left) {
+        int row, col;
+        if constexpr (FOLD == 2) {
+            const int wu = wave + u * NWV, strip = wu % NSTRIP, c = wu / NSTRIP;
+            row = n0 + c * 4 + (i16 & 3), col = m0 + strip * 128 + grp * 32 + (i16 >> 2) * 8;
+        } else {
+            int j, m, cbk;
+            decode(tid + u * NT, j, m, cbk);
+            row = m0 + m, col = n0 + cbk * BLK_COLS + j * 8;
+        }
+        poff = (long)row * g.upd_cols + col;
+        left = g.upd_cols - col;
+        return row < g.upd_rows && left > 0;
+    };
+    auto load_param = [&]() {
+#pragma unroll
+        for (int u = 0; u < NLE; ++u) {
+            long poff;
+            int left;
+            if (!piece(u, poff, left)) continue;
+            if (pbf) fold_load(pv[u], (const bf16_t*)pbase + poff, pvec, left);
+            else fold_load(pv[u], (const float*)pbase + poff, pvec, left);
+        }
+    };
+    if constexpr (FOLD && PRELOAD && (PART & EPI_LOADS)) load_param();
+    if constexpr (!(PART & EPI_REST)) return;
     __syncthreads();  // the operand stages are no longer read
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -363,28 +436,9 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
         // ds_read_b64_tr_b16 (the gather of the symmetric epilogue): lane i16 of a group of 16 receives
         // T[m .. m+7][4c + i16 % 4] with m = strip * 128 + grp * 32 + (i16 / 4) * 8, i.e. 16 bytes of row 4c + i16 % 4
         // of the parameter tile; a wave instruction covers 4 parameter rows x 128 columns.
-        constexpr int NSTRIP = BM / 128, NQUAD = BN / 4, NWV = NT / 64;
-        constexpr int NUNIT = NSTRIP * NQUAD / NWV;
-        static_assert(BM % 128 == 0 && (NSTRIP * NQUAD) % NWV == 0, "whole 128-row strips per wave");
-        void* pbase = const_cast<void*>(g.upd_ptrs[tc.bidx]);
-        const bool pvec = (g.upd_cols % 8 == 0) && ((((uintptr_t)pbase) & 15) == 0);
-        const bool pbf = g.upd_dtype == MUON_HIP_BF16;
-        const int grp = lane >> 4, i16 = lane & 15;
-        auto piece = [&](int u, long& poff, int& left) {
-            const int wu = wave + u * NWV, strip = wu % NSTRIP, c = wu / NSTRIP;
-            const int row = n0 + c * 4 + (i16 & 3), col = m0 + strip * 128 + grp * 32 + (i16 >> 2) * 8;
-            poff = (long)row * g.upd_cols + col;
-            left = g.upd_cols - col;
-            return row < g.upd_rows && left > 0;
-        };
-        FoldPiece pv[NUNIT];
-#pragma unroll
-        for (int u = 0; u < NUNIT; ++u) {
-            long poff;
-            int left;
-            if (piece(u, poff, left))
-                pv[u] = pbf ? fold_load<bf16_t>((const bf16_t*)pbase + poff, pvec, left) : fold_load<float>((const float*)pbase + poff, pvec, left);
-        }
+        constexpr int NQUAD = BN / 4, NUNIT = NSTRIP * NQUAD / NWV;
+        static_assert(BM % 128 == 0 && NUNIT * NWV == NSTRIP * NQUAD && NUNIT == NLE, "whole 128-row strips per wave");
+        if constexpr (!PRELOAD) load_param();
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < NLE; ++u) {
@@ -410,47 +464,28 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
             int left;
             if (piece(u, poff, left)) {
                 const bf16x8 o = *(const bf16x8*)&t8;
-                if (pbf) fold_apply<bf16_t>((bf16_t*)pbase + poff, pv[u], o, pvec, left, g);
-                else fold_apply<float>((float*)pbase + poff, pv[u], o, pvec, left, g);
+                if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, pvec, left, g);
+                else fold_apply((float*)pbase + poff, pv[u], o, pvec, left, g);
             }
         }
         return;
     }
-    void* pbase = const_cast<void*>(g.upd_ptrs[tc.bidx]);
-    const bool pvec = (g.upd_cols % 8 == 0) && ((((uintptr_t)pbase) & 15) == 0);
-    const bool pbf = g.upd_dtype == MUON_HIP_BF16;
     // The parameter pieces are fetched here, with the accumulators already in LDS, so that their latency passes
     // behind the barrier.
-    auto piece = [&](int c, long& poff, int& left) {
-        int j, m, cbk;
-        decode(c, j, m, cbk);
-        const int row = m0 + m, col = n0 + cbk * BLK_COLS + j * 8;
-        poff = (long)row * g.upd_cols + col;
-        left = g.upd_cols - col;
-        return row < g.upd_rows && left > 0;
-    };
-    FoldPiece pv[NLE];
-#pragma unroll
-    for (int u = 0; u < NLE; ++u) {
-        long poff;
-        int left;
-        if (piece(tid + u * NT, poff, left))
-            pv[u] = pbf ? fold_load<bf16_t>((const bf16_t*)pbase + poff, pvec, left) : fold_load<float>((const float*)pbase + poff, pvec, left);
-    }
+    if constexpr (!PRELOAD) load_param();
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < NLE; ++u) {
         long goff, poff;
         int loff, left;
-        const int c = tid + u * NT;
-        tile_chunk(c, g.cbC, goff, loff);
+        tile_chunk(tid + u * NT, g.cbC, goff, loff);
         const bf16x8 t = *(const bf16x8*)(smem + loff);
         bf16x8 o;
 #pragma unroll
         for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[u][k])) + bf2f(t[k]));
-        if (piece(c, poff, left)) {
-            if (pbf) fold_apply<bf16_t>((bf16_t*)pbase + poff, pv[u], o, pvec, left, g);
-            else fold_apply<float>((float*)pbase + poff, pv[u], o, pvec, left, g);
+        if (piece(u, poff, left)) {
+            if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, pvec, left, g);
+            else fold_apply((float*)pbase + poff, pv[u], o, pvec, left, g);
         }
     }
 }
@@ -471,24 +506,29 @@ __device__ __forceinline__ unsigned pack_bf16x2(float a, float b) {
 // SPLIT: rows of the tile that the first of its two wave rows holds.  The wave rows may differ (variable-height tiles of the
 // persistent kernel).  FMU: fragment rows this wave holds.  IN_BLOCK: the tile lies inside one row block, so that fragment rows
 // are instruction offsets apart; otherwise each is addressed on its own, with scalar arithmetic.
-template <int BN, int WGN, int SPLIT, int FMU, bool IN_BLOCK, int FM, int FN>
-__device__ __forceinline__ void epilogue_nn_reg(const GemmArgs& g, int bidx, int m0, int n0, f32x4 (&acc)[FM][FN]) {
+template <int BN, int WGN, int SPLIT, int FMU, bool IN_BLOCK, bool COH, int PART, int FM, int FN, int NEV>
+__device__ __forceinline__ void epilogue_nn_reg(const GemmArgs& g, int bidx, int m0, int n0, f32x4 (&acc)[FM][FN], bf16x8 (&ev)[NEV]) {
     constexpr int WTN = BN / WGN;
     static_assert(FN % 2 == 0 && FN * 16 == WTN && BLK_COLS == 32, "a pair of fragments is one column block");
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tid = thread_number<COH>(), lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN, row = lane >> 4;
     // piece (i, t): row m0 + wm*SPLIT + 16 i + lane%16, columns n0 + wn*WTN + 32 t + 16 (row & 1) + 8 (row >> 1) .. + 7
     const int lane_off = (lane & 15) * BLK_COLS + (row & 1) * 16 + (row >> 1) * 8;
     const int m = m0 + wm * SPLIT;
     auto at = [&](int i, int cb) { return IN_BLOCK ? panel_offset(m, cb) + i * 16 * BLK_COLS : panel_offset(m + i * 16, cb); };
-    const bf16_t* Et = g.Et + bidx * g.strideEt + (long)((n0 >> BLK_SHIFT) + wn * (WTN / 32)) * BLK_ELEMS + lane_off;
+    const long et_off = (long)((n0 >> BLK_SHIFT) + wn * (WTN / 32)) * BLK_ELEMS + lane_off;
+    const bf16_t* Et = g.Et + bidx * g.strideEt + (COH ? 0 : et_off);  // (COH: the same in every lane)
     bf16_t* C = g.C + bidx * g.strideC + (long)((n0 >> BLK_SHIFT) + wn * (WTN / 32)) * BLK_ELEMS + lane_off;
-    bf16x8 ev[FMU][FN / 2];
+    static_assert(NEV >= FMU * (FN / 2), "pieces of the a.X term");
+    if constexpr (PART & EPI_LOADS) {
 #pragma unroll
-    for (int i = 0; i < FMU; ++i)
+        for (int i = 0; i < FMU; ++i)
 #pragma unroll
-        for (int t = 0; t < FN / 2; ++t) ev[i][t] = *(const bf16x8*)(Et + at(i, g.cbEt) + (long)t * BLK_ELEMS);
+            for (int t = 0; t < FN / 2; ++t) 
+                ev[i * (FN / 2) + t] = load16<COH>(Et, (COH ? et_off : 0) + at(i, g.cbEt) + (long)t * BLK_ELEMS);
+    }
+    if constexpr (!(PART & EPI_REST)) return;
 #pragma unroll
     for (int i = 0; i < FMU; ++i)
 #pragma unroll
@@ -500,7 +540,7 @@ __device__ __forceinline__ void epilogue_nn_reg(const GemmArgs& g, int bidx, int
             const bf16x8 tv = *(const bf16x8*)&tw;
             bf16x8 o;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[i][t][k])) + bf2f(tv[k]));
+            for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[i * (FN / 2) + t][k])) + bf2f(tv[k]));
             *(bf16x8*)(C + at(i, g.cbC) + (long)t * BLK_ELEMS) = o;
         }
 }
@@ -525,15 +565,15 @@ __device__ __forceinline__ void quad_transpose_b16(unsigned& p0, unsigned& p1, u
     p0 = upper ? recv : p0;
     p1 = upper ? p1 : recv;
 }
-template <int BM, int BN, int WGM, int WGN, int EPI, unsigned MASK = 0>
+template <int BM, int BN, int WGM, int WGN, int EPI, unsigned MASK, bool COH, int PART, int NEV>
 __device__ __forceinline__ void epilogue_sym_reg(const GemmArgs& g, const TileCoord& tc,
-                                                 f32x4 (&acc)[BM / WGM / 16][BN / WGN / 16]) {
+                                                 f32x4 (&acc)[BM / WGM / 16][BN / WGN / 16], bf16x8 (&ev)[NEV]) {
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
     constexpr int FM = WTM / 16, FN = WTN / 16;
     static_assert(FM % 2 == 0 && FN % 2 == 0 && BLK_COLS == 32, "a pair of fragments is one column block");
     static_assert(EPI == EPI_SYRK || EPI == EPI_SYMPOLY, "symmetric products");
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tid = thread_number<COH>(), lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN, row = lane >> 4;
     const int m0 = tc.ti * BM, n0 = tc.tj * BN;
     const bool diag = tc.ti == tc.tj;
@@ -548,17 +588,18 @@ __device__ __forceinline__ void epilogue_sym_reg(const GemmArgs& g, const TileCo
     const bool upper = (lane & 2) != 0;
     // SYMPOLY: the b.A pieces of EV_AHEAD rows of pairs are in flight at a time; those of row t + EV_AHEAD are fetched
     // when row t starts (all of them at once do not fit beside the accumulators in the persistent kernel)
-    bf16x8 ev[EPI == EPI_SYMPOLY ? FM / 2 : 1][EPI == EPI_SYMPOLY ? FN : 1];
-    const bf16_t* Et = g.Et + tc.bidx * g.strideEt + panel_offset(n0, g.cbEt) + ct_off;
-    constexpr int EV_AHEAD = 2 < FM / 2 ? 2 : FM / 2;  // measured: 3 no faster, 4 spills an accumulator fragment
+    static_assert(NEV >= (EPI == EPI_SYMPOLY ? FM / 2 * FN : 1), "pieces of the b.A term");
+    const bf16_t* Et = g.Et + tc.bidx * g.strideEt + panel_offset(n0, g.cbEt) + (COH ? 0 : ct_off);  // (COH: the same in every lane)
+    constexpr int EV_AHEAD = PART == EPI_REST ? FM / 2 : 2 < FM / 2 ? 2 : FM / 2;  // measured: 3 no faster, 4 spills an accumulator fragment
     auto load_ev = [&](int t) {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) ev[t][j] = *(const bf16x8*)(Et + j * 16 * BLK_COLS + (long)t * BLK_ELEMS);
+        for (int j = 0; j < FN; ++j) ev[t * FN + j] = load16<COH>(Et, (COH ? ct_off : 0) + j * 16 * BLK_COLS + (long)t * BLK_ELEMS);
     };
-    if constexpr (EPI == EPI_SYMPOLY) {
+    if constexpr (EPI == EPI_SYMPOLY && (PART & EPI_LOADS)) {
 #pragma unroll
-        for (int t = 0; t < EV_AHEAD; ++t) load_ev(t);
+        for (int t = 0; t < (PART == EPI_LOADS ? FM / 2 : EV_AHEAD); ++t) load_ev(t);
     }
+    if constexpr (!(PART & EPI_REST)) return;
     auto rounded = [&](float v) {
         v = rbf(v);
         if (EPI == EPI_SYMPOLY) v = g.s1 * v;
@@ -586,7 +627,7 @@ __device__ __forceinline__ void epilogue_sym_reg(const GemmArgs& g, const TileCo
                 const bf16x8 tv = *(const bf16x8*)&tw;
                 bf16x8 o;
 #pragma unroll
-                for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[t][j][k])) + bf2f(tv[k]));
+                for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[t * FN + j][k])) + bf2f(tv[k]));
                 *(bf16x8*)(Ct + j * 16 * BLK_COLS + (long)t * BLK_ELEMS) = o;
                 if (diag && mblk == nblk) continue;
                 const u32x4 ow = *(const u32x4*)&o;
@@ -790,8 +831,10 @@ __global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pipe_kernel(const GemmL
         }
     }
     WAIT_VM(0);  // the dummy loads of the last two tails must not land in the epilogue's tile
-    if constexpr (QT) epilogue_nn<BM, BN, WGM, WGN, epi_fold_mode(EPI)>(g, tc, acc, smem);
-    else epilogue<BM, BN, WGM, WGN, EPI, false>(g, tc, acc, smem);
+    bf16x8 ev[tile_pieces<BM, BN, WGM, WGN>()];
+    FoldPiece<false> pv[tile_pieces<BM, BN, WGM, WGN>()];
+    if constexpr (QT) epilogue_nn<BM, BN, WGM, WGN, epi_fold_mode(EPI), false, EPI_ALL>(g, tc, acc, smem, ev, pv);
+    else epilogue<BM, BN, WGM, WGN, EPI, false, false, EPI_ALL>(g, tc, acc, smem, ev);
 }
 
 // 16x16 fragments (i, j) of wave `wave` of a WGM x WGN wave grid whose enclosing 32x32 block lies entirely below
@@ -831,8 +874,14 @@ __device__ __forceinline__ int pp_swizzle(int rg) { return (0x78 >> (2 * rg)) & 
 // group 1 runs M(t) in p=2t+1 and C(t) in p=2t+2.  Stage t&3 is last read in p=2t+1, the
 // loads of k-tile t+4 into it are issued in p=2t+2 / 2t+3, each wave waits for its own at the
 // end of its M phase two k-tiles later (p=2t+6 / 2t+7), and k-tile t+4 is first read in p=2t+8.
-template <int BM, int BN, int WGM, int WGN, int EPI>
-__device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, unsigned char* smem) {
+//
+// COH: operands and elementwise terms are read at device scope (load16).  before_loads() runs in front of the first load, after_loop()
+// between the k loop and the epilogue.
+struct Nothing {
+    __device__ void operator()() const {}
+};
+template <int BM, int BN, int WGM, int WGN, int EPI, bool COH = false, typename F0 = Nothing, typename F1 = Nothing>
+__device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, unsigned char* smem, F0 before_loads = F0(), F1 after_loop = F1()) {
     constexpr int NW = WGM * WGN;
     constexpr int BK4 = 32, ROWB = 64;
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
@@ -845,7 +894,7 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     static_assert(BM % (16 * NW) == 0 && BN % (16 * NW) == 0, "dma split");
     static_assert(epi_is_bx(EPI) || BM == BN, "triangular tiles are square");
 
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = thread_number<COH>(), lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 2;
     const int wm = wave / WGN, wn = wave % WGN;
@@ -880,10 +929,16 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     // global_load_lds_dwordx4 with a scalar base and a 32-bit vector offset; the LDS destination
     // of lane 0 goes through M0 (the wave's 64 lanes fill 1 KB from there in lane order).
     auto dma = [&](const char* base, unsigned voff, unsigned lds_byte) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :
-                     : "s"(lds_byte), "v"(voff), "s"(base)
-                     : "memory");
+        if constexpr (COH)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 sc1"
+                         :
+                         : "s"(lds_byte), "v"(voff), "s"(base)
+                         : "memory");
+        else
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                         :
+                         : "s"(lds_byte), "v"(voff), "s"(base)
+                         : "memory");
     };
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_void_ptr)smem;
     auto issue_tile = [&](int kt) {  // kt may run past the end: re-load the last k-tile
@@ -917,6 +972,25 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     const int a_off = (wm * WTM + (lane & 15)) * ROWB + co;
     const int b_off = A_BYTES + (wn * WTN + (lane & 15)) * ROWB + co;
 
+    // The elementwise term and the parameter's pieces first, where they fit (128-tiles).  They lie before the k-tiles in the queue,
+    // which returns in order, so the counts below stay what they are.
+    constexpr bool PRE = BM == 128;
+    // The epilogues that need no LDS.  Measured: on whole 256-tiles b.A + c.A.A is 0.5 % faster without it, X.Xt 0.6 % slower; on
+    // 128-tiles a launch of either is 1 % slower, but in the kernel with COH, where every tile is waited for, two barriers fewer are
+    // worth 3 to 10 % of a chain (1400 sets of matrices of 65 to 1536 rows).
+    constexpr bool REG = EPI == EPI_BX;
+    constexpr bool SREG = (EPI == EPI_SYMPOLY && BM == 256) || (!QT && COH);
+    constexpr int NEV = tile_pieces<BM, BN, WGM, WGN>(), LATE = PRE ? EPI_REST : EPI_ALL;
+    bf16x8 ev[NEV];
+    FoldPiece<PRE> pv[NEV];
+    before_loads();
+    if constexpr (PRE) {
+        if constexpr (REG) epilogue_nn_reg<BN, WGN, WTM, FM, true, COH, EPI_LOADS>(g, tc.bidx, tc.ti * BM, tc.tj * BN, acc, ev);
+        else if constexpr (QT) epilogue_nn<BM, BN, WGM, WGN, epi_fold_mode(EPI), COH, EPI_LOADS>(g, tc, acc, smem, ev, pv);
+        else if constexpr (SREG) epilogue_sym_reg<BM, BN, WGM, WGN, EPI, 0, COH, EPI_LOADS>(g, tc, acc, ev);
+        else epilogue<BM, BN, WGM, WGN, EPI, true, COH, EPI_LOADS>(g, tc, acc, smem, ev);
+    }
+
     issue_tile(0);
     issue_tile(1);
     issue_tile(2);
@@ -938,8 +1012,11 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
             rb[half][h] = QT ? smem + half * 2 * STAGE + A_BYTES + (wn * WTN / 32) * 2048 + qt_lane_offset(lane, h)
                              : smem + half * 2 * STAGE + b_off;
     }
-    auto body = [&](int kt, auto stage_c, auto mask_c) {
-        constexpr int SIDX = decltype(stage_c)::value;
+    // LATER: k-tiles behind kt that are still to come, as far as it matters: 3 where kt + 3 is (or, on 256-tiles, the last k-tile
+    // is loaded once more in its place, into a stage that nobody reads: a straight loop), fewer in the last three of a 128-tile,
+    // where a short loop would wait for such loads in front of its epilogue.
+    auto body = [&](int kt, auto stage_c, auto mask_c, auto later_c) {
+        constexpr int SIDX = decltype(stage_c)::value, LATER = decltype(later_c)::value;
         constexpr unsigned MASK = decltype(mask_c)::value;
         auto kept = [](int i, int j) { return !((MASK >> (i * FN + j)) & 1); };
         // ---- M(kt)
@@ -960,9 +1037,9 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
             if (QT) fb[j] = lds_read_qt(rb[SIDX >> 1][j & 1] + (SIDX & 1) * STAGE + (j >> 1) * 2048);
             else fb[j] = *(const bf16x8*)(rb[SIDX >> 1][0] + (SIDX & 1) * STAGE + j * 16 * ROWB);
         }
-        issue_tile(kt + 3);
+        if constexpr (LATER == 3) issue_tile(kt + 3);
         WAIT_LGKM0();
-        WAIT_VM(2 * NLD);  // own loads of k-tile kt+1 have landed
+        if constexpr (LATER > 0) WAIT_VM((LATER - 1) * NLD);  // own loads of k-tile kt+1 have landed
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -988,11 +1065,23 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     };
     // nk is a multiple of 4 (k extents are multiples of 128)
     auto k_loop = [&](auto mask_c) {
-        for (int kt = 0; kt < nk; kt += 4) {
-            body(kt, std::integral_constant<int, 0>{}, mask_c);
-            body(kt + 1, std::integral_constant<int, 1>{}, mask_c);
-            body(kt + 2, std::integral_constant<int, 2>{}, mask_c);
-            body(kt + 3, std::integral_constant<int, 3>{}, mask_c);
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I3 = std::integral_constant<int, 3>;
+        constexpr bool PEEL = BM == 128 && !epi_fold_mode(EPI);  // (with the parameter's pieces held as well a second copy spills)
+        const int whole = PEEL ? nk - 4 : nk;
+        for (int kt = 0; kt < whole; kt += 4) {
+            body(kt, I0{}, mask_c, I3{});
+            body(kt + 1, I1{}, mask_c, I3{});
+            body(kt + 2, I2{}, mask_c, I3{});
+            body(kt + 3, I3{}, mask_c, I3{});
+        }
+        if constexpr (PEEL) {
+            body(nk - 4, I0{}, mask_c, I3{});
+            body(nk - 3, I1{}, mask_c, I2{});
+            body(nk - 2, I2{}, mask_c, I1{});
+            body(nk - 1, I3{}, mask_c, I0{});
         }
     };
     // One copy of the loop per distinct mask (the masks are compile-time facts of the wave grid), chosen once per
@@ -1017,24 +1106,24 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
         run_if_mine(std::integral_constant<int, 7>{});
     }
     if (!grp) __builtin_amdgcn_s_barrier();
-    if constexpr (EPI == EPI_BX) {
+    after_loop();
+    if constexpr (REG) {
         // no LDS in this epilogue: the loads issued past the end may land while it runs (its own loads are behind
         // them in the queue, so they have landed before the wave ends)
-        epilogue_nn_reg<BN, WGN, WTM, FM, true>(g, tc.bidx, tc.ti * BM, tc.tj * BN, acc);
+        epilogue_nn_reg<BN, WGN, WTM, FM, true, COH, LATE>(g, tc.bidx, tc.ti * BM, tc.tj * BN, acc, ev);
         return;
     }
-    if constexpr (EPI == EPI_SYMPOLY && BM == 256) {
-        // measured: without LDS b.A + c.A.A is 0.5 % faster on whole 256-tiles, X.Xt 0.6 % slower
-        epilogue_sym_reg<BM, BN, WGM, WGN, EPI>(g, tc, acc);
+    if constexpr (SREG) {
+        epilogue_sym_reg<BM, BN, WGM, WGN, EPI, 0, COH, LATE>(g, tc, acc, ev);
         return;
     }
     WAIT_VM(0);  // the loads issued past the end must not land in the epilogue's tile
-    if constexpr (QT) epilogue_nn<BM, BN, WGM, WGN, epi_fold_mode(EPI)>(g, tc, acc, smem);
-    else epilogue<BM, BN, WGM, WGN, EPI, true>(g, tc, acc, smem);
+    if constexpr (QT) epilogue_nn<BM, BN, WGM, WGN, epi_fold_mode(EPI), COH, LATE>(g, tc, acc, smem, ev, pv);
+    else epilogue<BM, BN, WGM, WGN, EPI, true, COH, LATE>(g, tc, acc, smem, ev);
 }
 
 template <int BM, int BN, int WGM, int WGN, int EPI>
-__global__ void __launch_bounds__(WGM* WGN * 64) gemm_nt_pp_kernel(const GemmList l) {
+__global__ void __launch_bounds__(WGM* WGN * 64, BM == 128 ? 4 : 2) gemm_nt_pp_kernel(const GemmList l) {
     extern __shared__ __align__(16) unsigned char smem[];
     const int logical = xcd_remap(blockIdx.x, gridDim.x, l.xcd_shift), entry = list_entry(l, logical);
     pp_tile<BM, BN, WGM, WGN, EPI>(l.g[entry], tile_of<EPI>(l.g[entry], logical - l.start[entry]), smem);
@@ -1185,8 +1274,9 @@ __global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmList l) {
     tail_pair(std::integral_constant<int, 6>{});
     tail_pair(std::integral_constant<int, 4>{});
     tail_pair(std::integral_constant<int, 2>{});
-    if constexpr (QT) epilogue_nn_reg<BN, WGN, WTM, FM, true>(g, tc.bidx, tc.ti * BM, tc.tj * BN, acc);
-    else epilogue_sym_reg<BM, BN, WGM, WGN, EPI>(g, tc, acc);
+    bf16x8 ev[tile_pieces<BM, BN, WGM, WGN>()];
+    if constexpr (QT) epilogue_nn_reg<BN, WGN, WTM, FM, true, false, EPI_ALL>(g, tc.bidx, tc.ti * BM, tc.tj * BN, acc, ev);
+    else epilogue_sym_reg<BM, BN, WGM, WGN, EPI, 0, false, EPI_ALL>(g, tc, acc, ev);
 }
 
 // The same with a split tail: when the tile count leaves the last round of the compute units mostly empty,
@@ -1449,9 +1539,11 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmList l) {
             // reduction by the compiler, which then waits for the answer on the spot); the answer is needed at the end.
             if (has_next && tid == 0) fetched = atomicInc(&ctr.next[xcd][0], 0xffffffffu);
             if constexpr (QT) {
-                epilogue_nn_reg<BN, WGN, WTM, MASK == 0 ? F0 : F1, WHOLE>(g, cur.tc.bidx, cur.tc.ti * BM, cur.tc.tj * BN, acc);
+                bf16x8 ev[(MASK == 0 ? F0 : F1) * (FN / 2)];
+                epilogue_nn_reg<BN, WGN, WTM, MASK == 0 ? F0 : F1, WHOLE, false, EPI_ALL>(g, cur.tc.bidx, cur.tc.ti * BM, cur.tc.tj * BN, acc, ev);
             } else {
-                epilogue_sym_reg<BM, BN, WGM, WGN, EPI, MASK>(g, cur.tc, acc);
+                bf16x8 ev[FM * FN / 2];
+                epilogue_sym_reg<BM, BN, WGM, WGN, EPI, MASK, false, EPI_ALL>(g, cur.tc, acc, ev);
                 // What says that this wave's share of the next tile's first k-tiles has landed: B.X and b.A + c.A.A consume
                 // loads that were issued after them (the queue returns in order).  X.Xt loads nothing, and in a diagonal
                 // tile a wave may have nothing to finish at all: there the count is explicit (48 stores went out after the
@@ -1502,6 +1594,186 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmList l) {
         if (atomicAdd(&ctr.done[0], 1u) == (unsigned)grid - 1) {
             for (int x = 0; x < xcds; ++x) atomicExch(&ctr.next[x][0], 0u);
             atomicExch(&ctr.done[0], 0u);
+        }
+    }
+}
+
+// ---- kernel 4: the whole chain of many small matrices in one launch ------------------------------
+// A set of a few dozen matrices makes fifteen dependent launches of one to three rounds of tiles, and in each of them most compute
+// units wait for the last tiles and for the next launch to start.  Here a matrix belongs to one XCD for all of its products:
+// what one compute unit writes, another of the same XCD reads out of the L2 that they share, so that a product may start as
+// soon as the one before it has finished for that matrix, with a counter in memory between them and no launch.  (The same over all
+// XCDs has to write through to memory: a handover between 32 workgroups of an XCD takes 1.3 us, between all 256 with
+// written-through stores 5 to 13, with cache write-backs 49; a launch 2.5 to 2.9.)
+//
+// The host deals the matrices to as many groups as there are XCDs.  A workgroup finds out which XCD it runs on, takes that
+// XCD's group (the first of an XCD to ask fetches a group for it; an XCD that has finished one fetches another, so the groups
+// are served whatever XCDs the workgroups land on) and then tiles of it by a counter, in the order iteration, product, matrix,
+// tile.  A tile waits until its matrix has finished every tile of the product before.  Tiles are taken in order, and a tile waits
+// only for tiles that come before its own, which workgroups that are running hold: the earliest unfinished tile never waits, so
+// every wait ends.  (Each is bounded all the same, by some minutes, after which the launch drains.)
+//
+// Memory order.  Producer: the tile's stores, `s_waitcnt vmcnt(0)` in every wave (they are in L2), the workgroup's barrier, the
+// matrix's counter.  Consumer: the counter, the barrier, then loads that read past the compute unit's own vector cache (load16,
+// sc1 on the operand loads; the buffers of X are written again two iterations later and may be in it).  Measured, sc1 costs the
+// loads nothing: the XCD's L2 serves them.
+//
+// 128x128 tiles on the ping-pong loop, two workgroups per compute unit: one waits, starts and drains while the other computes.
+struct FlowControl {
+    unsigned tile[GEMM_MAX_XCDS][16];           // per group: tiles handed out
+    unsigned group_of[GEMM_MAX_XCC_IDS][16];    // the n-th group of an XCD: 0 nobody has asked, 1 being fetched, group + 2
+    unsigned next_group[16];
+    unsigned abandoned[16];                     // a wait has given up: everybody leaves
+};
+static_assert(sizeof(FlowControl) == GEMM_FLOW_CONTROL_BYTES && GEMM_MAX_XCDS < 16, "the size the header promises");
+
+__device__ __forceinline__ unsigned flow_load(const unsigned* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Waits until *p, a count, has reached `want`; false if the launch is being abandoned.  Polls seldom while much is missing: on the
+// line that sixty workgroups poll the increments themselves have to queue.
+__device__ __forceinline__ bool flow_wait(const unsigned* p, unsigned want, unsigned* abandoned) {
+    for (unsigned spins = 0;; ++spins) {
+        const unsigned have = flow_load(p);
+        if (have >= want) return true;
+        if (want - have > 16) __builtin_amdgcn_s_sleep(32);
+        else if (want - have > 4) __builtin_amdgcn_s_sleep(8);
+        else __builtin_amdgcn_s_sleep(2);
+        if ((spins & 1023) == 1023 && flow_load(abandoned)) return false;
+        if (spins == 1u << 27) {
+            atomicExch(abandoned, 1u);
+            return false;
+        }
+    }
+}
+
+constexpr int kFlowStages = 4 * (128 + 128) * 64;
+// What thread 0 of a workgroup keeps, and what it tells the others: the tile (entry, matrix, tile, product, iteration; entry < 0: none
+// is left).
+struct FlowSlot {
+    int entry, matrix, tile, stage, it;
+    bool gone;           // a wait has been given up
+    int epoch, group;    // the XCD's group that the workgroup takes tiles of, -1 before it knows
+    unsigned want;       // tiles of the matrix that come before the tile's product
+    unsigned* done;      // the matrix's counter
+};
+// The next tile of this XCD, in order: false when there is none left.  have: tile `t` of the group has been asked for already.
+__device__ __forceinline__ bool flow_next(const FlowList& l, FlowControl& ctl, FlowSlot* slot, bool have, int t) {
+    int g = slot->group, epoch = slot->epoch;
+    if (slot->gone) return false;
+    for (;;) {
+        if (g < 0) {
+            if (epoch == l.groups) return false;
+            unsigned id;
+            asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(id));
+            unsigned* const mine = &ctl.group_of[id & (GEMM_MAX_XCC_IDS - 1)][epoch];
+            unsigned v = atomicCAS(mine, 0u, 1u);
+            if (v == 0) {
+                v = atomicAdd(&ctl.next_group[0], 1u) + 2;
+                atomicExch(mine, v);
+            } else if (v == 1) {
+                if (!flow_wait(mine, 2, &ctl.abandoned[0])) return false;
+                v = flow_load(mine);
+            }
+            g = (int)v - 2;
+            if (g >= l.groups) return false;
+        }
+        if (!have) t = (int)atomicAdd(&ctl.tile[g][0], 1u);
+        have = false;
+        if (t < flow_tiles(l, g)) break;
+        g = -1;
+        ++epoch;
+    }
+    slot->group = g;
+    slot->epoch = epoch;
+    const FlowPlace p = flow_place(l, g, t);
+    slot->entry = p.entry;
+    slot->matrix = p.matrix;
+    slot->tile = p.tile;
+    slot->stage = p.stage;
+    slot->it = p.it;
+    slot->done = l.e[p.entry].done + p.matrix * GEMM_FLOW_LINE;
+    slot->want = (unsigned)p.before;
+    return true;
+}
+
+__global__ void __launch_bounds__(512, 4) gemm_nt_flow_kernel(const FlowList l) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    FlowSlot* const slot = (FlowSlot*)(smem + kFlowStages);  // behind the four stages
+    FlowControl& ctl = *(FlowControl*)l.control;
+    const int tid = threadIdx.x;
+    if (tid == 0) slot->epoch = 0, slot->group = -1, slot->gone = false;
+    int fetched = 0;             // thread 0: the tile asked for while the one before was in its epilogue
+    unsigned* finished = nullptr;  // the counter of the matrix that the tile before belongs to
+    auto ask = [&]() {
+        // (atomicInc: an atomicAdd of a uniform value becomes a wave-wide reduction whose result the compiler waits for on the spot)
+        if (tid == 0) fetched = (int)atomicInc(&ctl.tile[slot->group][0], 0xffffffffu);
+    };
+    auto wait = [&]() {  // everything in front of this is done while the matrix is not ready yet
+        if (tid == 0 && !flow_wait(slot->done, slot->want, &ctl.abandoned[0])) slot->gone = true;
+        __syncthreads();
+    };
+    for (;;) {
+        if (tid == 0 && !flow_next(l, ctl, slot, finished != nullptr, fetched)) slot->entry = -1;
+        // every wave's stores of the tile before are in L2, and every wave has read what it needs from LDS
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0 && finished) __hip_atomic_fetch_add(finished, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const int entry = __builtin_amdgcn_readfirstlane(slot->entry);
+        if (entry < 0) break;
+        const FlowEntry& e = l.e[entry];
+        const int tile = __builtin_amdgcn_readfirstlane(slot->tile), stage = __builtin_amdgcn_readfirstlane(slot->stage);
+        const int it = __builtin_amdgcn_readfirstlane(slot->it), cur = it & 1;
+        GemmArgs a = {};
+        a.cbP = e.Mp / BLK_COLS;
+        a.kdim = e.Mp;
+        TileCoord tc{__builtin_amdgcn_readfirstlane(slot->matrix), 0, 0};
+        finished = e.done + tc.bidx * GEMM_FLOW_LINE;
+        auto run = [&](auto epi_c) { pp_tile<128, 128, 2, 4, decltype(epi_c)::value, true>(a, tc, smem, wait, ask); };
+        if (stage == 2) {
+            a.tiles_m = e.Mp / 128;
+            a.tiles_n = e.Kr / 128;
+            rect_decode<4>(tile, a.tiles_m, a.tiles_n, tc.ti, tc.tj);
+            a.P = e.B;
+            a.strideP = e.strideA;
+            a.Q = a.Et = e.X[cur];
+            a.C = e.X[cur ^ 1];
+            a.strideQ = a.strideEt = a.strideC = e.strideX;
+            a.cbQ = a.cbEt = a.cbC = e.Kp / BLK_COLS;
+            a.s0 = l.a;
+            if (!e.p_ptrs || it < l.steps - 1) {
+                run(std::integral_constant<int, EPI_BX>{});
+            } else {
+                a.upd_ptrs = e.p_ptrs;
+                a.upd_dtype = l.p_dtype;
+                a.upd_rows = e.rows;
+                a.upd_cols = e.cols;
+                a.upd_scale = e.scale;
+                a.upd_decay = l.decay;
+                a.upd_alpha = l.alpha;
+                if (e.rows <= e.cols) run(std::integral_constant<int, EPI_BX_UPD>{});
+                else run(std::integral_constant<int, EPI_BX_UPD_T>{});
+            }
+        } else {
+            tri_decode<4>(tile, e.Mp / 128, tc.ti, tc.tj);
+            a.strideC = a.strideCt = e.strideA;
+            a.cbC = a.cbCt = e.Mp / BLK_COLS;
+            if (stage == 0) {
+                a.P = a.Q = e.X[cur];
+                a.strideP = a.strideQ = e.strideX;
+                a.cbP = e.Kp / BLK_COLS;
+                a.kdim = e.Kr;
+                a.C = a.Ct = e.A;
+                run(std::integral_constant<int, EPI_SYRK>{});
+            } else {
+                a.P = a.Q = a.Et = e.A;
+                a.strideP = a.strideQ = a.strideEt = e.strideA;
+                a.cbEt = e.Mp / BLK_COLS;
+                a.C = a.Ct = e.B;
+                a.s0 = l.b;
+                a.s1 = l.c;
+                run(std::integral_constant<int, EPI_SYMPOLY>{});
+            }
         }
     }
 }
@@ -1764,6 +2036,76 @@ int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* r
         ++launches;
     }
     return launches;
+}
+
+bool plan_flow(FlowList& l, int xcds) {
+    l.groups = xcds;
+    if (l.n < 1 || l.n > GEMM_MAX_LIST || xcds < 1 || xcds > GEMM_MAX_XCDS || l.steps < 1) return false;
+    // Dearest matrices first, each to the group with the least work so far.  Work in k-tiles of 32 columns, the start and the
+    // epilogue of a tile as twelve more.
+    double load[GEMM_MAX_XCDS] = {}, cost[GEMM_MAX_LIST], mean = 0, most = 0, chain = 0;
+    int order[GEMM_MAX_LIST];
+    for (int i = 0; i < l.n; ++i) {
+        FlowEntry& e = l.e[i];
+        const double tm = e.Mp / 128, tn = e.Kr / 128, tri = tm * (tm + 1) / 2;
+        if (tm * tn > 0xffff) return false;
+        e.sym = (int)tri;
+        e.rect = (int)(tm * tn);
+        cost[i] = tri * (4 * tn + 12) + (tri + tm * tn) * (4 * tm + 12);
+        chain = std::max(chain, 4 * tn + 8 * tm + 36);
+        mean += cost[i] * e.batch / xcds;
+        order[i] = i;
+    }
+    std::stable_sort(order, order + l.n, [&](int x, int y) { return cost[x] > cost[y]; });
+    for (int k = 0; k < l.n; ++k) {
+        FlowEntry& e = l.e[order[k]];
+        int count[GEMM_MAX_XCDS];
+        for (int g = 0; g < xcds; ++g) {
+            count[g] = e.batch / xcds;
+            load[g] += cost[order[k]] * count[g];
+        }
+        for (int r = e.batch % xcds; r > 0; --r) {
+            const int least = (int)(std::min_element(load, load + xcds) - load);
+            ++count[least];
+            load[least] += cost[order[k]];
+        }
+        e.first[0] = 0;
+        for (int g = 0; g < xcds; ++g) e.first[g + 1] = e.first[g] + count[g];
+    }
+    for (int g = 0; g < xcds; ++g) {
+        long sym = 0, rect = 0;
+        for (int i = 0; i < l.n; ++i) {
+            const FlowEntry& e = l.e[i];
+            sym += (long)(e.first[g + 1] - e.first[g]) * e.sym;
+            rect += (long)(e.first[g + 1] - e.first[g]) * e.rect;
+        }
+        if ((2 * sym + rect) * l.steps > 0x3fffffffL) return false;  // (what is asked for past the end stays below 2^31)
+        l.sym[g] = (int)sym;
+        l.rect[g] = (int)rect;
+        most = std::max(most, load[g]);
+    }
+    // Measured on 1400 sets of one to four shapes of 65 to 1536 rows, 2 to 800 matrices, against launches of their own: the XCD with
+    // the most work and, where there is little, the chain of one matrix through an iteration set its time, launches of their own
+    // share the work evenly but pay for each other's last rounds.  The line below takes 598 of them, 15 % faster in the mean (up to
+    // 30 %) and 18 slower by more than 3 % (8 % at most).  Beyond `mean` of 30000 the 256-tiles of large launches are worth more than
+    // what is lost between them (1.02 of their time).
+    if (mean < 30000 && most < 1.35 * mean - 15 * chain + 600) return true;
+    // A step over very little: the device takes as long either way (94 against 86 us for 14 matrices of 128 x 128 to 384), but the
+    // caller waits for his own 14 launches less (whole step of that model 240 us with, 190 without them).
+    return l.e[0].p_ptrs && 0.032 * most + 0.64 * chain + 55 < 120;
+}
+
+hipError_t launch_flow(const FlowList& l, hipStream_t stream) {
+    MachineShape ms;
+    if (hipError_t e = machine_shape(ms); e != hipSuccess) return e;
+    constexpr int smem = kFlowStages + (int)sizeof(FlowSlot);
+    static std::atomic<unsigned long long> configured{0};
+    if (hipError_t e = allow_dynamic_lds((const void*)gemm_nt_flow_kernel, smem, configured); e != hipSuccess) return e;
+    // two workgroups per compute unit, but no more than have something to do: the others would only poll
+    int most = 1;
+    for (int g = 0; g < l.groups; ++g) most = std::max(most, l.sym[g] + l.rect[g]);
+    hipLaunchKernelGGL(gemm_nt_flow_kernel, dim3(l.groups * std::min(2 * ms.cus / l.groups, most)), dim3(512), smem, stream, l);
+    return hipGetLastError();
 }
 
 hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t stream) {
