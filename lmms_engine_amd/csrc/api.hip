@@ -696,6 +696,48 @@ int muon_hip_syrk_bf16(const void* X, void* A, int Mp, int Kp, int batch, int cf
     return launch_items(MUON_HIP_K_SYRK, "syrk launch", &it, 1, use.adapt, (hipStream_t)stream);
 }
 
+// Whether the kernels read X where it lies.  They can when its rows are whole k-tiles and 16-byte pieces, a panel of 256 rows is
+// addressed with 32 bits, and nothing that they write is still to be read.  They should, but for 128-tiles of an X that the L2s do not
+// hold: those read 64 bytes of a row at a time, and rows whose pitch is a multiple of the L2 channels crowd into few of them.
+// Measured, packed | in place: 64-tiles 896 x 4864 28.0 | 18.8 us; 128-tiles 2048 x 1024 18.5 | 11.6, 2048 x 2176 27.3 | 23.4, 2800 x
+// 3968 45.1 | 42.9, 2048 x 5632 46.4 | 47.6, 3072 x 3072 50.4 | 58.0, 1536 x 6144 47.6 | 56.1; 256-tiles 4096 x 1024 38.4 | 29.7,
+// 4096 x 12288 214 | 204, 8192 x 16384 899 | 900.
+static bool mmt_reads_x(const void* X, const void* Y, int M, int K) {
+    const uintptr_t x = (uintptr_t)X, y = (uintptr_t)Y;
+    const bool apart = y + 2 * (size_t)M * M <= x || x + 2 * (size_t)M * K <= y;
+    if (K % 128 || K > (1 << 22) || (x & 15) || !apart) return false;
+    MachineShape ms;
+    if (machine_shape(ms) != hipSuccess) return false;  // the launch will report it
+    const long t = round_up(M, 128) / 128, t128 = t * (t + 1) / 2, t64 = t * (2 * t + 1);
+    const bool small = t64 <= ms.cus, large = use_tile256(M) && t128 > 2 * ms.cus;  // as plan_gemm_nt has it
+    return small || large || (long)M * K <= 5L << 20;
+}
+static int mmt_tile(int M) { return use_tile256(M) ? 256 : 128; }
+
+long muon_hip_mmt_scratch_elems(const void* X, const void* Y, int M, int K) {
+    if (M <= 0 || K <= 0) return 0;
+    const int tile = mmt_tile(M);
+    return mmt_reads_x(X, Y, M, K) ? 0 : blocked_elems(round_up(M, tile), round_up(K, tile));
+}
+
+int muon_hip_mmt_bf16(const void* X, void* Y, int M, int K, void* scratch, void* stream) {
+    if (M <= 0 || K <= 0) return fail(MUON_HIP_EINVAL, "sizes must be positive");
+    if (!X || !Y) return fail(MUON_HIP_EINVAL, "null operand");
+    const int tile = mmt_tile(M), Mp = (int)round_up(M, tile), Kp = (int)round_up(K, tile);
+    const bool reads_x = mmt_reads_x(X, Y, M, K);
+    if (!reads_x) {
+        if (!scratch || ((uintptr_t)scratch & 15)) return fail(MUON_HIP_EINVAL, "this X needs scratch, 16-byte aligned");
+        hipError_t e = launch_pack((const bf16_t*)X, 0, K, M, K, (bf16_t*)scratch, 0, Mp, Kp, 1, (hipStream_t)stream);
+        if (e != hipSuccess) return hip_fail(e, "pack launch");
+    }
+    const int cfg = tile == 256 && M > 512 ? GEMM_CFG_256_PINGPONG : GEMM_CFG_128_PINGPONG;
+    GemmItem it = syrk_item(cfg, (const bf16_t*)(reads_x ? X : scratch), (bf16_t*)Y, Mp, (int)round_up(K, 128), Kp, 1, nullptr);
+    it.epi = EPI_MMT;
+    it.g.dense_rows = M;
+    it.g.dense_pitch = reads_x ? K : 0;
+    return launch_items(MUON_HIP_K_SYRK, "mmt launch", &it, 1, true, (hipStream_t)stream);
+}
+
 int muon_hip_sympoly_bf16(const void* A, void* B, int Mp, int batch, double b, double c, int cfg, void* counters,
                           void* stream) {
     const Cfg use = cfg == MUON_HIP_CFG_AUTO ? pick_cfg(Mp, EPI_SYMPOLY) : Cfg{cfg, false};

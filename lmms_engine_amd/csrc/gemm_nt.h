@@ -5,7 +5,8 @@
 
 // EPI_BX_UPD is EPI_BX with the parameter update folded into the epilogue (GemmArgs::upd_*) instead of writing X';
 // EPI_BX_UPD_T is the same for a parameter that is the transpose of X (rows > cols)
-enum { EPI_SYRK = 0, EPI_SYMPOLY = 1, EPI_BX = 2, EPI_BX_UPD = 3, EPI_BX_UPD_T = 4 };
+// EPI_MMT is EPI_SYRK with a row-major result, and a left operand that may be row-major too (matmul_transpose on its own)
+enum { EPI_SYRK = 0, EPI_SYMPOLY = 1, EPI_BX = 2, EPI_BX_UPD = 3, EPI_BX_UPD_T = 4, EPI_MMT = 5 };
 constexpr bool epi_is_bx(int e) { return e == EPI_BX || e == EPI_BX_UPD || e == EPI_BX_UPD_T; }
 // how the B.X epilogue finishes: 0 writes X', 1 updates a parameter in the orientation of X, 2 a transposed one
 constexpr int epi_fold_mode(int e) { return e == EPI_BX_UPD ? 1 : e == EPI_BX_UPD_T ? 2 : 0; }
@@ -50,6 +51,9 @@ struct GemmArgs {
     int upd_dtype;                // MUON_HIP_F32 or MUON_HIP_BF16
     int upd_rows, upd_cols;       // the parameter's own (unpadded) shape
     float upd_scale, upd_decay, upd_alpha;  // python-double scale, 1 - lr*wd and -lr, as fp32
+    // EPI_MMT: C is row-major, dense_rows x dense_rows (rows, cols: in whole 128-tiles as ever).  dense_pitch: P and Q are too, with
+    // that many elements from row to row and dense_rows rows; 0: they are blocked.
+    int dense_rows, dense_pitch;
     unsigned* ppx;          // tile counters of the persistent kernel (GEMM_PPX_COUNTER_BYTES, zero between launches);
                             // null: the launcher takes the one-tile kernels instead
 };

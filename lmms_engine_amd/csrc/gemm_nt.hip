@@ -131,6 +131,34 @@ __device__ __forceinline__ long panel_offset(int row0, int cb) {
     return (long)(row0 >> 8) * cb * BLK_ELEMS + (row0 & 255) * BLK_COLS;
 }
 
+// EPI_MMT: rows of a row-major C.  Pieces of 16 and 8 bytes where its rows are whole numbers of them, element by element otherwise
+// and at the edge.
+__device__ __forceinline__ bool dense_vec(const GemmArgs& g) { return g.dense_rows % 8 == 0 && (((uintptr_t)g.C) & 15) == 0; }
+template <typename V>
+__device__ __forceinline__ void dense_store(const GemmArgs& g, bool vec, int row, int col, const V& v) {
+    constexpr int N = sizeof(V) / 2;
+    bf16_t* p = g.C + (long)row * g.dense_rows + col;
+    if (row >= g.dense_rows) return;
+    if (vec && col + N <= g.dense_rows) {
+        *(V*)p = v;
+    } else {
+        const bf16_t* e = (const bf16_t*)&v;
+#pragma unroll
+        for (int k = 0; k < N; ++k)
+            if (col + k < g.dense_rows) p[k] = e[k];
+    }
+}
+
+// EPI_MMT of a row-major X: where the panel of rows row0.. starts, and row r of it from there.  Past the last row of X that row
+// again: what it gives lies outside C.
+__device__ __forceinline__ long dense_panel(const GemmArgs& g, int row0) {
+    return (long)(row0 < g.dense_rows ? row0 : g.dense_rows - 1) * g.dense_pitch;
+}
+__device__ __forceinline__ int dense_row(const GemmArgs& g, int row0, int r) {
+    const int left = row0 < g.dense_rows ? g.dense_rows - 1 - row0 : 0;
+    return (r < left ? r : left) * g.dense_pitch;
+}
+
 // ---- epilogue ------------------------------------------------------------------------------
 // One LDS copy of the tile, both output orientations written as 16-byte vectors.  The tile
 // lives in LDS as Tt[n][m] (n = local column, m = local row of the accumulator tile), the
@@ -222,6 +250,15 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const TileCoord& tc,
         // rows of Tt leave as rows of Ct; SYMPOLY adds the rounded b.A term here and, when the tile itself is
         // gathered from LDS afterwards, puts the finished pieces back
         bf16_t* Ct = g.Ct + tc.bidx * g.strideCt;
+        if constexpr (EPI == EPI_MMT) {  // whole tile rows: a wave covers 64 pieces of a row, 256 or 512 bytes at a time
+            const bool vec = dense_vec(g);
+#pragma unroll
+            for (int u = 0; u < NLE; ++u) {
+                const int c = tid + u * NT, n = c / (BM / 8), piece = c % (BM / 8);
+                if (MASKED && diag && (piece >> 2) > (n >> 5)) continue;
+                dense_store(g, vec, n0 + n, m0 + piece * 8, *(const u32x4*)(smem + n * S + piece * 16));
+            }
+        } else
 #pragma unroll
         for (int u = 0; u < NLE; ++u) {
             long goff;
@@ -257,7 +294,10 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, const TileCoord& tc,
             const s16x8 o = {lo[0], lo[1], lo[2], lo[3], hi4[0], hi4[1], hi4[2], hi4[3]};
             // a diagonal tile: the pieces strictly above the diagonal fragments (row block c/8 < column block);
             // the Ct pass has written the rest
-            if (!diag || (c >> 3) < strip * 4 + grp)
+            if (diag && (c >> 3) >= strip * 4 + grp) continue;
+            if constexpr (EPI == EPI_MMT)
+                dense_store(g, dense_vec(g), m0 + c * 4 + (i16 & 3), n0 + strip * 128 + grp * 32 + (i16 >> 2) * 8, o);
+            else
                 *(s16x8*)(dst + (long)strip * (128 / BLK_COLS) * BLK_ELEMS + c * 4 * BLK_COLS) = o;
         }
     }
@@ -571,7 +611,9 @@ __device__ __forceinline__ void epilogue_sym_reg(const GemmArgs& g, const TileCo
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
     constexpr int FM = WTM / 16, FN = WTN / 16;
     static_assert(FM % 2 == 0 && FN % 2 == 0 && BLK_COLS == 32, "a pair of fragments is one column block");
-    static_assert(EPI == EPI_SYRK || EPI == EPI_SYMPOLY, "symmetric products");
+    static_assert(EPI == EPI_SYRK || EPI == EPI_SYMPOLY || EPI == EPI_MMT, "symmetric products");
+    constexpr bool DENSE = EPI == EPI_MMT;
+    const bool vec = DENSE && dense_vec(g);
     const int tid = thread_number<COH>(), lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN, row = lane >> 4;
@@ -636,11 +678,19 @@ __device__ __forceinline__ void epilogue_sym_reg(const GemmArgs& g, const TileCo
                 a01 = lo[0], b01 = lo[1], a23 = hi[0], b23 = hi[1];
             } else {
                 const u32x4 tw = {lo[0], hi[0], lo[1], hi[1]};
-                *(u32x4*)(Ct + j * 16 * BLK_COLS + (long)t * BLK_ELEMS) = tw;
+                if constexpr (DENSE)
+                    dense_store(g, vec, n0 + wn * WTN + 16 * j + (lane & 15), m0 + wm * WTM + 32 * t + 16 * (row & 1) + 8 * (row >> 1), tw);
+                else *(u32x4*)(Ct + j * 16 * BLK_COLS + (long)t * BLK_ELEMS) = tw;
                 if (diag && mblk == nblk) continue;
             }
             quad_transpose_b16(a01, a23, sel, upper);
             quad_transpose_b16(b01, b23, sel, upper);
+            if constexpr (DENSE) {
+                const int r = m0 + wm * WTM + 32 * t + 4 * row + (lane & 3), c = n0 + wn * WTN + 16 * j + ((lane >> 2) & 3) * 4;
+                dense_store(g, vec, r, c, u32x2v{a01, a23});
+                dense_store(g, vec, r + 16, c, u32x2v{b01, b23});
+                continue;
+            }
             bf16_t* cp = C + (2 * t) * 16 * BLK_COLS + (long)(j >> 1) * BLK_ELEMS + (j & 1) * 16;
             *(u32x2v*)cp = u32x2v{a01, a23};
             *(u32x2v*)(cp + 16 * BLK_COLS) = u32x2v{b01, b23};
@@ -900,9 +950,14 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     const int wm = wave / WGN, wn = wave % WGN;
     constexpr bool QT = epi_is_bx(EPI);  // Q is X itself, rows = reduction index
     const int kb = g.cbP;
-    const bf16_t* Pb = uniform_ptr(g.P + tc.bidx * g.strideP + panel_offset(tc.ti * BM, kb));
+    const bool dense = EPI == EPI_MMT && g.dense_pitch != 0;
+    auto panel = [&](int row0) { return dense ? dense_panel(g, row0) : panel_offset(row0, kb); };
+    auto in_panel = [&](int row0, int r, int ch) {  // element offset of row r, column ch of a k-tile from the panel's start
+        return dense ? dense_row(g, row0, r) + ch : r * BLK_COLS + ch;
+    };
+    const bf16_t* Pb = uniform_ptr(g.P + tc.bidx * g.strideP + panel(tc.ti * BM));
     const bf16_t* Qb = uniform_ptr(g.Q + tc.bidx * g.strideQ +
-                                   (QT ? (long)(tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel_offset(tc.tj * BN, kb)));
+                                   (QT ? (long)(tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel(tc.tj * BN)));
 
     // Loads: a wave-uniform base pointer (advanced along k with scalar adds) plus a 32-bit byte
     // offset per lane, so that no vector ALU instruction is needed per load: in the memory phase
@@ -911,7 +966,7 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     const int dch = ((lane & 3) ^ pp_swizzle((lane >> 4) & 3)) * 8;
     unsigned offa[LA], offb[LB];
 #pragma unroll
-    for (int n = 0; n < LA; ++n) offa[n] = (unsigned)(((wave * 16 * LA + n * 16 + drow) * BLK_COLS + dch) * 2);
+    for (int n = 0; n < LA; ++n) offa[n] = (unsigned)in_panel(tc.ti * BM, wave * 16 * LA + n * 16 + drow, dch) * 2;
     // BX: a k-tile of Q is BN/32 pieces of 32 rows x 32 columns, each a contiguous 2 KB run of one block; load
     // instruction t of the tile (1 KB) is the half t%2 of piece t/2, in lane order, with the two 32-byte halves
     // of a row swapped in rows whose k has bit 3 set (see qt_lane_offset)
@@ -920,11 +975,12 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     for (int n = 0; n < LB; ++n) {
         const int t = wave * LB + n;
         offb[n] = QT ? (unsigned)(((t >> 1) * BLK_ELEMS + ((t & 1) * 16 + drow) * BLK_COLS + qch) * 2)
-                     : (unsigned)(((wave * 16 * LB + n * 16 + drow) * BLK_COLS + dch) * 2);
+                     : (unsigned)in_panel(tc.tj * BN, wave * 16 * LB + n * 16 + drow, dch) * 2;
     }
     const int lds_a = wave * 16 * LA * ROWB;
     const int lds_b = A_BYTES + wave * 16 * LB * ROWB;
     const int nk = g.kdim / BK4;
+    const int kstep = dense ? BK4 : BLK_ELEMS;  // elements from k-tile to k-tile
 
     // global_load_lds_dwordx4 with a scalar base and a 32-bit vector offset; the LDS destination
     // of lane 0 goes through M0 (the wave's 64 lanes fill 1 KB from there in lane order).
@@ -943,7 +999,8 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_void_ptr)smem;
     auto issue_tile = [&](int kt) {  // kt may run past the end: re-load the last k-tile
         const int k0 = (kt < nk ? kt : nk - 1) * BK4;
-        const long koff = (long)(k0 >> BLK_SHIFT) * BLK_ELEMS + (k0 & (BLK_COLS - 1));
+        static_assert(BLK_COLS == BK4, "a k-tile is one block of columns");
+        const long koff = (long)(k0 >> BLK_SHIFT) * kstep;
         const char* ba = (const char*)(Pb + koff);
         const char* bb = (const char*)(Qb + (QT ? (long)(k0 >> 8) * g.cbQ * BLK_ELEMS + (k0 & 255) * BLK_COLS : koff));
         const unsigned st = lds_base + (kt & 3) * STAGE;
@@ -1142,7 +1199,7 @@ __global__ void __launch_bounds__(WGM* WGN * 64, BM == 128 ? 4 : 2) gemm_nt_pp_k
 // the persistent kernel, and every element sums its products in the same order: the results are the other kernels' bit for bit.
 template <int EPI>
 __global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmList l) {
-    static_assert(EPI == EPI_BX || EPI == EPI_SYRK || EPI == EPI_SYMPOLY, "the epilogues that need no LDS");
+    static_assert(EPI == EPI_BX || EPI == EPI_SYRK || EPI == EPI_SYMPOLY || EPI == EPI_MMT, "the epilogues that need no LDS");
     constexpr int BM = 64, BN = 64, WGM = 2, WGN = 2, NW = 4;
     constexpr int WTM = BM / WGM, WTN = BN / WGN, FM = WTM / 16, FN = WTN / 16;
     constexpr int A_BYTES = BM * ROW_BYTES, STAGE = A_BYTES + BN * ROW_BYTES, NST = 8;
@@ -1157,22 +1214,27 @@ __global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmList l) {
     const GemmArgs& g = l.g[entry];
     const TileCoord tc = tile_of<EPI>(g, logical - l.start[entry]);
     const int kb = g.cbP;
-    const bf16_t* Pb = uniform_ptr(g.P + tc.bidx * g.strideP + panel_offset(tc.ti * BM, kb));
+    // a row-major X of EPI_MMT: as in pp_tile
+    const bool dense = EPI == EPI_MMT && g.dense_pitch != 0;
+    auto panel = [&](int row0) { return dense ? dense_panel(g, row0) : panel_offset(row0, kb); };
+    auto in_panel = [&](int row0, int r) { return dense ? dense_row(g, row0, r) : r * BLK_COLS; };
+    const bf16_t* Pb = uniform_ptr(g.P + tc.bidx * g.strideP + panel(tc.ti * BM));
     const bf16_t* Qb = uniform_ptr(g.Q + tc.bidx * g.strideQ +
-                                   (QT ? (long)(tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel_offset(tc.tj * BN, kb)));
+                                   (QT ? (long)(tc.tj * BN >> BLK_SHIFT) * BLK_ELEMS : panel(tc.tj * BN)));
     const int drow = lane >> 3;
     // byte offsets of this lane's 16 bytes of each load instruction, from the scalar base of the k-tile (ping-pong kernel: no
     // vector ALU work per load)
-    auto chunk_off = [](int e) { return (e >> BLK_SHIFT) * BLK_ELEMS + (e & (BLK_COLS - 1)); };
+    const int kstep = dense ? BLK_COLS : BLK_ELEMS;  // elements from 32 columns to the next 32
+    auto chunk_off = [&](int e) { return (e >> BLK_SHIFT) * kstep + (e & (BLK_COLS - 1)); };
     unsigned offa[LA], offb[LB];
 #pragma unroll
     for (int n = 0; n < LA; ++n)  // LA is even: instruction n of a wave covers an even or an odd group of eight rows
-        offa[n] = (unsigned)(((wave * LA + n) * 8 + drow) * BLK_COLS + chunk_off(((lane & 7) ^ (((n & 1) << 2) | (drow >> 1))) * 8)) * 2;
+        offa[n] = (unsigned)(in_panel(tc.ti * BM, (wave * LA + n) * 8 + drow) + chunk_off(((lane & 7) ^ (((n & 1) << 2) | (drow >> 1))) * 8)) * 2;
 #pragma unroll
     for (int n = 0; n < LB; ++n) {
         const int t = wave * LB + n;
         offb[n] = QT ? (unsigned)((t >> 2) * BLK_ELEMS + ((t & 3) * 16 + (lane >> 2)) * BLK_COLS + ((lane & 3) ^ (((lane >> 5) & 1) << 1)) * 8) * 2
-                     : (unsigned)((t * 8 + drow) * BLK_COLS + chunk_off(((lane & 7) ^ (((n & 1) << 2) | (drow >> 1))) * 8)) * 2;
+                     : (unsigned)(in_panel(tc.tj * BN, t * 8 + drow) + chunk_off(((lane & 7) ^ (((n & 1) << 2) | (drow >> 1))) * 8)) * 2;
     }
     constexpr int KT_BLOCKS = 64 / BLK_COLS;
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_void_ptr)smem;
@@ -1184,7 +1246,7 @@ __global__ void __launch_bounds__(256) gemm_nt_deep_kernel(const GemmList l) {
     };
     auto issue_one = [&](int n, int kt) {  // load instruction n of k-tile kt: rows of P first, then Q
         const unsigned st = lds_base + (kt & (NST - 1)) * STAGE;
-        const long koff = (long)kt * KT_BLOCKS * BLK_ELEMS;
+        const long koff = (long)kt * KT_BLOCKS * kstep;
         const int k0 = kt * 64;
         if (n < LA) dma((const char*)(Pb + koff), offa[n], st + (wave * LA + n) * 8 * ROW_BYTES);
         else
@@ -1846,8 +1908,12 @@ hipError_t launch_pp_tail(GemmList& l, int nblocks, int rest, hipStream_t stream
 template <int EPI>
 hipError_t launch_cfg(int cfg, GemmList& l, int nblocks, int cus, hipStream_t stream) {
     switch (cfg) {
-        case GEMM_CFG_128_PIPE: return launch_one<128, 128, 2, 2, EPI, 0>(l, nblocks, stream);
-        case GEMM_CFG_256_PIPE: return launch_one<256, 256, 2, 4, EPI, 0>(l, nblocks, stream);
+        case GEMM_CFG_128_PIPE:
+            if constexpr (EPI == EPI_MMT) return hipErrorInvalidValue;
+            else return launch_one<128, 128, 2, 2, EPI, 0>(l, nblocks, stream);
+        case GEMM_CFG_256_PIPE:
+            if constexpr (EPI == EPI_MMT) return hipErrorInvalidValue;
+            else return launch_one<256, 256, 2, 4, EPI, 0>(l, nblocks, stream);
         case GEMM_CFG_256_PINGPONG: {
             // Split the tiles of a last round that would fill at most a quarter of the CUs (a 128x128 tile takes about 0.6 of
             // the time of a 256x256 one, so one round of quarters beats a round of whole tiles).
@@ -1870,6 +1936,7 @@ hipError_t launch_epi(int epi, int cfg, GemmList& l, int nblocks, int cus, hipSt
         case EPI_BX: return launch_cfg<EPI_BX>(cfg, l, nblocks, cus, stream);
         case EPI_BX_UPD: return launch_cfg<EPI_BX_UPD>(cfg, l, nblocks, cus, stream);
         case EPI_BX_UPD_T: return launch_cfg<EPI_BX_UPD_T>(cfg, l, nblocks, cus, stream);
+        case EPI_MMT: return launch_cfg<EPI_MMT>(cfg, l, nblocks, cus, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1886,6 +1953,7 @@ bool tiles_fit(const GemmItem& it, int height, int width) {
     const GemmArgs& g = it.g;
     auto up = [](int v, int m) { return (v + m - 1) / m * m; };
     if (up(g.rows, height) > up(g.rows, BLK_ROWS)) return false;
+    if (it.epi == EPI_MMT) return g.rows % height == 0 && g.dense_rows <= g.rows && g.dense_rows > g.rows - 128;
     if (!epi_is_bx(it.epi)) return g.rows % height == 0 && g.rows <= g.cbC * BLK_COLS;
     const int cols = up(g.cols, width);
     return cols <= g.cbC * BLK_COLS && cols <= g.cbQ * BLK_COLS && cols <= g.cbEt * BLK_COLS;

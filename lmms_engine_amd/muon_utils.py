@@ -145,19 +145,14 @@ def matmul_transpose_assign(d_in: Tensor, d_out: Tensor) -> None:
     if d_in.dtype != torch.bfloat16:
         raise TypeError(f"the MI355X kernel multiplies bfloat16 operands, got {d_in.dtype}")
     M, K = d_in.shape
-    tile = 256 if (-(-M // 128) % 2 == 0 and M > 384) else 128
-    cfg = _abi.CFG_AUTO  # the library picks the kernel for the padded size
-    Mp, Kp = -(-M // tile) * tile, -(-K // tile) * tile
     lib = _abi.lib()
     with torch.cuda.device(d_in.device):
-        s = _abi.stream_ptr(d_in.device)
         src = d_in.contiguous()
-        x = torch.empty(lib.muon_hip_blocked_elems(Mp, Kp), dtype=torch.bfloat16, device=d_in.device)
-        a = torch.empty(lib.muon_hip_blocked_elems(Mp, Mp), dtype=torch.bfloat16, device=d_in.device)
-        _abi.check(lib.muon_hip_pack_bf16(src.data_ptr(), 0, K, M, K, x.data_ptr(), Mp, Kp, 1, s), "pack")
-        _abi.check(lib.muon_hip_syrk_bf16(x.data_ptr(), a.data_ptr(), Mp, Kp, 1, cfg, None, s), "syrk")
         out = d_out if d_out.is_contiguous() else torch.empty_like(d_out, memory_format=torch.contiguous_format)
-        _abi.check(lib.muon_hip_unpack_bf16(a.data_ptr(), Mp, Mp, out.data_ptr(), 0, M, M, M, 1, s), "unpack")
+        x, y = src.data_ptr(), out.data_ptr()
+        n = lib.muon_hip_mmt_scratch_elems(x, y, M, K)
+        scratch = torch.empty(n, dtype=torch.bfloat16, device=d_in.device) if n else None
+        _abi.check(lib.muon_hip_mmt_bf16(x, y, M, K, scratch.data_ptr() if n else None, _abi.stream_ptr(d_in.device)), "mmt")
         if out is not d_out:
             d_out.copy_(out)
 
