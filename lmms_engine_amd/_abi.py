@@ -121,10 +121,28 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_scan = None
+
+
+def scan():
+    """The native reader of tensor lists (csrc/scan.cpp)."""
+    global _scan
+    if _scan is None:
+        try:
+            from . import _scan as module
+        except ImportError as e:
+            raise MuonHipError(f"lmms_engine_amd/_scan.so cannot be loaded ({e}): build it with `python -m lmms_engine_amd.build`") from e
+        _scan = module
+    return _scan
+
+
 def check(rc: int, what: str = "") -> None:
     if rc != 0:
         msg = lib().muon_hip_last_error().decode()
         raise MuonHipError(f"{what or 'muon_hip'} failed (code {rc}): {msg}")
+
+
+DTYPES = {F32: torch.float32, BF16: torch.bfloat16}
 
 
 def dtype_code(dt: torch.dtype) -> int:

@@ -1,4 +1,4 @@
-"""Builds lmms_engine_amd/libmuon_hip.so from csrc/ with hipcc for gfx950.
+"""Builds lmms_engine_amd/libmuon_hip.so from csrc/ with hipcc for gfx950, and the host-side module _scan.so beside it.
 
 Run as `python -m lmms_engine_amd.build` or call build_library().  The library is built
 in-tree, next to this file, so it travels with the source tree.
@@ -18,6 +18,8 @@ SOURCES = ["gemm_nt.hip", "elementwise.hip", "small_chain.hip", "multi_tensor.hi
 PROBE_LIB = os.path.join(HERE, "libmuon_probe.so")
 PROBE_SOURCES = ["probe.hip"]
 # Packed-fp32 VALU forms stay off for every device function.
+# Reads lists of torch tensors for the optimizer step (host code; a Python module, since it handles Python objects).
+SCAN_LIB = os.path.join(HERE, "_scan.so")
 HIP_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -55,10 +57,27 @@ def _compile_and_link(sources, lib, hipcc, verbose):
     return lib
 
 
+def _build_scan(verbose):
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *[f"-isystem{p}" for p in include_paths()], f"-isystem{sysconfig.get_paths()['include']}", os.path.join(CSRC, "scan.cpp"), "-o", SCAN_LIB,
+           *[f"-L{p}" for p in library_paths()], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on scan.cpp:\n{r.stdout}")
+
+
 def build_library(verbose: bool = False) -> str:
     hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
     if not os.path.exists(hipcc):
         raise RuntimeError("hipcc not found; cannot build libmuon_hip.so")
+    _build_scan(verbose)
     _compile_and_link(PROBE_SOURCES, PROBE_LIB, hipcc, verbose)
     return _compile_and_link(SOURCES, LIB, hipcc, verbose)
 

@@ -29,6 +29,13 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
     norm_type = float(norm_type)
     if norm_type != norm_type:
         raise ValueError("norm_type is NaN")
+    plain = _abi.scan().grads(parameters, _abi.MULTI_CHUNK)
+    if plain is not None:
+        index, lists = plain
+        dev = torch.device("cuda", index)
+        return _clip(dev, sum(n for _, n, _, _ in lists), [code for code, *_ in lists],
+                     lambda: [TensorListTable.of_words(words, 1, n, chunks, dev, _abi.DTYPES[code]) for code, n, chunks, words in lists],
+                     max_norm, norm_type, error_if_nonfinite)
     grads = [g for g in [p.grad for p in parameters] if g is not None]
     if len(grads) == 0:
         return torch.tensor(0.0)  # what _get_total_norm returns for an empty list
@@ -49,23 +56,29 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
         if same is None:
             same = groups[g.dtype] = []
         same.append(c)
+    total = _clip(dev, len(grads), [_abi.dtype_code(dt) for dt in groups], lambda: [TensorListTable([gs]) for gs in groups.values()], max_norm,
+                  norm_type, error_if_nonfinite)
+    for g, c in strided:
+        g.copy_(c)
+    return total
+
+
+def _clip(dev, n_total, codes, make_tables, max_norm, norm_type, error_if_nonfinite) -> Tensor:
+    """The norm of the lists that make_tables() describes, one per dtype code, and their scaling."""
     lib = _abi.lib()
     # torch stacks the per-tensor norms of all dtype groups; stacking promotes, so the total has the widest dtype
-    out_dtype = torch.float32 if torch.float32 in groups else torch.bfloat16
-    n_total = len(grads)
+    out_dtype = torch.float32 if _abi.F32 in codes else torch.bfloat16
     with torch.cuda.device(dev):
         s = _abi.stream_ptr(dev)
         norms = torch.empty(n_total, dtype=torch.float32, device=dev)
         total_f32 = torch.empty(1, dtype=torch.float32, device=dev)
         total = torch.empty((), dtype=out_dtype, device=dev)
-        tables, off = [], 0
-        for dt, gs in groups.items():
-            tab = TensorListTable([gs])
-            tables.append((dt, tab))
+        tables, off = make_tables(), 0
+        for code, tab in zip(codes, tables):
             if tab.chunks > 0:
                 partials = torch.empty(tab.chunks, dtype=torch.float32, device=dev)
                 _abi.check(lib.muon_hip_grad_norms(tab.role_ptrs[0], tab.numel_ptr, tab.chunk_start_ptr, tab.n, tab.chunks,
-                                                   _abi.dtype_code(dt), norm_type, partials.data_ptr(), norms.data_ptr() + 4 * off, s),
+                                                   code, norm_type, partials.data_ptr(), norms.data_ptr() + 4 * off, s),
                            "grad_norms")
             else:
                 norms[off:off + tab.n].zero_()
@@ -77,13 +90,11 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
                 f"The total norm of order {norm_type} for gradients from `parameters` is non-finite, so it "
                 "cannot be clipped. To disable this error and scale the gradients by the non-finite norm anyway, "
                 "set `error_if_nonfinite=False`")
-        for dt, tab in tables:
+        for code, tab in zip(codes, tables):
             if tab.chunks > 0:
                 _abi.check(lib.muon_hip_clip_scale(tab.role_ptrs[0], tab.numel_ptr, tab.chunk_start_ptr, tab.n, tab.chunks,
-                                                   _abi.dtype_code(dt), total_f32.data_ptr(), _abi.dtype_code(out_dtype),
+                                                   code, total_f32.data_ptr(), _abi.dtype_code(out_dtype),
                                                    float(max_norm), s), "clip_scale")
-        for g, c in strided:
-            g.copy_(c)
     return total
 
 

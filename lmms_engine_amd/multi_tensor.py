@@ -50,13 +50,26 @@ class TensorListTable:
             words.extend([t.data_ptr() for t in r])
         words.extend(numel)
         words.extend(starts)
+        self._put(bytearray(words.tobytes()), len(roles), doubles)
+        self._keep += ([list(r) for r in roles],)  # the tensors stay alive while kernels may read them
+
+    @classmethod
+    def of_words(cls, words: bytearray, roles: int, n: int, chunks: int, device, dtype, doubles: Sequence[Sequence[float]] = ()):
+        """A table whose rows `_abi.scan()` has put together: pointers of `roles` roles, element counts, first chunks."""
+        self = cls.__new__(cls)
+        self.n, self.chunks, self.device, self.dtype = n, chunks, device, dtype
+        self._put(words, roles, doubles)
+        return self
+
+    def _put(self, words: bytearray, k: int, doubles) -> None:
+        n = self.n
         for d in doubles:
-            words.frombytes(array("d", d).tobytes())
-        host = torch.empty(len(words), dtype=torch.int64, pin_memory=True)
+            words += array("d", d).tobytes()
+        host = torch.empty(len(words) // 8, dtype=torch.int64, pin_memory=True)
         host.copy_(torch.frombuffer(words, dtype=torch.int64))
         self.table = host.to(self.device, non_blocking=True)
-        self._keep = (host, [list(r) for r in roles])  # the tensors stay alive while kernels may read them
-        base, k = self.table.data_ptr(), len(roles)
+        self._keep = (host,)
+        base = self.table.data_ptr()
         self.role_ptrs = [base + 8 * n * i for i in range(k)]
         self.numel_ptr = base + 8 * n * k
         self.chunk_start_ptr = self.numel_ptr + 8 * n

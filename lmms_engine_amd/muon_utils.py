@@ -22,6 +22,7 @@ Differences from the reference, all deliberate:
 from __future__ import annotations
 
 import logging
+from array import array
 from collections import OrderedDict, deque
 from itertools import chain
 from typing import Optional, Protocol
@@ -76,11 +77,15 @@ def _workspace(nbytes: int, device) -> Tensor:
     return torch.empty(nbytes, dtype=torch.uint8, device=device)
 
 
-def _pointer_table(tensors, device, cache=None, key=None) -> Tensor:
-    """Device table of the tensors' base pointers.  With a cache (a _TableCache), a table whose pointers have not changed
+def _pointers(tensors) -> bytes:
+    """The tensors' base pointers as 64-bit words."""
+    return array("q", [t.data_ptr() for t in tensors]).tobytes()
+
+
+def _pointer_table(ptrs: bytes, device, cache=None, key=None) -> Tensor:
+    """Device table of base pointers (_pointers).  With a cache (a _TableCache), a table whose pointers have not changed
     since the last call under `key` is handed back as it is: no host allocation and no copy, which is what lets a step
     over static tensors be recorded into a HIP graph (and saves the copy otherwise)."""
-    ptrs = tuple(t.data_ptr() for t in tensors)
     if cache is not None:
         hit = cache.tables.get(key)
         if hit is not None and hit[0] == ptrs and hit[1].device == device:
@@ -93,7 +98,8 @@ def _pointer_table(tensors, device, cache=None, key=None) -> Tensor:
             "and momentum buffers must keep their addresses (run an eager step first and do not re-allocate grads, "
             "e.g. zero_grad(set_to_none=False))"
         )
-    host = torch.tensor(ptrs, dtype=torch.int64, pin_memory=True)
+    host = torch.empty(len(ptrs) // 8, dtype=torch.int64, pin_memory=True)
+    host.copy_(torch.frombuffer(bytearray(ptrs), dtype=torch.int64))
     table = host.to(device, non_blocking=True)
     if cache is not None:
         cache.replace(key, ptrs, table)
@@ -239,7 +245,7 @@ def apply_momentum(grad: Tensor, momentum: Tensor, beta: float, nesterov: bool) 
     rows, cols = g2.shape
     with torch.cuda.device(grad.device):
         ws = _workspace(_abi.workspace_bytes(rows, cols, 1), grad.device)
-        gt, mt = _pointer_table([gc], grad.device), _pointer_table([mc], grad.device)
+        gt, mt = _pointer_table(_pointers([gc]), grad.device), _pointer_table(_pointers([mc]), grad.device)
         _abi.check(
             _abi.lib().muon_hip_momentum_norm(gt.data_ptr(), mt.data_ptr(), _abi.dtype_code(grad.dtype),
                                               _abi.dtype_code(momentum.dtype), ws.data_ptr(), rows, cols, 1,
@@ -356,49 +362,44 @@ def _held_workspace(ws_holder, dev, need: int) -> Tensor:
     return ws
 
 
-def _muon_buckets_step(buckets, group, ns_steps, nesterov, write_back_grad, ws_holder, ws_limit, tables=None):
-    """All stages of the Muon step for `buckets`, a list of (params, grads, moms) of one shape each; all of them on one
-    device and of the same three dtypes.
+def _muon_buckets_step(buckets, dev, codes, group, ns_steps, nesterov, write_back_grad, ws_holder, ws_limit, tables=None):
+    """All stages of the Muon step for `buckets` on `dev`, a list of (rows, cols, matrices, pointers of the parameters, of the
+    gradients, of the momentum buffers) of one shape each (_pointers); `codes`: the three dtype codes of all of them.
 
     Buckets that fit the workspace limit together share one library call, whose launches work on all of them: the matrices of
     one shape alone leave most of the machine idle in a small model (56 matrices of four shapes: 77 launches, 993 us of
     kernels).  A bucket that exceeds the limit on its own is cut into chunks, one call each."""
     lib = _abi.lib()
-    p0, g0, m0 = (t[0] for t in buckets[0])
-    dev = p0.device
-    codes = (_abi.dtype_code(p0.dtype), _abi.dtype_code(g0.dtype), _abi.dtype_code(m0.dtype))
     hyper = (float(group["lr"]), float(group["weight_decay"]), float(group["momentum"]), int(bool(nesterov)), int(ns_steps), *NS_COEFFS,
              int(bool(write_back_grad)))
-    calls = []  # lists of (rows, cols, params, grads, moms)
+    calls = []  # lists of buckets
     together, used = [], 0
-    for params, grads, moms in buckets:
-        rows, cols = params[0].shape
-        n = len(params)
+    for rows, cols, n, *roles in buckets:
         chunk = _pick_chunk(n, max(1, min(ws_limit // _abi.workspace_bytes(rows, cols, 1), 65535)), rows, cols, _cu_count(dev))
         if chunk < n:
             for lo in range(0, n, chunk):
-                calls.append([(rows, cols, params[lo:lo + chunk], grads[lo:lo + chunk], moms[lo:lo + chunk])])
+                calls.append([(rows, cols, min(chunk, n - lo), *[r[8 * lo:8 * (lo + chunk)] for r in roles])])
             continue
         need = _abi.workspace_bytes(rows, cols, n)
         if together and (used + need > ws_limit or len(together) == _abi.MAX_BUCKETS):
             calls.append(together)
             together, used = [], 0
-        together.append((rows, cols, params, grads, moms))
+        together.append((rows, cols, n, *roles))
         used += need
     if together:
         calls.append(together)
     with torch.cuda.device(dev):
         s = _abi.stream_ptr(dev)
         for index, call in enumerate(calls):
-            ws = _held_workspace(ws_holder, dev, sum(_abi.workspace_bytes(rows, cols, len(ps)) for rows, cols, ps, _, _ in call))
-            tensors = [t for _, _, ps, gs, ms in call for t in chain(ps, gs, ms)]
-            table = _pointer_table(tensors, dev, tables, (id(group), dev, codes, index))
+            ws = _held_workspace(ws_holder, dev, sum(_abi.workspace_bytes(rows, cols, n) for rows, cols, n, *_ in call))
+            ptrs = b"".join([r for _, _, _, *roles in call for r in roles])
+            table = _pointer_table(ptrs, dev, tables, (id(group), dev, codes, index))
             at = table.data_ptr()
             args = (_abi.Bucket * len(call))()
-            for arg, (rows, cols, ps, _, _) in zip(args, call):
-                step = 8 * len(ps)
+            for arg, (rows, cols, n, *_) in zip(args, call):
+                step = 8 * n
                 arg.p_ptrs, arg.g_ptrs, arg.m_ptrs = at, at + step, at + 2 * step
-                arg.rows, arg.cols, arg.batch = rows, cols, len(ps)
+                arg.rows, arg.cols, arg.batch = rows, cols, n
                 arg.scale = scale_factor(rows, cols, group["rms_scale"])
                 at += 3 * step
             _abi.check(lib.muon_hip_step_multi(args, len(call), *codes, ws.data_ptr(), *hyper, s), "step_multi")
@@ -458,8 +459,9 @@ class SingelDeviceWork:
         ns_steps, nesterov = g["ns_steps"], g["nesterov"]
         if self.reference_bug_compat:
             ns_steps, nesterov = int(bool(g["nesterov"])), bool(g["ns_steps"])
-        _muon_buckets_step([([self.param], [self.param.grad], [self.state["momentum_buffer"]])], g, ns_steps, nesterov,
-                           self.write_back_grad, {}, 1 << 62)
+        trio = (self.param, self.param.grad, self.state["momentum_buffer"])
+        _muon_buckets_step([(*self.param.shape, 1, *[_pointers([t]) for t in trio])], self.param.device,
+                           tuple(_abi.dtype_code(t.dtype) for t in trio), g, ns_steps, nesterov, self.write_back_grad, {}, 1 << 62)
 
     def finish(self):
         pass
@@ -585,6 +587,10 @@ class Muon(torch.optim.Optimizer):
         self._recorded = False
 
     def _adam_group_step(self, group) -> None:
+        plain = _abi.scan().adam(group["params"], self.state, _abi.MULTI_CHUNK)
+        if plain is not None:
+            _adamw_plain(plain, group)
+            return
         items = []
         for p in group["params"]:
             if p.grad is None:
@@ -617,6 +623,11 @@ class Muon(torch.optim.Optimizer):
             state["momentum_buffer"] = torch.zeros_like(p, dtype=self.momentum_dtype or p.dtype)
         return state
 
+    def _plain_work(self) -> bool:
+        """Whether every plain tensor takes the single-device work with its state as this class keeps it."""
+        cls = type(self)
+        return cls._get_work_class is Muon._get_work_class and cls._init_muon_state is Muon._init_muon_state
+
     @torch.no_grad()
     def step_fsdp(self, closure=None):
         loss = None
@@ -630,6 +641,18 @@ class Muon(torch.optim.Optimizer):
             self._recorded = True
         for group in self.param_groups:
             if group["use_muon"]:
+                ns_steps, nesterov = group["ns_steps"], group["nesterov"]
+                if self.reference_bug_compat:
+                    ns_steps, nesterov = int(bool(group["nesterov"])), bool(group["ns_steps"])
+                how = (group, ns_steps, nesterov, self.write_back_grad, self._workspaces, self.workspace_limit_bytes, self._pointer_tables)
+                plain = _abi.scan().muon(group["params"], self.state) if self._plain_work() else None
+                if plain is not None:
+                    alike = {}
+                    for dev, rows, cols, *codes, n, p, g, m in plain:
+                        alike.setdefault((dev, *codes), []).append((rows, cols, n, p, g, m))
+                    for (dev, *codes), bs in alike.items():
+                        _muon_buckets_step(bs, torch.device("cuda", dev), tuple(codes), *how)
+                    continue
                 buckets: "OrderedDict[tuple, list]" = OrderedDict()
                 strided = []
                 for i, p in enumerate(group["params"]):
@@ -663,15 +686,11 @@ class Muon(torch.optim.Optimizer):
                     if same is None:
                         same = buckets[key] = []
                     same.append((pc, g, mc))
-                ns_steps, nesterov = group["ns_steps"], group["nesterov"]
-                if self.reference_bug_compat:
-                    ns_steps, nesterov = int(bool(group["nesterov"])), bool(group["ns_steps"])
-                alike: "OrderedDict[tuple, list]" = OrderedDict()  # buckets of one device and the same dtypes
-                for (dev, _, *dtypes), items in buckets.items():
-                    alike.setdefault((dev, *dtypes), []).append(tuple(list(t) for t in zip(*items)))
-                for bs in alike.values():
-                    _muon_buckets_step(bs, group, ns_steps, nesterov, self.write_back_grad, self._workspaces,
-                                       self.workspace_limit_bytes, self._pointer_tables)
+                alike = {}  # buckets of one device and the same dtypes
+                for (dev, shape, *dtypes), items in buckets.items():
+                    alike.setdefault((dev, *dtypes), []).append((*shape, len(items), *[_pointers(t) for t in zip(*items)]))
+                for (dev, *dtypes), bs in alike.items():
+                    _muon_buckets_step(bs, torch.device("cuda", dev), tuple(_abi.dtype_code(dt) for dt in dtypes), *how)
                 for p, pc, m, mc, g in strided:
                     if pc is not p:
                         p.copy_(pc)
@@ -688,6 +707,32 @@ class Muon(torch.optim.Optimizer):
             work.finish()
 
         return loss
+
+
+def _adamw_plain(plain, group: dict) -> None:
+    """_adamw_group for a list that needs no decision (csrc/scan.cpp)."""
+    from .multi_tensor import TensorListTable
+
+    index, code, steps, chunks, words = plain
+    dev = torch.device("cuda", index)
+    b1, b2 = float(group["betas"][0]), float(group["betas"][1])
+    with torch.cuda.device(dev):
+        _adamw_launch(TensorListTable.of_words(words, 4, len(steps), chunks, dev, _abi.DTYPES[code], _bias(steps, b1, b2)), code, group)
+
+
+def _bias(steps, b1: float, b2: float):
+    once = {st: (1 - b1 ** st, 1 - b2 ** st) for st in set(steps)}
+    return [[once[st][0] for st in steps], [once[st][1] for st in steps]]
+
+
+def _adamw_launch(tab, code: int, group: dict) -> None:
+    _abi.check(
+        _abi.lib().muon_hip_adamw_multi(
+            *tab.role_ptrs, tab.numel_ptr, tab.chunk_start_ptr, *tab.double_ptrs, tab.n, tab.chunks, code, float(group["lr"]),
+            float(group["betas"][0]), float(group["betas"][1]), float(group["eps"]), float(group["weight_decay"]), _abi.stream_ptr(tab.device),
+        ),
+        "adamw_multi",
+    )
 
 
 def _adamw_group(items, group: dict) -> None:
@@ -716,15 +761,7 @@ def _adamw_group(items, group: dict) -> None:
     for (dev, dt), its in buckets.items():
         ps, gs, e1s, e2s, steps = (list(t) for t in zip(*its))
         with torch.cuda.device(dev):
-            tab = TensorListTable([ps, gs, e1s, e2s], doubles=[[1 - b1 ** st for st in steps], [1 - b2 ** st for st in steps]])
-            _abi.check(
-                _abi.lib().muon_hip_adamw_multi(
-                    *tab.role_ptrs, tab.numel_ptr, tab.chunk_start_ptr, *tab.double_ptrs, tab.n, tab.chunks,
-                    _abi.dtype_code(dt), float(group["lr"]), b1, b2, float(group["eps"]), float(group["weight_decay"]),
-                    _abi.stream_ptr(dev),
-                ),
-                "adamw_multi",
-            )
+            _adamw_launch(TensorListTable([ps, gs, e1s, e2s], doubles=_bias(steps, b1, b2)), _abi.dtype_code(dt), group)
     for t, c in strided:
         t.copy_(c)
 

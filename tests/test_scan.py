@@ -1,0 +1,127 @@
+"""The native reader of tensor lists: what it takes, what it leaves to the callers' own loops, and that both give the same step."""
+import numpy as np
+import pytest
+import torch
+
+from lmms_engine_amd import _abi
+from tests.test_gpu_parity import env  # noqa: F401
+
+
+def test_cpu_tensors_and_other_things_are_left_to_the_caller():
+    scan = _abi.scan()
+    p = torch.nn.Parameter(torch.zeros(3, 4))
+    p.grad = torch.ones(3, 4)
+    state = {p: {"momentum_buffer": torch.zeros(3, 4), "exp_avg": torch.zeros(3, 4), "exp_avg_sq": torch.zeros(3, 4), "step": 4}}
+    for params in ([p], (p,), [], [None], "p", [torch.nn.Parameter(torch.zeros(0))]):
+        assert scan.grads(params, 16384) is None
+        assert scan.muon(params, state) is None or params == []
+        assert scan.adam(params, state, 16384) is None
+    assert scan.muon([p], None) is None and scan.adam([p], [], 16384) is None and scan.grads([p], 0) is None
+    assert state[p]["step"] == 4
+
+
+def _set(dev, dtype, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    shapes = [(96, 40), (128, 256), (96, 40), (300, 20), (128, 256)]
+    mats = [torch.nn.Parameter((0.02 * torch.randn(*s, generator=g)).to(dtype).to(dev)) for s in shapes]
+    rest = [torch.nn.Parameter(torch.randn(n, generator=g).to(dtype).to(dev)) for n in (5, 16384 * 2 + 3, 7)]
+    for p in mats + rest:
+        p.grad = torch.randn(p.shape, generator=g).to(dtype).to(dev)
+    return mats, rest
+
+
+def _optimizer(mu, mats, rest, mdtype=None):
+    return mu.Muon([dict(params=list(mats), use_muon=True, lr=0.02, momentum=0.95, nesterov=True, weight_decay=0.01, ns_steps=5, rms_scale=True),
+                    dict(params=list(rest), use_muon=False, lr=1e-3, betas=(0.9, 0.95), eps=1e-8, weight_decay=0.01)], momentum_dtype=mdtype)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,mdtype", [(torch.float32, None), (torch.bfloat16, torch.float32)])
+def test_step_and_clipping_equal_the_callers_own_loops(env, monkeypatch, dtype, mdtype):
+    from lmms_engine_amd.clip_grad import clip_grad_norm_
+
+    mu, dev = env["mu"], env["dev"]
+
+    class Loops:
+        grads = muon = adam = staticmethod(lambda *a: None)
+
+    out = []
+    for own in (False, True):
+        mats, rest = _set(dev, dtype)
+        opt = _optimizer(mu, mats, rest, mdtype)
+        opt.step()  # makes the state: nobody's fast path
+        scan = _abi.scan()
+        assert scan.muon(opt.param_groups[0]["params"], opt.state) and scan.grads(mats + rest, 16384)
+        with monkeypatch.context() as m:
+            if own:
+                m.setattr(_abi, "scan", lambda: Loops)
+            totals = []
+            for _ in range(3):
+                totals.append(clip_grad_norm_(mats + rest, 1.0).clone())
+                opt.step()
+        torch.cuda.synchronize()
+        out.append((mats + rest, totals, [opt.state[p]["step"] for p in rest], [opt.state[p]["momentum_buffer"] for p in mats],
+                    [p.grad for p in mats + rest], [opt.state[p]["exp_avg_sq"] for p in rest]))
+    a, b = out
+    assert a[2] == b[2] == [4, 4, 4]
+    for x, y in zip(a[0] + a[1] + a[3] + a[4] + a[5], b[0] + b[1] + b[3] + b[4] + b[5]):
+        assert torch.equal(x.detach(), y.detach())
+
+
+@pytest.mark.gpu
+def test_addresses_sizes_and_order(env):
+    mats, rest = _set(env["dev"], torch.float32)
+    opt = _optimizer(env["mu"], mats, rest)
+    opt.step()
+    ps = opt.param_groups[0]["params"]
+    for dev, rows, cols, pc, gc, mc, n, p, g, m in _abi.scan().muon(ps, opt.state):
+        mine = [q for q in ps if tuple(q.shape) == (rows, cols)]
+        assert (dev, pc, gc, mc, n) == (mats[0].get_device(), 0, 0, 0, len(mine))
+        for words, ts in ((p, mine), (g, [q.grad for q in mine]), (m, [opt.state[q]["momentum_buffer"] for q in mine])):
+            assert np.frombuffer(words, np.int64).tolist() == [t.data_ptr() for t in ts]
+    _, ((code, n, chunks, words),) = _abi.scan().grads(rest, 16384)
+    assert (code, n, chunks) == (0, 3, 1 + 3 + 1)
+    assert np.frombuffer(words, np.int64).tolist() == [p.grad.data_ptr() for p in rest] + [p.numel() for p in rest] + [0, 1, 4, 5]
+
+
+@pytest.mark.gpu
+def test_lists_that_need_a_decision_are_left_to_the_caller(env):
+    dev, scan = env["dev"], _abi.scan()
+    for change in ("no grad", "strided grad", "strided parameter", "grad of another dtype", "no state", "shape", "subclass", "float step", "twice"):
+        mats, rest = _set(dev, torch.float32)
+        opt = _optimizer(env["mu"], mats, rest)
+        opt.step()
+        p, q, params = mats[0], rest[1], list(rest)
+        if change == "no grad":
+            p.grad = q.grad = None
+        elif change == "strided grad":
+            p.grad = torch.randn(40, 96, device=dev).t()
+            q.grad = torch.randn(q.numel(), 2, device=dev)[:, 0]
+        elif change == "strided parameter":
+            p.data = torch.randn(40, 96, device=dev).t()
+            q.data = torch.randn(q.numel(), 2, device=dev)[:, 0]
+        elif change == "grad of another dtype":
+            p.data, q.data = p.data.bfloat16(), q.data.bfloat16()
+            opt.state[p]["momentum_buffer"] = opt.state[p]["momentum_buffer"].half()
+        elif change == "no state":
+            opt.state[p], opt.state[q] = {}, {}
+        elif change == "shape":
+            opt.state[p]["momentum_buffer"] = torch.zeros(40, 96, device=dev)
+            opt.state[q]["exp_avg"] = torch.zeros(3, device=dev)
+        elif change == "subclass":
+            class Sub(torch.nn.Parameter):
+                pass
+            for old in (p, q):
+                new = Sub(old.detach().clone())
+                new.grad, opt.state[new] = old.grad, opt.state[old]
+                mats, params = [new if t is old else t for t in mats], [new if t is old else t for t in params]
+        elif change == "float step":
+            opt.state[q]["step"] = 2.0
+            opt.state[p]["momentum_buffer"] = None
+        elif change == "twice":
+            params.append(q)
+            opt.state[p]["momentum_buffer"] = opt.state[p]["momentum_buffer"].cpu()
+        before = [opt.state[t].get("step") for t in rest]
+        assert scan.muon(mats, opt.state) is None, change
+        assert scan.adam(params, opt.state, 16384) is None, change
+        assert [opt.state[t].get("step") for t in rest] == before, change
