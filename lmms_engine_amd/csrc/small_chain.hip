@@ -43,37 +43,57 @@ __device__ __forceinline__ float update_one(float p, bf16_t x, float scale, floa
     return fmaf(alpha, os, pd);
 }
 
-// Eight consecutive columns of one row of X to the parameter: a piece of its row, or (turned) of its column.
+// Eight consecutive columns of one row of X meet the parameter: a piece of its row, or (turned) of its column.  In two halves, so that
+// the loads of several pieces are in flight before the first store (the compiler cannot know that the pieces are apart: one after the
+// other they cost a trip to memory each, eight for a turned piece; see kBatch).
+struct Piece {
+    float v[8];
+};
+__device__ __forceinline__ bool whole_rows(const void* p, int cols, bool turn) { return !turn && cols % 8 == 0 && (((uintptr_t)p) & 15) == 0; }
 template <typename PT>
-__device__ __forceinline__ void update8(PT* p, const bf16x8& x, int row, int col, int cols, int M, int K, bool turn, float scale,
-                                        float decay, float alpha) {
-    if (turn) {
-        for (int e = 0; e < 8 && col + e < K; ++e) {
-            PT* d = p + (long)(col + e) * M + row;
-            *d = (PT)update_one<PT>((float)*d, x[e], scale, decay, alpha);
+__device__ __forceinline__ void load8(Piece& o, const PT* p, int row, int col, int cols, int M, int K, bool turn, bool whole) {
+    if (whole) {  // eight columns are all there or none is
+        const PT* d = p + (long)row * cols + col;
+        if constexpr (sizeof(PT) == 2) {
+            const bf16x8 v = *(const bf16x8*)d;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o.v[e] = bf2f(v[e]);
+        } else {
+            const f32x4 v = *(const f32x4*)d, w = *(const f32x4*)(d + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o.v[e] = v[e], o.v[4 + e] = w[e];
         }
         return;
     }
-    PT* d = p + (long)row * cols + col;
-    if (cols % 8 == 0 && (((uintptr_t)p) & 15) == 0) {  // eight columns are all there or none is
-        if constexpr (sizeof(PT) == 2) {
-            bf16x8 v = *(const bf16x8*)d;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = f2bf(update_one<PT>(bf2f(v[e]), x[e], scale, decay, alpha));
+    for (int e = 0; e < 8; ++e)
+        if (col + e < K) o.v[e] = (float)p[turn ? (long)(col + e) * M + row : (long)row * cols + col + e];
+}
+template <typename PT>
+__device__ __forceinline__ void store8(PT* p, const Piece& o, const bf16x8& x, int row, int col, int cols, int M, int K, bool turn, bool whole, float scale,
+                                       float decay, float alpha) {
+    if (whole) {
+        PT* d = p + (long)row * cols + col;
+        if constexpr (sizeof(PT) == 2) {
+            bf16x8 v;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = f2bf(update_one<PT>(o.v[e], x[e], scale, decay, alpha));
             *(bf16x8*)d = v;
         } else {
-            f32x4 v = *(const f32x4*)d, w = *(const f32x4*)(d + 4);
+            f32x4 v, w;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                v[e] = update_one<PT>(v[e], x[e], scale, decay, alpha);
-                w[e] = update_one<PT>(w[e], x[4 + e], scale, decay, alpha);
+                v[e] = update_one<PT>(o.v[e], x[e], scale, decay, alpha);
+                w[e] = update_one<PT>(o.v[4 + e], x[4 + e], scale, decay, alpha);
             }
             *(f32x4*)d = v;
             *(f32x4*)(d + 4) = w;
         }
         return;
     }
-    for (int e = 0; e < 8 && col + e < K; ++e) d[e] = (PT)update_one<PT>((float)d[e], x[e], scale, decay, alpha);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        if (col + e < K) p[turn ? (long)(col + e) * M + row : (long)row * cols + col + e] = (PT)update_one<PT>(o.v[e], x[e], scale, decay, alpha);
 }
 
 // The row that lane i of 16 holds in block t of 16 rows.  The turned fragment of a block has rows i = 4q .. 4q+3 of it in lane group
@@ -101,12 +121,24 @@ __device__ __forceinline__ bf16x8 gather_rows16(const bf16x4& v) {
 constexpr int CHAIN_WAVES = 8;
 constexpr int CHAIN_FRAGS = 32;  // fragments of X a lane can hold: 128 of the 256 registers of a wave
 
+// Fragments that a lane loads from memory (the blend; the parameter) together, while those before them are still on their way: loads and
+// stores leave the queue in order, so a load that is issued behind a store waits for it as well.  One at a time, as written before, 56
+// matrices of 5632 x 16 in fp32 took 142 us, now 117 (with four 117 as well, at the cost of 20 to 50 registers); 168 + 84 + 56 of 2048 and 512 columns
+// 60 and 53; 256 of 2048 x 64 296 and 212.  Asking for the parameter before the iterations, through LDS, gave nothing on top.
+constexpr int kBatch = 2;
+
 // MT blocks of 16 rows (1, 2 or 4), up to NCH chunks of 32 columns per wave.
 template <int MT, int NCH>
 __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainList l, const ChainMath cm) {
     constexpr int NP = (MT + 1) / 2;         // 32-deep reductions over the rows
     constexpr int PITCH = 32 * NP + 8;       // of A and B in LDS; with MT = 1 columns 16 to 31 stay zero
     constexpr int NF = MT * (MT + 1) / 2;    // 16 x 16 blocks of A on or above the diagonal
+    constexpr int BATCH = kBatch < MT ? 1 : kBatch / MT;  // chunks that are loaded from memory together
+    constexpr bool TWO = MT < 4;             // while the next ones are on their way (with four blocks a chunk is enough, and two spill)
+    // Chunks without a branch between them: 40 -> 30 ns for each MFMA of the chain through 176 chunks (16 x 5632).  Four blocks have
+    // ten MFMAs between two branches anyway.
+    constexpr int RUN = MT == 4 ? 1 : 4;
+    static_assert(NCH % RUN == 0, "whole runs");
     constexpr int LEG = MT == 4 ? 2 : 1, NLEG = NF / LEG;  // blocks that a wave adds its chunks to at a time
     __shared__ __align__(16) f32x4 sum[NF][64];
     __shared__ __align__(16) bf16_t As[MT * 16][PITCH], Bs[MT * 16][PITCH];
@@ -141,22 +173,41 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
     // Normalised fragments, zero past the matrix's edges.  Through the work area, so that the loop over loads of every kind
     // (ragged, turned) and divisions need not be unrolled over the register array.
     const bool vec = !turn && K % 8 == 0;
-#pragma unroll 4
-    for (int j = 0; j < per; ++j) {
+    {
+        bf16x8 v[TWO ? 2 : 1][BATCH][MT];
+        auto each = [&](int j0, auto f) {
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            const int row = chain_row<MT>(t, i), col = col0 + j * 32;
-            bf16x8 v;
-            if (vec && row < M && col < K) {
-                v = *(const bf16x8*)(u + (long)row * K + col);
-            } else {
+            for (int jj = 0; jj < BATCH; ++jj)
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    v[e] = (row < M && col + e < K) ? u[turn ? (long)(col + e) * M + row : (long)row * K + col + e] : (bf16_t)0.f;
+                for (int t = 0; t < MT; ++t)
+                    if (j0 + jj < per) f(jj, t, chain_row<MT>(t, i), col0 + (j0 + jj) * 32);
+        };
+        auto load = [&](int j0, bf16x8 (&w)[BATCH][MT]) {
+            each(j0, [&](int jj, int t, int row, int col) {
+                if (vec && row < M && col < K) {
+                    w[jj][t] = *(const bf16x8*)(u + (long)row * K + col);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        w[jj][t][e] = (row < M && col + e < K) ? u[turn ? (long)(col + e) * M + row : (long)row * K + col + e] : (bf16_t)0.f;
+                }
+            });
+        };
+        auto put = [&](int j0, bf16x8 (&w)[BATCH][MT]) {
+            each(j0, [&](int jj, int t, int, int) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) w[jj][t][e] = f2bf(__fdiv_rn(bf2f(w[jj][t][e]), d));
+                mine[((j0 + jj) * MT + t) * 64] = w[jj][t];
+            });
+        };
+        if constexpr (TWO) load(0, v[0]);
+        for (int j0 = 0; j0 < per; j0 += (TWO ? 2 : 1) * BATCH) {
+            load(TWO ? j0 + BATCH : j0, v[TWO ? 1 : 0]);
+            put(j0, v[0]);
+            if constexpr (TWO) {
+                load(j0 + 2 * BATCH, v[0]);
+                put(j0 + BATCH, v[1]);
             }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = f2bf(__fdiv_rn(bf2f(v[e]), d));
-            mine[(j * MT + t) * 64] = v;
         }
     }
     bf16x8 zero8, unit[2];  // unit[h]: selects columns 8q' + 4h + 0..3 (q' = 0..3) of a chunk
@@ -178,8 +229,10 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
 #pragma unroll
         for (int f = 0; f < LEG; ++f) acc[f] = wave == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum[F0 + f][lane];
 #pragma unroll
-        for (int j = 0; j < NCH; ++j)
-            if (j < per) {
+        for (int j0 = 0; j0 < NCH; j0 += RUN) {
+            if (j0 >= per) continue;
+#pragma unroll
+            for (int j = j0; j < j0 + RUN; ++j) {  // (past the wave's last chunk x is zero, and the sum plus zero is the sum)
                 int f = 0;
 #pragma unroll
                 for (int ti = 0; ti < MT; ++ti)
@@ -187,6 +240,7 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
                     for (int tj = ti; tj < MT; ++tj, ++f)
                         if (f >= F0 && f < F0 + LEG) acc[f - F0] = mfma(x[j][ti], x[j][tj], acc[f - F0]);
             }
+        }
 #pragma unroll
         for (int f = 0; f < LEG; ++f) sum[F0 + f][lane] = acc[f];
     };
@@ -263,8 +317,16 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
                 }
         };
 #pragma unroll
-        for (int j = 0; j < NCH; ++j)
-            if (j < per) next_chunk(x[j]);
+        for (int j0 = 0; j0 < NCH; j0 += RUN) {
+            if (j0 + RUN <= per) {
+#pragma unroll
+                for (int j = j0; j < j0 + RUN; ++j) next_chunk(x[j]);
+            } else {  // (nothing is computed past the last chunk: with an infinite B its zeros would not stay zero)
+#pragma unroll
+                for (int j = j0; j < j0 + RUN - 1; ++j)
+                    if (j < per) next_chunk(x[j]);
+            }
+        }
     }
 
     if (!k.p_ptrs) {
@@ -283,15 +345,44 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         for (int t = 0; t < MT; ++t)
             if (j < per) mine[(j * MT + t) * 64] = x[j][t];
     void* p = const_cast<void*>(k.p_ptrs[b]);
-    for (int j = 0; j < per; ++j)
+    const bool whole = whole_rows(p, k.cols, turn);
+    auto update = [&](auto* pp) {
+        struct Batch {
+            Piece o[BATCH][MT];
+            bf16x8 v[BATCH][MT];
+        } w[TWO ? 2 : 1];
+        auto each = [&](int j0, auto f) {
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            const int row = chain_row<MT>(t, i), col = col0 + j * 32;
-            if (row >= M || col >= K) continue;
-            const bf16x8 v = mine[(j * MT + t) * 64];
-            if (cm.p_dtype == MUON_HIP_BF16) update8((bf16_t*)p, v, row, col, k.cols, M, K, turn, k.scale, cm.decay, cm.alpha);
-            else update8((float*)p, v, row, col, k.cols, M, K, turn, k.scale, cm.decay, cm.alpha);
+            for (int jj = 0; jj < BATCH; ++jj)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    const int row = chain_row<MT>(t, i), col = col0 + (j0 + jj) * 32;
+                    if (j0 + jj < per && row < M && col < K) f(jj, t, row, col);
+                }
+        };
+        auto load = [&](int j0, Batch& w) {
+            each(j0, [&](int jj, int t, int row, int col) {
+                w.v[jj][t] = mine[((j0 + jj) * MT + t) * 64];
+                load8(w.o[jj][t], pp, row, col, k.cols, M, K, turn, whole);
+            });
+        };
+        auto store = [&](int j0, Batch& w) {
+            each(j0, [&](int jj, int t, int row, int col) {
+                store8(pp, w.o[jj][t], w.v[jj][t], row, col, k.cols, M, K, turn, whole, k.scale, cm.decay, cm.alpha);
+            });
+        };
+        if constexpr (TWO) load(0, w[0]);
+        for (int j0 = 0; j0 < per; j0 += (TWO ? 2 : 1) * BATCH) {
+            load(TWO ? j0 + BATCH : j0, w[TWO ? 1 : 0]);
+            store(j0, w[0]);
+            if constexpr (TWO) {
+                load(j0 + 2 * BATCH, w[0]);
+                store(j0 + BATCH, w[1]);
+            }
         }
+    };
+    if (cm.p_dtype == MUON_HIP_BF16) update((bf16_t*)p);
+    else update((float*)p);
 }
 
 int chain_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
