@@ -6,11 +6,11 @@
 // the parameter) written once; what bounds it is the chain of dependent steps inside a workgroup (five iterations of the sums of
 // X Xt handed from wave to wave, a walk over the wave's chunks, and three barriers) times the rounds of workgroups, not memory.
 // fast_newtonschulz, us, tiles | this:
-//      16 x  512, 1 | 256 | 1024 matrices   97 |  191 |  609    20 |  25 |  50
-//      16 x 5632                           217 | 1414 | 5461    82 | 118 | 511
-//      32 x 4096                           181 | 1087 | 4229    90 | 160 | 635
-//      64 x 2048                           137 |  556 | 2322    97 | 165 | 660
-//    2048 x   64                           139 |  567 | 2363   109 | 191 | 747
+//      16 x  512, 1 | 256 | 1024 matrices   97 |  191 |  609    18 |  24 |  49
+//      16 x 5632                           217 | 1414 | 5461    72 | 107 | 461
+//      32 x 4096                           181 | 1087 | 4229    80 | 147 | 590
+//      64 x 2048                           137 |  556 | 2322    97 | 163 | 644
+//    2048 x   64                           139 |  567 | 2363   103 | 181 | 701
 // It wins wherever the registers hold the matrix, so that is the rule (chain_fits); larger ones take the tiled products.
 //
 // Eight waves share the columns of X in chunks of 32, a run of consecutive chunks each.  Lane (i = l%16, q = l/16) of a wave holds
@@ -25,7 +25,7 @@
 // Results are those of the tiled kernels bit for bit: the same rounding points (bf(X Xt); bf(bf(bA) + bf(c bf(AA)));
 // bf(bf(aX) + bf(BX))), and every fp32 sum in their order, ascending in 32-deep MFMAs with the reduction index in its natural
 // place.  That order is why a block of X Xt is one chain through the waves and not eight partial sums, which take 3 to 30 % less
-// time (16 x 5632: 57 | 95 | 415, 64 x 2048: 87 | 160 | 621): a bf16 value that rounds the other way moves through the remaining
+// time (16 x 5632: 57 | 95 | 415 when this took 82 | 118 | 511, 64 x 2048: 87 | 160 | 621 against 97 | 165 | 660): a bf16 value that rounds the other way moves through the remaining
 // iterations, up to 1e-3 of the result in norm.
 #include "small_chain.h"
 #include <type_traits>
@@ -124,7 +124,7 @@ constexpr int CHAIN_FRAGS = 32;  // fragments of X a lane can hold: 128 of the 2
 // Fragments that a lane loads from memory (the blend; the parameter) together, while those before them are still on their way: loads and
 // stores leave the queue in order, so a load that is issued behind a store waits for it as well.  One at a time, as written before, 56
 // matrices of 5632 x 16 in fp32 took 142 us, now 117 (with four 117 as well, at the cost of 20 to 50 registers); 168 + 84 + 56 of 2048 and 512 columns
-// 60 and 53; 256 of 2048 x 64 296 and 212.  Asking for the parameter before the iterations, through LDS, gave nothing on top.
+// 60 and 53; 256 of 2048 x 64 296 and 205 (a whole step; 256 of 64 x 2048 199 and 203 in fp32, 190 and 182 in bf16).  Asking for the parameter before the iterations, through LDS, gave nothing on top.
 constexpr int kBatch = 2;
 
 // MT blocks of 16 rows (1, 2 or 4), up to NCH chunks of 32 columns per wave.
@@ -136,8 +136,9 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
     constexpr int BATCH = kBatch < MT ? 1 : kBatch / MT;  // chunks that are loaded from memory together
     constexpr bool TWO = MT < 4;             // while the next ones are on their way (with four blocks a chunk is enough, and two spill)
     // Chunks without a branch between them: 40 -> 30 ns for each MFMA of the chain through 176 chunks (16 x 5632).  Four blocks have
-    // ten MFMAs between two branches anyway.
-    constexpr int RUN = MT == 4 ? 1 : 4;
+    // ten MFMAs between two branches anyway; and where a wave has four chunks at most, those that are not there cost as much as the
+    // branches (111 of 20 x 56, one chunk: 17.5 with runs, 16.0 without).
+    constexpr int RUN = MT == 4 || NCH < 8 ? 1 : 4;
     static_assert(NCH % RUN == 0, "whole runs");
     constexpr int LEG = MT == 4 ? 2 : 1, NLEG = NF / LEG;  // blocks that a wave adds its chunks to at a time
     __shared__ __align__(16) f32x4 sum[NF][64];
@@ -173,40 +174,47 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
     // Normalised fragments, zero past the matrix's edges.  Through the work area, so that the loop over loads of every kind
     // (ragged, turned) and divisions need not be unrolled over the register array.
     const bool vec = !turn && K % 8 == 0;
-    {
-        bf16x8 v[TWO ? 2 : 1][BATCH][MT];
-        auto each = [&](int j0, auto f) {
+    auto fetch = [&](bf16x8& v, int j, int t) {
+        const int row = chain_row<MT>(t, i), col = col0 + j * 32;
+        if (vec && row < M && col < K) {
+            v = *(const bf16x8*)(u + (long)row * K + col);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                v[e] = (row < M && col + e < K) ? u[turn ? (long)(col + e) * M + row : (long)row * K + col + e] : (bf16_t)0.f;
+        }
+    };
+    auto norm = [&](bf16x8& v, int j, int t) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = f2bf(__fdiv_rn(bf2f(v[e]), d));
+        mine[(j * MT + t) * 64] = v;
+    };
+    if constexpr (TWO) {
+        bf16x8 v[2][BATCH][MT];
+        auto each = [&](int j0, bf16x8 (&w)[BATCH][MT], auto f) {
 #pragma unroll
             for (int jj = 0; jj < BATCH; ++jj)
 #pragma unroll
                 for (int t = 0; t < MT; ++t)
-                    if (j0 + jj < per) f(jj, t, chain_row<MT>(t, i), col0 + (j0 + jj) * 32);
+                    if (j0 + jj < per) f(w[jj][t], j0 + jj, t);
         };
-        auto load = [&](int j0, bf16x8 (&w)[BATCH][MT]) {
-            each(j0, [&](int jj, int t, int row, int col) {
-                if (vec && row < M && col < K) {
-                    w[jj][t] = *(const bf16x8*)(u + (long)row * K + col);
-                } else {
+        each(0, v[0], fetch);
+        for (int j0 = 0; j0 < per; j0 += 2 * BATCH) {
+            each(j0 + BATCH, v[1], fetch);
+            each(j0, v[0], norm);
+            each(j0 + 2 * BATCH, v[0], fetch);
+            each(j0 + BATCH, v[1], norm);
+        }
+    } else {
+        // Four blocks in one order: a chunk's loads together would gain 4 % at 256 of 64 x 2048 and lose 9 % at 2048 x 64 (its elements
+        // come one by one) and 5 % at 111 of 34 x 56.
+#pragma unroll 4
+        for (int j = 0; j < per; ++j) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        w[jj][t][e] = (row < M && col + e < K) ? u[turn ? (long)(col + e) * M + row : (long)row * K + col + e] : (bf16_t)0.f;
-                }
-            });
-        };
-        auto put = [&](int j0, bf16x8 (&w)[BATCH][MT]) {
-            each(j0, [&](int jj, int t, int, int) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) w[jj][t][e] = f2bf(__fdiv_rn(bf2f(w[jj][t][e]), d));
-                mine[((j0 + jj) * MT + t) * 64] = w[jj][t];
-            });
-        };
-        if constexpr (TWO) load(0, v[0]);
-        for (int j0 = 0; j0 < per; j0 += (TWO ? 2 : 1) * BATCH) {
-            load(TWO ? j0 + BATCH : j0, v[TWO ? 1 : 0]);
-            put(j0, v[0]);
-            if constexpr (TWO) {
-                load(j0 + 2 * BATCH, v[0]);
-                put(j0 + BATCH, v[1]);
+            for (int t = 0; t < MT; ++t) {
+                bf16x8 v;
+                fetch(v, j, t);
+                norm(v, j, t);
             }
         }
     }
@@ -230,7 +238,7 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         for (int f = 0; f < LEG; ++f) acc[f] = wave == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum[F0 + f][lane];
 #pragma unroll
         for (int j0 = 0; j0 < NCH; j0 += RUN) {
-            if (j0 >= per) continue;
+            if (j0 >= per) break;
 #pragma unroll
             for (int j = j0; j < j0 + RUN; ++j) {  // (past the wave's last chunk x is zero, and the sum plus zero is the sum)
                 int f = 0;
