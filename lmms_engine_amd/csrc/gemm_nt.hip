@@ -2159,7 +2159,8 @@ bool plan_flow(FlowList& l, int xcds) {
     // what is lost between them (1.02 of their time).
     if (mean < 30000 && most < 1.35 * mean - 15 * chain + 600) return true;
     // A step over very little: the device takes as long either way (94 against 86 us for 14 matrices of 128 x 128 to 384), but the
-    // caller waits for his own 14 launches less (whole step of that model 240 us with, 190 without them).
+    // caller waits for his own 14 launches less (whole step of that model 240 us with, 190 without them;
+    // 150 since its tensor lists are read in native code).
     return l.e[0].p_ptrs && 0.032 * most + 0.64 * chain + 55 < 120;
 }
 
