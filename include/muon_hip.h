@@ -133,6 +133,11 @@ int muon_hip_apply_update(const void* const* p_ptrs, int p_dtype, void* workspac
  * the return value of fast_newtonschulz (muon_utils.py:154-156). */
 int muon_hip_ns_output(void* workspace, int rows, int cols, int batch, int steps, void* out, void* stream);
 
+/* muon_hip_ns_grouped and muon_hip_ns_output in one call, the same bits.  Matrices with a short side of at most 64 whose chain
+ * runs in one workgroup write `out` from there where that is faster; the workspace then does not hold the result. */
+int muon_hip_ns_result(void* workspace, int rows, int cols, int batch, int steps, double a, double b, double c, void* out,
+                       void* stream);
+
 /* The whole Muon step for one bucket: SingelDeviceWork.start (muon_utils.py:315-325) for
  * `batch` same-shape parameters in one grouped dispatch per stage.  With ns_steps >= 1 the scaling,
  * decay and update lines (:167-175, :324-325) run in the epilogue of the last B.X product, so the

@@ -61,6 +61,7 @@ SIGNATURES = {
     "muon_hip_ns_grouped": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_double, c_double, c_double, c_void_p]),
     "muon_hip_apply_update": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_double, c_double,
                                       c_double, c_void_p]),
+    "muon_hip_ns_result": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_double, c_double, c_double, c_void_p, c_void_p]),
     "muon_hip_ns_output": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p]),
     "muon_hip_step_grouped": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_int, c_int,
                                       c_double, c_double, c_double, c_int, c_int, c_double, c_double, c_double,

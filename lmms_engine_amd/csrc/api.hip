@@ -417,7 +417,8 @@ bool flow_of(const Work& w, int steps, double a, double b, double c, const Updat
 }
 
 // Normalise, then `steps` iterations; with `upd` the last B.X applies the parameter update instead of writing X'.
-int ns_chain(const Work& all, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s) {
+// `out`: where the result of small matrices goes, dense (one bucket; null: X).
+int ns_chain(const Work& all, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s, bf16_t* out = nullptr) {
     if (steps < 0) return fail(MUON_HIP_EINVAL, "steps must be >= 0");
     Work w;  // the matrices that go through the tiled products
     if (steps > 0) {
@@ -430,7 +431,7 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
                 continue;
             }
             small[n++] = ChainBucket{k.at(k.p.offX[1]), k.p.strideU, (const float*)(k.ws + k.p.offParts), k.at(k.p.offX[0]), k.p.strideX,
-                                     upd ? k.p_ptrs : nullptr, (float)k.scale, k.p.Kp / BLK_COLS, k.p.nparts, k.p.rows, k.p.cols, k.p.batch};
+                                     upd ? k.p_ptrs : nullptr, out, (float)k.scale, k.p.Kp / BLK_COLS, k.p.nparts, k.p.rows, k.p.cols, k.p.batch};
         }
         if (n) {
             ChainMath cm{steps, (float)a, (float)b, (float)c, 0, 1.f, 0.f};
@@ -537,6 +538,15 @@ int muon_hip_ns_grouped(void* workspace, int rows, int cols, int batch, int step
     Work w;
     if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
     return ns_chain(w, steps, a, b, c, nullptr, (hipStream_t)stream);
+}
+
+int muon_hip_ns_result(void* workspace, int rows, int cols, int batch, int steps, double a, double b, double c, void* out, void* stream) {
+    Work w;
+    if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
+    if (!out) return fail(MUON_HIP_EINVAL, "bad output pointer");
+    const bool direct = w.b[0].p.small && steps > 0 && chain_writes(rows, cols, batch, out);
+    if (int rc = ns_chain(w, steps, a, b, c, nullptr, (hipStream_t)stream, direct ? (bf16_t*)out : nullptr)) return rc;
+    return direct ? 0 : muon_hip_ns_output(workspace, rows, cols, batch, steps, out, stream);
 }
 
 int muon_hip_apply_update(const void* const* p_ptrs, int p_dtype, void* workspace, int rows, int cols, int batch,

@@ -8,9 +8,10 @@ struct ChainBucket {
     const bf16_t* U;             // the blend, dense in the parameter's layout, strideU elements per matrix
     long strideU;
     const float* partials;       // nparts sums of squares per matrix
-    bf16_t* X;                   // work area of strideX elements per matrix; without p_ptrs the result, blocked with cbx column blocks
+    bf16_t* X;                   // work area of strideX elements per matrix; without p_ptrs and out the result, blocked with cbx column blocks
     long strideX;
-    const void* const* p_ptrs;   // device table of the parameters to update; null: the result goes to X
+    const void* const* p_ptrs;   // device table of the parameters to update; null: the result goes to `out`
+    bf16_t* out;                 // the result, dense in the parameter's layout, one matrix after the other; null: it goes to X
     float scale;
     int cbx, nparts, rows, cols, batch;
 };
@@ -29,5 +30,7 @@ struct ChainMath {
 
 // A short side of M, a long side of K: whether the registers of one workgroup hold the matrix.
 bool chain_fits(int M, int K);
+// Whether a bucket's result is better written to `out` by the chain than copied there from X.
+bool chain_writes(int rows, int cols, int batch, const void* out);
 // Every bucket must fit; steps >= 1.
 hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, hipStream_t stream);

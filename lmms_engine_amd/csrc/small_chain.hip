@@ -6,11 +6,11 @@
 // the parameter) written once; what bounds it is the chain of dependent steps inside a workgroup (five iterations of the sums of
 // X Xt handed from wave to wave, a walk over the wave's chunks, and three barriers) times the rounds of workgroups, not memory.
 // fast_newtonschulz, us, tiles | this:
-//      16 x  512, 1 | 256 | 1024 matrices   97 |  191 |  609    18 |  24 |  49
-//      16 x 5632                           217 | 1414 | 5461    72 | 107 | 461
-//      32 x 4096                           181 | 1087 | 4229    80 | 147 | 590
-//      64 x 2048                           137 |  556 | 2322    97 | 163 | 644
-//    2048 x   64                           139 |  567 | 2363   103 | 181 | 701
+//      16 x  512, 1 | 256 | 1024 matrices   97 |  191 |  609    17 |  20 |  44
+//      16 x 5632                           217 | 1414 | 5461    72 |  94 | 395
+//      32 x 4096                           181 | 1087 | 4229    81 | 116 | 481
+//      64 x 2048                           137 |  556 | 2322    97 | 134 | 558
+//    2048 x   64                           139 |  567 | 2363   103 | 177 | 694
 // It wins wherever the registers hold the matrix, so that is the rule (chain_fits); larger ones take the tiled products.
 //
 // Eight waves share the columns of X in chunks of 32, a run of consecutive chunks each.  Lane (i = l%16, q = l/16) of a wave holds
@@ -28,6 +28,7 @@
 // time (16 x 5632: 57 | 95 | 415 when this took 82 | 118 | 511, 64 x 2048: 87 | 160 | 621 against 97 | 165 | 660): a bf16 value that rounds the other way moves through the remaining
 // iterations, up to 1e-3 of the result in norm.
 #include "small_chain.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -337,13 +338,15 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         }
     }
 
-    if (!k.p_ptrs) {
+    bf16_t* out = k.out + (long)b * M * K;
+    const bool whole_out = !turn && K % 8 == 0 && (((uintptr_t)k.out) & 15) == 0;
+    if (!k.p_ptrs && (!k.out || whole_out)) {
 #pragma unroll
         for (int j = 0; j < NCH; ++j)
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 const int row = chain_row<MT>(t, i), col = col0 + j * 32;
-                if (j < per && row < M && col < K) *(bf16x8*)(area + blocked_offset(row, col, k.cbx)) = x[j][t];
+                if (j < per && row < M && col < K) *(bf16x8*)(k.out ? out + (long)row * K + col : area + blocked_offset(row, col, k.cbx)) = x[j][t];
             }
         return;
     }
@@ -352,6 +355,18 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
 #pragma unroll
         for (int t = 0; t < MT; ++t)
             if (j < per) mine[(j * MT + t) * 64] = x[j][t];
+    if (!k.p_ptrs) {  // turned, or of rows that are no whole pieces: element by element
+        for (int j = 0; j < per; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const int row = chain_row<MT>(t, i), col = col0 + j * 32;
+                const bf16x8 v = mine[(j * MT + t) * 64];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (row < M && col + e < K) out[turn ? (long)(col + e) * M + row : (long)row * K + col + e] = v[e];
+            }
+        return;
+    }
     void* p = const_cast<void*>(k.p_ptrs[b]);
     const bool whole = whole_rows(p, k.cols, turn);
     auto update = [&](auto* pp) {
@@ -407,6 +422,16 @@ void launch_as(int nch, const ChainList& l, const ChainMath& cm, hipStream_t str
 }  // namespace
 
 bool chain_fits(int M, int K) { return M <= 64 && K <= 8192 && chain_per_wave(K) * chain_blocks(M) <= CHAIN_FRAGS; }
+
+// Whole pieces of rows cost the chain nothing (32 x 4096, 1 | 256 matrices: 80 | 147 us with the copy, 80 | 116 without).  Element by
+// element a workgroup pays 0.6 us for a fragment, which few matrices of many fragments feel more than the copy (one of 512 x 64,
+// eight fragments: 43 and 45.5; of 4096 x 32, 32 of them: 97 and 118; of 512 x 16, two: 20.4 and 19.2); from as many on as leave few
+// compute units idle, the copy is a pass over memory and costs more (256 of 512 x 64 61 and 55, of 4096 x 32 190 and 159, of 2048 x 64 181 and
+// 175, of 5632 x 16 182 and 124).
+bool chain_writes(int rows, int cols, int batch, const void* out) {
+    if (rows <= cols && cols % 8 == 0 && ((uintptr_t)out & 15) == 0) return true;
+    return batch >= 192 || chain_per_wave(std::max(rows, cols)) * chain_blocks(std::min(rows, cols)) <= 4;
+}
 
 // One launch per kernel: blocks of rows, and 8, 16 or 32 fragments of X per lane (fewer registers, more workgroups in flight).
 hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, hipStream_t stream) {

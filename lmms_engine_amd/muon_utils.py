@@ -225,8 +225,7 @@ def fast_newtonschulz(G: Tensor, steps: int = 5) -> Tensor:
         s = _abi.stream_ptr(G.device)
         _abi.check(lib.muon_hip_cast_norm(Gc.data_ptr(), _abi.dtype_code(Gc.dtype), ws.data_ptr(), rows, cols, batch, s),
                    "cast_norm")
-        _abi.check(lib.muon_hip_ns_grouped(ws.data_ptr(), rows, cols, batch, int(steps), a, b, c, s), "ns_grouped")
-        _abi.check(lib.muon_hip_ns_output(ws.data_ptr(), rows, cols, batch, int(steps), out.data_ptr(), s), "ns_output")
+        _abi.check(lib.muon_hip_ns_result(ws.data_ptr(), rows, cols, batch, int(steps), a, b, c, out.data_ptr(), s), "ns_result")
     return out
 
 

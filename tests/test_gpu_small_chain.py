@@ -135,3 +135,28 @@ def test_small_chain_in_a_step_equals_the_stages_bitwise(env, pdtype):
         abi.check(lib.muon_hip_apply_update(tp, code, area.data_ptr(), *s, 1, 5, mu.scale_factor(*s, True), hp["lr"], hp["weight_decay"], 0))
         torch.cuda.synchronize()
         assert torch.equal(p.detach(), q), s
+
+
+@pytest.mark.parametrize("rows,cols,batch", [(16, 2048, 3), (13, 333, 2), (13, 2049, 2), (64, 2048, 1), (64, 520, 200), (333, 7, 2), (2048, 64, 3),
+                                             (2048, 64, 192), (515, 33, 193), (1, 1, 1), (4096, 32, 192)])
+def test_small_chain_writes_its_result_where_the_copy_would(env, rows, cols, batch):
+    """muon_hip_ns_result against muon_hip_ns_grouped and muon_hip_ns_output: the same bits, on aligned outputs and on others, and nothing
+    around them."""
+    print(f"small chain result {batch} x {rows}x{cols}", flush=True)
+    lib, abi, dev = env["lib"], env["abi"], env["dev"]
+    G = torch.randn(batch, rows, cols, generator=torch.Generator().manual_seed(rows + cols)).to(dev)
+    ws = torch.empty(lib.muon_hip_workspace_bytes(rows, cols, batch), dtype=torch.uint8, device=dev)
+    n = G.numel()
+    for shift in (8, 1):
+        buf = torch.full((n + 16,), 7.0, dtype=torch.bfloat16, device=dev)
+        ref = torch.empty(G.shape, dtype=torch.bfloat16, device=dev)
+        for direct in (True, False):
+            abi.check(lib.muon_hip_cast_norm(G.data_ptr(), abi.dtype_code(G.dtype), ws.data_ptr(), rows, cols, batch, 0))
+            if direct:
+                abi.check(lib.muon_hip_ns_result(ws.data_ptr(), rows, cols, batch, 5, 3.4445, -4.775, 2.0315, buf.data_ptr() + 2 * shift, 0))
+            else:
+                abi.check(lib.muon_hip_ns_grouped(ws.data_ptr(), rows, cols, batch, 5, 3.4445, -4.775, 2.0315, 0))
+                abi.check(lib.muon_hip_ns_output(ws.data_ptr(), rows, cols, batch, 5, ref.data_ptr(), 0))
+        torch.cuda.synchronize()
+        assert torch.equal(buf[shift:shift + n].view(G.shape), ref), shift
+        assert bool((buf[:shift] == 7).all()) and bool((buf[shift + n:] == 7).all())
