@@ -560,13 +560,21 @@ __device__ __forceinline__ void epilogue_nn_reg(const GemmArgs& g, int bidx, int
     const long et_off = (long)((n0 >> BLK_SHIFT) + wn * (WTN / 32)) * BLK_ELEMS + lane_off;
     const bf16_t* Et = g.Et + bidx * g.strideEt + (COH ? 0 : et_off);  // (COH: the same in every lane)
     bf16_t* C = g.C + bidx * g.strideC + (long)((n0 >> BLK_SHIFT) + wn * (WTN / 32)) * BLK_ELEMS + lane_off;
-    static_assert(NEV >= FMU * (FN / 2), "pieces of the a.X term");
+    static_assert(PART == EPI_ALL || NEV >= FMU * (FN / 2), "pieces of the a.X term");
+    // Where nothing comes between the two parts the pieces are an array of this function's own: in the caller's they cost the 224-row
+    // persistent kernel (251 registers like this) four more registers, 12 bytes of scratch a lane and 0.5 to 1 % (median us: 60 of 640 x
+    // 2560 159.0 and 157.6 like this, 48 of 896 x 896 77.7 and 76.7).
+    bf16x8 own[PART == EPI_ALL ? FMU : 1][FN / 2];
+    auto piece = [&](int i, int t) -> bf16x8& {
+        if constexpr (PART == EPI_ALL) return own[i][t];
+        else return ev[i * (FN / 2) + t];
+    };
     if constexpr (PART & EPI_LOADS) {
 #pragma unroll
         for (int i = 0; i < FMU; ++i)
 #pragma unroll
-            for (int t = 0; t < FN / 2; ++t) 
-                ev[i * (FN / 2) + t] = load16<COH>(Et, (COH ? et_off : 0) + at(i, g.cbEt) + (long)t * BLK_ELEMS);
+            for (int t = 0; t < FN / 2; ++t)
+                piece(i, t) = load16<COH>(Et, (COH ? et_off : 0) + at(i, g.cbEt) + (long)t * BLK_ELEMS);
     }
     if constexpr (!(PART & EPI_REST)) return;
 #pragma unroll
@@ -580,7 +588,7 @@ __device__ __forceinline__ void epilogue_nn_reg(const GemmArgs& g, int bidx, int
             const bf16x8 tv = *(const bf16x8*)&tw;
             bf16x8 o;
 #pragma unroll
-            for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[i * (FN / 2) + t][k])) + bf2f(tv[k]));
+            for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(piece(i, t)[k])) + bf2f(tv[k]));
             *(bf16x8*)(C + at(i, g.cbC) + (long)t * BLK_ELEMS) = o;
         }
 }
@@ -1601,8 +1609,8 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmList l) {
             // reduction by the compiler, which then waits for the answer on the spot); the answer is needed at the end.
             if (has_next && tid == 0) fetched = atomicInc(&ctr.next[xcd][0], 0xffffffffu);
             if constexpr (QT) {
-                bf16x8 ev[(MASK == 0 ? F0 : F1) * (FN / 2)];
-                epilogue_nn_reg<BN, WGN, WTM, MASK == 0 ? F0 : F1, WHOLE, false, EPI_ALL>(g, cur.tc.bidx, cur.tc.ti * BM, cur.tc.tj * BN, acc, ev);
+                bf16x8 none[1];
+                epilogue_nn_reg<BN, WGN, WTM, MASK == 0 ? F0 : F1, WHOLE, false, EPI_ALL>(g, cur.tc.bidx, cur.tc.ti * BM, cur.tc.tj * BN, acc, none);
             } else {
                 bf16x8 ev[FM * FN / 2];
                 epilogue_sym_reg<BM, BN, WGM, WGN, EPI, MASK, false, EPI_ALL>(g, cur.tc, acc, ev);

@@ -5,6 +5,8 @@ symbol include/muon_hip.h declares (no compute calls here)."""
 import ctypes
 import os
 import re
+import struct
+import subprocess
 
 import pytest
 import torch
@@ -180,6 +182,27 @@ def test_missing_library_is_an_error(monkeypatch):
     monkeypatch.setattr(_abi, "LIB_PATH", "/nonexistent/libmuon_hip.so")
     with pytest.raises(_abi.MuonHipError, match="no fallback"):
         _abi.lib()
+
+
+def test_no_kernel_uses_scratch_memory(tmp_path):
+    """A spilled register is a trip to memory per lane; reads the metadata of the code objects that the library was linked from."""
+    readelf = "/opt/rocm/llvm/bin/llvm-readelf"
+    if not os.path.exists(readelf):
+        pytest.skip("no llvm-readelf")
+    blob, kernels = open(_abi.LIB_PATH, "rb").read(), {}
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    for found in re.finditer(magic, blob):
+        base, at = found.start(), found.end() + 8
+        for _ in range(struct.unpack_from("<Q", blob, found.end())[0]):
+            start, size, name = struct.unpack_from("<QQQ", blob, at)
+            target, at = blob[at + 24:at + 24 + name], at + 24 + name
+            if b"gfx950" in target:
+                elf = tmp_path / f"{base}.elf"
+                elf.write_bytes(blob[base + start:base + start + size])
+                notes = subprocess.run([readelf, "--notes", str(elf)], stdout=subprocess.PIPE, text=True, check=True).stdout
+                kernels.update(zip(re.findall(r"^    \.name:\s+(\S+)", notes, re.M), re.findall(r"\.private_segment_fixed_size: (\d+)", notes)))
+    assert len(kernels) > 50
+    assert not {k: v for k, v in kernels.items() if v != "0"}
 
 
 # ---- the C ABI ----------------------------------------------------------------------------
