@@ -21,8 +21,9 @@
  *  - The Newton-Schulz operands live, in a blocked layout (below), in a caller-allocated workspace of
  *    muon_hip_workspace_bytes() bytes, 256-byte aligned, which the entry points partition
  *    identically; its contents between calls are private to the library.
- *  - Concurrency.  The library keeps no device state of its own (the one exception is
- *    muon_hip_grad_norms_static, which says so).  Everything a call shares between its kernels lives in
+ *  - Concurrency.  The library keeps no device state of its own (the exceptions are
+ *    muon_hip_grad_norms_static, which says so, and the word of host memory per device behind
+ *    muon_hip_chain_status).  Everything a call shares between its kernels lives in
  *    the caller's workspace, the tile counters of the persistent GEMM kernels included (the
  *    normalisation stage clears them, every persistent launch leaves them zero).  Calls that use
  *    different workspaces may run at the same time on different streams, also a replayed HIP graph beside
@@ -43,6 +44,7 @@ extern "C" {
 
 #define MUON_HIP_EINVAL (-1)  /* bad argument (null pointer, non-positive size, unknown dtype/config) */
 #define MUON_HIP_ESHAPE (-2)  /* shape is not a whole number of tiles / exceeds a launch limit */
+#define MUON_HIP_ECHAIN (-3)  /* an earlier chain of this device was abandoned (muon_hip_chain_status) */
 
 /* kernel ids for muon_hip_timing_read */
 #define MUON_HIP_K_MOMENTUM 0
@@ -92,6 +94,16 @@ size_t muon_hip_workspace_bytes(int rows, int cols, int batch);
  * each under MUON_HIP_CFG_AUTO only), so it stays as it is from muon_hip_workspace_bytes to the call that reads the result; meant
  * for benchmarking sweeps. */
 int muon_hip_set_gemm_config(int cfg);
+
+/* Many small matrices run their iterations in one launch whose workgroups wait for each other (muon_hip_flow_tiles).  By their order
+ * every wait ends; should one not end within some minutes all the same, the launch is abandoned: tiles that lack an operand are neither
+ * computed nor stored, so that some parameters have been updated and others have not.  The first of muon_hip_ns_grouped,
+ * muon_hip_ns_result, muon_hip_step_grouped, muon_hip_step_multi and this function that is called for the device afterwards returns
+ * MUON_HIP_ECHAIN and does nothing else; the ones after it work again.  0 otherwise.  Waits for nothing: synchronise with the stream
+ * first. */
+int muon_hip_chain_status(void);
+/* Polls after which such a wait is given up in launches of the calling thread, the default again with a negative number.  For tests. */
+int muon_hip_set_chain_polls(long polls);
 
 /* ---- stage entry points (workspace based) ------------------------------------------- */
 

@@ -54,6 +54,8 @@ SIGNATURES = {
     "muon_hip_geometry": (c_int, [c_int, c_int] + [POINTER(c_int)] * 5),
     "muon_hip_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),
     "muon_hip_set_gemm_config": (c_int, [c_int]),
+    "muon_hip_chain_status": (c_int, []),
+    "muon_hip_set_chain_polls": (c_int, [c_long]),
     "muon_hip_momentum_norm": (c_int, [c_void_p, c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int, c_double,
                                        c_int, c_int, c_void_p]),
     "muon_hip_cast_norm": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_void_p]),

@@ -93,6 +93,48 @@ struct Timed {
     }
 };
 
+// ---- chains that were given up ---------------------------------------------------------
+// A word of host memory per device, a line each, that a chain in one launch sets when it gives up a wait (gemm_nt.h).  Allocated with the
+// first such launch and never freed: kernels may hold its address.
+constexpr int kAlarmDevices = 64, kAlarmLine = 16;
+constexpr unsigned kChainPolls = 1u << 27;  // some minutes
+thread_local unsigned g_chain_polls = kChainPolls;
+std::mutex g_alarm_mu;
+std::atomic<unsigned*> g_alarm{nullptr};
+
+int chain_alarm(unsigned** word) {
+    int dev = 0;
+    if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return hip_fail(e, "hipGetDevice");
+    if (dev >= kAlarmDevices) return fail(MUON_HIP_EINVAL, "device %d", dev);
+    unsigned* p = g_alarm.load(std::memory_order_acquire);
+    if (!p) {
+        std::lock_guard<std::mutex> lock(g_alarm_mu);
+        if (p = g_alarm.load(std::memory_order_relaxed); !p) {
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;  // (the launch may be one that is being recorded)
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            const hipError_t e = hipHostMalloc((void**)&p, kAlarmDevices * kAlarmLine * sizeof(unsigned),
+                                               hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (e != hipSuccess) return hip_fail(e, "hipHostMalloc");
+            std::fill(p, p + kAlarmDevices * kAlarmLine, 0u);
+            g_alarm.store(p, std::memory_order_release);
+        }
+    }
+    *word = p + dev * kAlarmLine;
+    return 0;
+}
+
+// Reports an abandoned chain of the current device, once.
+int chain_status() {
+    unsigned* p = g_alarm.load(std::memory_order_acquire);
+    int dev = 0;
+    if (!p || hipGetDevice(&dev) != hipSuccess || dev >= kAlarmDevices) return 0;
+    p += dev * kAlarmLine;
+    if (!__atomic_load_n(p, __ATOMIC_RELAXED) || !__atomic_exchange_n(p, 0u, __ATOMIC_ACQ_REL)) return 0;
+    return fail(MUON_HIP_ECHAIN, "an earlier chain of Newton-Schulz iterations on device %d gave up waiting for its own tiles: the parameters or "
+                                 "results of that call are incomplete", dev);
+}
+
 // ---- geometry / workspace ------------------------------------------------------------
 struct Plan {
     int rows, cols, batch, M, K, Mp, Kp, tile, nparts;
@@ -451,8 +493,11 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
     MachineShape ms;
     if (hipError_t e = machine_shape(ms); e != hipSuccess) return hip_fail(e, "device shape");
     const bool flow = steps > 0 && flow_of(w, steps, a, b, c, upd, 1 << ms.xcd_shift, fl);
+    if (flow)
+        if (int rc = chain_alarm(&fl.alarm)) return rc;
     if (int rc = do_normalize(w, flow, s)) return rc;
     if (flow) {
+        fl.polls = g_chain_polls;
         Timed t(MUON_HIP_K_FLOW_CHAIN, s);
         hipError_t e = launch_flow(fl, s);
         return e == hipSuccess ? 0 : hip_fail(e, "ns_flow launch");
@@ -485,6 +530,14 @@ const char* muon_hip_last_error(void) { return g_err; }
 int muon_hip_set_gemm_config(int cfg) {
     if (cfg != MUON_HIP_CFG_AUTO && cfg != MUON_HIP_CFG_STAGED && gemm_cfg_tile(cfg) == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration %d", cfg);
     g_forced_cfg.store(cfg, std::memory_order_relaxed);
+    return 0;
+}
+
+int muon_hip_chain_status(void) { return chain_status(); }
+
+int muon_hip_set_chain_polls(long polls) {
+    if (polls > kChainPolls) return fail(MUON_HIP_EINVAL, "at most %u polls", kChainPolls);
+    g_chain_polls = polls < 0 ? kChainPolls : (unsigned)polls;
     return 0;
 }
 
@@ -537,6 +590,7 @@ int muon_hip_ns_grouped(void* workspace, int rows, int cols, int batch, int step
                         void* stream) {
     Work w;
     if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
+    if (int rc = chain_status()) return rc;
     return ns_chain(w, steps, a, b, c, nullptr, (hipStream_t)stream);
 }
 
@@ -544,6 +598,7 @@ int muon_hip_ns_result(void* workspace, int rows, int cols, int batch, int steps
     Work w;
     if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
     if (!out) return fail(MUON_HIP_EINVAL, "bad output pointer");
+    if (int rc = chain_status()) return rc;
     const bool direct = w.b[0].p.small && steps > 0 && chain_writes(rows, cols, batch, out);
     if (int rc = ns_chain(w, steps, a, b, c, nullptr, (hipStream_t)stream, direct ? (bf16_t*)out : nullptr)) return rc;
     return direct ? 0 : muon_hip_ns_output(workspace, rows, cols, batch, steps, out, stream);
@@ -594,6 +649,7 @@ int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int 
         w.b[i].scale = in.scale;
         base += w.b[i].p.total;
     }
+    if (int rc = chain_status()) return rc;
     hipStream_t s = (hipStream_t)stream;
     if (int rc = do_momentum(w, g_dtype, m_dtype, beta, nesterov, write_back_grad, s)) return rc;
     // The parameter is updated by the epilogue of the last B.X (for rows > cols through a transposing gather out of

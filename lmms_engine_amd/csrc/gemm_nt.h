@@ -123,6 +123,8 @@ struct FlowList {
     int n, groups, steps, p_dtype;
     float a, b, c, decay, alpha;
     unsigned* control;         // GEMM_FLOW_CONTROL_BYTES, zero before the launch
+    unsigned* alarm;           // host memory, set when a wait is given up: the results are then not what was asked for
+    unsigned polls;            // after which a wait is given up
     int sym[GEMM_MAX_XCDS], rect[GEMM_MAX_XCDS];  // per group: tiles of each symmetric product, of a.X + B.X
     FlowEntry e[GEMM_MAX_LIST];
 };

@@ -934,12 +934,17 @@ __device__ __forceinline__ int pp_swizzle(int rg) { return (0x78 >> (2 * rg)) & 
 // end of its M phase two k-tiles later (p=2t+6 / 2t+7), and k-tile t+4 is first read in p=2t+8.
 //
 // COH: operands and elementwise terms are read at device scope (load16).  before_loads() runs in front of the first load, after_loop()
-// between the k loop and the epilogue.
+// between the k loop and the epilogue.  Where wanted(), asked with the first loads on their way, says no in every wave, the tile ends there:
+// nothing is stored, and the loads are still in flight.
 struct Nothing {
     __device__ void operator()() const {}
 };
-template <int BM, int BN, int WGM, int WGN, int EPI, bool COH = false, typename F0 = Nothing, typename F1 = Nothing>
-__device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, unsigned char* smem, F0 before_loads = F0(), F1 after_loop = F1()) {
+struct Always {
+    __device__ bool operator()() const { return true; }
+};
+template <int BM, int BN, int WGM, int WGN, int EPI, bool COH = false, typename F0 = Nothing, typename F1 = Nothing, typename F2 = Always>
+__device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, unsigned char* smem, F0 before_loads = F0(), F1 after_loop = F1(),
+                                        F2 wanted = F2()) {
     constexpr int NW = WGM * WGN;
     constexpr int BK4 = 32, ROWB = 64;
     constexpr int WTM = BM / WGM, WTN = BN / WGN;
@@ -1059,6 +1064,7 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     issue_tile(0);
     issue_tile(1);
     issue_tile(2);
+    if (!wanted()) return;
     WAIT_VM(2 * NLD);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -1681,7 +1687,8 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmList l) {
 // are served whatever XCDs the workgroups land on) and then tiles of it by a counter, in the order iteration, product, matrix,
 // tile.  A tile waits until its matrix has finished every tile of the product before.  Tiles are taken in order, and a tile waits
 // only for tiles that come before its own, which workgroups that are running hold: the earliest unfinished tile never waits, so
-// every wait ends.  (Each is bounded all the same, by some minutes, after which the launch drains.)
+// every wait ends.  Each is bounded all the same, by some minutes: then the tile that waited stores nothing and is not counted, every
+// other workgroup leaves at its next wait in vain, and FlowList::alarm, a word of host memory, says so to the next call.
 //
 // Memory order.  Producer: the tile's stores, `s_waitcnt vmcnt(0)` in every wave (they are in L2), the workgroup's barrier, the
 // matrix's counter.  Consumer: the counter, the barrier, then loads that read past the compute unit's own vector cache (load16,
@@ -1702,7 +1709,7 @@ __device__ __forceinline__ unsigned flow_load(const unsigned* p) {
 }
 // Waits until *p, a count, has reached `want`; false if the launch is being abandoned.  Polls seldom while much is missing: on the
 // line that sixty workgroups poll the increments themselves have to queue.
-__device__ __forceinline__ bool flow_wait(const unsigned* p, unsigned want, unsigned* abandoned) {
+__device__ __forceinline__ bool flow_wait(const FlowList& l, const unsigned* p, unsigned want, unsigned* abandoned) {
     for (unsigned spins = 0;; ++spins) {
         const unsigned have = flow_load(p);
         if (have >= want) return true;
@@ -1710,8 +1717,9 @@ __device__ __forceinline__ bool flow_wait(const unsigned* p, unsigned want, unsi
         else if (want - have > 4) __builtin_amdgcn_s_sleep(8);
         else __builtin_amdgcn_s_sleep(2);
         if ((spins & 1023) == 1023 && flow_load(abandoned)) return false;
-        if (spins == 1u << 27) {
+        if (spins >= l.polls) {
             atomicExch(abandoned, 1u);
+            __hip_atomic_store(l.alarm, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             return false;
         }
     }
@@ -1722,7 +1730,7 @@ constexpr int kFlowStages = 4 * (128 + 128) * 64;
 // is left).
 struct FlowSlot {
     int entry, matrix, tile, stage, it;
-    bool gone;           // a wait has been given up
+    int gone;            // a wait has been given up
     int epoch, group;    // the XCD's group that the workgroup takes tiles of, -1 before it knows
     unsigned want;       // tiles of the matrix that come before the tile's product
     unsigned* done;      // the matrix's counter
@@ -1742,7 +1750,7 @@ __device__ __forceinline__ bool flow_next(const FlowList& l, FlowControl& ctl, F
                 v = atomicAdd(&ctl.next_group[0], 1u) + 2;
                 atomicExch(mine, v);
             } else if (v == 1) {
-                if (!flow_wait(mine, 2, &ctl.abandoned[0])) return false;
+                if (!flow_wait(l, mine, 2, &ctl.abandoned[0])) return false;
                 v = flow_load(mine);
             }
             g = (int)v - 2;
@@ -1772,7 +1780,7 @@ __global__ void __launch_bounds__(512, 4) gemm_nt_flow_kernel(const FlowList l) 
     FlowSlot* const slot = (FlowSlot*)(smem + kFlowStages);  // behind the four stages
     FlowControl& ctl = *(FlowControl*)l.control;
     const int tid = threadIdx.x;
-    if (tid == 0) slot->epoch = 0, slot->group = -1, slot->gone = false;
+    if (tid == 0) slot->epoch = 0, slot->group = -1, slot->gone = 0;
     int fetched = 0;             // thread 0: the tile asked for while the one before was in its epilogue
     unsigned* finished = nullptr;  // the counter of the matrix that the tile before belongs to
     auto ask = [&]() {
@@ -1780,8 +1788,13 @@ __global__ void __launch_bounds__(512, 4) gemm_nt_flow_kernel(const FlowList l) 
         if (tid == 0) fetched = (int)atomicInc(&ctl.tile[slot->group][0], 0xffffffffu);
     };
     auto wait = [&]() {  // everything in front of this is done while the matrix is not ready yet
-        if (tid == 0 && !flow_wait(slot->done, slot->want, &ctl.abandoned[0])) slot->gone = true;
+        if (tid == 0 && !flow_wait(l, slot->done, slot->want, &ctl.abandoned[0])) slot->gone = 1;
         __syncthreads();
+    };
+    auto ready = [&]() {  // whether that wait found the matrix ready; if not, the workgroup leaves
+        const bool yes = !__builtin_amdgcn_readfirstlane(slot->gone);
+        if (!yes) finished = nullptr;
+        return yes;
     };
     for (;;) {
         if (tid == 0 && !flow_next(l, ctl, slot, finished != nullptr, fetched)) slot->entry = -1;
@@ -1799,7 +1812,7 @@ __global__ void __launch_bounds__(512, 4) gemm_nt_flow_kernel(const FlowList l) 
         a.kdim = e.Mp;
         TileCoord tc{__builtin_amdgcn_readfirstlane(slot->matrix), 0, 0};
         finished = e.done + tc.bidx * GEMM_FLOW_LINE;
-        auto run = [&](auto epi_c) { pp_tile<128, 128, 2, 4, decltype(epi_c)::value, true>(a, tc, smem, wait, ask); };
+        auto run = [&](auto epi_c) { pp_tile<128, 128, 2, 4, decltype(epi_c)::value, true>(a, tc, smem, wait, ask, ready); };
         if (stage == 2) {
             a.tiles_m = e.Mp / 128;
             a.tiles_n = e.Kr / 128;

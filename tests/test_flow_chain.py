@@ -142,6 +142,48 @@ def test_replays_and_two_streams_equal_eager_steps_bitwise(env):
         assert torch.equal(p.detach(), w.detach()) and torch.equal(q.detach(), w.detach()), tuple(p.shape)
 
 
+@pytest.mark.gpu
+def test_an_abandoned_chain_stores_nothing_unfinished_and_is_reported(env):
+    """A wait that gives up at its second poll: every workgroup leaves, no element of a parameter is computed from operands that were not
+    there, and the next call says what happened, once."""
+    mu, dev, lib = env["mu"], env["dev"], env["lib"]
+    assert _abi.flow_tiles(sorted(MIXED, reverse=True), 5, True)
+    ps, ws, opt = _steps(mu, dev, MIXED, torch.bfloat16, torch.float32, _abi.CFG_AUTO, steps=1)
+    want, _, _ = _steps(mu, dev, MIXED, torch.bfloat16, torch.float32, _abi.CFG_STAGED, steps=2)
+    before = [p.detach().clone() for p in ps]
+    moms = [opt.state[p]["momentum_buffer"].clone() for p in ps]
+    assert lib.muon_hip_chain_status() == 0
+    print("an abandoned chain", flush=True)
+    _abi.check(lib.muon_hip_set_chain_polls(1))
+    try:
+        opt.step()
+    finally:
+        _abi.check(lib.muon_hip_set_chain_polls(-1))
+    torch.cuda.synchronize()
+    left = [p.detach().clone() for p in ps]
+    changed = 0
+    for p, b, w in zip(left, before, want):
+        same = p == b
+        assert bool((same | (p == w.detach())).all()), tuple(p.shape)
+        changed += int(not bool(same.all()))
+    assert changed < len(ps)
+    with pytest.raises(_abi.MuonHipError, match="gave up waiting"):
+        opt.step()
+    torch.cuda.synchronize()
+    assert lib.muon_hip_chain_status() == 0
+    for p, q in zip(ps, left):
+        assert torch.equal(p.detach(), q)
+    # as a program goes on from its last checkpoint
+    for p, b, m in zip(ps, before, moms):
+        p.detach().copy_(b)
+        opt.state[p]["momentum_buffer"].copy_(m)
+    opt.step()
+    torch.cuda.synchronize()
+    assert lib.muon_hip_chain_status() == 0
+    for p, w in zip(ps, want):
+        assert torch.equal(p.detach(), w.detach())
+
+
 # the lists of the persistent kernel that calls of these sizes run when every product has a launch of its own
 @pytest.mark.gpu
 @pytest.mark.parametrize("shapes", [[(512, 1024, 40), (256, 384, 3), (300, 100, 2), (1024, 1100, 1)], [(512, 1408, 24), (512, 512, 16)]])
