@@ -29,7 +29,8 @@ def clip_grad_norm_(parameters, max_norm, norm_type=2.0, error_if_nonfinite=Fals
     norm_type = float(norm_type)
     if norm_type != norm_type:
         raise ValueError("norm_type is NaN")
-    plain = _abi.scan().grads(parameters, _abi.MULTI_CHUNK)
+    held = []  # the gradients' memory, until this call has launched everything
+    plain = _abi.scan().grads(parameters, _abi.MULTI_CHUNK, held)
     if plain is not None:
         index, lists = plain
         dev = torch.device("cuda", index)

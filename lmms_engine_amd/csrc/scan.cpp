@@ -5,9 +5,14 @@
 // Each function takes lists in which nothing needs a decision: plain parameters on one kind of device with plain contiguous
 // gradients and state.  Anything else (a missing gradient or state, a CPU tensor, other strides, a subclass such as DTensor, an
 // empty tensor) makes it return None before it has changed anything, and the caller goes through the list itself.
+//
+// What a function returns are addresses.  Given a list as `held`, it appends an object to it that keeps the memory behind them alive: the
+// caller's launches give up the interpreter lock, and another thread may drop a gradient there.  The caller lets go after the last
+// launch that uses the addresses (9 ns a tensor; memory that a kernel on the stream still reads is the allocator's affair, as ever).
 #define PY_SSIZE_T_CLEAN
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <memory>
 #include <string>
 #include <unordered_set>
 #include <vector>
@@ -26,6 +31,21 @@ PyObject* none() {
     if (PyErr_Occurred()) PyErr_Clear();  // a look-up that raised: the caller's own loop raises it again
     Py_RETURN_NONE;
 }
+
+// The storages of tensors whose addresses a function hands out.
+using Held = std::vector<c10::Storage>;
+void let_go(PyObject* capsule) { delete (Held*)PyCapsule_GetPointer(capsule, nullptr); }
+// Appends them to the caller's list (null: the caller holds the tensors himself); false with an exception set.
+bool hand_over(PyObject* list, std::unique_ptr<Held> held) {
+    if (!list) return true;
+    PyObject* capsule = PyCapsule_New(held.get(), nullptr, let_go);
+    if (!capsule) return false;
+    (void)held.release();
+    const bool ok = PyList_Append(list, capsule) == 0;
+    Py_DECREF(capsule);
+    return ok;
+}
+bool is_holder(PyObject* list) { return !list || PyList_CheckExact(list); }
 
 // state[p][key], borrowed; null if there is no such thing in plain dictionaries
 PyObject* state_of(PyObject* state, PyObject* p) {
@@ -51,13 +71,14 @@ long long put_sizes(std::string& words, const std::vector<long long>& numel, lon
     return at;
 }
 
-// grads(params, chunk): (device index, [(dtype code, tensors, chunks, table words)]) of the gradients that there are, by dtype in the
+// grads(params, chunk, held = nothing): (device index, [(dtype code, tensors, chunks, table words)]) of the gradients that there are, by dtype in the
 // order of their first gradient.
 PyObject* grads(PyObject*, PyObject* args) {
-    PyObject* params;
+    PyObject *params, *held_list = nullptr;
     long long chunk;
-    if (!PyArg_ParseTuple(args, "OL", &params, &chunk)) return nullptr;
-    if (!PyList_CheckExact(params) || chunk < 1) return none();
+    if (!PyArg_ParseTuple(args, "OL|O", &params, &chunk, &held_list)) return nullptr;
+    auto held = std::make_unique<Held>();
+    if (!PyList_CheckExact(params) || !is_holder(held_list) || chunk < 1) return none();
     struct Group {
         int code;
         std::string ptrs;
@@ -80,8 +101,10 @@ PyObject* grads(PyObject*, PyObject* args) {
         if (k == groups.size()) groups.push_back(Group{code, {}, {}});
         put(groups[k].ptrs, (long long)g.data_ptr());
         groups[k].numel.push_back(g.numel());
+        if (held_list) held->push_back(g.storage());
     }
     if (groups.empty()) return none();
+    if (!hand_over(held_list, std::move(held))) return nullptr;
     PyObject* list = PyList_New(0);
     if (!list) return nullptr;
     for (Group& g : groups) {
@@ -97,12 +120,13 @@ PyObject* grads(PyObject*, PyObject* args) {
     return Py_BuildValue("(iN)", device, list);
 }
 
-// muon(params, state): [(device index, rows, cols, parameter, gradient and momentum dtype codes, matrices, their addresses)] by shape and
+// muon(params, state, held = nothing): [(device index, rows, cols, parameter, gradient and momentum dtype codes, matrices, their addresses)] by shape and
 // dtypes, in the order of their first parameter; the addresses as three strings of 64-bit words.
 PyObject* muon(PyObject*, PyObject* args) {
-    PyObject *params, *state;
-    if (!PyArg_ParseTuple(args, "OO", &params, &state)) return nullptr;
-    if (!PyList_CheckExact(params) || !PyDict_Check(state)) return none();
+    PyObject *params, *state, *held_list = nullptr;
+    if (!PyArg_ParseTuple(args, "OO|O", &params, &state, &held_list)) return nullptr;
+    auto held = std::make_unique<Held>();
+    if (!PyList_CheckExact(params) || !PyDict_Check(state) || !is_holder(held_list)) return none();
     struct Bucket {
         int device, codes[3];
         long long rows, cols, n;
@@ -140,7 +164,10 @@ PyObject* muon(PyObject*, PyObject* args) {
         put(b.ptrs[0], (long long)p.data_ptr());
         put(b.ptrs[1], (long long)g.data_ptr());
         put(b.ptrs[2], (long long)m.data_ptr());
+        if (held_list)
+            for (const at::Tensor* t : {&p, &g, &m}) held->push_back(t->storage());
     }
+    if (!hand_over(held_list, std::move(held))) return nullptr;
     PyObject* list = PyList_New((Py_ssize_t)buckets.size());
     if (!list) return nullptr;
     for (size_t k = 0; k < buckets.size(); ++k) {
@@ -157,13 +184,14 @@ PyObject* muon(PyObject*, PyObject* args) {
     return list;
 }
 
-// adam(params, state, chunk): (device index, dtype code, steps, chunks, table words) of parameters of one device and dtype; every step count
+// adam(params, state, chunk, held = nothing): (device index, dtype code, steps, chunks, table words) of parameters of one device and dtype; every step count
 // is one higher afterwards.
 PyObject* adam(PyObject*, PyObject* args) {
-    PyObject *params, *state;
+    PyObject *params, *state, *held_list = nullptr;
     long long chunk;
-    if (!PyArg_ParseTuple(args, "OOL", &params, &state, &chunk)) return nullptr;
-    if (!PyList_CheckExact(params) || !PyDict_Check(state) || chunk < 1) return none();
+    if (!PyArg_ParseTuple(args, "OOL|O", &params, &state, &chunk, &held_list)) return nullptr;
+    auto held = std::make_unique<Held>();
+    if (!PyList_CheckExact(params) || !PyDict_Check(state) || !is_holder(held_list) || chunk < 1) return none();
     const Py_ssize_t n = PyList_GET_SIZE(params);
     if (n == 0) return none();
     int device = -1, code = -1;
@@ -193,6 +221,7 @@ PyObject* adam(PyObject*, PyObject* args) {
         for (int k = 0; k < 4; ++k) {
             if (plain(*t[k]) != code || t[k]->get_device() != device || t[k]->numel() != p.numel()) return none();
             put(ptrs[k], (long long)t[k]->data_ptr());
+            if (held_list) held->push_back(t[k]->storage());
         }
         if (!seen.insert(s).second) return none();  // a parameter that is listed twice steps twice
         numel.push_back(p.numel());
@@ -201,6 +230,7 @@ PyObject* adam(PyObject*, PyObject* args) {
     }
     std::string words = ptrs[0] + ptrs[1] + ptrs[2] + ptrs[3];
     const long long chunks = put_sizes(words, numel, chunk);
+    if (!hand_over(held_list, std::move(held))) return nullptr;
     PyObject* list = PyList_New(n);
     if (!list) return nullptr;
     for (Py_ssize_t i = 0; i < n; ++i) {

@@ -586,7 +586,8 @@ class Muon(torch.optim.Optimizer):
         self._recorded = False
 
     def _adam_group_step(self, group) -> None:
-        plain = _abi.scan().adam(group["params"], self.state, _abi.MULTI_CHUNK)
+        held = []  # the tensors' memory, until the launch
+        plain = _abi.scan().adam(group["params"], self.state, _abi.MULTI_CHUNK, held)
         if plain is not None:
             _adamw_plain(plain, group)
             return
@@ -644,7 +645,8 @@ class Muon(torch.optim.Optimizer):
                 if self.reference_bug_compat:
                     ns_steps, nesterov = int(bool(group["nesterov"])), bool(group["ns_steps"])
                 how = (group, ns_steps, nesterov, self.write_back_grad, self._workspaces, self.workspace_limit_bytes, self._pointer_tables)
-                plain = _abi.scan().muon(group["params"], self.state) if self._plain_work() else None
+                held = []  # the tensors' memory, until the last launch
+                plain = _abi.scan().muon(group["params"], self.state, held) if self._plain_work() else None
                 if plain is not None:
                     alike = {}
                     for dev, rows, cols, *codes, n, p, g, m in plain:

@@ -125,3 +125,40 @@ def test_lists_that_need_a_decision_are_left_to_the_caller(env):
         assert scan.muon(mats, opt.state) is None, change
         assert scan.adam(params, opt.state, 16384) is None, change
         assert [opt.state[t].get("step") for t in rest] == before, change
+
+
+@pytest.mark.gpu
+def test_memory_lives_until_the_last_launch(env, monkeypatch):
+    """Gradients that their parameters give up between the reading of the addresses and the launches (another thread may, while a call
+    waits or launches) stay allocated until the call is through."""
+    from lmms_engine_amd.clip_grad import clip_grad_norm_
+
+    mu, dev = env["mu"], env["dev"]
+    mats = [torch.nn.Parameter(torch.zeros(256, 4096, device=dev)) for _ in range(4)]
+    rest = [torch.nn.Parameter(torch.zeros(1 << 20, device=dev)) for _ in range(4)]
+    both = _optimizer(mu, mats, rest)
+    stream_ptr, seen = _abi.stream_ptr, []
+
+    def drop(device):
+        before = torch.cuda.memory_allocated()
+        for p in dropped:
+            p.grad = None
+        seen.append(before - torch.cuda.memory_allocated())
+        return stream_ptr(device)
+
+    def set_grads():
+        for p in mats + rest:
+            p.grad = torch.ones_like(p)
+
+    set_grads()
+    both.step()  # makes the state
+    for call, dropped in ((lambda: clip_grad_norm_(mats + rest, 1.0, error_if_nonfinite=True), mats + rest), (both.step, mats),
+                          (lambda: both._adam_group_step(both.param_groups[1]), rest)):
+        set_grads()
+        del seen[:]
+        with monkeypatch.context() as m:
+            m.setattr(_abi, "stream_ptr", drop)
+            call()
+        assert seen and not any(seen), seen
+        assert all(p.grad is None for p in dropped)
+    torch.cuda.synchronize()
