@@ -624,9 +624,9 @@ class Muon(torch.optim.Optimizer):
         return state
 
     def _plain_work(self) -> bool:
-        """Whether every plain tensor takes the single-device work with its state as this class keeps it."""
-        cls = type(self)
-        return cls._get_work_class is Muon._get_work_class and cls._init_muon_state is Muon._init_muon_state
+        """Whether every plain tensor takes the single-device work with its state as this class keeps it: nobody has put methods of
+        their own in the place of these two, in a subclass, on the class or on the instance."""
+        return tuple(getattr(m, "__func__", None) for m in (self._get_work_class, self._init_muon_state)) == _PLAIN_WORK
 
     @torch.no_grad()
     def step_fsdp(self, closure=None):
@@ -708,6 +708,9 @@ class Muon(torch.optim.Optimizer):
             work.finish()
 
         return loss
+
+
+_PLAIN_WORK = (Muon._get_work_class, Muon._init_muon_state)
 
 
 def _adamw_plain(plain, group: dict) -> None:

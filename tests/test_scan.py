@@ -20,6 +20,48 @@ def test_cpu_tensors_and_other_things_are_left_to_the_caller():
     assert state[p]["step"] == 4
 
 
+@pytest.mark.parametrize("where", ["subclass", "class", "instance"])
+@pytest.mark.parametrize("name", ["_get_work_class", "_init_muon_state"])
+def test_methods_of_the_callers_own_are_asked(monkeypatch, where, name):
+    """A step reads its lists in native code only where nobody has replaced the methods that choose a parameter's work and make its state."""
+    from lmms_engine_amd import muon_utils
+
+    started = []
+
+    class OwnWork:
+        def __init__(self, param, state, group, index):
+            self.param = param
+
+        def start(self):
+            started.append(self.param)
+
+        def finish(self):
+            pass
+
+    def own(*args):  # (self is the first argument but for an instance's)
+        if name == "_get_work_class":
+            return OwnWork, 1
+        started.append(args[-1])
+        raise KeyboardInterrupt
+
+    monkeypatch.setattr(_abi, "scan", lambda: pytest.fail("read in native code"))
+    cls = type("Sub", (muon_utils.Muon,), {name: own}) if where == "subclass" else muon_utils.Muon
+    p = torch.nn.Parameter(torch.zeros(3, 4))
+    p.grad = torch.ones(3, 4)
+    opt = cls([dict(params=[p], use_muon=True)])
+    assert (where == "subclass") != opt._plain_work()
+    if where == "class":
+        monkeypatch.setattr(muon_utils.Muon, name, own)
+    elif where == "instance":
+        monkeypatch.setattr(opt, name, own)
+    if name == "_get_work_class":
+        opt.step()
+    else:
+        with pytest.raises(KeyboardInterrupt):
+            opt.step()
+    assert len(started) == 1 and started[0] is p
+
+
 def _set(dev, dtype, seed=0):
     g = torch.Generator().manual_seed(seed)
     shapes = [(96, 40), (128, 256), (96, 40), (300, 20), (128, 256)]
