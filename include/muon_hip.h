@@ -187,9 +187,12 @@ typedef struct {
 int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cus, muon_hip_route* out);
 
 /* The tiles of a call whose `steps` iterations run as one launch on a device of `xcds` XCDs, group after group (the matrices of a
- * group belong to one XCD) in the order in which the workgroups of an XCD take them; update: the call updates parameters.  Writes at
- * most `capacity` of them; *count is how many there are, 0 for a call whose products are launched one by one.  A tile starts when
- * `before` tiles of its matrix are finished.  Touches no device; for tests and measurements. */
+ * group belong to one XCD) in the order in which the workgroups of an XCD take them; update: 0, or 1 for a call that updates
+ * parameters, plus MUON_HIP_FLOW_RECORDED for one that is being recorded into a graph (over very little work only a call that is not
+ * takes this way, for the sake of its launches).  Writes at most `capacity` of them; *count is how many there are, 0 for a call whose
+ * products are launched one by one.  A tile starts when `before` tiles of its matrix are finished.  Touches no device; for tests and
+ * measurements. */
+#define MUON_HIP_FLOW_RECORDED 0x100
 typedef struct {
     int group, bucket, matrix, iteration;
     int product; /* MUON_HIP_K_SYRK, MUON_HIP_K_SYMPOLY or MUON_HIP_K_BX */

@@ -16,6 +16,7 @@ LIB_PATH = os.path.join(_HERE, "libmuon_hip.so")
 
 F32, BF16 = 0, 1
 CFG_STAGED = -2
+FLOW_RECORDED = 0x100  # MUON_HIP_FLOW_RECORDED
 CFG_AUTO, CFG_128_PIPE, CFG_256_PIPE, CFG_256_PINGPONG, CFG_128_PINGPONG, CFG_256_PERSIST, CFG_64_DEEP = -1, 0, 1, 2, 3, 4, 5
 GEMM_CONFIGS = list(range(4))
 K_MOMENTUM, K_NORMALIZE, K_SYRK, K_SYMPOLY, K_BX, K_UPDATE, K_ADAMW, K_ADAMW_MULTI, K_GRAD_NORM, K_CLIP_SCALE = range(10)
@@ -182,11 +183,11 @@ def routes(shapes, kernel: str, cus: int = 256):
     return [(r.cfg, r.height, r.launch) for r in out]
 
 
-def flow_tiles(shapes, steps: int, update: bool, xcds: int = 8):
+def flow_tiles(shapes, steps: int, update: bool, xcds: int = 8, recorded: bool = False):
     """The tiles of the (rows, cols, matrices) of one call whose iterations run as one launch, as FlowTile; empty where they do not."""
     buckets = (Bucket * len(shapes))(*[Bucket(rows=r, cols=c, batch=n) for r, c, n in shapes])
     count = c_long()
-    args = (buckets, len(shapes), int(steps), int(update), int(xcds))
+    args = (buckets, len(shapes), int(steps), int(update) + FLOW_RECORDED * int(recorded), int(xcds))
     check(lib().muon_hip_flow_tiles(*args, None, 0, ctypes.byref(count)), "flow_tiles")
     out = (FlowTile * count.value)()
     check(lib().muon_hip_flow_tiles(*args, out, count.value, ctypes.byref(count)), "flow_tiles")

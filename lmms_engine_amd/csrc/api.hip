@@ -68,14 +68,21 @@ int grow_pool(size_t want) {  // under g_tmu
     return 0;
 }
 
+// Whether what is launched on the stream goes into a graph (or cannot be told to be launched now).
+bool is_recorded(hipStream_t s) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
 struct Timed {
     EventPair* ev;
     hipStream_t s;
     Timed(int kid, hipStream_t st) : ev(nullptr), s(st) {
         if (!g_timing.load(std::memory_order_acquire)) return;
         // a launch that is being recorded into a graph has no time of its own: its events would become graph nodes
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        if (is_recorded(s)) {
             g_untimed.fetch_add(1, std::memory_order_relaxed);
             return;
         }
@@ -425,7 +432,7 @@ bool stage_items(const Work& w, int epi, int cur, double a, double b, double c, 
 }
 
 // The iterations as one launch (gemm_nt.h), where that is the faster way and nobody has named a configuration.
-bool flow_of(const Work& w, int steps, double a, double b, double c, const UpdateArgs* upd, int xcds, FlowList& l) {
+bool flow_of(const Work& w, int steps, double a, double b, double c, const UpdateArgs* upd, int xcds, bool recorded, FlowList& l) {
     if (g_forced_cfg.load(std::memory_order_relaxed) != MUON_HIP_CFG_AUTO) return false;
     l.n = w.n;
     l.steps = steps;
@@ -455,7 +462,7 @@ bool flow_of(const Work& w, int steps, double a, double b, double c, const Updat
         e.cols = p.cols;
         e.scale = (float)k.scale;
     }
-    return plan_flow(l, xcds);
+    return plan_flow(l, xcds, recorded);
 }
 
 // Normalise, then `steps` iterations; with `upd` the last B.X applies the parameter update instead of writing X'.
@@ -492,7 +499,7 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
     FlowList fl;
     MachineShape ms;
     if (hipError_t e = machine_shape(ms); e != hipSuccess) return hip_fail(e, "device shape");
-    const bool flow = steps > 0 && flow_of(w, steps, a, b, c, upd, 1 << ms.xcd_shift, fl);
+    const bool flow = steps > 0 && flow_of(w, steps, a, b, c, upd, 1 << ms.xcd_shift, upd && is_recorded(s), fl);
     if (flow)
         if (int rc = chain_alarm(&fl.alarm)) return rc;
     if (int rc = do_normalize(w, flow, s)) return rc;
@@ -690,6 +697,8 @@ int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cu
 
 int muon_hip_flow_tiles(const muon_hip_bucket* buckets, int n, int steps, int update, int xcds, muon_hip_flow_tile* out, long capacity,
                         long* count) {
+    const bool recorded = update & MUON_HIP_FLOW_RECORDED;
+    update &= ~MUON_HIP_FLOW_RECORDED;
     if (!buckets || !count || n < 1 || n > MUON_HIP_MAX_BUCKETS || capacity < 0 || (capacity && !out) || steps < 0 || xcds < 1 || xcds > GEMM_MAX_XCDS)
         return fail(MUON_HIP_EINVAL, "bad bucket list, steps, XCDs or output");
     *count = 0;
@@ -704,7 +713,7 @@ int muon_hip_flow_tiles(const muon_hip_bucket* buckets, int n, int steps, int up
     }
     FlowList l;
     const UpdateArgs u{};
-    if (!w.n || steps == 0 || !flow_of(w, steps, 1.0, 1.0, 1.0, update ? &u : nullptr, xcds, l)) return 0;
+    if (!w.n || steps == 0 || !flow_of(w, steps, 1.0, 1.0, 1.0, update ? &u : nullptr, xcds, recorded, l)) return 0;
     for (int g = 0; g < l.groups; ++g)
         for (int t = 0; t < flow_tiles(l, g); ++t, ++*count) {
             if (*count >= capacity) continue;

@@ -160,6 +160,7 @@ __host__ __device__ inline FlowPlace flow_place(const FlowList& l, int g, int t)
 }
 
 // Deals the matrices of l.e[0 .. l.n) to the XCDs (fills groups, sym and rect, here and in the entries, and every first); false where
-// launches of their own are the faster way.  Touches no device.
-bool plan_flow(FlowList& l, int xcds);
+// launches of their own are the faster way.  recorded: the call is being recorded into a graph, its launches cost the caller nothing.
+// Touches no device.
+bool plan_flow(FlowList& l, int xcds, bool recorded);
 hipError_t launch_flow(const FlowList& l, hipStream_t stream);

@@ -2127,7 +2127,7 @@ int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* r
     return launches;
 }
 
-bool plan_flow(FlowList& l, int xcds) {
+bool plan_flow(FlowList& l, int xcds, bool recorded) {
     l.groups = xcds;
     if (l.n < 1 || l.n > GEMM_MAX_LIST || xcds < 1 || xcds > GEMM_MAX_XCDS || l.steps < 1) return false;
     // Dearest matrices first, each to the group with the least work so far.  Work in k-tiles of 32 columns, the start and the
@@ -2181,8 +2181,9 @@ bool plan_flow(FlowList& l, int xcds) {
     if (mean < 30000 && most < 1.35 * mean - 15 * chain + 600) return true;
     // A step over very little: the device takes as long either way (94 against 86 us for 14 matrices of 128 x 128 to 384), but the
     // caller waits for his own 14 launches less (whole step of that model 240 us with, 190 without them;
-    // 150 since its tensor lists are read in native code).
-    return l.e[0].p_ptrs && 0.032 * most + 0.64 * chain + 55 < 120;
+    // 150 since its tensor lists are read in native code).  A step that is being recorded has no
+    // such launches when it is replayed (6 of 128 x 384 with 8 of 128 x 128: 94.5 us a replay in one launch, 74.0 without).
+    return !recorded && l.e[0].p_ptrs && 0.032 * most + 0.64 * chain + 55 < 120;
 }
 
 hipError_t launch_flow(const FlowList& l, hipStream_t stream) {

@@ -67,6 +67,13 @@ def test_calls_that_stay_with_a_launch_per_product():
             _abi.check(_abi.lib().muon_hip_set_gemm_config(_abi.CFG_AUTO))
 
 
+def test_a_recorded_step_over_very_little_keeps_its_launches():
+    """The one launch is the slower one on the device there; it saves the caller of an eager step his own launches, which a replay has not."""
+    assert _abi.flow_tiles(TINY, 5, True) and not _abi.flow_tiles(TINY, 5, True, recorded=True)
+    assert len(_abi.flow_tiles(MIXED, 5, True, recorded=True)) == len(_abi.flow_tiles(MIXED, 5, True)) > 0
+    assert _abi.flow_tiles([(256, 1024, 48)], 5, False, recorded=True)
+
+
 def _steps(mu, dev, shapes, dtype, mdtype, config, steps=2):
     g = torch.Generator().manual_seed(len(shapes))
     ws = [(0.02 * torch.randn(r, c, generator=g)).to(dtype) for r, c, n in shapes for _ in range(n)]
@@ -123,13 +130,15 @@ def test_stacks_equal_a_launch_per_product_bitwise(env, rows, cols, batch, steps
 
 
 @pytest.mark.gpu
-def test_replays_and_two_streams_equal_eager_steps_bitwise(env):
+@pytest.mark.parametrize("shapes", [MIXED, TINY])
+def test_replays_and_two_streams_equal_eager_steps_bitwise(env, shapes):
     """A recorded step replayed beside eager steps of another optimizer on a second stream, four times."""
     mu, dev = env["mu"], env["dev"]
-    assert _abi.flow_tiles(sorted(MIXED, reverse=True), 5, True)
-    want, _, _ = _steps(mu, dev, MIXED, torch.bfloat16, torch.float32, _abi.CFG_STAGED, steps=6)
-    pa, _, oa = _steps(mu, dev, MIXED, torch.bfloat16, torch.float32, _abi.CFG_AUTO, steps=2)
-    pb, _, ob = _steps(mu, dev, MIXED, torch.bfloat16, torch.float32, _abi.CFG_AUTO, steps=2)
+    assert _abi.flow_tiles(sorted(shapes, reverse=True), 5, True)
+    assert bool(_abi.flow_tiles(sorted(shapes, reverse=True), 5, True, recorded=True)) == (shapes is MIXED)
+    want, _, _ = _steps(mu, dev, shapes, torch.bfloat16, torch.float32, _abi.CFG_STAGED, steps=6)
+    pa, _, oa = _steps(mu, dev, shapes, torch.bfloat16, torch.float32, _abi.CFG_AUTO, steps=2)
+    pb, _, ob = _steps(mu, dev, shapes, torch.bfloat16, torch.float32, _abi.CFG_AUTO, steps=2)
     graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
     with torch.cuda.graph(graph):
         oa.step()
