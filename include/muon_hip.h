@@ -225,9 +225,8 @@ int muon_hip_unpack_bf16(const void* src, int rows_p, int cols_p, void* dst, lon
 #define MUON_HIP_PPX_COUNTER_BYTES 576
 
 /* Y (M x M) = bf16(X Xt) for X (M x K), both row-major and contiguous: matmul_transpose_assign + mmt_kernel, muon_utils.py:95-119 and
- * :28-92.  `scratch`: muon_hip_mmt_scratch_elems bf16 elements, 16-byte aligned, for an X that has to be packed first (a K that is no
- * multiple of 128, an X that is not 16-byte aligned or overlaps Y); 0 elements, and a null pointer, otherwise.  Chooses its kernel by
- * itself, whatever muon_hip_set_gemm_config says. */
+ * :28-92.  `scratch`: muon_hip_mmt_scratch_elems bf16 elements, 16-byte aligned, for an X that is packed first; 0 elements, and a null
+ * pointer, where it is read as it lies. */
 long muon_hip_mmt_scratch_elems(const void* X, const void* Y, int M, int K);
 int muon_hip_mmt_bf16(const void* X, void* Y, int M, int K, void* scratch, void* stream);
 

@@ -787,30 +787,40 @@ static bool mmt_reads_x(const void* X, const void* Y, int M, int K) {
     const bool small = t64 <= ms.cus, large = use_tile256(M) && t128 > 2 * ms.cus;  // as plan_gemm_nt has it
     return small || large || (long)M * K <= 5L << 20;
 }
-static int mmt_tile(int M) { return use_tile256(M) ? 256 : 128; }
+struct MmtPlan {
+    Cfg use;
+    int Mp, Kp;
+    bool reads_x;  // a named configuration multiplies packed operands, which every kernel takes
+};
+static MmtPlan mmt_plan(const void* X, const void* Y, int M, int K) {
+    const int forced = g_forced_cfg.load(std::memory_order_relaxed), tile = use_tile256(M) ? 256 : 128;
+    const int own = tile == 256 && M > 512 ? GEMM_CFG_256_PINGPONG : GEMM_CFG_128_PINGPONG;
+    return MmtPlan{forced >= 0 ? Cfg{forced, false} : Cfg{own, true}, (int)round_up(M, tile), (int)round_up(K, tile),
+                   forced < 0 && mmt_reads_x(X, Y, M, K)};
+}
 
 long muon_hip_mmt_scratch_elems(const void* X, const void* Y, int M, int K) {
     if (M <= 0 || K <= 0) return 0;
-    const int tile = mmt_tile(M);
-    return mmt_reads_x(X, Y, M, K) ? 0 : blocked_elems(round_up(M, tile), round_up(K, tile));
+    const MmtPlan p = mmt_plan(X, Y, M, K);
+    return p.reads_x ? 0 : blocked_elems(p.Mp, p.Kp);
 }
 
 int muon_hip_mmt_bf16(const void* X, void* Y, int M, int K, void* scratch, void* stream) {
     if (M <= 0 || K <= 0) return fail(MUON_HIP_EINVAL, "sizes must be positive");
     if (!X || !Y) return fail(MUON_HIP_EINVAL, "null operand");
-    const int tile = mmt_tile(M), Mp = (int)round_up(M, tile), Kp = (int)round_up(K, tile);
-    const bool reads_x = mmt_reads_x(X, Y, M, K);
-    if (!reads_x) {
+    const MmtPlan p = mmt_plan(X, Y, M, K);
+    int tile;
+    if (int rc = check_gemm(p.use.id, p.Mp, p.Kp, 1, tile)) return rc;
+    if (!p.reads_x) {
         if (!scratch || ((uintptr_t)scratch & 15)) return fail(MUON_HIP_EINVAL, "this X needs scratch, 16-byte aligned");
-        hipError_t e = launch_pack((const bf16_t*)X, 0, K, M, K, (bf16_t*)scratch, 0, Mp, Kp, 1, (hipStream_t)stream);
+        hipError_t e = launch_pack((const bf16_t*)X, 0, K, M, K, (bf16_t*)scratch, 0, p.Mp, p.Kp, 1, (hipStream_t)stream);
         if (e != hipSuccess) return hip_fail(e, "pack launch");
     }
-    const int cfg = tile == 256 && M > 512 ? GEMM_CFG_256_PINGPONG : GEMM_CFG_128_PINGPONG;
-    GemmItem it = syrk_item(cfg, (const bf16_t*)(reads_x ? X : scratch), (bf16_t*)Y, Mp, (int)round_up(K, 128), Kp, 1, nullptr);
+    GemmItem it = syrk_item(p.use.id, (const bf16_t*)(p.reads_x ? X : scratch), (bf16_t*)Y, p.Mp, (int)round_up(K, 128), p.Kp, 1, nullptr);
     it.epi = EPI_MMT;
     it.g.dense_rows = M;
-    it.g.dense_pitch = reads_x ? K : 0;
-    return launch_items(MUON_HIP_K_SYRK, "mmt launch", &it, 1, true, (hipStream_t)stream);
+    it.g.dense_pitch = p.reads_x ? K : 0;
+    return launch_items(MUON_HIP_K_SYRK, "mmt launch", &it, 1, p.use.adapt, (hipStream_t)stream);
 }
 
 int muon_hip_sympoly_bf16(const void* A, void* B, int Mp, int batch, double b, double c, int cfg, void* counters,

@@ -1929,12 +1929,8 @@ hipError_t launch_pp_tail(GemmList& l, int nblocks, int rest, hipStream_t stream
 template <int EPI>
 hipError_t launch_cfg(int cfg, GemmList& l, int nblocks, int cus, hipStream_t stream) {
     switch (cfg) {
-        case GEMM_CFG_128_PIPE:
-            if constexpr (EPI == EPI_MMT) return hipErrorInvalidValue;
-            else return launch_one<128, 128, 2, 2, EPI, 0>(l, nblocks, stream);
-        case GEMM_CFG_256_PIPE:
-            if constexpr (EPI == EPI_MMT) return hipErrorInvalidValue;
-            else return launch_one<256, 256, 2, 4, EPI, 0>(l, nblocks, stream);
+        case GEMM_CFG_128_PIPE: return launch_one<128, 128, 2, 2, EPI, 0>(l, nblocks, stream);
+        case GEMM_CFG_256_PIPE: return launch_one<256, 256, 2, 4, EPI, 0>(l, nblocks, stream);
         case GEMM_CFG_256_PINGPONG: {
             // Split the tiles of a last round that would fill at most a quarter of the CUs (a 128x128 tile takes about 0.6 of
             // the time of a 256x256 one, so one round of quarters beats a round of whole tiles).
@@ -1974,6 +1970,8 @@ bool tiles_fit(const GemmItem& it, int height, int width) {
     const GemmArgs& g = it.g;
     auto up = [](int v, int m) { return (v + m - 1) / m * m; };
     if (up(g.rows, height) > up(g.rows, BLK_ROWS)) return false;
+    // (the two-stage kernels read blocked operands only)
+    if (it.epi == EPI_MMT && g.dense_pitch && (it.cfg == GEMM_CFG_128_PIPE || it.cfg == GEMM_CFG_256_PIPE)) return false;
     if (it.epi == EPI_MMT) return g.rows % height == 0 && g.dense_rows <= g.rows && g.dense_rows > g.rows - 128;
     if (!epi_is_bx(it.epi)) return g.rows % height == 0 && g.rows <= g.cbC * BLK_COLS;
     const int cols = up(g.cols, width);

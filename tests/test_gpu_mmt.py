@@ -59,3 +59,26 @@ def test_a_result_over_its_own_input(env):
     mu.matmul_transpose_assign(a, b)
     torch.cuda.synchronize()
     assert torch.equal(x, ref) and torch.equal(b, ref2)
+
+
+@pytest.mark.parametrize("M,K", [(100, 130), (512, 384), (896, 128), (1030, 256), (2048, 1024)])
+def test_a_named_configuration_multiplies(env, M, K):
+    """muon_hip_set_gemm_config holds for matmul_transpose: the same bits on each kernel, an error where its tiles do not divide the padded
+    matrix."""
+    print(f"mmt {M} x {K} on named configurations", flush=True)
+    mu, lib, dev = env["mu"], env["lib"], env["dev"]
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).bfloat16().to(dev)
+    ref = mu.matmul_transpose(x)
+    whole256 = -(-M // 128) % 2 == 0 and M > 384
+    for cfg in (*_abi.GEMM_CONFIGS, _abi.CFG_256_PERSIST, _abi.CFG_64_DEEP):
+        refused = not whole256 and cfg in (_abi.CFG_256_PIPE, _abi.CFG_256_PINGPONG, _abi.CFG_256_PERSIST)
+        _abi.check(lib.muon_hip_set_gemm_config(cfg))
+        try:
+            if refused:
+                with pytest.raises(_abi.MuonHipError, match="multiples of the 256 tile"):
+                    mu.matmul_transpose(x)
+            else:
+                assert lib.muon_hip_mmt_scratch_elems(x.data_ptr(), ref.data_ptr(), M, K) > 0
+                assert torch.equal(mu.matmul_transpose(x), ref), cfg
+        finally:
+            _abi.check(lib.muon_hip_set_gemm_config(_abi.CFG_AUTO))
