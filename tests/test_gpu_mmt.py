@@ -38,6 +38,22 @@ def test_read_in_place_equals_packed_bitwise(env, M, K):
     assert ((got.cpu().double() - exact).abs() <= exact.abs() * 2.0**-8 + K * 2.0**-24 * (x.double().abs() @ x.double().abs().T)).all()
 
 
+# aligned operands that are packed because of their size
+@pytest.mark.parametrize("M,K", [(2048, 5632), (3072, 3072), (1536, 6144), (1700, 3200)])
+def test_large_operands_on_128_tiles_are_packed(env, M, K):
+    print(f"mmt {M} x {K}", flush=True)
+    lib, dev = env["lib"], env["dev"]
+    x = torch.randn(M, K, generator=torch.Generator().manual_seed(M)).bfloat16().to(dev)
+    out = torch.empty(M, M, dtype=torch.bfloat16, device=dev)
+    assert lib.muon_hip_mmt_scratch_elems(x.data_ptr(), out.data_ptr(), M, K) >= M * K
+    assert lib.muon_hip_mmt_bf16(x.data_ptr(), out.data_ptr(), M, K, None, 0) < 0  # scratch that the caller has not brought
+    got, n = _mmt(lib, x, out)
+    torch.cuda.synchronize()
+    assert n > 0 and torch.equal(got, got.T)
+    exact, bound = x.double() @ x.double().T, x.double().abs() @ x.double().abs().T
+    assert ((got.double() - exact).abs() <= exact.abs() * 2.0**-8 + K * 2.0**-24 * bound).all()
+
+
 def test_result_stays_inside_its_rows(env):
     lib, dev = env["lib"], env["dev"]
     for M, K in [(130, 128), (1030, 128), (2047, 256), (3001, 100)]:
