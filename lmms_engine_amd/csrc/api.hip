@@ -606,7 +606,9 @@ int muon_hip_ns_result(void* workspace, int rows, int cols, int batch, int steps
     if (int rc = one_bucket(rows, cols, batch, workspace, w)) return rc;
     if (!out) return fail(MUON_HIP_EINVAL, "bad output pointer");
     if (int rc = chain_status()) return rc;
-    const bool direct = w.b[0].p.small && steps > 0 && chain_writes(rows, cols, batch, out);
+    MachineShape ms;
+    if (hipError_t e = machine_shape(ms); e != hipSuccess) return hip_fail(e, "device shape");
+    const bool direct = w.b[0].p.small && steps > 0 && chain_writes(rows, cols, batch, out, ms.cus);
     if (int rc = ns_chain(w, steps, a, b, c, nullptr, (hipStream_t)stream, direct ? (bf16_t*)out : nullptr)) return rc;
     return direct ? 0 : muon_hip_ns_output(workspace, rows, cols, batch, steps, out, stream);
 }

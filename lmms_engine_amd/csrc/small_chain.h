@@ -30,7 +30,7 @@ struct ChainMath {
 
 // A short side of M, a long side of K: whether the registers of one workgroup hold the matrix.
 bool chain_fits(int M, int K);
-// Whether a bucket's result is better written to `out` by the chain than copied there from X.
-bool chain_writes(int rows, int cols, int batch, const void* out);
+// Whether a bucket's result is better written to `out` by the chain than copied there from X, on a device of `cus` compute units.
+bool chain_writes(int rows, int cols, int batch, const void* out, int cus);
 // Every bucket must fit; steps >= 1.
 hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, hipStream_t stream);

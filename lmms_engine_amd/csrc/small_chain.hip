@@ -427,10 +427,10 @@ bool chain_fits(int M, int K) { return M <= 64 && K <= 8192 && chain_per_wave(K)
 // element a workgroup pays 0.6 us for a fragment, which few matrices of many fragments feel more than the copy (one of 512 x 64,
 // eight fragments: 43 and 45.5; of 4096 x 32, 32 of them: 97 and 118; of 512 x 16, two: 20.4 and 19.2); from as many on as leave few
 // compute units idle, the copy is a pass over memory and costs more (256 of 512 x 64 61 and 55, of 4096 x 32 190 and 159, of 2048 x 64 181 and
-// 175, of 5632 x 16 182 and 124).
-bool chain_writes(int rows, int cols, int batch, const void* out) {
+// 175, of 5632 x 16 182 and 124): three quarters of the compute units.
+bool chain_writes(int rows, int cols, int batch, const void* out, int cus) {
     if (rows <= cols && cols % 8 == 0 && ((uintptr_t)out & 15) == 0) return true;
-    return batch >= 192 || chain_per_wave(std::max(rows, cols)) * chain_blocks(std::min(rows, cols)) <= 4;
+    return 4L * batch >= 3L * cus || chain_per_wave(std::max(rows, cols)) * chain_blocks(std::min(rows, cols)) <= 4;
 }
 
 // One launch per kernel: blocks of rows, and 8, 16 or 32 fragments of X per lane (fewer registers, more workgroups in flight).
