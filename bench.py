@@ -432,9 +432,9 @@ def main():
     from lmms_engine_amd import _abi
     from lmms_engine_amd.muon_utils import Muon
 
-    if not os.path.exists(_abi.LIB_PATH):
-        from lmms_engine_amd.build import build_library
+    from lmms_engine_amd.build import build_library, built
 
+    if not built():
         build_library()
     assert torch.cuda.is_available(), "bench.py needs a GPU"
     dev = torch.device("cuda:0")

@@ -135,7 +135,11 @@ def scan():
         try:
             from . import _scan as module
         except ImportError as e:
-            raise MuonHipError(f"lmms_engine_amd/_scan.so cannot be loaded ({e}): build it with `python -m lmms_engine_amd.build`") from e
+            raise MuonHipError(f"the module lmms_engine_amd._scan cannot be loaded ({e}): build it with `python -m lmms_engine_amd.build`") from e
+        of = getattr(module, "torch_version", "of another kind")
+        if of != torch.__version__:  # it reads torch's objects as that version lays them out
+            raise MuonHipError(f"lmms_engine_amd._scan was built for torch {of}, this is {torch.__version__}: "
+                               "build it again with `python -m lmms_engine_amd.build`")
         _scan = module
     return _scan
 

@@ -1,4 +1,4 @@
-"""Builds lmms_engine_amd/libmuon_hip.so from csrc/ with hipcc for gfx950, and the host-side module _scan.so beside it.
+"""Builds lmms_engine_amd/libmuon_hip.so from csrc/ with hipcc for gfx950, and the host-side Python module _scan beside it.
 
 Run as `python -m lmms_engine_amd.build` or call build_library().  The library is built
 in-tree, next to this file, so it travels with the source tree.
@@ -9,6 +9,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -17,9 +18,10 @@ SOURCES = ["gemm_nt.hip", "elementwise.hip", "small_chain.hip", "multi_tensor.hi
 # Measurement kernels (MFMA-only loops) for the benchmark's operand-power legs: a library of their own, no part of the product.
 PROBE_LIB = os.path.join(HERE, "libmuon_probe.so")
 PROBE_SOURCES = ["probe.hip"]
+# Reads lists of torch tensors for the optimizer step (host code; a Python module, since it handles Python objects).  Its name says
+# which Python it is for, and it carries the version of the torch whose headers it was compiled with (checked when it is loaded).
+SCAN_LIB = os.path.join(HERE, "_scan" + sysconfig.get_config_var("EXT_SUFFIX"))
 # Packed-fp32 VALU forms stay off for every device function.
-# Reads lists of torch tensors for the optimizer step (host code; a Python module, since it handles Python objects).
-SCAN_LIB = os.path.join(HERE, "_scan.so")
 HIP_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -58,19 +60,22 @@ def _compile_and_link(sources, lib, hipcc, verbose):
 
 
 def _build_scan(verbose):
-    import sysconfig
-
     import torch
     from torch.utils.cpp_extension import include_paths, library_paths
 
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *[f"-isystem{p}" for p in include_paths()], f"-isystem{sysconfig.get_paths()['include']}", os.path.join(CSRC, "scan.cpp"), "-o", SCAN_LIB,
+           f'-DSCAN_TORCH_VERSION="{torch.__version__}"', *[f"-isystem{p}" for p in include_paths()], f"-isystem{sysconfig.get_paths()['include']}", os.path.join(CSRC, "scan.cpp"), "-o", SCAN_LIB,
            *[f"-L{p}" for p in library_paths()], "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"g++ failed on scan.cpp:\n{r.stdout}")
+
+
+def built() -> bool:
+    """Whether everything that the package loads is there."""
+    return os.path.exists(LIB) and os.path.exists(SCAN_LIB)
 
 
 def build_library(verbose: bool = False) -> str:

@@ -269,5 +269,7 @@ PyMODINIT_FUNC PyInit__scan() {
     key_exp_avg = PyUnicode_InternFromString("exp_avg");
     key_exp_avg_sq = PyUnicode_InternFromString("exp_avg_sq");
     key_step = PyUnicode_InternFromString("step");
-    return PyModule_Create(&module);
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", SCAN_TORCH_VERSION) < 0) Py_CLEAR(m);
+    return m;
 }

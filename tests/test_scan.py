@@ -20,6 +20,25 @@ def test_cpu_tensors_and_other_things_are_left_to_the_caller():
     assert state[p]["step"] == 4
 
 
+def test_a_module_for_another_torch_is_refused(monkeypatch):
+    scan = _abi.scan()
+    assert scan.torch_version == torch.__version__
+    monkeypatch.setattr(_abi, "_scan", None)
+    monkeypatch.setattr(torch, "__version__", "0.0")
+    with pytest.raises(_abi.MuonHipError, match="built for torch"):
+        _abi.scan()
+
+
+def test_nothing_counts_as_built_while_a_library_is_missing(monkeypatch):
+    from lmms_engine_amd import build
+
+    assert build.built()
+    for name in ("LIB", "SCAN_LIB"):
+        with monkeypatch.context() as m:
+            m.setattr(build, name, "/nonexistent/" + name)
+            assert not build.built()
+
+
 @pytest.mark.parametrize("where", ["subclass", "class", "instance"])
 @pytest.mark.parametrize("name", ["_get_work_class", "_init_muon_state"])
 def test_methods_of_the_callers_own_are_asked(monkeypatch, where, name):
