@@ -31,25 +31,27 @@ def _check_order(shapes, steps, update, xcds):
     for i, (rows, cols, n) in enumerate(shapes):
         tm, tn = -(-min(rows, cols) // 128), -(-max(rows, cols) // 128)
         want = sorted(((it, s), k) for it in range(steps) for s in range(3) for k in range(tm * tn if s == 2 else tm * (tm + 1) // 2))
-        for k in range(n):
-            if (i, k) in done:
-                assert sorted(done[i, k]) == want
-    return tiles, done
+        for k in range(n if tiles and min(rows, cols) > 64 else 0):
+            assert sorted(done.pop((i, k))) == want
+    assert not done
+    return tiles
 
 
 @pytest.mark.parametrize("xcds", [1, 2, 4, 8])
-@pytest.mark.parametrize("shapes,steps,update", [(MIXED, 5, True), (TINY, 5, True), ([(256, 1024, 48)], 1, False), ([(130, 700, 33)], 3, False)])
-def test_every_tile_once_and_after_what_it_waits_for(shapes, steps, update, xcds):
-    tiles, done = _check_order(shapes, steps, update, xcds)
-    if xcds == 8 and shapes in (MIXED, TINY):
-        assert len(done) == sum(n for r, c, n in shapes if min(r, c) > 64)
+@pytest.mark.parametrize("shapes,steps,update,not_on", [
+    (MIXED, 5, True, (1, 2)),  # there a launch of its own per product is full
+    (TINY, 5, True, ()), ([(256, 1024, 48)], 1, False, ()), ([(130, 700, 64)], 3, False, ()),
+    ([(130, 700, 33)], 3, False, (8,)),  # 33 matrices: one XCD has a quarter more than the others
+])
+def test_every_tile_once_and_after_what_it_waits_for(shapes, steps, update, not_on, xcds):
+    assert bool(_check_order(shapes, steps, update, xcds)) == (xcds not in not_on)
 
 
 def test_every_tile_once_for_drawn_calls():
     rng, taken = random.Random(3), 0
     for _ in range(60):
         shapes = [(rng.randint(65, 700), rng.randint(65, 1500), rng.randint(1, 40)) for _ in range(rng.randint(1, 5))]
-        taken += bool(_check_order(shapes, rng.randint(1, 3), rng.random() < 0.5, rng.choice([1, 2, 4, 8]))[0])
+        taken += bool(_check_order(shapes, rng.randint(1, 3), rng.random() < 0.5, rng.choice([1, 2, 4, 8])))
     assert taken > 20
 
 
@@ -74,11 +76,12 @@ def test_a_recorded_step_over_very_little_keeps_its_launches():
     assert _abi.flow_tiles([(256, 1024, 48)], 5, False, recorded=True)
 
 
-def _steps(mu, dev, shapes, dtype, mdtype, config, steps=2):
+def _steps(mu, dev, shapes, dtype, mdtype, config, steps=2, offset=0):
     g = torch.Generator().manual_seed(len(shapes))
     ws = [(0.02 * torch.randn(r, c, generator=g)).to(dtype) for r, c, n in shapes for _ in range(n)]
     gs = [(1e-3 * torch.randn(w.shape, generator=g)).to(dtype) for w in ws]
-    ps = [torch.nn.Parameter(w.clone().to(dev)) for w in ws]
+    places = [torch.full((w.numel() + offset + 8,), 7.0, dtype=dtype, device=dev) for w in ws]
+    ps = [torch.nn.Parameter(b[offset:offset + w.numel()].view(w.shape).copy_(w)) for b, w in zip(places, ws)]
     for p, gr in zip(ps, gs):
         p.grad = gr.to(dev)
     opt = mu.Muon([dict(params=list(ps), use_muon=True, lr=0.02, momentum=0.95, nesterov=True, weight_decay=0.01, ns_steps=5, rms_scale=True)],
@@ -90,23 +93,29 @@ def _steps(mu, dev, shapes, dtype, mdtype, config, steps=2):
         torch.cuda.synchronize()
     finally:
         _abi.check(_abi.lib().muon_hip_set_gemm_config(_abi.CFG_AUTO))
+    for b, w in zip(places, ws):  # nothing around a parameter has been written
+        assert bool((b[:offset] == 7).all()) and bool((b[offset + w.numel():] == 7).all())
     return ps, ws, opt
 
 
-# both orientations, ragged edges, odd numbers of tiles, a parameter in an unaligned place of a larger buffer's rows (odd column counts)
+# both orientations, ragged edges, odd numbers of tiles, odd column counts, parameters of whole 16-byte pieces that lie one element
+# behind a 16-byte boundary
 @pytest.mark.gpu
-@pytest.mark.parametrize("name,shapes,dtype,mdtype", [
-    ("mixed", MIXED, torch.bfloat16, torch.float32),
-    ("tiny", TINY, torch.float32, None),
-    ("ragged", [(200, 333, 24), (333, 200, 16), (130, 130, 16), (901, 257, 8)], torch.bfloat16, None),
-    ("ragged fp32", [(70, 129, 40), (500, 411, 32), (129, 1000, 8)], torch.float32, None),
+@pytest.mark.parametrize("name,shapes,dtype,mdtype,offset", [
+    ("mixed", MIXED, torch.bfloat16, torch.float32, 0),
+    ("tiny", TINY, torch.float32, None, 0),
+    ("ragged", [(200, 333, 24), (333, 200, 16), (130, 130, 16), (901, 257, 8)], torch.bfloat16, None, 0),
+    ("ragged fp32", [(70, 129, 40), (500, 411, 32), (129, 1000, 8)], torch.float32, None, 0),
+    ("unaligned", MIXED, torch.bfloat16, torch.float32, 1),
+    ("unaligned fp32", [(256, 384, 24), (384, 256, 24), (128, 512, 8)], torch.float32, None, 1),
 ])
-def test_steps_equal_a_launch_per_product_bitwise(env, name, shapes, dtype, mdtype):
+def test_steps_equal_a_launch_per_product_bitwise(env, name, shapes, dtype, mdtype, offset):
     print(f"one launch: {name}", flush=True)
     assert _abi.flow_tiles(sorted(shapes, reverse=True), 5, True)
     mu, dev = env["mu"], env["dev"]
-    a, ws, _ = _steps(mu, dev, shapes, dtype, mdtype, _abi.CFG_AUTO)
+    a, ws, _ = _steps(mu, dev, shapes, dtype, mdtype, _abi.CFG_AUTO, offset=offset)
     b, _, _ = _steps(mu, dev, shapes, dtype, mdtype, _abi.CFG_STAGED)
+    assert all(p.data_ptr() % 16 for p in a) if offset else not any(p.data_ptr() % 16 for p in a)
     for p, q, w in zip(a, b, ws):
         assert bool(torch.isfinite(p.detach().float()).all())
         assert torch.equal(p.detach(), q.detach()) and not torch.equal(p.detach().cpu(), w), tuple(p.shape)
