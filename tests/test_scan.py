@@ -130,6 +130,38 @@ def test_step_and_clipping_equal_the_callers_own_loops(env, monkeypatch, dtype, 
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("first", [torch.float32, torch.bfloat16])
+def test_clipping_gradients_of_two_dtypes_and_of_none_equals_the_callers_own_loop(env, monkeypatch, first):
+    from lmms_engine_amd.clip_grad import clip_grad_norm_
+
+    class Loops:
+        grads = staticmethod(lambda *a: None)
+
+    dev, out = env["dev"], []
+    other = torch.bfloat16 if first == torch.float32 else torch.float32
+    for own in (False, True):
+        g = torch.Generator().manual_seed(5)
+        ps = []
+        for n, dtype in ((7, first), (16384 + 5, other), (300, first), (16384 * 3, first), (64, other), (9, other)):
+            p = torch.nn.Parameter(torch.zeros(n, dtype=dtype, device=dev))
+            p.grad = torch.randn(n, generator=g).to(dtype).to(dev)
+            ps.append(p)
+        ps[2].grad = ps[5].grad = None
+        ps.insert(0, torch.nn.Parameter(torch.zeros(4)))  # no gradient, not on the device either
+        lists = _abi.scan().grads(ps, 16384)[1]
+        assert [(code, n, chunks) for code, n, chunks, _ in lists] == [(_abi.dtype_code(first), 2, 4), (_abi.dtype_code(other), 2, 3)]
+        with monkeypatch.context() as m:
+            if own:
+                m.setattr(_abi, "scan", lambda: Loops)
+            totals = [clip_grad_norm_(ps, 1.0, norm_type=t) for t in (2.0, float("inf"))]
+        torch.cuda.synchronize()
+        out.append((totals, [p.grad for p in ps]))
+    for x, y in zip(out[0][0] + out[0][1], out[1][0] + out[1][1]):
+        assert (x is None) == (y is None) and (x is None or (x.dtype == y.dtype and torch.equal(x, y)))
+    assert out[0][0][0].dtype == torch.float32
+
+
+@pytest.mark.gpu
 def test_addresses_sizes_and_order(env):
     mats, rest = _set(env["dev"], torch.float32)
     opt = _optimizer(env["mu"], mats, rest)
@@ -183,8 +215,11 @@ def test_lists_that_need_a_decision_are_left_to_the_caller(env):
             params.append(q)
             opt.state[p]["momentum_buffer"] = opt.state[p]["momentum_buffer"].cpu()
         before = [opt.state[t].get("step") for t in rest]
-        assert scan.muon(mats, opt.state) is None, change
-        assert scan.adam(params, opt.state, 16384) is None, change
+        held = []
+        if change in ("strided grad", "subclass"):
+            assert scan.grads(mats, 16384, held) is None and scan.grads(params, 16384, held) is None and not held, change
+        assert scan.muon(mats, opt.state, held) is None, change
+        assert scan.adam(params, opt.state, 16384, held) is None and not held, change
         assert [opt.state[t].get("step") for t in rest] == before, change
 
 
