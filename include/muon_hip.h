@@ -227,8 +227,8 @@ int muon_hip_unpack_bf16(const void* src, int rows_p, int cols_p, void* dst, lon
 /* Y (M x M) = bf16(X Xt) for X (M x K), both row-major and contiguous: matmul_transpose_assign + mmt_kernel, muon_utils.py:95-119 and
  * :28-92.  `scratch`: muon_hip_mmt_scratch_elems bf16 elements, 16-byte aligned, for an X that is packed first; 0 elements, and a null
  * pointer, where X is read as it lies.  An X with a K that is no multiple of 128 or above 2^22, one that is not 16-byte aligned or
- * overlaps Y, and every X under a named configuration is packed; others are where that is faster, which depends on M, K and the
- * current device (on 256 compute units 2048 x 5632 is, 2048 x 1024 is not).  So the size is asked for with the same pointers, sizes,
+ * overlaps Y, and every X under a named configuration is packed; others are where that is faster, which depends on M, K, the
+ * boundary that X lies on (16 to 128 bytes) and the current device (on 256 compute units 2048 x 5632 is, 2048 x 1024 is not).  So the size is asked for with the same pointers, sizes,
  * configuration and device as the call: a call that lacks its scratch returns MUON_HIP_EINVAL and launches nothing. */
 long muon_hip_mmt_scratch_elems(const void* X, const void* Y, int M, int K);
 int muon_hip_mmt_bf16(const void* X, void* Y, int M, int K, void* scratch, void* stream);

@@ -774,11 +774,16 @@ int muon_hip_syrk_bf16(const void* X, void* A, int Mp, int Kp, int batch, int cf
 }
 
 // Whether the kernels read X where it lies.  They can when its rows are whole k-tiles and 16-byte pieces, a panel of 256 rows is
-// addressed with 32 bits, and nothing that they write is still to be read.  They should, but for 128-tiles of an X that the L2s do not
-// hold: those read 64 bytes of a row at a time, and rows whose pitch is a multiple of the L2 channels crowd into few of them.
-// Measured, packed | in place: 64-tiles 896 x 4864 28.0 | 18.8 us; 128-tiles 2048 x 1024 18.5 | 11.6, 2048 x 2176 27.3 | 23.4, 2800 x
-// 3968 45.1 | 42.9, 2048 x 5632 46.4 | 47.6, 3072 x 3072 50.4 | 58.0, 1536 x 6144 47.6 | 56.1; 256-tiles 4096 x 1024 38.4 | 29.7,
-// 4096 x 12288 214 | 204, 8192 x 16384 899 | 900.
+// addressed with 32 bits, and nothing that they write is still to be read.  They should, but
+//  - where the 64 (64-tiles: 128) bytes of a row that a load instruction takes straddle two cache lines: rows are whole numbers of lines, so
+//    it is the address of X that decides;
+//  - on 128-tiles of an X that the L2s do not hold: those read 64 bytes of a row at a time, and rows whose pitch is a multiple of the L2
+//    channels crowd into few of them.
+// A small X is the better read in place in both.  Measured (profiles/mmt_packed_or_in_place.txt), packed | in place | in place on a boundary
+// of 32 bytes: 64-tiles 896 x 4864 26.5 | 18.7 | 26.0 us, 896 x 32768 117 | 98 | 139; 128-tiles 2048 x 1024 18.9 | 12.0 | 13.3, 2048 x 2048
+// 25.6 | 20.4 | 29.4, 2048 x 5632 44.1 | 47.7 | 70.8, 3072 x 3072 48.0 | 56.4 | 77.8; 256-tiles 4096 x 512 28.2 | 22.0 | 24.4, 4096 x 12288
+// 213 | 203 | 300, 8192 x 16384 901 | 876 | 1161.  The line at 5 Mi elements is one of many shapes: on 128-tiles 2048 x 2560 would be 7 %
+// faster packed, 2800 x 1920 and 2560 x 4096 13 and 7 % faster in place.
 static bool mmt_reads_x(const void* X, const void* Y, int M, int K) {
     const uintptr_t x = (uintptr_t)X, y = (uintptr_t)Y;
     const bool apart = y + 2 * (size_t)M * M <= x || x + 2 * (size_t)M * K <= y;
@@ -787,7 +792,8 @@ static bool mmt_reads_x(const void* X, const void* Y, int M, int K) {
     if (machine_shape(ms) != hipSuccess) return false;  // the launch will report it
     const long t = round_up(M, 128) / 128, t128 = t * (t + 1) / 2, t64 = t * (2 * t + 1);
     const bool small = t64 <= ms.cus, large = use_tile256(M) && t128 > 2 * ms.cus;  // as plan_gemm_nt has it
-    return small || large || (long)M * K <= 5L << 20;
+    const bool whole = x % (small ? 128 : 64) == 0;
+    return (long)M * K <= (whole ? 5L : 2L) << 20 || (whole && (small || large));
 }
 struct MmtPlan {
     Cfg use;
