@@ -1679,8 +1679,8 @@ __global__ void __launch_bounds__(512) gemm_nt_ppx_kernel(const GemmList l) {
 // units wait for the last tiles and for the next launch to start.  Here a matrix belongs to one XCD for all of its products:
 // what one compute unit writes, another of the same XCD reads out of the L2 that they share, so that a product may start as
 // soon as the one before it has finished for that matrix, with a counter in memory between them and no launch.  (The same over all
-// XCDs has to write through to memory: a handover between 32 workgroups of an XCD takes 1.3 us, between all 256 with
-// written-through stores 5 to 13, with cache write-backs 49; a launch 2.5 to 2.9.)
+// XCDs has to write through to memory: a hand-over of 8 KB each between 32 workgroups of an XCD takes 1.9 us, between all 256 with
+// written-through stores 6.4, with cache write-backs 77; a launch without any work 2.4.  profiles/flow_chain_hand_over.txt)
 //
 // The host deals the matrices to as many groups as there are XCDs.  A workgroup finds out which XCD it runs on, takes that
 // XCD's group (the first of an XCD to ask fetches a group for it; an XCD that has finished one fetches another, so the groups
@@ -2171,16 +2171,16 @@ bool plan_flow(FlowList& l, int xcds, bool recorded) {
         l.rect[g] = (int)rect;
         most = std::max(most, load[g]);
     }
-    // Measured on 1400 sets of one to four shapes of 65 to 1536 rows, 2 to 800 matrices, against launches of their own: the XCD with
-    // the most work and, where there is little, the chain of one matrix through an iteration set its time, launches of their own
-    // share the work evenly but pay for each other's last rounds.  The line below takes 598 of them, 15 % faster in the mean (up to
-    // 30 %) and 18 slower by more than 3 % (8 % at most).  Beyond `mean` of 30000 the 256-tiles of large launches are worth more than
-    // what is lost between them (1.02 of their time).
+    // The XCD with the most work and, where there is little, the chain of one matrix through an iteration set the time of one launch;
+    // launches of their own share the work evenly but pay for each other's last rounds.  Measured on 500 sets of one to four shapes of 65
+    // to 1536 rows, 2 to 800 matrices (recorded steps, profiles/flow_chain_or_launches.txt): the line below takes 298 of them, 13 % faster in
+    // the mean (up to 32 %) and 3 slower by more than 3 % (5 % at most); of the 141 others below it 21 would be faster by more than 3 %,
+    // and all of them 12 % slower in the mean.  Beyond `mean` of 30000 the 256-tiles of large launches are worth what is lost between them.
+    // (The figures are of XCDs of 32 compute units, which gfx950 has however it is partitioned.)
     if (mean < 30000 && most < 1.35 * mean - 15 * chain + 600) return true;
-    // A step over very little: the device takes as long either way (94 against 86 us for 14 matrices of 128 x 128 to 384), but the
-    // caller waits for his own 14 launches less (whole step of that model 240 us with, 190 without them;
-    // 150 since its tensor lists are read in native code).  A step that is being recorded has no
-    // such launches when it is replayed (6 of 128 x 384 with 8 of 128 x 128: 94.5 us a replay in one launch, 74.0 without).
+    // A step over very little takes longer on the device (replays: 6 of 128 x 384 with 8 of 128 x 128 94.5 us in one launch, 74.0 without),
+    // but the caller waits for his own 14 launches less: steps of a model of 14 such matrices, one behind the other, 149 us and 199.  A
+    // step that is being recorded has no such launches when it is replayed.
     return !recorded && l.e[0].p_ptrs && 0.032 * most + 0.64 * chain + 55 < 120;
 }
 

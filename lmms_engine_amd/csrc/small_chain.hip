@@ -423,11 +423,13 @@ void launch_as(int nch, const ChainList& l, const ChainMath& cm, hipStream_t str
 
 bool chain_fits(int M, int K) { return M <= 64 && K <= 8192 && chain_per_wave(K) * chain_blocks(M) <= CHAIN_FRAGS; }
 
-// Whole pieces of rows cost the chain nothing (32 x 4096, 1 | 256 matrices: 80 | 147 us with the copy, 80 | 116 without).  Element by
-// element a workgroup pays 0.6 us for a fragment, which few matrices of many fragments feel more than the copy (one of 512 x 64,
-// eight fragments: 43 and 45.5; of 4096 x 32, 32 of them: 97 and 118; of 512 x 16, two: 20.4 and 19.2); from as many on as leave few
-// compute units idle, the copy is a pass over memory and costs more (256 of 512 x 64 61 and 55, of 4096 x 32 190 and 159, of 2048 x 64 181 and
-// 175, of 5632 x 16 182 and 124): three quarters of the compute units.
+// Measured (profiles/low_rank_result_copy.txt, iterations and result), with the copy | written by the chain.  Whole pieces of rows cost the
+// chain nothing: 32 x 4096, one | 256 matrices 78 | 77 and 124 | 95 us.  Element by element a workgroup pays 0.6 us for a fragment, which
+// few matrices of many fragments feel more than the copy: one of 4096 x 32 (32 fragments) 93 | 112, of 512 x 64 (eight) 40.5 | 42.8, of
+// 512 x 16 (two) 18.1 | 16.5.  With many matrices the copy, a pass over memory, costs more.  The lines cross between 64 matrices (5632 x 16,
+// 512 x 64) and 160 (2048 x 64); at three quarters of the compute units the chain is ahead everywhere: 192 of 5632 x 16 144 | 106, of
+// 4096 x 32 147 | 130, of 2048 x 64 143 | 135.  (Rows that are no whole pieces and not turned are the exception: 33 x 515, 192 matrices
+// 60.5 | 58.4, 1024 229 | 237.)
 bool chain_writes(int rows, int cols, int batch, const void* out, int cus) {
     if (rows <= cols && cols % 8 == 0 && ((uintptr_t)out & 15) == 0) return true;
     return 4L * batch >= 3L * cus || chain_per_wave(std::max(rows, cols)) * chain_blocks(std::min(rows, cols)) <= 4;
