@@ -1047,7 +1047,7 @@ __device__ __forceinline__ void pp_tile(const GemmArgs& g, const TileCoord& tc, 
     constexpr bool PRE = BM == 128;
     // The epilogues that need no LDS.  Measured: on whole 256-tiles b.A + c.A.A is 0.5 % faster without it, X.Xt 0.6 % slower; on
     // 128-tiles a launch of either is 1 % slower, but in the kernel with COH, where every tile is waited for, two barriers fewer are
-    // worth 3 to 10 % of a chain (1400 sets of matrices of 65 to 1536 rows).
+    // worth 2 % of the chain's launch in the mean and up to 8 % (56 drawn sets, profiles/flow_chain_or_launches.txt).
     constexpr bool REG = EPI == EPI_BX;
     constexpr bool SREG = (EPI == EPI_SYMPOLY && BM == 256) || (!QT && COH);
     constexpr int NEV = tile_pieces<BM, BN, WGM, WGN>(), LATE = PRE ? EPI_REST : EPI_ALL;
