@@ -469,6 +469,8 @@ bool flow_of(const Work& w, int steps, double a, double b, double c, const Updat
 // `out`: where the result of small matrices goes, dense (one bucket; null: X).
 int ns_chain(const Work& all, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s, bf16_t* out = nullptr) {
     if (steps < 0) return fail(MUON_HIP_EINVAL, "steps must be >= 0");
+    MachineShape ms;
+    if (hipError_t e = machine_shape(ms); e != hipSuccess) return hip_fail(e, "device shape");
     Work w;  // the matrices that go through the tiled products
     if (steps > 0) {
         ChainBucket small[MUON_HIP_MAX_BUCKETS];
@@ -490,15 +492,13 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
                 cm.alpha = (float)(-upd->lr);
             }
             Timed t(MUON_HIP_K_SMALL_CHAIN, s);
-            if (hipError_t e = launch_ns_chain(small, n, cm, s); e != hipSuccess) return hip_fail(e, "ns_chain launch");
+            if (hipError_t e = launch_ns_chain(small, n, cm, ms.cus, s); e != hipSuccess) return hip_fail(e, "ns_chain launch");
         }
         if (!w.n) return 0;
     } else {
         w = all;
     }
     FlowList fl;
-    MachineShape ms;
-    if (hipError_t e = machine_shape(ms); e != hipSuccess) return hip_fail(e, "device shape");
     const bool flow = steps > 0 && flow_of(w, steps, a, b, c, upd, 1 << ms.xcd_shift, upd && is_recorded(s), fl);
     if (flow)
         if (int rc = chain_alarm(&fl.alarm)) return rc;

@@ -50,6 +50,49 @@ __device__ __forceinline__ float materialized(float x) {
     return x;
 }
 
+// Two values rounded to bf16 in one instruction, the first in the low half; and back.
+__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{f2bf(a), f2bf(b)});
+}
+__device__ __forceinline__ float low_bf16(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
+__device__ __forceinline__ float high_bf16(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
+// bf(bf(a x) + v) for both halves of x and v
+__device__ __forceinline__ uint32_t axpy_bf16x2(float a, uint32_t x, uint32_t v) {
+    const uint32_t p = pack_bf16x2(a * low_bf16(x), a * high_bf16(x));
+    return pack_bf16x2(low_bf16(p) + low_bf16(v), high_bf16(p) + high_bf16(v));
+}
+
+// bf(u / d) with IEEE division, for bf16 values u and one bf16 value d.  u times the reciprocal of d rounds to the same value: a quotient of
+// two 8-bit significands is never halfway between two bf16 values (u = m d with an odd 9-bit m needs more than 8 bits) and at least 2^-17 of
+// itself away from there, and the product is off by 2^-22.  What that leaves out is a quotient among the subnormal numbers, where fewer bits
+// are kept, and a d whose reciprocal is one: those are divided.
+struct DivideBf16 {
+    float d, r;
+    bool fast;
+    __device__ __forceinline__ explicit DivideBf16(float d_) : d(d_), r(__fdiv_rn(1.0f, d_)), fast(d_ >= 0x1p-100f && d_ <= 0x1p100f) {}
+    // out is right where true is returned
+    __device__ __forceinline__ bool quick(bf16x8& out, const bf16x8& u) const {
+        const u32x4 w = __builtin_bit_cast(u32x4, u);
+        u32x4 o;
+        bool normal = fast;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float a = low_bf16(w[e]) * r, b = high_bf16(w[e]) * r;
+            normal &= !__builtin_amdgcn_classf(a, 0x90) & !__builtin_amdgcn_classf(b, 0x90);  // the subnormal numbers of either sign
+            o[e] = pack_bf16x2(a, b);
+        }
+        out = __builtin_bit_cast(bf16x8, o);
+        return normal;
+    }
+    __device__ __forceinline__ bf16x8 slow(const bf16x8& u) const {
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = f2bf(__fdiv_rn(bf2f(u[e]), d));
+        return o;
+    }
+};
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);

@@ -32,5 +32,5 @@ struct ChainMath {
 bool chain_fits(int M, int K);
 // Whether a bucket's result is better written to `out` by the chain than copied there from X, on a device of `cus` compute units.
 bool chain_writes(int rows, int cols, int batch, const void* out, int cus);
-// Every bucket must fit; steps >= 1.
-hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, hipStream_t stream);
+// Every bucket must fit; steps >= 1.  cus: compute units of the device.
+hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, int cus, hipStream_t stream);

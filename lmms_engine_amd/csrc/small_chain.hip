@@ -6,11 +6,15 @@
 // the parameter) written once; what bounds it is the chain of dependent steps inside a workgroup (five iterations of the sums of
 // X Xt handed from wave to wave, a walk over the wave's chunks, and three barriers) times the rounds of workgroups, not memory.
 // fast_newtonschulz, us, tiles | this:
-//      16 x  512, 1 | 256 | 1024 matrices   97 |  191 |  609    17 |  20 |  44
-//      16 x 5632                           217 | 1414 | 5461    72 |  94 | 395
-//      32 x 4096                           181 | 1087 | 4229    81 | 116 | 481
-//      64 x 2048                           137 |  556 | 2322    97 | 134 | 558
-//    2048 x   64                           139 |  567 | 2363   103 | 177 | 694
+//      16 x  512, 1 | 256 | 1024 matrices   97 |  191 |  609    20 |  22 |  50
+//      16 x 5632                           217 | 1414 | 5461    60 |  81 | 325
+//    5632 x   16                                                65 |  85 | 352
+//      32 x 4096                           181 | 1087 | 4229    75 | 109 | 431
+//      64 x 2048                           137 |  556 | 2322    87 | 118 | 497
+//    2048 x   64                           139 |  567 | 2363    96 | 131 | 509
+// What a workgroup spends (cycles, one 16 x 5632 with an fp32 parameter, 175000 in all): an iteration 20000, of which the sums of X Xt 9500 (48
+// for each of 176 MFMAs, hand-over included) and X' 10000; blend and norm 22000; the parameter, 720 KB through one compute unit, 48000.
+// With the blend divided element by element and the parameter in pairs of chunks these were 24000, 32000 and 60000.
 // It wins wherever the registers hold the matrix, so that is the rule (chain_fits); larger ones take the tiled products.
 //
 // Eight waves share the columns of X in chunks of 32, a run of consecutive chunks each.  Lane (i = l%16, q = l/16) of a wave holds
@@ -18,10 +22,11 @@
 // v_mfma_f32_16x16x32_bf16 as it stands, so
 //   A = X Xt      contracts such fragments with one another; the sum of a 16x16 block goes from wave to wave through LDS;
 //   B = bA + cAA  is a handful of MFMAs on A in LDS;
-//   X' = aX + BX  contracts rows, for which a chunk is turned by multiplying it with selected columns of the identity (exact:
-//                 one product is the element, the others are zero): the result's four registers are four rows of one column,
-//                 and the rows are dealt to the lanes so that two blocks make eight consecutive rows, the fragment that B's rows
-//                 meet; what comes out lies as X lay.
+//   X' = aX + BX  contracts rows, for which a chunk is turned on its way through 1 KB of LDS: a transposing read gives four rows of
+//                 one column, and the rows are dealt to the lanes so that two blocks make eight consecutive rows, the fragment
+//                 that B's rows meet; what comes out lies as X lay.
+// A matrix of a parameter that is taller than wide (X is its transpose) is read and written the same way where its rows are whole pieces
+// of four: a chunk is then a run of the parameter, 2 KB of it for 16 columns in fp32, and not 32 columns element by element.
 // Results are those of the tiled kernels bit for bit: the same rounding points (bf(X Xt); bf(bf(bA) + bf(c bf(AA)));
 // bf(bf(aX) + bf(BX))), and every fp32 sum in their order, ascending in 32-deep MFMAs with the reduction index in its natural
 // place.  That order is why a block of X Xt is one chain through the waves and not eight partial sums, which take 3 to 30 % less
@@ -44,112 +49,143 @@ __device__ __forceinline__ float update_one(float p, bf16_t x, float scale, floa
     return fmaf(alpha, os, pd);
 }
 
-// Eight consecutive columns of one row of X meet the parameter: a piece of its row, or (turned) of its column.  In two halves, so that
-// the loads of several pieces are in flight before the first store (the compiler cannot know that the pieces are apart: one after the
-// other they cost a trip to memory each, eight for a turned piece; see kBatch).
+// Four elements of the parameter that lie next to one another, and four of X (two registers) that meet them.
+template <typename PT>
+using FourOf = PT __attribute__((ext_vector_type(4)));
+template <typename PT>
+__device__ __forceinline__ FourOf<PT> update_four(const FourOf<PT>& p, uint32_t x01, uint32_t x23, float scale, float decay, float alpha) {
+    FourOf<PT> o;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const uint32_t x = e ? x23 : x01, os = pack_bf16x2(low_bf16(x) * scale, high_bf16(x) * scale);
+        if constexpr (sizeof(PT) == 2) {
+            const uint32_t pd = pack_bf16x2(bf2f(p[2 * e]) * decay, bf2f(p[2 * e + 1]) * decay);
+            o[2 * e] = f2bf(fmaf(alpha, low_bf16(os), low_bf16(pd)));
+            o[2 * e + 1] = f2bf(fmaf(alpha, high_bf16(os), high_bf16(pd)));
+        } else {
+            o[2 * e] = fmaf(alpha, low_bf16(os), p[2 * e] * decay);
+            o[2 * e + 1] = fmaf(alpha, high_bf16(os), p[2 * e + 1] * decay);
+        }
+    }
+    return o;
+}
+// Where the parameter is read and written in whole pieces: rows of X are rows of it (eight columns are all there or none is), or X is its
+// transpose and four rows of X lie next to one another there.
+__device__ __forceinline__ bool whole_rows(const void* p, int cols, bool turn) { return !turn && cols % 8 == 0 && (((uintptr_t)p) & 15) == 0; }
+__device__ __forceinline__ bool turned_pieces(const void* p, int M, bool turn, int elem) { return turn && M % 4 == 0 && ((uintptr_t)p & (4 * elem - 1)) == 0; }
+
+// Elsewhere element by element, eight columns of a row of X at a time.  In two halves, so that the loads of several pieces are in flight
+// before the first store (the compiler cannot know that the pieces are apart: one after the other they cost a trip to memory each, eight for
+// a turned piece; see kBatch).
 struct Piece {
     float v[8];
 };
-__device__ __forceinline__ bool whole_rows(const void* p, int cols, bool turn) { return !turn && cols % 8 == 0 && (((uintptr_t)p) & 15) == 0; }
 template <typename PT>
-__device__ __forceinline__ void load8(Piece& o, const PT* p, int row, int col, int cols, int M, int K, bool turn, bool whole) {
-    if (whole) {  // eight columns are all there or none is
-        const PT* d = p + (long)row * cols + col;
-        if constexpr (sizeof(PT) == 2) {
-            const bf16x8 v = *(const bf16x8*)d;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o.v[e] = bf2f(v[e]);
-        } else {
-            const f32x4 v = *(const f32x4*)d, w = *(const f32x4*)(d + 4);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) o.v[e] = v[e], o.v[4 + e] = w[e];
-        }
-        return;
-    }
+__device__ __forceinline__ void load_each(Piece& o, const PT* p, int row, int col, int cols, int M, int K, bool turn) {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
         if (col + e < K) o.v[e] = (float)p[turn ? (long)(col + e) * M + row : (long)row * cols + col + e];
 }
 template <typename PT>
-__device__ __forceinline__ void store8(PT* p, const Piece& o, const bf16x8& x, int row, int col, int cols, int M, int K, bool turn, bool whole, float scale,
-                                       float decay, float alpha) {
-    if (whole) {
-        PT* d = p + (long)row * cols + col;
-        if constexpr (sizeof(PT) == 2) {
-            bf16x8 v;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = f2bf(update_one<PT>(o.v[e], x[e], scale, decay, alpha));
-            *(bf16x8*)d = v;
-        } else {
-            f32x4 v, w;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                v[e] = update_one<PT>(o.v[e], x[e], scale, decay, alpha);
-                w[e] = update_one<PT>(o.v[4 + e], x[4 + e], scale, decay, alpha);
-            }
-            *(f32x4*)d = v;
-            *(f32x4*)(d + 4) = w;
-        }
-        return;
-    }
+__device__ __forceinline__ void store_each(PT* p, const Piece& o, const bf16x8& x, int row, int col, int cols, int M, int K, bool turn, float scale, float decay,
+                                           float alpha) {
 #pragma unroll
     for (int e = 0; e < 8; ++e)
         if (col + e < K) p[turn ? (long)(col + e) * M + row : (long)row * cols + col + e] = (PT)update_one<PT>(o.v[e], x[e], scale, decay, alpha);
 }
 
+// A block of 16 rows and 32 columns turned within a wave, through LDS of its own (a wave's LDS instructions are carried out in order,
+// so it needs no barrier).  lds_read_tr16: in a group of 16 lanes, lane i receives element i%4 of the 8-byte pieces addressed by lanes
+// i/4, 4 + i/4, 8 + i/4, 12 + i/4.
+constexpr int TURN_ZEROS = 16, TURN_BYTES = (TURN_ZEROS + 4) * 64;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ bf16x4 lds_read_tr16(const unsigned char* p) {
+    typedef __attribute__((address_space(3))) void* lds_void_ptr;
+    return __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(lds_void_ptr)p));
+}
+// v: four rows 4 (l%4) .. of columns l/4 and 16 + l/4 in lane l  ->  columns 8q .. 8q+7 of row i
+__device__ __forceinline__ bf16x8 turn_in(unsigned char* lds, const bf16x8& v, int lane) {
+    const int i = lane & 15, q = lane >> 4;
+    asm volatile("" ::: "memory");
+    *(bf16x4*)(lds + lane * 8) = bf16x4{v[0], v[1], v[2], v[3]};
+    *(bf16x4*)(lds + 512 + lane * 8) = bf16x4{v[4], v[5], v[6], v[7]};
+    asm volatile("" ::: "memory");
+    const unsigned char* r = lds + (8 * q + (i >> 2)) * 32 + (i & 3) * 8;
+    const bf16x4 lo = lds_read_tr16(r), hi = lds_read_tr16(r + 128);
+    asm volatile("" ::: "memory");
+    return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+// v: columns 8q .. 8q+7 of row i in lane (i, q)  ->  rows row .. row+3 of columns 8 (i/4) + i%4 and 8 (i/4) + 4 + i%4.  Without v: of the
+// block that is there.  Row TURN_ZEROS and those after it are zeros.
+__device__ __forceinline__ bf16x8 turn_rows(unsigned char* lds, const bf16x8* v, int row, int lane) {
+    const int i = lane & 15, q = lane >> 4;
+    if (v) {
+        asm volatile("" ::: "memory");
+        *(bf16x8*)(lds + i * 64 + q * 16) = *v;
+        asm volatile("" ::: "memory");
+    }
+    const unsigned char* r = lds + (row + (i >> 2)) * 64 + (i & 3) * 16;
+    const bf16x4 lo = lds_read_tr16(r), hi = lds_read_tr16(r + 8);
+    asm volatile("" ::: "memory");
+    return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+// v: columns 8q .. 8q+7 of row i in lane (i, q)  ->  rows 4q .. 4q+3 of column i, then of column 16 + i
+__device__ __forceinline__ bf16x8 turn_out(unsigned char* lds, const bf16x8& v, int lane) {
+    const int i = lane & 15, q = lane >> 4;
+    asm volatile("" ::: "memory");
+    *(bf16x8*)(lds + i * 64 + q * 16) = v;
+    asm volatile("" ::: "memory");
+    const unsigned char* r = lds + (4 * q + (i >> 2)) * 64 + (i & 3) * 8;
+    const bf16x4 lo = lds_read_tr16(r), hi = lds_read_tr16(r + 32);
+    asm volatile("" ::: "memory");
+    return bf16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+}
+
 // The row that lane i of 16 holds in block t of 16 rows.  The turned fragment of a block has rows i = 4q .. 4q+3 of it in lane group
 // q; in this order blocks 2p and 2p + 1 put rows 32p + 8q .. 32p + 8q + 7 there, which is where an MFMA has them.  A single block
-// (MT = 1) is in natural order: its fragment is put together by lane swaps instead.
+// (MT = 1) is in natural order: its fragment is two reads of four rows, and zeros.
 template <int MT>
 __device__ __forceinline__ int chain_row(int t, int i) {
     return MT == 1 ? i : 32 * (t >> 1) + 8 * (i >> 2) + 4 * (t & 1) + (i & 3);
 }
 
-// Rows 4q .. 4q+3 of a column in lane group q = l/16 become rows 8q .. 8q+7 in groups 0 and 1, and zeros in 2 and 3.
-__device__ __forceinline__ bf16x8 gather_rows16(const bf16x4& v) {
-    u32x2 r = __builtin_bit_cast(u32x2, v);
-    u32x4 o;
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const auto half = __builtin_amdgcn_permlane32_swap(r[e], 0u, false, false);      // groups 0, 1 and 2, 3, each before zeros
-        const auto part = __builtin_amdgcn_permlane16_swap(half[0], half[1], false, false);  // groups 0, 2 and 1, 3
-        o[e] = part[0];
-        o[2 + e] = part[1];
-    }
-    return __builtin_bit_cast(bf16x8, o);
-}
-
 constexpr int CHAIN_WAVES = 8;
 constexpr int CHAIN_FRAGS = 32;  // fragments of X a lane can hold: 128 of the 256 registers of a wave
 
-// Fragments that a lane loads from memory (the blend; the parameter) together, while those before them are still on their way: loads and
-// stores leave the queue in order, so a load that is issued behind a store waits for it as well.  One at a time, as written before, 56
-// matrices of 5632 x 16 in fp32 took 142 us, now 117 (with four 117 as well, at the cost of 20 to 50 registers); 168 + 84 + 56 of 2048 and 512 columns
-// 60 and 53; 256 of 2048 x 64 296 and 205 (a whole step; 256 of 64 x 2048 199 and 203 in fp32, 190 and 182 in bf16).  Asking for the parameter before the iterations, through LDS, gave nothing on top.
+// Where the parameter goes element by element: fragments that a lane asks for together, while those before them are still on their way
+// (loads and stores leave the queue in order, so a load that is issued behind a store waits for it as well).
 constexpr int kBatch = 2;
 
-// MT blocks of 16 rows (1, 2 or 4), up to NCH chunks of 32 columns per wave.
+template <int MT>
+struct ChainShared {
+    static constexpr int PITCH = 32 * ((MT + 1) / 2) + 8;  // of A and B; with MT = 1 columns 16 to 31 stay zero
+    f32x4 sum[MT * (MT + 1) / 2][64];
+    bf16_t A[MT * 16][PITCH], B[MT * 16][PITCH];
+    unsigned char turned[CHAIN_WAVES][TURN_BYTES];
+    float red[4];
+    int left[MT * (MT + 1) / 2];  // per leg: waves that have left it, of all iterations
+};
+
+// Matrix b of bucket k.  MT blocks of 16 rows (1, 2 or 4), up to NCH chunks of 32 columns per wave.
 template <int MT, int NCH>
-__global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainList l, const ChainMath cm) {
+__device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const ChainMath& cm, ChainShared<MT>& sh) {
     constexpr int NP = (MT + 1) / 2;         // 32-deep reductions over the rows
-    constexpr int PITCH = 32 * NP + 8;       // of A and B in LDS; with MT = 1 columns 16 to 31 stay zero
+    constexpr int PITCH = ChainShared<MT>::PITCH;
     constexpr int NF = MT * (MT + 1) / 2;    // 16 x 16 blocks of A on or above the diagonal
-    constexpr int BATCH = kBatch < MT ? 1 : kBatch / MT;  // chunks that are loaded from memory together
+    constexpr int BATCH = kBatch < MT ? 1 : kBatch / MT;  // chunks of the parameter that are loaded together
     constexpr bool TWO = MT < 4;             // while the next ones are on their way (with four blocks a chunk is enough, and two spill)
     // Chunks without a branch between them: 40 -> 30 ns for each MFMA of the chain through 176 chunks (16 x 5632).  Four blocks have
     // ten MFMAs between two branches anyway; and where a wave has four chunks at most, those that are not there cost as much as the
     // branches (111 of 20 x 56, one chunk: 17.5 with runs, 16.0 without).
     constexpr int RUN = MT == 4 || NCH < 8 ? 1 : 4;
-    static_assert(NCH % RUN == 0, "whole runs");
+    constexpr int GROUP = MT == 4 || RUN == 1 ? 1 : 4 / MT;  // chunks of X' that are computed together
+    static_assert(NCH % RUN == 0 && RUN % GROUP == 0, "whole runs");
     constexpr int LEG = MT == 4 ? 2 : 1, NLEG = NF / LEG;  // blocks that a wave adds its chunks to at a time
-    __shared__ __align__(16) f32x4 sum[NF][64];
-    __shared__ __align__(16) bf16_t As[MT * 16][PITCH], Bs[MT * 16][PITCH];
-    __shared__ float red[4];
-
-    int bucket = 0;
-    while (bucket + 1 < l.n && (int)blockIdx.x >= l.start[bucket + 1]) ++bucket;
-    const ChainBucket& k = l.b[__builtin_amdgcn_readfirstlane(bucket)];
-    const int b = blockIdx.x - l.start[__builtin_amdgcn_readfirstlane(bucket)];
+    auto& sum = sh.sum;
+    auto& As = sh.A;
+    auto& Bs = sh.B;
+    auto& turned = sh.turned;
+    auto& red = sh.red;
     const bool turn = k.rows > k.cols;
     const int M = turn ? k.cols : k.rows, K = turn ? k.rows : k.cols;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15, q = lane >> 4;
@@ -164,79 +200,94 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         (&As[0][0])[t] = (bf16_t)0.f;
         (&Bs[0][0])[t] = (bf16_t)0.f;
     }
-    // d = bf(bf(sqrt(sum)) + 1e-7), in the order of the normalisation kernel: both halves of the workgroup add the same sums
-    float s = 0.f;
-    for (int t = tid & 255; t < k.nparts; t += 256) s += k.partials[(long)b * k.nparts + t];
-    s = wave_sum(s);
-    if (lane == 0 && wave < 4) red[wave] = s;
-    __syncthreads();
-    const float d = rbf(rbf(sqrtf((red[0] + red[1]) + (red[2] + red[3]))) + 1e-7f);
-
-    // Normalised fragments, zero past the matrix's edges.  Through the work area, so that the loop over loads of every kind
-    // (ragged, turned) and divisions need not be unrolled over the register array.
-    const bool vec = !turn && K % 8 == 0;
-    auto fetch = [&](bf16x8& v, int j, int t) {
-        const int row = chain_row<MT>(t, i), col = col0 + j * 32;
-        if (vec && row < M && col < K) {
-            v = *(const bf16x8*)(u + (long)row * K + col);
-        } else {
+    *(unsigned*)&turned[wave][TURN_ZEROS * 64 + lane * 4] = 0u;
+    if (tid < NLEG) sh.left[tid] = 0;
+    // The matrix in whole pieces (turned: four rows of two columns, turned below), every load in flight together; zero past its edges.
+    const bool vec = !turn && K % 8 == 0, tvec = turned_pieces(u, M, turn, 2);
+    unsigned char* const tl = turned[wave];
+    float s = (tid & 255) < k.nparts ? k.partials[(long)b * k.nparts + (tid & 255)] : 0.f;  // asked for ahead of them
+    bf16x8 zero8;
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                v[e] = (row < M && col + e < K) ? u[turn ? (long)(col + e) * M + row : (long)row * K + col + e] : (bf16_t)0.f;
-        }
-    };
-    auto norm = [&](bf16x8& v, int j, int t) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = f2bf(__fdiv_rn(bf2f(v[e]), d));
-        mine[(j * MT + t) * 64] = v;
-    };
-    if constexpr (TWO) {
-        bf16x8 v[2][BATCH][MT];
-        auto each = [&](int j0, bf16x8 (&w)[BATCH][MT], auto f) {
-#pragma unroll
-            for (int jj = 0; jj < BATCH; ++jj)
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    if (j0 + jj < per) f(w[jj][t], j0 + jj, t);
-        };
-        each(0, v[0], fetch);
-        for (int j0 = 0; j0 < per; j0 += 2 * BATCH) {
-            each(j0 + BATCH, v[1], fetch);
-            each(j0, v[0], norm);
-            each(j0 + 2 * BATCH, v[0], fetch);
-            each(j0 + BATCH, v[1], norm);
-        }
-    } else {
-        // Four blocks in one order: a chunk's loads together would gain 4 % at 256 of 64 x 2048 and lose 9 % at 2048 x 64 (its elements
-        // come one by one) and 5 % at 111 of 34 x 56.
-#pragma unroll 4
-        for (int j = 0; j < per; ++j) {
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                bf16x8 v;
-                fetch(v, j, t);
-                norm(v, j, t);
-            }
-        }
-    }
-    bf16x8 zero8, unit[2];  // unit[h]: selects columns 8q' + 4h + 0..3 (q' = 0..3) of a chunk
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        zero8[e] = (bf16_t)0.f;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) unit[h][e] = (bf16_t)((q == i >> 2 && e == 4 * h + (i & 3)) ? 1.f : 0.f);
-    }
+    for (int e = 0; e < 8; ++e) zero8[e] = (bf16_t)0.f;
     bf16x8 x[NCH][MT];
 #pragma unroll
     for (int j = 0; j < NCH; ++j)
 #pragma unroll
-        for (int t = 0; t < MT; ++t) x[j][t] = j < per ? mine[(j * MT + t) * 64] : zero8;
-    // The sum of leg `leg` (LEG blocks of A) over this wave's chunks, on top of the waves' before it.
-    auto add_leg = [&](auto leg_c) {
-        constexpr int F0 = decltype(leg_c)::value * LEG;
-        f32x4 acc[LEG];
+        for (int t = 0; t < MT; ++t) x[j][t] = zero8;
+    if (vec) {
 #pragma unroll
-        for (int f = 0; f < LEG; ++f) acc[f] = wave == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : sum[F0 + f][lane];
+        for (int j = 0; j < NCH; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const int row = chain_row<MT>(t, i), col = col0 + j * 32;
+                if (j < per && row < M && col < K) x[j][t] = *(const bf16x8*)(u + (long)row * K + col);
+            }
+    } else if (tvec) {
+#pragma unroll
+        for (int j = 0; j < NCH; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const int row = chain_row<MT>(t, 4 * (lane & 3)), col = (wave * per + j) * 32 + (lane >> 2);
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (j < per && row < M && col + 16 * h < K) {
+                        const bf16x4 p = *(const bf16x4*)(u + (long)(col + 16 * h) * M + row);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) x[j][t][4 * h + e] = p[e];
+                    }
+            }
+    }
+    // d = bf(bf(sqrt(sum)) + 1e-7), in the order of the normalisation kernel: both halves of the workgroup add the same sums
+    for (int t = (tid & 255) + 256; t < k.nparts; t += 256) s += k.partials[(long)b * k.nparts + t];
+    s = wave_sum(s);
+    if (lane == 0 && wave < 4) red[wave] = s;
+    __syncthreads();
+    const DivideBf16 div(rbf(rbf(sqrtf((red[0] + red[1]) + (red[2] + red[3]))) + 1e-7f));
+    bool exact = (vec || tvec) && div.fast;
+    if (exact) {
+#pragma unroll
+        for (int j = 0; j < NCH; ++j)
+            if (j < per) {
+#pragma unroll
+                for (int t = 0; t < MT; ++t) exact &= div.quick(x[j][t], tvec ? turn_in(tl, x[j][t], lane) : x[j][t]);
+            }
+    }
+    if (!__all(exact)) {
+        // Element by element, or divided one by one: a fragment at a time through the work area, so that the loop need not be unrolled over
+        // the register array.
+#pragma unroll 4
+        for (int j = 0; j < per; ++j) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const int row = chain_row<MT>(t, i), col = col0 + j * 32;
+                bf16x8 v;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = (row < M && col + e < K) ? u[turn ? (long)(col + e) * M + row : (long)row * K + col + e] : (bf16_t)0.f;
+                mine[(j * MT + t) * 64] = div.slow(v);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NCH; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) x[j][t] = j < per ? mine[(j * MT + t) * 64] : zero8;
+    }
+    // The sum of leg `leg` (LEG blocks of A) over this wave's chunks, on top of the waves' before it.
+    auto add_leg = [&](auto leg_c, int before) {
+        constexpr int F0 = decltype(leg_c)::value * LEG;
+        int* const left = &sh.left[decltype(leg_c)::value];
+        f32x4 acc[LEG];
+        for (;;) {  // the count and the sums in one trip to LDS (a wave's LDS instructions are carried out in order)
+            const int n = __hip_atomic_load(left, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int f = 0; f < LEG; ++f) acc[f] = sum[F0 + f][lane];
+            if (n == before) break;
+        }
+        if (wave == 0) {
+#pragma unroll
+            for (int f = 0; f < LEG; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        __builtin_amdgcn_s_setprio(3);
 #pragma unroll
         for (int j0 = 0; j0 < NCH; j0 += RUN) {
             if (j0 >= per) break;
@@ -252,20 +303,26 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         }
 #pragma unroll
         for (int f = 0; f < LEG; ++f) sum[F0 + f][lane] = acc[f];
+        __builtin_amdgcn_s_setprio(0);
+        asm volatile("" ::: "memory");
+        if (lane == 0) __hip_atomic_store(left, before + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
 
+    const int active = ((K + 31) / 32 + per - 1) / per;  // waves that have columns
     for (int it = 0; it < cm.steps; ++it) {
-        // A wave starts a leg when the wave before it has left it, so the legs follow one another through the waves.
-        for (int slot = 0; slot < NLEG + CHAIN_WAVES - 1; ++slot) {
-            const int leg = slot - wave;
-            if (leg == 0) add_leg(std::integral_constant<int, 0>{});
-            if constexpr (NLEG > 1) if (leg == 1) add_leg(std::integral_constant<int, 1>{});
-            if constexpr (NLEG > 2) if (leg == 2) add_leg(std::integral_constant<int, 2>{});
-            if constexpr (NLEG > 3) if (leg == 3) add_leg(std::integral_constant<int, 3>{});
-            if constexpr (NLEG > 4) if (leg == 4) add_leg(std::integral_constant<int, 4>{});
+        // A wave starts a leg when the wave before it has left it, so the legs follow one another through the waves; the first ones go
+        // ahead while the last are still at X' of the iteration before.  Every wave of the workgroup runs, and waits only for the one
+        // before it.
+        if (wave < active) {
+            const int before = it * active + wave;
+            add_leg(std::integral_constant<int, 0>{}, before);
+            if constexpr (NLEG > 1) add_leg(std::integral_constant<int, 1>{}, before);
+            if constexpr (NLEG > 2) add_leg(std::integral_constant<int, 2>{}, before);
+            if constexpr (NLEG > 3) add_leg(std::integral_constant<int, 3>{}, before);
+            if constexpr (NLEG > 4) add_leg(std::integral_constant<int, 4>{}, before);
             static_assert(NLEG <= 5 && NLEG * LEG == NF, "every leg has its branch");
-            __syncthreads();
         }
+        __syncthreads();
         for (int t = tid; t < NF * 64; t += 64 * CHAIN_WAVES) {
             const int ln = t & 63;
             int f = t >> 6, ti = 0;
@@ -300,42 +357,65 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int p = 0; p < NP; ++p) bfr[t][p] = *(const bf16x8*)&Bs[chain_row<MT>(t, i)][p * 32 + 8 * q];
-        auto next_chunk = [&](bf16x8 (&xc)[MT]) {
-            bf16x8 xt[2][NP];
+        // GROUP chunks together, so that one's way through LDS and the products passes behind the others'
+        auto next_chunks = [&](int j0, auto count_c) {
+            constexpr int N = decltype(count_c)::value;
+            bf16x8 xt[N][2][NP];  // xt[.][h][p]: rows 32p + 8q .. + 7 of column 8 (i/4) + 4h + i%4, the operand that B's rows meet
 #pragma unroll
-            for (int h = 0; h < 2; ++h)
+            for (int n = 0; n < N; ++n) {
+                bf16x8(&xc)[MT] = x[j0 + n];
+                if constexpr (MT == 1) {
+                    const bf16x8 lo = turn_rows(tl, &xc[0], q < 2 ? 8 * q : TURN_ZEROS, lane), hi = turn_rows(tl, nullptr, q < 2 ? 8 * q + 4 : TURN_ZEROS, lane);
 #pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    const f32x4 v = mfma(xc[t], unit[h], f32x4{0.f, 0.f, 0.f, 0.f});
-                    if constexpr (MT == 1) {
-                        xt[h][0] = gather_rows16(bf16x4{f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3])});
-                    } else {
+                    for (int h = 0; h < 2; ++h)
+                        xt[n][h][0] = bf16x8{lo[4 * h], lo[4 * h + 1], lo[4 * h + 2], lo[4 * h + 3], hi[4 * h], hi[4 * h + 1], hi[4 * h + 2], hi[4 * h + 3]};
+                } else {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) xt[h][t / 2][4 * (t & 1) + e] = f2bf(v[e]);
+                    for (int t = 0; t < MT; ++t) {
+                        const bf16x8 v = turn_rows(tl, &xc[t], 4 * q, lane);
+#pragma unroll
+                        for (int h = 0; h < 2; ++h)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) xt[n][h][t / 2][4 * (t & 1) + e] = v[4 * h + e];
                     }
                 }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            f32x4 v[N][MT][2];
 #pragma unroll
-            for (int t = 0; t < MT; ++t)
+            for (int p = 0; p < NP; ++p)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+                for (int n = 0; n < N; ++n)
 #pragma unroll
-                    for (int p = 0; p < NP; ++p) v = mfma(xt[h][p], bfr[t][p], v);
+                    for (int t = 0; t < MT; ++t)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) xc[t][4 * h + e] = f2bf(rbf(cm.a * bf2f(xc[t][4 * h + e])) + rbf(v[e]));
+                        for (int h = 0; h < 2; ++h) v[n][t][h] = mfma(xt[n][h][p], bfr[t][p], p ? v[n][t][h] : f32x4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    u32x4 xw = __builtin_bit_cast(u32x4, x[j0 + n][t]);
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int e = 0; e < 2; ++e) xw[2 * h + e] = axpy_bf16x2(cm.a, xw[2 * h + e], pack_bf16x2(v[n][t][h][2 * e], v[n][t][h][2 * e + 1]));
+                    x[j0 + n][t] = __builtin_bit_cast(bf16x8, xw);
                 }
         };
+        // (waves w and w + 4 share a SIMD: the first four are done in half of the time, and the sums of the next iteration can start)
+        if (wave < CHAIN_WAVES / 2) __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int j0 = 0; j0 < NCH; j0 += RUN) {
             if (j0 + RUN <= per) {
 #pragma unroll
-                for (int j = j0; j < j0 + RUN; ++j) next_chunk(x[j]);
+                for (int j = j0; j < j0 + RUN; j += GROUP) next_chunks(j, std::integral_constant<int, GROUP>{});
             } else {  // (nothing is computed past the last chunk: with an infinite B its zeros would not stay zero)
 #pragma unroll
                 for (int j = j0; j < j0 + RUN - 1; ++j)
-                    if (j < per) next_chunk(x[j]);
+                    if (j < per) next_chunks(j, std::integral_constant<int, 1>{});
             }
         }
+        __builtin_amdgcn_s_setprio(0);
     }
 
     bf16_t* out = k.out + (long)b * M * K;
@@ -350,6 +430,59 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
             }
         return;
     }
+    if (!k.p_ptrs && turned_pieces(k.out, M, turn, 2)) {
+#pragma unroll
+        for (int j = 0; j < NCH; ++j)
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                if (j >= per) continue;
+                const bf16x8 v = turn_out(tl, x[j][t], lane);
+                const int row = chain_row<MT>(t, 4 * q), col = (wave * per + j) * 32 + i;
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (row < M && col + 16 * h < K)
+                        *(bf16x4*)(out + (long)(col + 16 * h) * M + row) = bf16x4{v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+            }
+        return;
+    }
+    void* const p = k.p_ptrs ? const_cast<void*>(k.p_ptrs[b]) : nullptr;
+    auto piece_update = [&](auto* pp, auto turned_c) {
+        using PT = std::remove_pointer_t<decltype(pp)>;
+        constexpr bool TURNED = decltype(turned_c)::value;
+        // fragments whose pieces are asked for together: what the registers hold beside X
+        constexpr int G = sizeof(PT) == 4 || NCH * MT == 8 ? (NCH * MT == 8 ? 4 : 8) : 16;
+#pragma unroll
+        for (int f0 = 0; f0 < NCH * MT; f0 += G) {
+            if (f0 / MT >= per) break;
+            FourOf<PT> o[G][2];
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int j = (f0 + g) / MT, t = (f0 + g) % MT, row = chain_row<MT>(t, TURNED ? 4 * q : i), col = TURNED ? (wave * per + j) * 32 + i : col0 + j * 32;
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (j < per && row < M && col + (TURNED ? 16 * h : 0) < K)
+                        o[g][h] = *(const FourOf<PT>*)(pp + (TURNED ? (long)(col + 16 * h) * M + row : (long)row * K + col + 4 * h));
+            }
+#pragma unroll
+            for (int g = 0; g < G; ++g) {
+                const int j = (f0 + g) / MT, t = (f0 + g) % MT, row = chain_row<MT>(t, TURNED ? 4 * q : i), col = TURNED ? (wave * per + j) * 32 + i : col0 + j * 32;
+                if (j >= per) continue;
+                const bf16x8 v = TURNED ? turn_out(tl, x[j][t], lane) : x[j][t];
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (row < M && col + (TURNED ? 16 * h : 0) < K)
+                        *(FourOf<PT>*)(pp + (TURNED ? (long)(col + 16 * h) * M + row : (long)row * K + col + 4 * h)) =
+                            update_four<PT>(o[g][h], __builtin_bit_cast(u32x4, v)[2 * h], __builtin_bit_cast(u32x4, v)[2 * h + 1], k.scale, cm.decay, cm.alpha);
+            }
+        }
+    };
+    auto try_pieces = [&](auto* pp) {
+        if (turned_pieces(p, M, turn, sizeof(*pp))) piece_update(pp, std::true_type{});
+        else if (whole_rows(p, k.cols, turn)) piece_update(pp, std::false_type{});
+        else return false;
+        return true;
+    };
+    if (k.p_ptrs && (cm.p_dtype == MUON_HIP_BF16 ? try_pieces((bf16_t*)p) : try_pieces((float*)p))) return;
 #pragma unroll
     for (int j = 0; j < NCH; ++j)
 #pragma unroll
@@ -367,9 +500,7 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
             }
         return;
     }
-    void* p = const_cast<void*>(k.p_ptrs[b]);
-    const bool whole = whole_rows(p, k.cols, turn);
-    auto update = [&](auto* pp) {
+    auto each_update = [&](auto* pp) {  // element by element, BATCH chunks asked for ahead of the stores of the BATCH before
         struct Batch {
             Piece o[BATCH][MT];
             bf16x8 v[BATCH][MT];
@@ -386,13 +517,11 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
         auto load = [&](int j0, Batch& w) {
             each(j0, [&](int jj, int t, int row, int col) {
                 w.v[jj][t] = mine[((j0 + jj) * MT + t) * 64];
-                load8(w.o[jj][t], pp, row, col, k.cols, M, K, turn, whole);
+                load_each(w.o[jj][t], pp, row, col, k.cols, M, K, turn);
             });
         };
         auto store = [&](int j0, Batch& w) {
-            each(j0, [&](int jj, int t, int row, int col) {
-                store8(pp, w.o[jj][t], w.v[jj][t], row, col, k.cols, M, K, turn, whole, k.scale, cm.decay, cm.alpha);
-            });
+            each(j0, [&](int jj, int t, int row, int col) { store_each(pp, w.o[jj][t], w.v[jj][t], row, col, k.cols, M, K, turn, k.scale, cm.decay, cm.alpha); });
         };
         if constexpr (TWO) load(0, w[0]);
         for (int j0 = 0; j0 < per; j0 += (TWO ? 2 : 1) * BATCH) {
@@ -404,12 +533,33 @@ __global__ void __launch_bounds__(64 * CHAIN_WAVES) ns_chain_kernel(const ChainL
             }
         }
     };
-    if (cm.p_dtype == MUON_HIP_BF16) update((bf16_t*)p);
-    else update((float*)p);
+    if (cm.p_dtype == MUON_HIP_BF16) each_update((bf16_t*)p);
+    else each_update((float*)p);
 }
 
-int chain_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
-int chain_per_wave(int K) { return ((K + 31) / 32 + CHAIN_WAVES - 1) / CHAIN_WAVES; }
+// Workgroup `id` of a list: its bucket, and the matrix there.
+__device__ __forceinline__ int chain_bucket(const ChainList& l, int id, int& b) {
+    int i = 0;
+    while (i + 1 < l.n && id >= l.start[i + 1]) ++i;
+    i = __builtin_amdgcn_readfirstlane(i);
+    b = id - l.start[i];
+    return i;
+}
+
+// (with 8 fragments two workgroups share a compute unit)
+template <int MT, int NCH>
+__global__ void __launch_bounds__(64 * CHAIN_WAVES, MT * NCH == 8 ? 4 : 2) ns_chain_kernel(const ChainList l, const ChainMath cm) {
+    __shared__ __align__(16) unsigned char shared[sizeof(ChainShared<MT>)];
+    int b;
+    const int i = chain_bucket(l, blockIdx.x, b);
+    chain_matrix<MT, NCH>(l.b[i], b, cm, *(ChainShared<MT>*)shared);
+}
+
+__host__ __device__ constexpr int chain_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
+__host__ __device__ constexpr int chain_per_wave(int K) { return ((K + 31) / 32 + CHAIN_WAVES - 1) / CHAIN_WAVES; }
+
+// Fragments of X per lane that a kernel is built for.
+__host__ __device__ constexpr int chain_class(int need) { return need <= 8 ? 8 : need <= 16 ? 16 : 32; }
 
 template <int MT>
 void launch_as(int nch, const ChainList& l, const ChainMath& cm, hipStream_t stream) {
@@ -423,41 +573,52 @@ void launch_as(int nch, const ChainList& l, const ChainMath& cm, hipStream_t str
 
 bool chain_fits(int M, int K) { return M <= 64 && K <= 8192 && chain_per_wave(K) * chain_blocks(M) <= CHAIN_FRAGS; }
 
-// Measured (profiles/low_rank_result_copy.txt, iterations and result), with the copy | written by the chain.  Whole pieces of rows cost the
-// chain nothing: 32 x 4096, one | 256 matrices 78 | 77 and 124 | 95 us.  Element by element a workgroup pays 0.6 us for a fragment, which
-// few matrices of many fragments feel more than the copy: one of 4096 x 32 (32 fragments) 93 | 112, of 512 x 64 (eight) 40.5 | 42.8, of
-// 512 x 16 (two) 18.1 | 16.5.  With many matrices the copy, a pass over memory, costs more.  The lines cross between 64 matrices (5632 x 16,
-// 512 x 64) and 160 (2048 x 64); at three quarters of the compute units the chain is ahead everywhere: 192 of 5632 x 16 144 | 106, of
-// 4096 x 32 147 | 130, of 2048 x 64 143 | 135.  (Rows that are no whole pieces and not turned are the exception: 33 x 515, 192 matrices
-// 60.5 | 58.4, 1024 229 | 237.)
+// Whole pieces, of rows or of a turned matrix's columns, cost the chain nothing.  Element by element a workgroup pays 0.6 us for a fragment,
+// which few matrices of many fragments feel more than the copy, while with many the copy, a pass over memory, costs more: the lines cross
+// between 64 and 160 matrices (profiles/low_rank_result_copy.txt); at three quarters of the compute units the chain is ahead everywhere.  (Rows
+// that are no whole pieces and not turned are the exception: 33 x 515, 192 matrices 60.5 with the copy, 58.4 without, 1024 229 and 237.)
 bool chain_writes(int rows, int cols, int batch, const void* out, int cus) {
     if (rows <= cols && cols % 8 == 0 && ((uintptr_t)out & 15) == 0) return true;
+    if (rows > cols && cols % 4 == 0 && ((uintptr_t)out & 7) == 0) return true;
     return 4L * batch >= 3L * cus || chain_per_wave(std::max(rows, cols)) * chain_blocks(std::min(rows, cols)) <= 4;
 }
 
-// One launch per kernel: blocks of rows, and 8, 16 or 32 fragments of X per lane (fewer registers, more workgroups in flight).
-hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, hipStream_t stream) {
+// One launch per number of row blocks, on the kernel that holds the widest matrices, or one per kernel (8, 16 or 32 fragments of X per
+// lane: fewer registers, more workgroups in flight).
+hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, int cus, hipStream_t stream) {
     if (n < 1 || n > CHAIN_MAX_LIST || cm.steps < 1) return hipErrorInvalidValue;
-    for (int mt = 4; mt >= 1; mt /= 2)
-        for (int frags = CHAIN_FRAGS; frags >= 8; frags /= 2) {
-            ChainList l;
-            l.n = 0;
-            l.start[0] = 0;
-            for (int i = 0; i < n; ++i) {
-                const ChainBucket& k = buckets[i];
-                const int M = k.rows < k.cols ? k.rows : k.cols, K = k.rows < k.cols ? k.cols : k.rows;
-                if (!chain_fits(M, K)) return hipErrorInvalidValue;
-                const int need = chain_per_wave(K) * chain_blocks(M);
-                if (chain_blocks(M) != mt || (need <= 8 ? 8 : need <= 16 ? 16 : 32) != frags) continue;
-                l.b[l.n] = k;
-                l.start[l.n + 1] = l.start[l.n] + k.batch;
-                ++l.n;
-            }
-            if (!l.n) continue;
-            if (mt == 4) launch_as<4>(frags / 4, l, cm, stream);
-            else if (mt == 2) launch_as<2>(frags / 2, l, cm, stream);
-            else launch_as<1>(frags, l, cm, stream);
-            if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    int order[CHAIN_MAX_LIST], need[CHAIN_MAX_LIST], blocks[CHAIN_MAX_LIST];
+    for (int i = 0; i < n; ++i) {
+        const ChainBucket& k = buckets[i];
+        const int M = std::min(k.rows, k.cols), K = std::max(k.rows, k.cols);
+        if (!chain_fits(M, K)) return hipErrorInvalidValue;
+        blocks[i] = chain_blocks(M);
+        need[i] = chain_per_wave(K) * blocks[i];
+        order[i] = i;
+    }
+    std::stable_sort(order, order + n, [&](int x, int y) { return blocks[x] != blocks[y] ? blocks[x] > blocks[y] : need[x] > need[y]; });
+    for (int at = 0; at < n;) {
+        const int mt = blocks[order[at]], frags = chain_class(need[order[at]]);
+        // The longest first, the others on the compute units that they leave: a launch of its own per width waits for the one before.  The
+        // narrow ones lose a place: two workgroups of 8 fragments share a compute unit on their own kernel, on a wider one each has its own.
+        // Steps (us, apart | together): 308 narrow with 84 of 16 x 5632 and 5632 x 16 178 | 140, a quarter of them 134 | 100; 12 of 24 x
+        // 1024 to 2624 in three widths 164 | 82; 504 narrow of 24 x 1024 with 168 of 24 x 2200 189 | 199; 616 with 168 of rank 16 272 | 262.
+        long narrow = 0;
+        for (int i = 0; i < n; ++i)
+            if (blocks[i] == mt && chain_class(need[i]) == 8) narrow += buckets[i].batch;
+        const bool together = 2 * narrow <= 3L * cus;
+        ChainList l;
+        l.n = 0;
+        l.start[0] = 0;
+        for (; at < n && blocks[order[at]] == mt && (together || chain_class(need[order[at]]) == frags); ++at) {
+            l.b[l.n] = buckets[order[at]];
+            l.start[l.n + 1] = l.start[l.n] + l.b[l.n].batch;
+            ++l.n;
         }
+        if (mt == 4) launch_as<4>(frags / 4, l, cm, stream);
+        else if (mt == 2) launch_as<2>(frags / 2, l, cm, stream);
+        else launch_as<1>(frags, l, cm, stream);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
     return hipSuccess;
 }
