@@ -50,10 +50,13 @@ __device__ __forceinline__ float materialized(float x) {
     return x;
 }
 
-// Two values rounded to bf16 in one instruction, the first in the low half; and back.
+// Two values rounded to bf16 in one instruction, the first in the low half; and back.  Left to itself the compiler rounds most of them one by
+// one, where the halves are used again: half an instruction more per element and rounding point.
 __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, bf16x2{f2bf(a), f2bf(b)});
+    uint32_t w = __builtin_bit_cast(uint32_t, bf16x2{f2bf(a), f2bf(b)});
+    asm("" : "+v"(w));  // (what is taken out of it again is taken out of this register)
+    return w;
 }
 __device__ __forceinline__ float low_bf16(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
 __device__ __forceinline__ float high_bf16(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
@@ -61,6 +64,10 @@ __device__ __forceinline__ float high_bf16(uint32_t w) { return __builtin_bit_ca
 __device__ __forceinline__ uint32_t axpy_bf16x2(float a, uint32_t x, uint32_t v) {
     const uint32_t p = pack_bf16x2(a * low_bf16(x), a * high_bf16(x));
     return pack_bf16x2(low_bf16(p) + low_bf16(v), high_bf16(p) + high_bf16(v));
+}
+__device__ __forceinline__ bf16x8 axpy_bf16x8(float a, const bf16x8& x, const bf16x8& v) {
+    const u32x4 xw = __builtin_bit_cast(u32x4, x), vw = __builtin_bit_cast(u32x4, v);
+    return __builtin_bit_cast(bf16x8, u32x4{axpy_bf16x2(a, xw[0], vw[0]), axpy_bf16x2(a, xw[1], vw[1]), axpy_bf16x2(a, xw[2], vw[2]), axpy_bf16x2(a, xw[3], vw[3])});
 }
 
 // bf(u / d) with IEEE division, for bf16 values u and one bf16 value d.  u times the reciprocal of d rounds to the same value: a quotient of
