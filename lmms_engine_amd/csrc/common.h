@@ -11,6 +11,10 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// Vectors at the address of any element: the hardware reads and writes them whole, at the cost of the cache lines that they touch.
+typedef bf16x8 __attribute__((aligned(2))) bf16x8_any;
+typedef f32x4 __attribute__((aligned(4))) f32x4_any;
+
 // dtype codes shared with the C ABI (include/muon_hip.h)
 #define MUON_HIP_F32 0
 #define MUON_HIP_BF16 1

@@ -247,6 +247,10 @@ __global__ void __launch_bounds__(256) frob_finalize_kernel(const EwList l) {
 // A parameter with rows > cols (X = u^T): a tile of 32 rows x 128 columns of u goes through an LDS transpose and leaves
 // as 128 rows of X, 32 elements each (the 64-byte rows of one column block, back to back).  32 x 128 measured best of
 // {32, 64} x {64, 128}: 5.5 to 5.7 TB/s against 5.2 to 5.5 for 64 x 128.
+//
+// Rows that are no whole pieces are read in pieces of 16 bytes all the same, from whatever address they start at: a piece costs at most one
+// cache line more.  12 of 1000 x 2731 element by element took 45 us, like this 34.
+// The quotients are products with the reciprocal (DivideBf16): 48 of 896 x 4864 160 -> 154 us, 16 of 512 x 1408 16.0 -> 14.4.
 constexpr int NORM_TR = 16, NORM_T_TR = 32, NORM_TC = 128;
 __global__ void __launch_bounds__(256) normalize_kernel(const EwList l) {
     constexpr int TC = NORM_TC, TR = NORM_T_TR, PITCH = TC + 8;
@@ -257,7 +261,7 @@ __global__ void __launch_bounds__(256) normalize_kernel(const EwList l) {
     if ((int)blockIdx.x == l.start[bucket])
         for (int i = threadIdx.x; i < e.clear_words; i += 256) e.clear[i] = 0u;
     const int rows = e.rows, cols = e.cols, cbx = e.Kp / BLK_COLS;
-    const bool vec = (cols % 8) == 0, turn = rows > cols;
+    const bool turn = rows > cols;
     // u's padded image is Mp x Kp, or Kp x Mp when it is turned; both are whole 128-tiles
     const int tiles_c = (turn ? e.Mp : e.Kp) / TC, per_mat = turn ? (e.Kp / TR) * tiles_c : (e.Mp / NORM_TR) * tiles_c;
     const int local = blockIdx.x - l.start[bucket], b = local / per_mat, t = local - b * per_mat;
@@ -266,8 +270,8 @@ __global__ void __launch_bounds__(256) normalize_kernel(const EwList l) {
     const int r0 = (t / tiles_c) * (turn ? TR : NORM_TR), c0 = (t % tiles_c) * TC;
     auto load8 = [&](int r, int c) {
         bf16x8 v;
-        if (r < rows && vec && c + 8 <= cols) {
-            v = *(const bf16x8*)(u + (long)r * cols + c);
+        if (r < rows && c + 8 <= cols) {
+            v = *(const bf16x8_any*)(u + (long)r * cols + c);
         } else {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[i] = (r < rows && c + i < cols) ? u[(long)r * cols + c + i] : (bf16_t)0.f;
@@ -279,10 +283,10 @@ __global__ void __launch_bounds__(256) normalize_kernel(const EwList l) {
     v[0] = load8(r0 + tr, c0 + tc);
     if (turn) v[1] = load8(r0 + tr + 16, c0 + tc);
     const float d = e.inline_norm ? frob_denom(e.partials + (long)b * e.nparts, e.nparts, red) : e.denom[b];
+    const DivideBf16 div(d);
     auto divide = [&](const bf16x8& a) {
         bf16x8 o;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = f2bf(__fdiv_rn(bf2f(a[i]), d));
+        if (!div.quick(o, a)) o = div.slow(a);
         return o;
     };
     if (!turn) {
@@ -411,8 +415,7 @@ apply_update_t_kernel(const void* const* p_ptrs, const bf16_t* O, long strideO, 
 // A blocked matrix, or its transpose, into a dense row-major bf16 tensor (row pitch ld): the NS output of
 // fast_newtonschulz called alone, and the result of a single GEMM.  One workgroup moves a tile of 64 output rows
 // x 128 output columns: straight (16-byte pieces of rows of the blocked image) or, for the transpose, from 128
-// rows x 64 columns of the blocked image through LDS.  Output rows leave as 16-byte vectors when the row pitch
-// and the base allow it.
+// rows x 64 columns of the blocked image through LDS.  Output rows leave as 16-byte vectors, wherever they start.
 __global__ void __launch_bounds__(256)
 unpack_kernel(bf16_t* out, long strideOut, int ld, const bf16_t* O, long strideO, int cbo, int rows, int cols,
               int transposed) {
@@ -423,7 +426,6 @@ unpack_kernel(bf16_t* out, long strideOut, int ld, const bf16_t* O, long strideO
     const bf16_t* o = O + b * strideO;
     const int tiles_c = (cols + TC - 1) / TC;
     const int r0 = (blockIdx.x / tiles_c) * TR, c0 = (blockIdx.x % tiles_c) * TC;
-    const bool vec = (ld % 8 == 0) && ((((uintptr_t)dst) & 15) == 0);
     const int pr = threadIdx.x >> 4, pc = (threadIdx.x & 15) * 8;  // 16 rows x 16 chunks per pass
     if (transposed) {
         // image rows c0..c0+127, columns r0..r0+63; the blocked image is padded to whole 128-tiles in both
@@ -446,8 +448,8 @@ unpack_kernel(bf16_t* out, long strideOut, int ld, const bf16_t* O, long strideO
             v = *(const bf16x8*)(o + blocked_offset(r, c, cbo));  // columns c..c+7 lie in one block row (c % 8 == 0)
         }
         bf16_t* d = dst + (long)r * ld + c;
-        if (vec && c + 8 <= cols) {
-            *(bf16x8*)d = v;
+        if (c + 8 <= cols) {
+            *(bf16x8_any*)d = v;
         } else {
             for (int i = 0; i < 8 && c + i < cols; ++i) d[i] = v[i];
         }
@@ -467,8 +469,8 @@ pack_kernel(const bf16_t* src, long strideSrc, int ld, int rows, int cols, bf16_
         const int c = (int)(i - r * (cols_p / 8)) * 8;
         bf16x8 v;
         const bf16_t* sp = src + b * strideSrc + r * ld + c;
-        if (r < rows && c + 8 <= cols && ((((uintptr_t)sp) & 15) == 0)) {
-            v = *(const bf16x8*)sp;
+        if (r < rows && c + 8 <= cols) {
+            v = *(const bf16x8_any*)sp;
         } else {
 #pragma unroll
             for (int k = 0; k < 8; ++k) v[k] = (r < rows && c + k < cols) ? sp[k] : (bf16_t)0.f;

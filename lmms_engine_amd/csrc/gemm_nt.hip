@@ -323,38 +323,43 @@ struct FoldPiece {
                               // the fetch of `lo` brought in
 };
 template <typename PT, bool WHOLE>
-__device__ __forceinline__ void fold_load(FoldPiece<WHOLE>& f, const PT* p, bool vec, int left) {
-    if (!vec || left < 8) return;
-    f.lo = __builtin_nontemporal_load((const f32x4*)p);
-    if constexpr (WHOLE && sizeof(PT) == 4) f.hi[0] = __builtin_nontemporal_load((const f32x4*)(p + 4));
+__device__ __forceinline__ void fold_load(FoldPiece<WHOLE>& f, const PT* p, int left) {
+    if (left < 8) return;
+    if constexpr (sizeof(PT) == 2) {
+        const bf16x8 v = __builtin_nontemporal_load((const bf16x8_any*)p);
+        f.lo = *(const f32x4*)&v;
+    } else {
+        f.lo = __builtin_nontemporal_load((const f32x4_any*)p);
+        if constexpr (WHOLE) f.hi[0] = __builtin_nontemporal_load((const f32x4_any*)(p + 4));
+    }
 }
 template <typename PT, bool WHOLE>
-__device__ __forceinline__ void fold_apply(PT* p, const FoldPiece<WHOLE>& f, const bf16x8& x, bool vec, int left, const GemmArgs& g) {
+__device__ __forceinline__ void fold_apply(PT* p, const FoldPiece<WHOLE>& f, const bf16x8& x, int left, const GemmArgs& g) {
     constexpr bool PBF = std::is_same<PT, bf16_t>::value;
     auto one = [&](float pv, bf16_t xv) {
         const float os = rbf(bf2f(xv) * g.upd_scale);
         const float pd = PBF ? rbf(pv * g.upd_decay) : pv * g.upd_decay;
         return fmaf(g.upd_alpha, os, pd);
     };
-    if (vec && left >= 8) {
+    if (left >= 8) {
         if constexpr (PBF) {
             bf16x8 pv = *(const bf16x8*)&f.lo;
 #pragma unroll
             for (int k = 0; k < 8; ++k) pv[k] = f2bf(one(bf2f(pv[k]), x[k]));
-            __builtin_nontemporal_store(pv, (bf16x8*)p);
+            __builtin_nontemporal_store(pv, (bf16x8_any*)p);
         } else {
             f32x4 a = f.lo, b;
             if constexpr (WHOLE) b = f.hi[0];
-            else b = __builtin_nontemporal_load((const f32x4*)(p + 4));
+            else b = __builtin_nontemporal_load((const f32x4_any*)(p + 4));
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 a[k] = one(a[k], x[k]);
                 b[k] = one(b[k], x[4 + k]);
             }
-            __builtin_nontemporal_store(a, (f32x4*)p);
-            __builtin_nontemporal_store(b, (f32x4*)(p + 4));
+            __builtin_nontemporal_store(a, (f32x4_any*)p);
+            __builtin_nontemporal_store(b, (f32x4_any*)(p + 4));
         }
-    } else {  // ragged row end or unaligned parameter: element by element
+    } else {  // the ragged end of a row: element by element
         for (int k = 0; k < 8 && k < left; ++k) {
             if constexpr (PBF) p[k] = f2bf(one(bf2f(p[k]), x[k]));
             else p[k] = one(p[k], x[k]);
@@ -414,7 +419,6 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
     }
     // FOLD: the parameter, and this thread's piece u of the tile in it
     void* pbase = FOLD ? const_cast<void*>(g.upd_ptrs[tc.bidx]) : nullptr;
-    const bool pvec = (g.upd_cols % 8 == 0) && ((((uintptr_t)pbase) & 15) == 0);
     const bool pbf = g.upd_dtype == MUON_HIP_BF16;
     constexpr int NSTRIP = BM / 128, NWV = NT / 64;
     const int grp = lane >> 4, i16 = lane & 15;
@@ -438,8 +442,8 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
             long poff;
             int left;
             if (!piece(u, poff, left)) continue;
-            if (pbf) fold_load(pv[u], (const bf16_t*)pbase + poff, pvec, left);
-            else fold_load(pv[u], (const float*)pbase + poff, pvec, left);
+            if (pbf) fold_load(pv[u], (const bf16_t*)pbase + poff, left);
+            else fold_load(pv[u], (const float*)pbase + poff, left);
         }
     };
     if constexpr (FOLD && PRELOAD && (PART & EPI_LOADS)) load_param();
@@ -504,8 +508,8 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
             int left;
             if (piece(u, poff, left)) {
                 const bf16x8 o = *(const bf16x8*)&t8;
-                if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, pvec, left, g);
-                else fold_apply((float*)pbase + poff, pv[u], o, pvec, left, g);
+                if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, left, g);
+                else fold_apply((float*)pbase + poff, pv[u], o, left, g);
             }
         }
         return;
@@ -524,8 +528,8 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
 #pragma unroll
         for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[u][k])) + bf2f(t[k]));
         if (piece(u, poff, left)) {
-            if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, pvec, left, g);
-            else fold_apply((float*)pbase + poff, pv[u], o, pvec, left, g);
+            if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, left, g);
+            else fold_apply((float*)pbase + poff, pv[u], o, left, g);
         }
     }
 }
