@@ -58,7 +58,7 @@ extern "C" {
 #define MUON_HIP_K_GRAD_NORM 8
 #define MUON_HIP_K_CLIP_SCALE 9
 #define MUON_HIP_K_BX_UPDATE 10 /* the a.X + B.X launch that carries the parameter update in its epilogue */
-#define MUON_HIP_K_SMALL_CHAIN 11 /* normalisation, iterations and update of matrices with a short side of at most 64 */
+#define MUON_HIP_K_SMALL_CHAIN 11 /* normalisation, iterations and update of matrices that one workgroup each holds */
 #define MUON_HIP_K_FLOW_CHAIN 12  /* the iterations and the update of many small matrices in one launch */
 #define MUON_HIP_K_COUNT 13
 
@@ -90,8 +90,9 @@ int muon_hip_geometry(int rows, int cols, int* M, int* K, int* Mp, int* Kp, int*
 size_t muon_hip_workspace_bytes(int rows, int cols, int batch);
 
 /* Force one tile configuration for every later call (MUON_HIP_CFG_AUTO restores the default).
- * Affects geometry, workspace size and where the iterations leave their result (short sides of at most 64 run in one workgroup
- * each under MUON_HIP_CFG_AUTO only), so it stays as it is from muon_hip_workspace_bytes to the call that reads the result; meant
+ * Affects geometry, workspace size and where the iterations leave their result (short sides of at most 64, and of at
+ * most 128 with long ones of at most 512, run in one workgroup each under MUON_HIP_CFG_AUTO; the latter are tiled under
+ * MUON_HIP_CFG_STAGED), so it stays as it is from muon_hip_workspace_bytes to the call that reads the result; meant
  * for benchmarking sweeps. */
 int muon_hip_set_gemm_config(int cfg);
 
@@ -190,7 +191,8 @@ int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cu
  * group belong to one XCD) in the order in which the workgroups of an XCD take them; update: 0, or 1 for a call that updates
  * parameters, plus MUON_HIP_FLOW_RECORDED for one that is being recorded into a graph (over very little work only a call that is not
  * takes this way, for the sake of its launches).  Writes at most `capacity` of them; *count is how many there are, 0 for a call whose
- * products are launched one by one.  A tile starts when `before` tiles of its matrix are finished.  Touches no device; for tests and
+ * products are launched one by one.  (Matrices with a short side beyond 64 that a workgroup each holds are answered for as if they were
+ * tiled too, as they are beside a named configuration; here and in muon_hip_routes.)  A tile starts when `before` tiles of its matrix are finished.  Touches no device; for tests and
  * measurements. */
 #define MUON_HIP_FLOW_RECORDED 0x100
 typedef struct {

@@ -193,7 +193,8 @@ int make_plan(int rows, int cols, int batch, Plan& p) {
     p.M = rows < cols ? rows : cols;
     p.K = rows < cols ? cols : rows;
     const Cfg cfg = pick_cfg(p.M);
-    p.small = cfg.adapt && chain_fits(p.M, p.K);  // a configuration that the caller has named is one of the tiled kernels
+    // a configuration that the caller has named is one of the tiled kernels; without one launch for many matrices those take the larger ones
+    p.small = cfg.adapt && chain_fits(p.M, p.K) && (p.M <= 64 || g_forced_cfg.load(std::memory_order_relaxed) == MUON_HIP_CFG_AUTO);
     p.tile = gemm_cfg_tile(cfg.id);
     if (p.tile == 0) return fail(MUON_HIP_EINVAL, "unknown GEMM configuration");
     if (p.tile < 128) p.tile = 128;  // the elementwise kernels move whole 128-tiles
@@ -684,7 +685,7 @@ int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cu
         out[i] = muon_hip_route{MUON_HIP_CFG_AUTO, 0, -1};
         Bucket& k = w.b[w.n];
         if (int rc = k.init(buckets[i].rows, buckets[i].cols, buckets[i].batch, nowhere)) return rc;
-        if (!k.p.small) from[w.n++] = i;
+        if (!k.p.small || k.p.M > 64) from[w.n++] = i;
     }
     if (!w.n) return 0;
     GemmItem items[MUON_HIP_MAX_BUCKETS];
@@ -711,7 +712,7 @@ int muon_hip_flow_tiles(const muon_hip_bucket* buckets, int n, int steps, int up
         Bucket& k = w.b[w.n];
         if (int rc = k.init(buckets[i].rows, buckets[i].cols, buckets[i].batch, nowhere)) return rc;
         k.p_ptrs = (const void* const*)nowhere;
-        if (!k.p.small) from[w.n++] = i;
+        if (!k.p.small || k.p.M > 64) from[w.n++] = i;
     }
     FlowList l;
     const UpdateArgs u{};

@@ -1,6 +1,7 @@
 // Host-side description of one batched NT GEMM launch (see gemm_nt.hip).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <atomic>
 #include "common.h"
 
 // EPI_BX_UPD is EPI_BX with the parameter update folded into the epilogue (GemmArgs::upd_*) instead of writing X';
@@ -84,6 +85,10 @@ struct MachineShape {
     int cus, xcd_shift;
 };
 hipError_t machine_shape(MachineShape& ms);
+
+// Dynamic LDS beyond 64 KB has to be allowed per kernel, and the attribute belongs to the device that is current when
+// it is set: once per (kernel instantiation, device), remembered as one bit per device in the instantiation's mask.
+hipError_t allow_dynamic_lds(const void* kern, int bytes, std::atomic<unsigned long long>& done);
 
 int gemm_cfg_tile(int cfg);
 // The products args[0..n) of one kind, each with the configuration that its shape asks for, in as few launches as their

@@ -1865,8 +1865,7 @@ __global__ void __launch_bounds__(512, 4) gemm_nt_flow_kernel(const FlowList l) 
     }
 }
 
-// Dynamic LDS beyond 64 KB has to be allowed per kernel, and the attribute belongs to the device that is current when
-// it is set: once per (kernel instantiation, device), remembered as one bit per device in the instantiation's mask.
+}  // namespace
 hipError_t allow_dynamic_lds(const void* kern, int bytes, std::atomic<unsigned long long>& done) {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
@@ -1878,6 +1877,7 @@ hipError_t allow_dynamic_lds(const void* kern, int bytes, std::atomic<unsigned l
     done.fetch_or(bit, std::memory_order_release);
     return hipSuccess;
 }
+namespace {
 
 template <int EPI, int F0, int F1, bool LIST>
 hipError_t launch_ppx_as(const GemmList& l, int nblocks, int cus, hipStream_t stream) {

@@ -1,4 +1,4 @@
-// The whole Newton-Schulz chain of a matrix with a short side of at most 64 in one workgroup (see small_chain.hip).
+// The whole Newton-Schulz chain of a matrix with a short side of at most 64, or 128, in one workgroup (see small_chain.hip).
 #pragma once
 #include <hip/hip_runtime.h>
 #include "common.h"

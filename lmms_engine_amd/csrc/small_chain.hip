@@ -1,5 +1,5 @@
-// Newton-Schulz for matrices with a short side of at most 64 (low-rank adapters): normalisation, every iteration and the
-// parameter update in one kernel, a workgroup per matrix, X in registers from the first product to the last.
+// Newton-Schulz for matrices with a short side of at most 64 (low-rank adapters), or 128 where the long one is at most 512 (toy models, heads):
+// normalisation, every iteration and the parameter update in one kernel, a workgroup per matrix, X in registers from the first product to the last.
 //
 // The tiled products of gemm_nt.hip pad a short side to 128 rows and stream X from memory three times an iteration: for 16 rows
 // that is 64 times the multiplications, eight times the bytes and 17 launches.  Here the matrix is read once and the result (or
@@ -15,6 +15,10 @@
 // What a workgroup spends (cycles, one 16 x 5632 with an fp32 parameter, 175000 in all): an iteration 20000, of which the sums of X Xt 9500 (48
 // for each of 176 MFMAs, hand-over included) and X' 10000; blend and norm 22000; the parameter, 720 KB through one compute unit, 48000.
 // With the blend divided element by element and the parameter in pairs of chunks these were 24000, 32000 and 60000.
+// and with a short side beyond 64, one | 64 | 1024 matrices (there the tiles already run in one launch):
+//     128 x  128                           80 |   85 |  239    48 |  51 | 198
+//     128 x  512                           88 |  107 |  654    78 |  84 | 359
+//     512 x   67                           91 |  108 |  616    86 |  93 | 404
 // It wins wherever the registers hold the matrix, so that is the rule (chain_fits); larger ones take the tiled products.
 //
 // Eight waves share the columns of X in chunks of 32, a run of consecutive chunks each.  Lane (i = l%16, q = l/16) of a wave holds
@@ -33,7 +37,9 @@
 // time (16 x 5632: 57 | 95 | 415 when this took 82 | 118 | 511, 64 x 2048: 87 | 160 | 621 against 97 | 165 | 660): a bf16 value that rounds the other way moves through the remaining
 // iterations, up to 1e-3 of the result in norm.
 #include "small_chain.h"
+#include "gemm_nt.h"
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 namespace {
@@ -74,7 +80,7 @@ __device__ __forceinline__ FourOf<PT> update_four(const FourOf<PT>& p, uint32_t 
 __device__ __forceinline__ bool whole_rows(const void* p, int cols, bool turn) { return !turn && cols % 8 == 0 && (((uintptr_t)p) & 15) == 0; }
 __device__ __forceinline__ bool turned_pieces(const void* p, int M, bool turn, int elem) { return turn && M % 4 == 0 && ((uintptr_t)p & (4 * elem - 1)) == 0; }
 
-// Elsewhere element by element, eight columns of a row of X at a time.  In two halves, so that the loads of several pieces are in flight
+// Elsewhere in pieces from any address, or element by element, eight columns of a row of X at a time.  In two halves, so that the loads of several pieces are in flight
 // before the first store (the compiler cannot know that the pieces are apart: one after the other they cost a trip to memory each, eight for
 // a turned piece; see kBatch).
 struct Piece {
@@ -82,6 +88,16 @@ struct Piece {
 };
 template <typename PT>
 __device__ __forceinline__ void load_each(Piece& o, const PT* p, int row, int col, int cols, int M, int K, bool turn) {
+    typedef FourOf<PT> __attribute__((aligned(sizeof(PT)))) four_any;
+    if (!turn && col + 8 <= K) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const FourOf<PT> v = *(const four_any*)(p + (long)row * cols + col + 4 * h);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o.v[4 * h + e] = (float)v[e];
+        }
+        return;
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e)
         if (col + e < K) o.v[e] = (float)p[turn ? (long)(col + e) * M + row : (long)row * cols + col + e];
@@ -89,6 +105,17 @@ __device__ __forceinline__ void load_each(Piece& o, const PT* p, int row, int co
 template <typename PT>
 __device__ __forceinline__ void store_each(PT* p, const Piece& o, const bf16x8& x, int row, int col, int cols, int M, int K, bool turn, float scale, float decay,
                                            float alpha) {
+    typedef FourOf<PT> __attribute__((aligned(sizeof(PT)))) four_any;
+    if (!turn && col + 8 <= K) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            FourOf<PT> v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = (PT)update_one<PT>(o.v[4 * h + e], x[4 * h + e], scale, decay, alpha);
+            *(four_any*)(p + (long)row * cols + col + 4 * h) = v;
+        }
+        return;
+    }
 #pragma unroll
     for (int e = 0; e < 8; ++e)
         if (col + e < K) p[turn ? (long)(col + e) * M + row : (long)row * cols + col + e] = (PT)update_one<PT>(o.v[e], x[e], scale, decay, alpha);
@@ -166,7 +193,7 @@ struct ChainShared {
     int left[MT * (MT + 1) / 2];  // per leg: waves that have left it, of all iterations
 };
 
-// Matrix b of bucket k.  MT blocks of 16 rows (1, 2 or 4), up to NCH chunks of 32 columns per wave.
+// Matrix b of bucket k.  MT blocks of 16 rows (1, 2, 4 or 8), up to NCH chunks of 32 columns per wave.
 template <int MT, int NCH>
 __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const ChainMath& cm, ChainShared<MT>& sh) {
     constexpr int NP = (MT + 1) / 2;         // 32-deep reductions over the rows
@@ -177,10 +204,10 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
     // Chunks without a branch between them: 40 -> 30 ns for each MFMA of the chain through 176 chunks (16 x 5632).  Four blocks have
     // ten MFMAs between two branches anyway; and where a wave has four chunks at most, those that are not there cost as much as the
     // branches (111 of 20 x 56, one chunk: 17.5 with runs, 16.0 without).
-    constexpr int RUN = MT == 4 || NCH < 8 ? 1 : 4;
-    constexpr int GROUP = MT == 4 || RUN == 1 ? 1 : 4 / MT;  // chunks of X' that are computed together
+    constexpr int RUN = MT >= 4 || NCH < 8 ? 1 : 4;
+    constexpr int GROUP = MT >= 4 || RUN == 1 ? 1 : 4 / MT;  // chunks of X' that are computed together
     static_assert(NCH % RUN == 0 && RUN % GROUP == 0, "whole runs");
-    constexpr int LEG = MT == 4 ? 2 : 1, NLEG = NF / LEG;  // blocks that a wave adds its chunks to at a time
+    constexpr int LEG = MT == 8 ? 6 : MT == 4 ? 2 : 1, NLEG = NF / LEG;  // blocks that a wave adds its chunks to at a time
     auto& sum = sh.sum;
     auto& As = sh.A;
     auto& Bs = sh.B;
@@ -253,18 +280,34 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             }
     }
     if (!__all(exact)) {
-        // Element by element, or divided one by one: a fragment at a time through the work area, so that the loop need not be unrolled over
-        // the register array.
-#pragma unroll 4
-        for (int j = 0; j < per; ++j) {
+        // In pieces from any address or element by element, or divided: a few fragments at a time through the work area, so that the loop
+        // need not be unrolled over the register array (their loads before the first store, which the compiler cannot tell apart from them).
+        constexpr int AHEAD = MT < 4 ? 4 / MT : 1;
+        for (int j0 = 0; j0 < per; j0 += AHEAD) {
+            bf16x8 v[AHEAD][MT];
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                const int row = chain_row<MT>(t, i), col = col0 + j * 32;
-                bf16x8 v;
+            for (int jj = 0; jj < AHEAD; ++jj)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = (row < M && col + e < K) ? u[turn ? (long)(col + e) * M + row : (long)row * K + col + e] : (bf16_t)0.f;
-                mine[(j * MT + t) * 64] = div.slow(v);
-            }
+                for (int t = 0; t < MT; ++t) {
+                    const int row = chain_row<MT>(t, i), col = col0 + (j0 + jj) * 32;
+                    if (j0 + jj >= per) continue;
+                    if (!turn && row < M && col + 8 <= K) {
+                        v[jj][t] = *(const bf16x8_any*)(u + (long)row * K + col);
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            v[jj][t][e] = (row < M && col + e < K) ? u[turn ? (long)(col + e) * M + row : (long)row * K + col + e] : (bf16_t)0.f;
+                    }
+                }
+#pragma unroll
+            for (int jj = 0; jj < AHEAD; ++jj)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    if (j0 + jj >= per) continue;
+                    bf16x8 o;
+                    if (!div.quick(o, v[jj][t])) o = div.slow(v[jj][t]);
+                    mine[((j0 + jj) * MT + t) * 64] = o;
+                }
         }
 #pragma unroll
         for (int j = 0; j < NCH; ++j)
@@ -320,7 +363,8 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             if constexpr (NLEG > 2) add_leg(std::integral_constant<int, 2>{}, before);
             if constexpr (NLEG > 3) add_leg(std::integral_constant<int, 3>{}, before);
             if constexpr (NLEG > 4) add_leg(std::integral_constant<int, 4>{}, before);
-            static_assert(NLEG <= 5 && NLEG * LEG == NF, "every leg has its branch");
+            if constexpr (NLEG > 5) add_leg(std::integral_constant<int, 5>{}, before);
+            static_assert(NLEG <= 6 && NLEG * LEG == NF, "every leg has its branch");
         }
         __syncthreads();
         for (int t = tid; t < NF * 64; t += 64 * CHAIN_WAVES) {
@@ -339,8 +383,10 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             }
         }
         __syncthreads();
-        for (int f = wave; f < MT * MT; f += CHAIN_WAVES) {
-            const int ti = f / MT, tj = f % MT;
+        for (int f0 = wave; f0 < NF; f0 += CHAIN_WAVES) {  // on and above the diagonal, and the mirror image
+            int ti = 0, f = f0;
+            while (f >= MT - ti) f -= MT - ti++;
+            const int tj = ti + f;
             f32x4 aa = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int p = 0; p < NP; ++p)
@@ -350,13 +396,23 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = f2bf(rbf(cm.b * bf2f(av[e])) + rbf(cm.c * rbf(aa[e])));
             *(bf16x4*)&Bs[tj * 16 + i][ti * 16 + 4 * q] = o;
+            if (ti != tj) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) Bs[ti * 16 + 4 * q + e][tj * 16 + i] = o[e];
+            }
         }
         __syncthreads();
-        bf16x8 bfr[MT][NP];  // B's rows, in the order of X's
+        // B's rows, in the order of X's.  Those of eight blocks do not fit beside X: they are read as they are met.
+        constexpr bool KEPT = MT < 8;
+        bf16x8 bfr[KEPT ? MT : 1][NP];
+        auto read_b = [&](int t, bf16x8 (&w)[NP]) {
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
+            for (int p = 0; p < NP; ++p) w[p] = *(const bf16x8*)&Bs[chain_row<MT>(t, i)][p * 32 + 8 * q];
+        };
+        if constexpr (KEPT) {
 #pragma unroll
-            for (int p = 0; p < NP; ++p) bfr[t][p] = *(const bf16x8*)&Bs[chain_row<MT>(t, i)][p * 32 + 8 * q];
+            for (int t = 0; t < MT; ++t) read_b(t, bfr[t]);
+        }
         // GROUP chunks together, so that one's way through LDS and the products passes behind the others'
         auto next_chunks = [&](int j0, auto count_c) {
             constexpr int N = decltype(count_c)::value;
@@ -381,26 +437,35 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-            f32x4 v[N][MT][2];
+            constexpr int TB = KEPT ? MT : 2;  // blocks whose products come before their sums with X
 #pragma unroll
-            for (int p = 0; p < NP; ++p)
+            for (int t0 = 0; t0 < MT; t0 += TB) {
+                f32x4 v[N][TB][2];
+                bf16x8 bt[KEPT ? 1 : TB][NP];
+                if constexpr (!KEPT) {
+#pragma unroll
+                    for (int t = 0; t < TB; ++t) read_b(t0 + t, bt[t]);
+                }
+#pragma unroll
+                for (int p = 0; p < NP; ++p)
+#pragma unroll
+                    for (int n = 0; n < N; ++n)
+#pragma unroll
+                        for (int t = 0; t < TB; ++t)
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) v[n][t][h] = mfma(xt[n][h][p], KEPT ? bfr[KEPT ? t : 0][p] : bt[KEPT ? 0 : t][p], p ? v[n][t][h] : f32x4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
                 for (int n = 0; n < N; ++n)
 #pragma unroll
-                    for (int t = 0; t < MT; ++t)
+                    for (int t = 0; t < TB; ++t) {
+                        u32x4 xw = __builtin_bit_cast(u32x4, x[j0 + n][t0 + t]);
 #pragma unroll
-                        for (int h = 0; h < 2; ++h) v[n][t][h] = mfma(xt[n][h][p], bfr[t][p], p ? v[n][t][h] : f32x4{0.f, 0.f, 0.f, 0.f});
+                        for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int n = 0; n < N; ++n)
-#pragma unroll
-                for (int t = 0; t < MT; ++t) {
-                    u32x4 xw = __builtin_bit_cast(u32x4, x[j0 + n][t]);
-#pragma unroll
-                    for (int h = 0; h < 2; ++h)
-#pragma unroll
-                        for (int e = 0; e < 2; ++e) xw[2 * h + e] = axpy_bf16x2(cm.a, xw[2 * h + e], pack_bf16x2(v[n][t][h][2 * e], v[n][t][h][2 * e + 1]));
-                    x[j0 + n][t] = __builtin_bit_cast(bf16x8, xw);
-                }
+                            for (int e = 0; e < 2; ++e) xw[2 * h + e] = axpy_bf16x2(cm.a, xw[2 * h + e], pack_bf16x2(v[n][t][h][2 * e], v[n][t][h][2 * e + 1]));
+                        x[j0 + n][t0 + t] = __builtin_bit_cast(bf16x8, xw);
+                    }
+            }
         };
         // (waves w and w + 4 share a SIMD: the first four are done in half of the time, and the sums of the next iteration can start)
         if (wave < CHAIN_WAVES / 2) __builtin_amdgcn_s_setprio(1);
@@ -450,7 +515,7 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
         using PT = std::remove_pointer_t<decltype(pp)>;
         constexpr bool TURNED = decltype(turned_c)::value;
         // fragments whose pieces are asked for together: what the registers hold beside X
-        constexpr int G = sizeof(PT) == 4 || NCH * MT == 8 ? (NCH * MT == 8 ? 4 : 8) : 16;
+        constexpr int G = NCH * MT == 8 ? 4 : sizeof(PT) == 4 ? 8 : 16;
 #pragma unroll
         for (int f0 = 0; f0 < NCH * MT; f0 += G) {
             if (f0 / MT >= per) break;
@@ -494,6 +559,8 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             for (int t = 0; t < MT; ++t) {
                 const int row = chain_row<MT>(t, i), col = col0 + j * 32;
                 const bf16x8 v = mine[(j * MT + t) * 64];
+                if (!turn && row < M && col + 8 <= K) *(bf16x8_any*)(out + (long)row * K + col) = v;
+                else
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                     if (row < M && col + e < K) out[turn ? (long)(col + e) * M + row : (long)row * K + col + e] = v[e];
@@ -548,30 +615,46 @@ __device__ __forceinline__ int chain_bucket(const ChainList& l, int id, int& b) 
 
 // (with 8 fragments two workgroups share a compute unit)
 template <int MT, int NCH>
-__global__ void __launch_bounds__(64 * CHAIN_WAVES, MT * NCH == 8 ? 4 : 2) ns_chain_kernel(const ChainList l, const ChainMath cm) {
-    __shared__ __align__(16) unsigned char shared[sizeof(ChainShared<MT>)];
+__global__ void __launch_bounds__(64 * CHAIN_WAVES, MT * NCH == 8 && MT < 8 ? 4 : 2) ns_chain_kernel(const ChainList l, const ChainMath cm) {
     int b;
     const int i = chain_bucket(l, blockIdx.x, b);
-    chain_matrix<MT, NCH>(l.b[i], b, cm, *(ChainShared<MT>*)shared);
+    if constexpr (MT == 8) {
+        extern __shared__ __align__(16) unsigned char dynamic[];
+        chain_matrix<MT, NCH>(l.b[i], b, cm, *(ChainShared<MT>*)dynamic);
+    } else {
+        __shared__ __align__(16) unsigned char shared[sizeof(ChainShared<MT>)];
+        chain_matrix<MT, NCH>(l.b[i], b, cm, *(ChainShared<MT>*)shared);
+    }
 }
 
-__host__ __device__ constexpr int chain_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : 4; }
+__host__ __device__ constexpr int chain_blocks(int M) { return M <= 16 ? 1 : M <= 32 ? 2 : M <= 64 ? 4 : 8; }
 __host__ __device__ constexpr int chain_per_wave(int K) { return ((K + 31) / 32 + CHAIN_WAVES - 1) / CHAIN_WAVES; }
 
 // Fragments of X per lane that a kernel is built for.
 __host__ __device__ constexpr int chain_class(int need) { return need <= 8 ? 8 : need <= 16 ? 16 : 32; }
 
+template <int MT, int NCH>
+hipError_t launch_chain(const ChainList& l, const ChainMath& cm, hipStream_t stream) {
+    int lds = 0;
+    if constexpr (MT == 8) {  // past the 64 KB that a kernel has without asking
+        lds = sizeof(ChainShared<MT>);
+        static std::atomic<unsigned long long> configured{0};  // per instantiation
+        if (hipError_t e = allow_dynamic_lds((const void*)ns_chain_kernel<MT, NCH>, lds, configured); e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((ns_chain_kernel<MT, NCH>), dim3(l.start[l.n]), dim3(64 * CHAIN_WAVES), lds, stream, l, cm);
+    return hipGetLastError();
+}
 template <int MT>
-void launch_as(int nch, const ChainList& l, const ChainMath& cm, hipStream_t stream) {
-    const dim3 grid(l.start[l.n]), block(64 * CHAIN_WAVES);
-    if (nch * MT == 8) hipLaunchKernelGGL((ns_chain_kernel<MT, 8 / MT>), grid, block, 0, stream, l, cm);
-    else if (nch * MT == 16) hipLaunchKernelGGL((ns_chain_kernel<MT, 16 / MT>), grid, block, 0, stream, l, cm);
-    else hipLaunchKernelGGL((ns_chain_kernel<MT, 32 / MT>), grid, block, 0, stream, l, cm);
+hipError_t launch_as(int frags, const ChainList& l, const ChainMath& cm, hipStream_t stream) {
+    if constexpr (MT < 8)
+        if (frags == 32) return launch_chain<MT, 32 / MT>(l, cm, stream);
+    return frags == 8 ? launch_chain<MT, 8 / MT>(l, cm, stream) : launch_chain<MT, 16 / MT>(l, cm, stream);
 }
 
 }  // namespace
 
-bool chain_fits(int M, int K) { return M <= 64 && K <= 8192 && chain_per_wave(K) * chain_blocks(M) <= CHAIN_FRAGS; }
+// (128 rows and four chunks a wave, 32 fragments, would fit the registers but for 100 bytes a lane.)
+bool chain_fits(int M, int K) { return M <= 128 && K <= 8192 && chain_per_wave(K) * chain_blocks(M) <= (M <= 64 ? CHAIN_FRAGS : 16); }
 
 // Whole pieces, of rows or of a turned matrix's columns, cost the chain nothing.  Element by element a workgroup pays 0.6 us for a fragment,
 // which few matrices of many fragments feel more than the copy, while with many the copy, a pass over memory, costs more: the lines cross
@@ -585,40 +668,50 @@ bool chain_writes(int rows, int cols, int batch, const void* out, int cus) {
 
 // One launch per number of row blocks, on the kernel that holds the widest matrices, or one per kernel (8, 16 or 32 fragments of X per
 // lane: fewer registers, more workgroups in flight).
+//
+// The longest come first, the others on the compute units that they leave: a launch of its own per width waits for the one before.  The
+// narrow ones lose a place: two workgroups of 8 fragments share a compute unit on their own kernel, on a wider one each has its own.
+// Steps (us, apart | together): 308 narrow with 84 of 16 x 5632 and 5632 x 16 178 | 140, a quarter of them 134 | 100; 12 of 24 x
+// 1024 to 2624 in three widths 164 | 82; 504 narrow of 24 x 1024 with 168 of 24 x 2200 189 | 199; 616 with 168 of rank 16 272 | 262.
+//
+// Matrices of fewer row blocks go along, as if their rows were padded, while every workgroup of the launch has a compute unit of its own and
+// their waves have no more columns than those of the launch have: then they end before those do.
 hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, int cus, hipStream_t stream) {
     if (n < 1 || n > CHAIN_MAX_LIST || cm.steps < 1) return hipErrorInvalidValue;
-    int order[CHAIN_MAX_LIST], need[CHAIN_MAX_LIST], blocks[CHAIN_MAX_LIST];
+    int order[CHAIN_MAX_LIST], per[CHAIN_MAX_LIST], blocks[CHAIN_MAX_LIST];
+    bool done[CHAIN_MAX_LIST] = {};
     for (int i = 0; i < n; ++i) {
         const ChainBucket& k = buckets[i];
         const int M = std::min(k.rows, k.cols), K = std::max(k.rows, k.cols);
         if (!chain_fits(M, K)) return hipErrorInvalidValue;
         blocks[i] = chain_blocks(M);
-        need[i] = chain_per_wave(K) * blocks[i];
+        per[i] = chain_per_wave(K);
         order[i] = i;
     }
-    std::stable_sort(order, order + n, [&](int x, int y) { return blocks[x] != blocks[y] ? blocks[x] > blocks[y] : need[x] > need[y]; });
-    for (int at = 0; at < n;) {
-        const int mt = blocks[order[at]], frags = chain_class(need[order[at]]);
-        // The longest first, the others on the compute units that they leave: a launch of its own per width waits for the one before.  The
-        // narrow ones lose a place: two workgroups of 8 fragments share a compute unit on their own kernel, on a wider one each has its own.
-        // Steps (us, apart | together): 308 narrow with 84 of 16 x 5632 and 5632 x 16 178 | 140, a quarter of them 134 | 100; 12 of 24 x
-        // 1024 to 2624 in three widths 164 | 82; 504 narrow of 24 x 1024 with 168 of 24 x 2200 189 | 199; 616 with 168 of rank 16 272 | 262.
+    std::stable_sort(order, order + n, [&](int x, int y) { return blocks[x] != blocks[y] ? blocks[x] > blocks[y] : per[x] > per[y]; });
+    for (int at = 0; at < n; ++at) {
+        const int head = order[at], mt = blocks[head], frags = chain_class(per[head] * mt);
+        if (done[head]) continue;
         long narrow = 0;
         for (int i = 0; i < n; ++i)
-            if (blocks[i] == mt && chain_class(need[i]) == 8) narrow += buckets[i].batch;
+            if (!done[i] && blocks[i] == mt && chain_class(per[i] * mt) == 8) narrow += buckets[i].batch;
         const bool together = 2 * narrow <= 3L * cus;
         ChainList l;
         l.n = 0;
         l.start[0] = 0;
-        for (; at < n && blocks[order[at]] == mt && (together || chain_class(need[order[at]]) == frags); ++at) {
-            l.b[l.n] = buckets[order[at]];
-            l.start[l.n + 1] = l.start[l.n] + l.b[l.n].batch;
+        for (int k = at; k < n; ++k) {
+            const int i = order[k];
+            if (done[i]) continue;
+            const bool own = blocks[i] == mt ? together || chain_class(per[i] * mt) == frags : per[i] <= per[head] && (long)l.start[l.n] + buckets[i].batch <= cus;
+            if (!own) continue;
+            l.b[l.n] = buckets[i];
+            l.start[l.n + 1] = l.start[l.n] + buckets[i].batch;
             ++l.n;
+            done[i] = true;
         }
-        if (mt == 4) launch_as<4>(frags / 4, l, cm, stream);
-        else if (mt == 2) launch_as<2>(frags / 2, l, cm, stream);
-        else launch_as<1>(frags, l, cm, stream);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        if (hipError_t e = mt == 8 ? launch_as<8>(frags, l, cm, stream) : mt == 4 ? launch_as<4>(frags, l, cm, stream)
+                           : mt == 2 ? launch_as<2>(frags, l, cm, stream) : launch_as<1>(frags, l, cm, stream);
+            e != hipSuccess) return e;
     }
     return hipSuccess;
 }
