@@ -216,12 +216,15 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
     const bool turn = k.rows > k.cols;
     const int M = turn ? k.cols : k.rows, K = turn ? k.rows : k.cols;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15, q = lane >> 4;
-    const int per = ((K + 31) / 32 + CHAIN_WAVES - 1) / CHAIN_WAVES;  // chunks per wave
-    const int col0 = wave * per * 32 + 8 * q;                         // this lane's first column in the wave's chunk 0
+    // The wave's chunks: `per` of them from chunk `first` on.  What is left over goes to the first waves, one chunk each: with equal runs 12
+    // chunks would give six waves two, and a SIMD that has two of those four, where it has three like this.
+    const int chunks = (K + 31) / 32, spare = chunks % CHAIN_WAVES;
+    const int per = chunks / CHAIN_WAVES + (wave < spare ? 1 : 0), first = wave * (chunks / CHAIN_WAVES) + (wave < spare ? wave : spare);
+    const int col0 = first * 32 + 8 * q;  // this lane's first column in chunk 0
     const bf16_t* u = k.U + b * k.strideU;
     bf16_t* area = k.X + b * k.strideX;
     // this lane's fragments in the work area: read and written by this lane only
-    bf16x8* mine = (bf16x8*)area + (long)wave * per * MT * 64 + lane;
+    bf16x8* mine = (bf16x8*)area + (long)first * MT * 64 + lane;
 
     for (int t = tid; t < MT * 16 * PITCH; t += 64 * CHAIN_WAVES) {
         (&As[0][0])[t] = (bf16_t)0.f;
@@ -254,7 +257,7 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
         for (int j = 0; j < NCH; ++j)
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                const int row = chain_row<MT>(t, 4 * (lane & 3)), col = (wave * per + j) * 32 + (lane >> 2);
+                const int row = chain_row<MT>(t, 4 * (lane & 3)), col = (first + j) * 32 + (lane >> 2);
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
                     if (j < per && row < M && col + 16 * h < K) {
@@ -351,7 +354,7 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
         if (lane == 0) __hip_atomic_store(left, before + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     };
 
-    const int active = ((K + 31) / 32 + per - 1) / per;  // waves that have columns
+    const int active = chunks < CHAIN_WAVES ? chunks : CHAIN_WAVES;  // waves that have columns
     for (int it = 0; it < cm.steps; ++it) {
         // A wave starts a leg when the wave before it has left it, so the legs follow one another through the waves; the first ones go
         // ahead while the last are still at X' of the iteration before.  Every wave of the workgroup runs, and waits only for the one
@@ -383,6 +386,24 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             }
         }
         __syncthreads();
+        if constexpr (MT == 8) {  // a row of blocks for each wave, whole: its operand is read once
+            bf16x8 own[NP];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) own[p] = *(const bf16x8*)&As[wave * 16 + i][p * 32 + 8 * q];
+#pragma unroll 4
+            for (int tj = 0; tj < MT; ++tj) {
+                f32x4 aa = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int p = 0; p < NP; ++p) aa = mfma(own[p], *(const bf16x8*)&As[tj * 16 + i][p * 32 + 8 * q], aa);
+                u32x2 o = *(const u32x2*)&As[tj * 16 + i][wave * 16 + 4 * q];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t w = pack_bf16x2(aa[2 * e], aa[2 * e + 1]);
+                    o[e] = axpy_bf16x2(cm.b, o[e], pack_bf16x2(cm.c * low_bf16(w), cm.c * high_bf16(w)));
+                }
+                *(u32x2*)&Bs[tj * 16 + i][wave * 16 + 4 * q] = o;
+            }
+        } else
         for (int f0 = wave; f0 < NF; f0 += CHAIN_WAVES) {  // on and above the diagonal, and the mirror image
             int ti = 0, f = f0;
             while (f >= MT - ti) f -= MT - ti++;
@@ -502,7 +523,7 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             for (int t = 0; t < MT; ++t) {
                 if (j >= per) continue;
                 const bf16x8 v = turn_out(tl, x[j][t], lane);
-                const int row = chain_row<MT>(t, 4 * q), col = (wave * per + j) * 32 + i;
+                const int row = chain_row<MT>(t, 4 * q), col = (first + j) * 32 + i;
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
                     if (row < M && col + 16 * h < K)
@@ -522,7 +543,7 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             FourOf<PT> o[G][2];
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const int j = (f0 + g) / MT, t = (f0 + g) % MT, row = chain_row<MT>(t, TURNED ? 4 * q : i), col = TURNED ? (wave * per + j) * 32 + i : col0 + j * 32;
+                const int j = (f0 + g) / MT, t = (f0 + g) % MT, row = chain_row<MT>(t, TURNED ? 4 * q : i), col = TURNED ? (first + j) * 32 + i : col0 + j * 32;
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
                     if (j < per && row < M && col + (TURNED ? 16 * h : 0) < K)
@@ -530,7 +551,7 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             }
 #pragma unroll
             for (int g = 0; g < G; ++g) {
-                const int j = (f0 + g) / MT, t = (f0 + g) % MT, row = chain_row<MT>(t, TURNED ? 4 * q : i), col = TURNED ? (wave * per + j) * 32 + i : col0 + j * 32;
+                const int j = (f0 + g) / MT, t = (f0 + g) % MT, row = chain_row<MT>(t, TURNED ? 4 * q : i), col = TURNED ? (first + j) * 32 + i : col0 + j * 32;
                 if (j >= per) continue;
                 const bf16x8 v = TURNED ? turn_out(tl, x[j][t], lane) : x[j][t];
 #pragma unroll
