@@ -433,14 +433,14 @@ bool stage_items(const Work& w, int epi, int cur, double a, double b, double c, 
 }
 
 // The iterations as one launch (gemm_nt.h), where that is the faster way and nobody has named a configuration.
-bool flow_of(const Work& w, int steps, double a, double b, double c, const UpdateArgs* upd, int xcds, bool recorded, FlowList& l) {
+bool flow_of(const Work& w, int steps, double a, double b, double c, const UpdateArgs* upd, bf16_t* out, int xcds, bool recorded, FlowList& l) {
     if (g_forced_cfg.load(std::memory_order_relaxed) != MUON_HIP_CFG_AUTO) return false;
     l.n = w.n;
     l.steps = steps;
     l.a = (float)a;
     l.b = (float)b;
     l.c = (float)c;
-    l.p_dtype = upd ? upd->p_dtype : 0;
+    l.p_dtype = upd ? upd->p_dtype : out ? GEMM_UPD_RESULT : 0;
     l.decay = upd ? (float)(1.0 - upd->lr * upd->weight_decay) : 0.f;
     l.alpha = upd ? (float)(-upd->lr) : 0.f;
     l.control = w.b[0].counters(kCtrFlow);
@@ -458,7 +458,7 @@ bool flow_of(const Work& w, int steps, double a, double b, double c, const Updat
         e.Kp = p.Kp;
         e.batch = p.batch;
         e.done = k.counters(kCtrMatrix);
-        e.p_ptrs = upd ? k.p_ptrs : nullptr;
+        e.p_ptrs = upd ? k.p_ptrs : (const void* const*)out;
         e.rows = p.rows;
         e.cols = p.cols;
         e.scale = (float)k.scale;
@@ -467,8 +467,9 @@ bool flow_of(const Work& w, int steps, double a, double b, double c, const Updat
 }
 
 // Normalise, then `steps` iterations; with `upd` the last B.X applies the parameter update instead of writing X'.
-// `out`: where the result of small matrices goes, dense (one bucket; null: X).
-int ns_chain(const Work& all, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s, bf16_t* out = nullptr) {
+// `out`: where the result goes, dense (one bucket; null: X).  Where the last product does not write it there, *left_in_x is set.
+int ns_chain(const Work& all, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s, bf16_t* out = nullptr,
+             bool* left_in_x = nullptr) {
     if (steps < 0) return fail(MUON_HIP_EINVAL, "steps must be >= 0");
     MachineShape ms;
     if (hipError_t e = machine_shape(ms); e != hipSuccess) return hip_fail(e, "device shape");
@@ -500,7 +501,7 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
         w = all;
     }
     FlowList fl;
-    const bool flow = steps > 0 && flow_of(w, steps, a, b, c, upd, 1 << ms.xcd_shift, upd && is_recorded(s), fl);
+    const bool flow = steps > 0 && flow_of(w, steps, a, b, c, upd, out, 1 << ms.xcd_shift, upd && is_recorded(s), fl);
     if (flow)
         if (int rc = chain_alarm(&fl.alarm)) return rc;
     if (int rc = do_normalize(w, flow, s)) return rc;
@@ -520,6 +521,19 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
         if (int rc = launch_items(MUON_HIP_K_SYMPOLY, "sympoly launch", items, w.n, adapt, s)) return rc;
         adapt = stage_items(w, EPI_BX, cur, a, b, c, ppx, items);
         const bool last = upd && it == steps - 1;
+        if (out && it == steps - 1) {
+            // Tiles of 128 write the result themselves.  Those of 256 that carry an epilogue through LDS are slower than the persistent ones by
+            // more than the copy takes (8192 x 8192: 70 us for 53).
+            GemmItem direct = items[0];
+            GemmRoute route;
+            direct.epi = all.b[0].p.rows <= all.b[0].p.cols ? EPI_BX_UPD : EPI_BX_UPD_T;
+            direct.g.upd_ptrs = (const void* const*)out;
+            direct.g.upd_dtype = GEMM_UPD_RESULT;
+            direct.g.upd_rows = all.b[0].p.rows;
+            direct.g.upd_cols = all.b[0].p.cols;
+            if (adapt && plan_gemm_nt(&direct, 1, adapt, ms.cus, &route) == 1 && route.cfg == GEMM_CFG_128_PINGPONG) items[0] = direct;
+            else *left_in_x = true;
+        }
         if (last)
             for (int i = 0; i < w.n; ++i) fold_update(items[i], w.b[i].p_ptrs, w.b[i].p.rows, w.b[i].p.cols, w.b[i].scale, *upd);
         if (int rc = launch_items(last ? MUON_HIP_K_BX_UPDATE : MUON_HIP_K_BX, "bx launch", items, w.n, adapt, s)) return rc;
@@ -609,9 +623,10 @@ int muon_hip_ns_result(void* workspace, int rows, int cols, int batch, int steps
     if (int rc = chain_status()) return rc;
     MachineShape ms;
     if (hipError_t e = machine_shape(ms); e != hipSuccess) return hip_fail(e, "device shape");
-    const bool direct = w.b[0].p.small && steps > 0 && chain_writes(rows, cols, batch, out, ms.cus);
-    if (int rc = ns_chain(w, steps, a, b, c, nullptr, (hipStream_t)stream, direct ? (bf16_t*)out : nullptr)) return rc;
-    return direct ? 0 : muon_hip_ns_output(workspace, rows, cols, batch, steps, out, stream);
+    const bool direct = steps > 0 && (!w.b[0].p.small || chain_writes(rows, cols, batch, out, ms.cus));
+    bool left_in_x = !direct;
+    if (int rc = ns_chain(w, steps, a, b, c, nullptr, (hipStream_t)stream, direct ? (bf16_t*)out : nullptr, &left_in_x)) return rc;
+    return !left_in_x ? 0 : muon_hip_ns_output(workspace, rows, cols, batch, steps, out, stream);
 }
 
 int muon_hip_apply_update(const void* const* p_ptrs, int p_dtype, void* workspace, int rows, int cols, int batch,
@@ -716,7 +731,7 @@ int muon_hip_flow_tiles(const muon_hip_bucket* buckets, int n, int steps, int up
     }
     FlowList l;
     const UpdateArgs u{};
-    if (!w.n || steps == 0 || !flow_of(w, steps, 1.0, 1.0, 1.0, update ? &u : nullptr, xcds, recorded, l)) return 0;
+    if (!w.n || steps == 0 || !flow_of(w, steps, 1.0, 1.0, 1.0, update ? &u : nullptr, nullptr, xcds, recorded, l)) return 0;
     for (int g = 0; g < l.groups; ++g)
         for (int t = 0; t < flow_tiles(l, g); ++t, ++*count) {
             if (*count >= capacity) continue;

@@ -25,6 +25,7 @@ enum {
     GEMM_CFG_COUNT = 6
 };
 
+constexpr int GEMM_UPD_RESULT = 2;
 struct GemmArgs {
     const bf16_t* P;        // left operand: rows x kdim, blocked
     const bf16_t* Q;        // right operand, blocked: rows x kdim (SYRK, SYMPOLY) or kdim x columns (BX)
@@ -49,7 +50,8 @@ struct GemmArgs {
     // BX, optional: fold apply_scaling and the parameter update into the epilogue instead of writing X'
     // (EPI_BX_UPD: the parameter is X's image, rows <= cols; EPI_BX_UPD_T: its transpose, rows > cols)
     const void* const* upd_ptrs;  // device table of parameter base pointers, one per matrix; null = write X'
-    int upd_dtype;                // MUON_HIP_F32 or MUON_HIP_BF16
+    int upd_dtype;                // MUON_HIP_F32 or MUON_HIP_BF16; GEMM_UPD_RESULT: no parameters, X' itself goes to the dense matrices at
+                                  // upd_ptrs (bf16, upd_rows x upd_cols each, one after the other)
     int upd_rows, upd_cols;       // the parameter's own (unpadded) shape
     float upd_scale, upd_decay, upd_alpha;  // python-double scale, 1 - lr*wd and -lr, as fp32
     // EPI_MMT: C is row-major, dense_rows x dense_rows (rows, cols: in whole 128-tiles as ever).  dense_pitch: P and Q are too, with
@@ -118,7 +120,8 @@ struct FlowEntry {
     long strideX, strideA;
     int Mp, Kr, Kp, batch;     // as GemmArgs: Kr columns in whole 128-tiles of storage for Kp
     unsigned* done;            // a counter per matrix, GEMM_FLOW_LINE words apart, zero before the launch
-    const void* const* p_ptrs; // device table of the parameters to update; null: the last iteration writes X'
+    const void* const* p_ptrs; // device table of the parameters to update (FlowList::p_dtype GEMM_UPD_RESULT: where X' goes, GemmArgs::upd_ptrs);
+                               // null: the last iteration writes X'
     int rows, cols;            // of the parameter
     float scale;
     int sym, rect;             // 128-tiles of a matrix: of a symmetric product, of a.X + B.X

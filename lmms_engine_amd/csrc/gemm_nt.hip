@@ -367,6 +367,14 @@ __device__ __forceinline__ void fold_apply(PT* p, const FoldPiece<WHOLE>& f, con
     }
 }
 
+__device__ __forceinline__ void result_store(bf16_t* p, const bf16x8& x, int left) {
+    if (left >= 8) {
+        *(bf16x8_any*)p = x;
+    } else {
+        for (int k = 0; k < 8 && k < left; ++k) p[k] = x[k];
+    }
+}
+
 // pv: the parameter's pieces, fetched with the a.X term.  PRELOAD: they are, with EPI_LOADS; otherwise this part comes later, with
 // the accumulators in LDS.
 template <int BM, int BN, int WGM, int WGN, int FOLD, bool COH, int PART, int NEV, bool PRELOAD, int NPV>
@@ -418,7 +426,8 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
         }
     }
     // FOLD: the parameter, and this thread's piece u of the tile in it
-    void* pbase = FOLD ? const_cast<void*>(g.upd_ptrs[tc.bidx]) : nullptr;
+    const bool result = FOLD && g.upd_dtype == GEMM_UPD_RESULT;
+    void* pbase = !FOLD ? nullptr : result ? (bf16_t*)g.upd_ptrs + (long)tc.bidx * g.upd_rows * g.upd_cols : const_cast<void*>(g.upd_ptrs[tc.bidx]);
     const bool pbf = g.upd_dtype == MUON_HIP_BF16;
     constexpr int NSTRIP = BM / 128, NWV = NT / 64;
     const int grp = lane >> 4, i16 = lane & 15;
@@ -437,6 +446,7 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
         return row < g.upd_rows && left > 0;
     };
     auto load_param = [&]() {
+        if (result) return;
 #pragma unroll
         for (int u = 0; u < NLE; ++u) {
             long poff;
@@ -508,7 +518,8 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
             int left;
             if (piece(u, poff, left)) {
                 const bf16x8 o = *(const bf16x8*)&t8;
-                if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, left, g);
+                if (result) result_store((bf16_t*)pbase + poff, o, left);
+                else if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, left, g);
                 else fold_apply((float*)pbase + poff, pv[u], o, left, g);
             }
         }
@@ -528,7 +539,8 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
 #pragma unroll
         for (int k = 0; k < 8; ++k) o[k] = f2bf(rbf(g.s0 * bf2f(ev[u][k])) + bf2f(t[k]));
         if (piece(u, poff, left)) {
-            if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, left, g);
+            if (result) result_store((bf16_t*)pbase + poff, o, left);
+            else if (pbf) fold_apply((bf16_t*)pbase + poff, pv[u], o, left, g);
             else fold_apply((float*)pbase + poff, pv[u], o, left, g);
         }
     }
@@ -2185,7 +2197,7 @@ bool plan_flow(FlowList& l, int xcds, bool recorded) {
     // A step over very little takes longer on the device (replays: 6 of 128 x 384 with 8 of 128 x 128 94.5 us in one launch, 74.0 without),
     // but the caller waits for his own 14 launches less: steps of a model of 14 such matrices, one behind the other, 149 us and 199.  A
     // step that is being recorded has no such launches when it is replayed.
-    return !recorded && l.e[0].p_ptrs && 0.032 * most + 0.64 * chain + 55 < 120;
+    return !recorded && l.e[0].p_ptrs && l.p_dtype != GEMM_UPD_RESULT && 0.032 * most + 0.64 * chain + 55 < 120;
 }
 
 hipError_t launch_flow(const FlowList& l, hipStream_t stream) {

@@ -60,3 +60,27 @@ def test_results_at_any_address_and_their_values(env, rows, cols, batch):
         torch.cuda.synchronize()
         assert torch.equal(buf[by:by + G.numel()].view(G.shape), want)
         assert bool((buf[:by] == 7).all()) and bool((buf[by + G.numel():] == 7).all())
+
+
+# one launch for all products, 64-tiles and 128-tiles in launches of their own, 256-tiles (where the result is copied), both orientations
+@pytest.mark.parametrize("rows,cols,batch,steps", [(1024, 256, 48, 5), (256, 1024, 48, 2), (130, 701, 64, 1), (701, 130, 33, 2), (896, 4864, 1, 5), (4864, 896, 1, 1),
+                                                   (300, 1001, 3, 2), (1001, 299, 3, 2), (640, 2560, 60, 1), (1408, 1408, 16, 1), (1024, 1024, 40, 2), (520, 512, 2, 0)])
+def test_results_written_by_the_last_product_equal_the_copy_bitwise(env, rows, cols, batch, steps):
+    print(f"result of {batch} x {rows}x{cols}, {steps} steps", flush=True)
+    lib, dev = env["lib"], env["dev"]
+    G = torch.randn(batch, rows, cols, generator=torch.Generator().manual_seed(rows + cols)).bfloat16().to(dev)
+    ws = torch.empty(lib.muon_hip_workspace_bytes(rows, cols, batch), dtype=torch.uint8, device=dev)
+    n, ref = G.numel(), torch.empty_like(G)
+    for by in (0, 1):
+        buf = torch.full((n + 16,), 7.0, dtype=torch.bfloat16, device=dev)
+        for direct in (True, False):
+            _abi.check(lib.muon_hip_cast_norm(G.data_ptr(), _abi.dtype_code(G.dtype), ws.data_ptr(), rows, cols, batch, 0))
+            if direct:
+                _abi.check(lib.muon_hip_ns_result(ws.data_ptr(), rows, cols, batch, steps, *NS, buf.data_ptr() + 16 + 2 * by, 0))
+            else:
+                _abi.check(lib.muon_hip_ns_grouped(ws.data_ptr(), rows, cols, batch, steps, *NS, 0))
+                _abi.check(lib.muon_hip_ns_output(ws.data_ptr(), rows, cols, batch, steps, ref.data_ptr(), 0))
+        torch.cuda.synchronize()
+        at = 8 + by
+        assert bool(torch.isfinite(ref.float()).all()) and torch.equal(buf[at:at + n].view(G.shape), ref), by
+        assert bool((buf[:at] == 7).all()) and bool((buf[at + n:] == 7).all())
