@@ -2073,6 +2073,22 @@ int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* r
             if (all128 <= 2 * cus && all64 <= cus && !fold) cfg[i] = GEMM_CFG_64_DEEP;
         }
     }
+    // Matrices of 129 to 256 rows (keys and values beside large weights) run on 128-tiles by themselves, after the launch of the large ones and
+    // on a few compute units.  Beside 256-tiles they go along, one tile a row of blocks, while that launch has eight times as many.  Steps, us,
+    // apart | along: 6 layers of 1000 x 1000, 200 x 1000 and 2731 x 1000 1638 | 1511, 12 of 768, 192 and 2048 1657 | 1520, 2 of 2048, 256 and
+    // 5632 3182 | 3018, 12 of 1024, 256 and 2816 3015 | 2901, 8 of 2048, 256 and 5632 (32 such matrices in 72 rounds) 10899 | 10895.
+    for (int epi : {EPI_SYRK, EPI_SYMPOLY, EPI_BX, EPI_BX_UPD, EPI_BX_UPD_T}) {
+        long large = 0, more = 0;
+        bool along[GEMM_MAX_LIST] = {};
+        for (int i = 0; i < n; ++i) {
+            if (!adapt || items[i].epi != epi) continue;
+            if (gemm_cfg_tile(cfg[i]) == 256) large += count_tiles(items[i], 256);
+            else if (cfg[i] == GEMM_CFG_128_PINGPONG && items[i].g.rows == 256 && items[i].g.kdim >= 256 && tiles_fit(items[i], 256, 256))
+                along[i] = true, more += count_tiles(items[i], 256);
+        }
+        for (int i = 0; i < n && 8 * more <= large; ++i)
+            if (along[i]) cfg[i] = GEMM_CFG_256_PERSIST;
+    }
     for (int i = 0; i < n; ++i)
         if (cfg[i] == GEMM_CFG_64_DEEP && epi_fold_mode(items[i].epi)) cfg[i] = GEMM_CFG_128_PINGPONG;
     // The persistent kernel: more tiles than compute units, and products with at least 8 k-tiles and a counter buffer; one launch
