@@ -146,8 +146,8 @@ int muon_hip_apply_update(const void* const* p_ptrs, int p_dtype, void* workspac
  * the return value of fast_newtonschulz (muon_utils.py:154-156). */
 int muon_hip_ns_output(void* workspace, int rows, int cols, int batch, int steps, void* out, void* stream);
 
-/* muon_hip_ns_grouped and muon_hip_ns_output in one call, the same bits.  Matrices with a short side of at most 64 whose chain
- * runs in one workgroup write `out` from there where that is faster; the workspace then does not hold the result. */
+/* muon_hip_ns_grouped and muon_hip_ns_output in one call, the same bits.  Matrices whose chain runs in one workgroup, and products on
+ * 128-tiles, write `out` from there where that is faster; the workspace then does not hold the result. */
 int muon_hip_ns_result(void* workspace, int rows, int cols, int batch, int steps, double a, double b, double c, void* out,
                        void* stream);
 

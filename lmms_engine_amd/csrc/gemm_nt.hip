@@ -2211,7 +2211,8 @@ bool plan_flow(FlowList& l, int xcds, bool recorded) {
     // (The figures are of XCDs of 32 compute units, which gfx950 has however it is partitioned.)
     if (mean < 30000 && most < 1.35 * mean - 15 * chain + 600) return true;
     // A step over very little takes longer on the device (replays: 6 of 128 x 384 with 8 of 128 x 128 94.5 us in one launch, 74.0 without),
-    // but the caller waits for his own 14 launches less: steps of a model of 14 such matrices, one behind the other, 149 us and 199.  A
+    // but the caller waits for his own 14 launches less: steps of a model of 14 such matrices, one behind the other, 149 us and 199 (matrices
+    // of those sizes run in a workgroup each since; the rule is for sets of slightly larger ones).  A
     // step that is being recorded has no such launches when it is replayed.
     return !recorded && l.e[0].p_ptrs && l.p_dtype != GEMM_UPD_RESULT && 0.032 * most + 0.64 * chain + 55 < 120;
 }

@@ -193,6 +193,22 @@ struct ChainShared {
     int left[MT * (MT + 1) / 2];  // per leg: waves that have left it, of all iterations
 };
 
+// Eight row blocks: the fragments of X of all waves (STAGE, 16 chunks) while A is summed, A and B in their place afterwards.
+template <>
+struct ChainShared<8> {
+    static constexpr int PITCH = 32 * 4 + 8, CHUNKS = 2 * CHAIN_WAVES;
+    union {
+        bf16x8 stage[CHUNKS * 8][64];
+        struct {
+            bf16_t A[128][PITCH], B[128][PITCH];
+        };
+        f32x4 sum[1][64];  // (the sums stay in registers)
+    };
+    unsigned char turned[CHAIN_WAVES][TURN_BYTES];
+    float red[4];
+    int left[1];
+};
+
 // Matrix b of bucket k.  MT blocks of 16 rows (1, 2, 4 or 8), up to NCH chunks of 32 columns per wave.
 template <int MT, int NCH>
 __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const ChainMath& cm, ChainShared<MT>& sh) {
@@ -207,7 +223,7 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
     constexpr int RUN = MT >= 4 || NCH < 8 ? 1 : 4;
     constexpr int GROUP = MT >= 4 || RUN == 1 ? 1 : 4 / MT;  // chunks of X' that are computed together
     static_assert(NCH % RUN == 0 && RUN % GROUP == 0, "whole runs");
-    constexpr int LEG = MT == 8 ? 6 : MT == 4 ? 2 : 1, NLEG = NF / LEG;  // blocks that a wave adds its chunks to at a time
+    constexpr int LEG = MT == 4 ? 2 : 1, NLEG = NF / LEG;  // blocks that a wave adds its chunks to at a time
     auto& sum = sh.sum;
     auto& As = sh.A;
     auto& Bs = sh.B;
@@ -226,12 +242,13 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
     // this lane's fragments in the work area: read and written by this lane only
     bf16x8* mine = (bf16x8*)area + (long)first * MT * 64 + lane;
 
+    if constexpr (MT < 8)
     for (int t = tid; t < MT * 16 * PITCH; t += 64 * CHAIN_WAVES) {
         (&As[0][0])[t] = (bf16_t)0.f;
         (&Bs[0][0])[t] = (bf16_t)0.f;
     }
     *(unsigned*)&turned[wave][TURN_ZEROS * 64 + lane * 4] = 0u;
-    if (tid < NLEG) sh.left[tid] = 0;
+    if (MT < 8 && tid < NLEG) sh.left[tid] = 0;
     // The matrix in whole pieces (turned: four rows of two columns, turned below), every load in flight together; zero past its edges.
     const bool vec = !turn && K % 8 == 0, tvec = turned_pieces(u, M, turn, 2);
     unsigned char* const tl = turned[wave];
@@ -359,6 +376,49 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
         // A wave starts a leg when the wave before it has left it, so the legs follow one another through the waves; the first ones go
         // ahead while the last are still at X' of the iteration before.  Every wave of the workgroup runs, and waits only for the one
         // before it.
+        if constexpr (MT == 8) {
+            // With at most two chunks a wave there is little to add between two hand-overs.  Here all of X goes through LDS, and a wave sums its
+            // own blocks of A over all chunks, the same sums: rows p and 7 - p have nine, five of row p for one wave and the others for the next.
+            const int p = wave >> 1, odd = wave & 1;
+            f32x4 acc[5];
+#pragma unroll
+            for (int f = 0; f < 5; ++f) acc[f] = f32x4{0.f, 0.f, 0.f, 0.f};
+            auto row_of = [&](int f) { return odd && 5 + f >= 8 - p ? 7 - p : p; };                     // block f of this wave
+            auto col_of = [&](int f) { return !odd ? p + f : 5 + f >= 8 - p ? 7 - p + (5 + f - (8 - p)) : p + 5 + f; };
+            __syncthreads();  // B is no longer read
+#pragma unroll
+            for (int j = 0; j < NCH; ++j)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+                    if (j < per) sh.stage[(first + j) * MT + t][lane] = x[j][t];
+            __syncthreads();
+            if (!odd) {
+#pragma unroll 2
+                for (int c = 0; c < chunks; ++c) {
+                    const bf16x8 own = sh.stage[c * MT + p][lane];
+#pragma unroll
+                    for (int f = 0; f < 5; ++f) acc[f] = mfma(own, sh.stage[c * MT + p + f][lane], acc[f]);
+                }
+            } else {
+#pragma unroll 2
+                for (int c = 0; c < chunks; ++c)
+#pragma unroll
+                    for (int f = 0; f < 4; ++f) acc[f] = mfma(sh.stage[c * MT + row_of(f)][lane], sh.stage[c * MT + col_of(f)][lane], acc[f]);
+            }
+            __syncthreads();  // X is no longer read
+#pragma unroll
+            for (int f = 0; f < 5; ++f) {
+                if (f == 4 && odd) break;
+                const int ti = row_of(f), tj = col_of(f), r = chain_row<MT>(ti, q * 4), c = chain_row<MT>(tj, i);
+                const u32x2 o = {pack_bf16x2(acc[f][0], acc[f][1]), pack_bf16x2(acc[f][2], acc[f][3])};
+                *(u32x2*)&As[c][r] = o;
+                if (ti != tj) {
+                    const bf16x4 v = __builtin_bit_cast(bf16x4, o);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) As[r + e][c] = v[e];
+                }
+            }
+        } else
         if (wave < active) {
             const int before = it * active + wave;
             add_leg(std::integral_constant<int, 0>{}, before);
@@ -366,10 +426,10 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             if constexpr (NLEG > 2) add_leg(std::integral_constant<int, 2>{}, before);
             if constexpr (NLEG > 3) add_leg(std::integral_constant<int, 3>{}, before);
             if constexpr (NLEG > 4) add_leg(std::integral_constant<int, 4>{}, before);
-            if constexpr (NLEG > 5) add_leg(std::integral_constant<int, 5>{}, before);
-            static_assert(NLEG <= 6 && NLEG * LEG == NF, "every leg has its branch");
+            static_assert(NLEG <= 5 && NLEG * LEG == NF, "every leg has its branch");
         }
         __syncthreads();
+        if constexpr (MT < 8) {
         for (int t = tid; t < NF * 64; t += 64 * CHAIN_WAVES) {
             const int ln = t & 63;
             int f = t >> 6, ti = 0;
@@ -386,6 +446,7 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             }
         }
         __syncthreads();
+        }
         if constexpr (MT == 8) {  // a row of blocks for each wave, whole: its operand is read once
             bf16x8 own[NP];
 #pragma unroll

@@ -166,7 +166,7 @@ def matmul_transpose_assign(d_in: Tensor, d_out: Tensor) -> None:
 def get_autotune_config():
     """muon_utils.py:13-25 lists the Triton tile shapes the autotuner tries.  The HIP kernels are not autotuned:
     this returns the fixed tile configurations of its large launches.  Launches that would leave compute units idle also take
-    64 x 64 tiles (CFG_64_DEEP), a.X + B.X tiles of 224 or 192 rows, and short sides of at most 64 one workgroup per matrix."""
+    64 x 64 tiles (CFG_64_DEEP), a.X + B.X tiles of 224 or 192 rows, and short sides of at most 64 (128 with long ones of at most 512) one workgroup per matrix."""
     return [
         dict(BLOCK_SIZE_M=128, BLOCK_SIZE_N=128, BLOCK_SIZE_K=64, num_stages=2, num_warps=4, config=_abi.CFG_128_PIPE),
         dict(BLOCK_SIZE_M=256, BLOCK_SIZE_N=256, BLOCK_SIZE_K=64, num_stages=2, num_warps=8, config=_abi.CFG_256_PIPE),
