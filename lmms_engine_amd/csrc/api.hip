@@ -477,9 +477,13 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
     if (steps > 0) {
         ChainBucket small[MUON_HIP_MAX_BUCKETS];
         int n = 0;
+        // Short sides beyond 64 cost little among the tiles of larger matrices, in one launch or one per product; a launch of their own in front
+        // of those would come on top (a step over such a mixture: 161 us among the tiles, 231 with a launch of their own).
+        bool tiles = false;
+        for (int i = 0; i < all.n; ++i) tiles |= upd && !all.b[i].p.small;
         for (int i = 0; i < all.n; ++i) {
             const Bucket& k = all.b[i];
-            if (!k.p.small) {
+            if (!k.p.small || (tiles && k.p.M > 64)) {
                 w.b[w.n++] = k;
                 continue;
             }
