@@ -16,9 +16,9 @@
 // for each of 176 MFMAs, hand-over included) and X' 10000; blend and norm 22000; the parameter, 720 KB through one compute unit, 48000.
 // With the blend divided element by element and the parameter in pairs of chunks these were 24000, 32000 and 60000.
 // and with a short side beyond 64, one | 64 | 1024 matrices (there the tiles already run in one launch):
-//     128 x  128                           80 |   85 |  239    48 |  51 | 198
-//     128 x  512                           88 |  107 |  654    78 |  84 | 359
-//     512 x   67                           91 |  108 |  616    86 |  93 | 404
+//     128 x  128                           80 |   85 |  239    35 |  36 | 147
+//     128 x  512                           88 |  107 |  654    73 |  78 | 359
+//     512 x   67                           91 |  108 |  616    79 |  86 | 388
 // It wins wherever the registers hold the matrix, so that is the rule (chain_fits); larger ones take the tiled products.
 //
 // Eight waves share the columns of X in chunks of 32, a run of consecutive chunks each.  Lane (i = l%16, q = l/16) of a wave holds
