@@ -2046,49 +2046,14 @@ hipError_t machine_shape(MachineShape& ms) {
     return hipSuccess;
 }
 
-int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* route) {
-    if (n < 1 || n > GEMM_MAX_LIST) return -1;
+namespace {
+
+// The launches of products with the configurations chosen[0..n).
+int place_launches(const GemmItem* items, int n, bool adapt, int cus, const int* chosen, GemmRoute* route) {
     int cfg[GEMM_MAX_LIST];
     bool done[GEMM_MAX_LIST] = {};
     int launches = 0;
-    long all128 = 0, own128 = 0, all64 = 0;
-    bool fold = false;
-    for (int i = 0; i < n; ++i) {
-        cfg[i] = items[i].cfg;
-        if (gemm_cfg_tile(cfg[i]) == 0) return -1;
-        all128 += count_tiles(items[i], 128);
-        if (gemm_cfg_tile(cfg[i]) == 256) own128 += count_tiles(items[i], 128);
-        all64 += count_tiles(items[i], 64);
-        fold |= epi_fold_mode(items[i].epi) != 0;
-    }
-    // Smaller tiles for launches that would not fill the machine (every configuration sums in the same order, so the result
-    // does not depend on the choice).  Measured on one to 48 matrices of 128 to 5120 rows, times per k-tile of 32 columns: a
-    // round of 256-tiles (one workgroup per compute unit) 460 ns, of 128-tiles 157 ns alone on a compute unit and 336 ns for
-    // two.  So 128-tiles win while they need no more than the two places per compute unit (X.Xt of 2048 x 5632: 84 -> 36 us,
-    // of 3072 x 8192 with 300 tiles 119 -> 91) and lose beyond (4096 x 4096 with 528: 68 -> 76); 64-tiles win while each has
-    // a compute unit of its own (896 x 4864: 30 -> 18) and lose with two (512 x 1408 x 8, 288 tiles: 11.7 -> 14.0).
-    if (adapt) {
-        for (int i = 0; i < n; ++i) {
-            if (gemm_cfg_tile(cfg[i]) == 256 && own128 <= 2 * cus) cfg[i] = GEMM_CFG_128_PINGPONG;
-            if (all128 <= 2 * cus && all64 <= cus && !fold) cfg[i] = GEMM_CFG_64_DEEP;
-        }
-    }
-    // Matrices of 129 to 256 rows (keys and values beside large weights) run on 128-tiles by themselves, after the launch of the large ones and
-    // on a few compute units.  Beside 256-tiles they go along, one tile a row of blocks, while that launch has eight times as many.  Steps, us,
-    // apart | along: 6 layers of 1000 x 1000, 200 x 1000 and 2731 x 1000 1638 | 1511, 12 of 768, 192 and 2048 1657 | 1520, 2 of 2048, 256 and
-    // 5632 3182 | 3018, 12 of 1024, 256 and 2816 3015 | 2901, 8 of 2048, 256 and 5632 (32 such matrices in 72 rounds) 10899 | 10895.
-    for (int epi : {EPI_SYRK, EPI_SYMPOLY, EPI_BX, EPI_BX_UPD, EPI_BX_UPD_T}) {
-        long large = 0, more = 0;
-        bool along[GEMM_MAX_LIST] = {};
-        for (int i = 0; i < n; ++i) {
-            if (!adapt || items[i].epi != epi) continue;
-            if (gemm_cfg_tile(cfg[i]) == 256) large += count_tiles(items[i], 256);
-            else if (cfg[i] == GEMM_CFG_128_PINGPONG && items[i].g.rows == 256 && items[i].g.kdim >= 256 && tiles_fit(items[i], 256, 256))
-                along[i] = true, more += count_tiles(items[i], 256);
-        }
-        for (int i = 0; i < n && 8 * more <= large; ++i)
-            if (along[i]) cfg[i] = GEMM_CFG_256_PERSIST;
-    }
+    std::copy(chosen, chosen + n, cfg);
     for (int i = 0; i < n; ++i)
         if (cfg[i] == GEMM_CFG_64_DEEP && epi_fold_mode(items[i].epi)) cfg[i] = GEMM_CFG_128_PINGPONG;
     // The persistent kernel: more tiles than compute units, and products with at least 8 k-tiles and a counter buffer; one launch
@@ -2155,6 +2120,67 @@ int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* r
         ++launches;
     }
     return launches;
+}
+
+}  // namespace
+
+int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* route) {
+    if (n < 1 || n > GEMM_MAX_LIST) return -1;
+    int cfg[GEMM_MAX_LIST];
+    long all128 = 0, own128 = 0, all64 = 0;
+    bool fold = false;
+    for (int i = 0; i < n; ++i) {
+        cfg[i] = items[i].cfg;
+        if (gemm_cfg_tile(cfg[i]) == 0) return -1;
+        all128 += count_tiles(items[i], 128);
+        if (gemm_cfg_tile(cfg[i]) == 256) own128 += count_tiles(items[i], 128);
+        all64 += count_tiles(items[i], 64);
+        fold |= epi_fold_mode(items[i].epi) != 0;
+    }
+    // Smaller tiles for launches that would not fill the machine (every configuration sums in the same order, so the result
+    // does not depend on the choice).  Measured on one to 48 matrices of 128 to 5120 rows, times per k-tile of 32 columns: a
+    // round of 256-tiles (one workgroup per compute unit) 460 ns, of 128-tiles 157 ns alone on a compute unit and 336 ns for
+    // two.  So 128-tiles win while they need no more than the two places per compute unit (X.Xt of 2048 x 5632: 84 -> 36 us,
+    // of 3072 x 8192 with 300 tiles 119 -> 91) and lose beyond (4096 x 4096 with 528: 68 -> 76); 64-tiles win while each has
+    // a compute unit of its own (896 x 4864: 30 -> 18) and lose with two (512 x 1408 x 8, 288 tiles: 11.7 -> 14.0).
+    if (adapt) {
+        for (int i = 0; i < n; ++i) {
+            if (gemm_cfg_tile(cfg[i]) == 256 && own128 <= 2 * cus) cfg[i] = GEMM_CFG_128_PINGPONG;
+            if (all128 <= 2 * cus && all64 <= cus && !fold) cfg[i] = GEMM_CFG_64_DEEP;
+        }
+    }
+    // Matrices of 129 to 256 rows (keys and values beside large weights) run on 128-tiles by themselves, after the launch of the large ones and
+    // on a few compute units.  Beside 256-tiles they go along, one tile a row of blocks, while that launch has eight times as many.  Steps, us,
+    // apart | along: 6 layers of 1000 x 1000, 200 x 1000 and 2731 x 1000 1638 | 1511, 12 of 768, 192 and 2048 1657 | 1520, 2 of 2048, 256 and
+    // 5632 3182 | 3018, 12 of 1024, 256 and 2816 3015 | 2901, 8 of 2048, 256 and 5632 (32 such matrices in 72 rounds) 10899 | 10895.
+    bool along[GEMM_MAX_LIST] = {};
+    for (int epi : {EPI_SYRK, EPI_SYMPOLY, EPI_BX, EPI_BX_UPD, EPI_BX_UPD_T}) {
+        long large = 0, more = 0;
+        bool short_side[GEMM_MAX_LIST] = {};
+        for (int i = 0; i < n; ++i) {
+            if (!adapt || items[i].epi != epi) continue;
+            if (gemm_cfg_tile(cfg[i]) == 256) large += count_tiles(items[i], 256);
+            else if (cfg[i] == GEMM_CFG_128_PINGPONG && items[i].g.rows == 256 && items[i].g.kdim >= 256 && tiles_fit(items[i], 256, 256))
+                short_side[i] = true, more += count_tiles(items[i], 256);
+        }
+        for (int i = 0; i < n && 8 * more <= large; ++i)
+            if (short_side[i]) cfg[i] = GEMM_CFG_256_PERSIST, along[i] = true;
+    }
+    // Large matrices and those that were to go along need not end in one launch (the persistent symmetric products take reductions of up to
+    // PPX_SYRK_MAXK columns): what has too few large ones beside it in its own launch goes back to its 128-tiles.  A step over 100 of 1024 x
+    // 2048 with 4 of 256 x 12288, whose four tiles of X.Xt were left alone like that: 5265 us, so 4994.
+    for (;;) {
+        const int launches = place_launches(items, n, adapt, cus, cfg, route);
+        bool alone = false;
+        for (int k = 0; k < launches; ++k) {
+            long large = 0, more = 0;
+            for (int i = 0; i < n; ++i)
+                if (route[i].launch == k && gemm_cfg_tile(cfg[i]) == 256) (along[i] ? more : large) += count_tiles(items[i], 256);
+            for (int i = 0; i < n && 8 * more > large; ++i)
+                if (along[i] && route[i].launch == k) cfg[i] = GEMM_CFG_128_PINGPONG, along[i] = false, alone = true;
+        }
+        if (!alone) return launches;
+    }
 }
 
 bool plan_flow(FlowList& l, int xcds, bool recorded) {

@@ -1,4 +1,6 @@
 """Matrices of one row of 256-tiles beside large ones: in the launches of those up to an eighth of their tiles, on 128-tiles beyond; the same bits."""
+import random
+
 import pytest
 import torch
 
@@ -26,6 +28,41 @@ def test_what_stays_on_128_tiles():
     assert _cfg(LARGE + [(100, 1000, 2)], "sympoly")[1] == _abi.CFG_128_PINGPONG  # 128 rows of storage
     assert _cfg(LARGE + [(200, 600, 2)], "bx_axpy")[1] == _abi.CFG_128_PINGPONG  # 640 columns of storage, no whole 256-tiles
     assert _cfg(LARGE + [(384, 1000, 2)], "sympoly")[1] == _abi.CFG_128_PINGPONG
+
+
+# The persistent symmetric products take reductions of at most 2048 columns: with large matrices on one side of that line and short ones on the
+# other they end in launches of their own.
+@pytest.mark.parametrize("shapes,along", [
+    ([(1024, 2048, 100), (256, 12288, 4)], False), ([(768, 2048, 384), (256, 4096, 4)], False), ([(1024, 2048, 100), (256, 2049, 4)], False),
+    ([(1024, 2048, 100), (256, 2048, 4)], True), ([(1024, 4096, 100), (256, 12288, 4)], True), ([(1024, 4096, 100), (256, 2048, 4)], True),
+    # some of each: those beyond the line keep their tiles where the large ones beyond it are too few
+    ([(1024, 2048, 100), (1024, 4096, 3), (256, 4096, 4)], False), ([(1024, 2048, 100), (1024, 4096, 4), (256, 4096, 4)], True),
+])
+def test_nothing_goes_along_in_a_launch_without_large_ones(shapes, along):
+    routes = _abi.routes(shapes, "syrk")
+    assert (routes[-1][0] != _abi.CFG_128_PINGPONG) == along, routes
+    assert (routes[-1][2] in [r[2] for r in routes[:-1]]) == along, routes
+
+
+def test_what_goes_along_shares_its_launch_for_drawn_calls():
+    """Every 256-tile of a matrix of one row of them lies in a launch with eight times as many of larger matrices."""
+    rng, taken = random.Random(5), 0
+    for _ in range(3000):
+        side = lambda: rng.choice([rng.randint(129, 256), 128 * rng.randint(3, 12), rng.randint(257, 2000)])  # noqa: E731
+        shapes = [(side(), rng.choice([512, 1000, 2048, 2049, 4096, 12288]), rng.randint(1, 120)) for _ in range(rng.randint(2, 5))]
+        for kind in ("syrk", "sympoly", "bx_axpy", "bx_axpy_update"):
+            own, along = {}, {}
+            for (r, c, n), (cfg, height, launch) in zip(shapes, _abi.routes(shapes, kind)):
+                if cfg == _abi.CFG_128_PINGPONG or launch < 0 or height != 256:
+                    continue
+                t, tn = -(-min(r, c) // 256), -(-max(r, c) // 256)
+                tiles = n * (t * tn if kind.startswith("bx") else t * (t + 1) // 2)
+                d = along if t == 1 else own
+                d[launch] = d.get(launch, 0) + tiles
+            for launch, tiles in along.items():
+                taken += 1
+                assert 8 * tiles <= own.get(launch, 0), (kind, shapes)
+    assert taken > 100
 
 
 @pytest.mark.gpu
