@@ -147,7 +147,7 @@ int muon_hip_apply_update(const void* const* p_ptrs, int p_dtype, void* workspac
 int muon_hip_ns_output(void* workspace, int rows, int cols, int batch, int steps, void* out, void* stream);
 
 /* muon_hip_ns_grouped and muon_hip_ns_output in one call, the same bits.  Matrices whose chain runs in one workgroup, and products on
- * 128-tiles, write `out` from there where that is faster; the workspace then does not hold the result. */
+ * 128-tiles (muon_hip_routes), write `out` from there where that is faster; the workspace then does not hold the result. */
 int muon_hip_ns_result(void* workspace, int rows, int cols, int batch, int steps, double a, double b, double c, void* out,
                        void* stream);
 
@@ -178,8 +178,9 @@ int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int 
                         int write_back_grad, void* stream);
 
 /* Which kernels the products of such a call take on a device of `cus` compute units where they are launched one by one, one entry per
- * bucket, for the product named by its MUON_HIP_K_ id (syrk, sympoly, bx, bx_update); touches no device.  For tests and
- * measurements. */
+ * bucket, for the product named by its MUON_HIP_K_ id (syrk, sympoly, bx, bx_update), or for the last one of muon_hip_ns_result over
+ * one bucket, on 128-tiles where it writes `out`; touches no device.  For tests and measurements. */
+#define MUON_HIP_ROUTE_RESULT 0x100
 typedef struct {
     int cfg;    /* MUON_HIP_CFG_256_PERSIST: the persistent kernel; otherwise the configuration of the one-tile kernel */
     int height; /* rows of a tile */

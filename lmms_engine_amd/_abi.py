@@ -17,6 +17,7 @@ LIB_PATH = os.path.join(_HERE, "libmuon_hip.so")
 F32, BF16 = 0, 1
 CFG_STAGED = -2
 FLOW_RECORDED = 0x100  # MUON_HIP_FLOW_RECORDED
+ROUTE_RESULT = 0x100  # MUON_HIP_ROUTE_RESULT
 CFG_AUTO, CFG_128_PIPE, CFG_256_PIPE, CFG_256_PINGPONG, CFG_128_PINGPONG, CFG_256_PERSIST, CFG_64_DEEP = -1, 0, 1, 2, 3, 4, 5
 GEMM_CONFIGS = list(range(4))
 K_MOMENTUM, K_NORMALIZE, K_SYRK, K_SYMPOLY, K_BX, K_UPDATE, K_ADAMW, K_ADAMW_MULTI, K_GRAD_NORM, K_CLIP_SCALE = range(10)
@@ -180,10 +181,11 @@ def workspace_bytes(rows: int, cols: int, batch: int) -> int:
 
 
 def routes(shapes, kernel: str, cus: int = 256):
-    """[(configuration, tile height, launch)] of the (rows, cols, matrices) of one call, for a product by its KERNEL_NAMES name."""
+    """[(configuration, tile height, launch)] of the (rows, cols, matrices) of one call, for a product by its KERNEL_NAMES name ("ns_result": the
+    last one of muon_hip_ns_result)."""
     buckets = (Bucket * len(shapes))(*[Bucket(rows=r, cols=c, batch=n) for r, c, n in shapes])
     out = (Route * len(shapes))()
-    check(lib().muon_hip_routes(buckets, len(shapes), KERNEL_NAMES.index(kernel), cus, out), "routes")
+    check(lib().muon_hip_routes(buckets, len(shapes), ROUTE_RESULT if kernel == "ns_result" else KERNEL_NAMES.index(kernel), cus, out), "routes")
     return [(r.cfg, r.height, r.launch) for r in out]
 
 

@@ -466,6 +466,28 @@ bool flow_of(const Work& w, int steps, double a, double b, double c, const Updat
     return plan_flow(l, xcds, recorded);
 }
 
+// The last product of a call that returns X, as one that writes `out` itself, where that is faster; whether it is.
+//
+// Only tiles of 128 do that.  Those of 256 that carry an epilogue through LDS are slower than the persistent ones by more than the copy takes
+// (8192 x 8192: 70 us for 53), and so are 128-tiles of large matrices where the product that writes X is a persistent one of tiles of their own
+// height: the difference grows with the reduction, the copy does not.  One iteration, us, copied | written here: 60 of 640 x 2560 486 | 444, 27 of
+// 1152 x 4304 833 | 783, 8 of 1664 x 6000 609 | 582, 8 of 1920 x 4096 503 | 503, 8 of 2432 x 2432 520 | 525, 6 of 2944 x 2944 652 | 673, 2 of 4480 x
+// 4480 656 | 686, one 8064 x 8064 1773 | 1898.
+constexpr int kResultRows = 2048;
+bool write_result(const Bucket& k, bool adapt, int cus, bf16_t* out, GemmItem& item) {
+    GemmItem direct = item;
+    GemmRoute plain, route;
+    direct.epi = k.p.rows <= k.p.cols ? EPI_BX_UPD : EPI_BX_UPD_T;
+    direct.g.upd_ptrs = (const void* const*)out;
+    direct.g.upd_dtype = GEMM_UPD_RESULT;
+    direct.g.upd_rows = k.p.rows;
+    direct.g.upd_cols = k.p.cols;
+    if (!adapt || plan_gemm_nt(&direct, 1, adapt, cus, &route) != 1 || route.cfg != GEMM_CFG_128_PINGPONG) return false;
+    if (k.p.Mp > kResultRows && plan_gemm_nt(&item, 1, adapt, cus, &plain) == 1 && plain.cfg == GEMM_CFG_256_PERSIST) return false;
+    item = direct;
+    return true;
+}
+
 // Normalise, then `steps` iterations; with `upd` the last B.X applies the parameter update instead of writing X'.
 // `out`: where the result goes, dense (one bucket; null: X).  Where the last product does not write it there, *left_in_x is set.
 int ns_chain(const Work& all, int steps, double a, double b, double c, const UpdateArgs* upd, hipStream_t s, bf16_t* out = nullptr,
@@ -525,19 +547,7 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
         if (int rc = launch_items(MUON_HIP_K_SYMPOLY, "sympoly launch", items, w.n, adapt, s)) return rc;
         adapt = stage_items(w, EPI_BX, cur, a, b, c, ppx, items);
         const bool last = upd && it == steps - 1;
-        if (out && it == steps - 1) {
-            // Tiles of 128 write the result themselves.  Those of 256 that carry an epilogue through LDS are slower than the persistent ones by
-            // more than the copy takes (8192 x 8192: 70 us for 53).
-            GemmItem direct = items[0];
-            GemmRoute route;
-            direct.epi = all.b[0].p.rows <= all.b[0].p.cols ? EPI_BX_UPD : EPI_BX_UPD_T;
-            direct.g.upd_ptrs = (const void* const*)out;
-            direct.g.upd_dtype = GEMM_UPD_RESULT;
-            direct.g.upd_rows = all.b[0].p.rows;
-            direct.g.upd_cols = all.b[0].p.cols;
-            if (adapt && plan_gemm_nt(&direct, 1, adapt, ms.cus, &route) == 1 && route.cfg == GEMM_CFG_128_PINGPONG) items[0] = direct;
-            else *left_in_x = true;
-        }
+        if (out && it == steps - 1 && !write_result(w.b[0], adapt, ms.cus, out, items[0])) *left_in_x = true;
         if (last)
             for (int i = 0; i < w.n; ++i) fold_update(items[i], w.b[i].p_ptrs, w.b[i].p.rows, w.b[i].p.cols, w.b[i].scale, *upd);
         if (int rc = launch_items(last ? MUON_HIP_K_BX_UPDATE : MUON_HIP_K_BX, "bx launch", items, w.n, adapt, s)) return rc;
@@ -696,7 +706,9 @@ int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int 
 int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cus, muon_hip_route* out) {
     if (!buckets || !out || n < 1 || n > MUON_HIP_MAX_BUCKETS || cus < 1) return fail(MUON_HIP_EINVAL, "bad bucket list or device");
     const int epi = kernel_id == MUON_HIP_K_SYRK ? EPI_SYRK : kernel_id == MUON_HIP_K_SYMPOLY ? EPI_SYMPOLY : EPI_BX;
-    if (epi == EPI_BX && kernel_id != MUON_HIP_K_BX && kernel_id != MUON_HIP_K_BX_UPDATE) return fail(MUON_HIP_EINVAL, "not a product");
+    const bool result = kernel_id == MUON_HIP_ROUTE_RESULT;
+    if (result && n != 1) return fail(MUON_HIP_EINVAL, "a result is that of one bucket");
+    if (epi == EPI_BX && !result && kernel_id != MUON_HIP_K_BX && kernel_id != MUON_HIP_K_BX_UPDATE) return fail(MUON_HIP_EINVAL, "not a product");
     Work w;
     int from[MUON_HIP_MAX_BUCKETS];
     alignas(256) static char nowhere[256];  // stands for a workspace: plans hold addresses, nothing is read through them
@@ -712,6 +724,7 @@ int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cu
     const bool adapt = stage_items(w, epi, 0, 1.0, 1.0, 1.0, ppx_counters(w), items);
     if (kernel_id == MUON_HIP_K_BX_UPDATE)
         for (int i = 0; i < w.n; ++i) fold_update(items[i], nullptr, w.b[i].p.rows, w.b[i].p.cols, 1.0, UpdateArgs{});
+    if (result) write_result(w.b[0], adapt, cus, (bf16_t*)nowhere, items[0]);
     if (plan_gemm_nt(items, w.n, adapt, cus, route) < 0) return fail(MUON_HIP_EINVAL, "no kernel takes these products");
     for (int i = 0; i < w.n; ++i) out[from[i]] = muon_hip_route{route[i].cfg, route[i].height, route[i].launch};
     return 0;

@@ -315,6 +315,18 @@ def test_tiles_of_odd_heights_where_the_matrices_fill_their_rounds(shape, height
     assert _abi.routes([shape], "bx_axpy")[0][1] == height
 
 
+@pytest.mark.parametrize("shape,direct", [
+    ((896, 4864, 1), True), ((640, 2560, 60), True), ((2560, 640, 60), True), ((1920, 8192, 4), True),
+    ((2176, 5632, 6), False), ((2944, 2944, 6), False), ((3456, 8192, 2), False), ((8064, 8064, 1), False), ((8192, 4480, 1), False), ((1024, 1024, 100), False),
+    ((2176, 2176, 1), True),  # (no persistent product to give up)
+])
+def test_the_last_product_writes_the_result_where_that_costs_less_than_the_copy(shape, direct):
+    """Short sides of an odd number of 128-tiles write a result on 128-tiles, X on persistent tiles of their own height."""
+    plain, result = (_abi.routes([shape], k)[0] for k in ("bx_axpy", "ns_result"))
+    assert (result[0] == _abi.CFG_128_PINGPONG) == direct, (plain, result)
+    assert direct or result == plain
+
+
 def test_clip_grad_norm_host_behaviour():
     """What clip_grad_norm_ decides before any kernel runs: the empty cases return what torch's
     _get_total_norm returns, a NaN order and CPU gradients are refused (no fallback path)."""
