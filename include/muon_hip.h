@@ -192,9 +192,8 @@ int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cu
  * group belong to one XCD) in the order in which the workgroups of an XCD take them; update: 0, or 1 for a call that updates
  * parameters, plus MUON_HIP_FLOW_RECORDED for one that is being recorded into a graph (over very little work only a call that is not
  * takes this way, for the sake of its launches).  Writes at most `capacity` of them; *count is how many there are, 0 for a call whose
- * products are launched one by one.  (Matrices with a short side beyond 64 that a workgroup each holds are answered for as if they were
- * tiled, as they are beside larger ones and under a named configuration; here and in muon_hip_routes.)  A tile starts when `before` tiles of its matrix are finished.  Touches no device; for tests and
- * measurements. */
+ * products are launched one by one or whose matrices run in a workgroup each.  A tile starts when `before` tiles of its matrix are
+ * finished.  Touches no device; for tests and measurements. */
 #define MUON_HIP_FLOW_RECORDED 0x100
 typedef struct {
     int group, bucket, matrix, iteration;

@@ -432,6 +432,15 @@ bool stage_items(const Work& w, int epi, int cur, double a, double b, double c, 
     return adapt;
 }
 
+// Whether a workgroup each takes the matrices of a bucket: where it holds them.  But short sides beyond 64 cost little among the tiles of larger
+// matrices, in one launch or one per product; a launch of their own in front of those would come on top (a step over such a mixture: 161 us
+// among the tiles, 231 with a launch of their own).
+bool in_workgroups(const Work& w, int i) {
+    bool tiles = false;
+    for (int k = 0; k < w.n; ++k) tiles |= !w.b[k].p.small;
+    return w.b[i].p.small && (w.b[i].p.M <= 64 || !tiles);
+}
+
 // The iterations as one launch (gemm_nt.h), where that is the faster way and nobody has named a configuration.
 bool flow_of(const Work& w, int steps, double a, double b, double c, const UpdateArgs* upd, bf16_t* out, int xcds, bool recorded, FlowList& l) {
     if (g_forced_cfg.load(std::memory_order_relaxed) != MUON_HIP_CFG_AUTO) return false;
@@ -499,13 +508,9 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
     if (steps > 0) {
         ChainBucket small[MUON_HIP_MAX_BUCKETS];
         int n = 0;
-        // Short sides beyond 64 cost little among the tiles of larger matrices, in one launch or one per product; a launch of their own in front
-        // of those would come on top (a step over such a mixture: 161 us among the tiles, 231 with a launch of their own).
-        bool tiles = false;
-        for (int i = 0; i < all.n; ++i) tiles |= upd && !all.b[i].p.small;
         for (int i = 0; i < all.n; ++i) {
             const Bucket& k = all.b[i];
-            if (!k.p.small || (tiles && k.p.M > 64)) {
+            if (!in_workgroups(all, i)) {
                 w.b[w.n++] = k;
                 continue;
             }
@@ -552,6 +557,25 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
             for (int i = 0; i < w.n; ++i) fold_update(items[i], w.b[i].p_ptrs, w.b[i].p.rows, w.b[i].p.cols, w.b[i].scale, *upd);
         if (int rc = launch_items(last ? MUON_HIP_K_BX_UPDATE : MUON_HIP_K_BX, "bx launch", items, w.n, adapt, s)) return rc;
     }
+    return 0;
+}
+
+// What a description of a call stands on in place of a workspace: plans hold addresses, nothing is read through them.
+alignas(256) char g_nowhere[256];
+
+// The buckets of a call whose products are tiled, as ns_chain parts them, and where they stand in the call.
+int tiled_buckets(const muon_hip_bucket* buckets, int n, Work& w, int* from) {
+    Work all;
+    all.n = n;
+    for (int i = 0; i < n; ++i) {
+        if (int rc = all.b[i].init(buckets[i].rows, buckets[i].cols, buckets[i].batch, g_nowhere)) return rc;
+        all.b[i].p_ptrs = (const void* const*)g_nowhere;
+    }
+    for (int i = 0; i < n; ++i)
+        if (!in_workgroups(all, i)) {
+            from[w.n] = i;
+            w.b[w.n++] = all.b[i];
+        }
     return 0;
 }
 
@@ -711,20 +735,15 @@ int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cu
     if (epi == EPI_BX && !result && kernel_id != MUON_HIP_K_BX && kernel_id != MUON_HIP_K_BX_UPDATE) return fail(MUON_HIP_EINVAL, "not a product");
     Work w;
     int from[MUON_HIP_MAX_BUCKETS];
-    alignas(256) static char nowhere[256];  // stands for a workspace: plans hold addresses, nothing is read through them
-    for (int i = 0; i < n; ++i) {
-        out[i] = muon_hip_route{MUON_HIP_CFG_AUTO, 0, -1};
-        Bucket& k = w.b[w.n];
-        if (int rc = k.init(buckets[i].rows, buckets[i].cols, buckets[i].batch, nowhere)) return rc;
-        if (!k.p.small || k.p.M > 64) from[w.n++] = i;
-    }
+    for (int i = 0; i < n; ++i) out[i] = muon_hip_route{MUON_HIP_CFG_AUTO, 0, -1};
+    if (int rc = tiled_buckets(buckets, n, w, from)) return rc;
     if (!w.n) return 0;
     GemmItem items[MUON_HIP_MAX_BUCKETS];
     GemmRoute route[MUON_HIP_MAX_BUCKETS];
     const bool adapt = stage_items(w, epi, 0, 1.0, 1.0, 1.0, ppx_counters(w), items);
     if (kernel_id == MUON_HIP_K_BX_UPDATE)
         for (int i = 0; i < w.n; ++i) fold_update(items[i], nullptr, w.b[i].p.rows, w.b[i].p.cols, 1.0, UpdateArgs{});
-    if (result) write_result(w.b[0], adapt, cus, (bf16_t*)nowhere, items[0]);
+    if (result) write_result(w.b[0], adapt, cus, (bf16_t*)g_nowhere, items[0]);
     if (plan_gemm_nt(items, w.n, adapt, cus, route) < 0) return fail(MUON_HIP_EINVAL, "no kernel takes these products");
     for (int i = 0; i < w.n; ++i) out[from[i]] = muon_hip_route{route[i].cfg, route[i].height, route[i].launch};
     return 0;
@@ -739,13 +758,7 @@ int muon_hip_flow_tiles(const muon_hip_bucket* buckets, int n, int steps, int up
     *count = 0;
     Work w;
     int from[MUON_HIP_MAX_BUCKETS];
-    alignas(256) static char nowhere[256];  // as in muon_hip_routes
-    for (int i = 0; i < n; ++i) {
-        Bucket& k = w.b[w.n];
-        if (int rc = k.init(buckets[i].rows, buckets[i].cols, buckets[i].batch, nowhere)) return rc;
-        k.p_ptrs = (const void* const*)nowhere;
-        if (!k.p.small || k.p.M > 64) from[w.n++] = i;
-    }
+    if (int rc = tiled_buckets(buckets, n, w, from)) return rc;
     FlowList l;
     const UpdateArgs u{};
     if (!w.n || steps == 0 || !flow_of(w, steps, 1.0, 1.0, 1.0, update ? &u : nullptr, nullptr, xcds, recorded, l)) return 0;

@@ -2236,10 +2236,10 @@ bool plan_flow(FlowList& l, int xcds, bool recorded) {
     // and all of them 12 % slower in the mean.  Beyond `mean` of 30000 the 256-tiles of large launches are worth what is lost between them.
     // (The figures are of XCDs of 32 compute units, which gfx950 has however it is partitioned.)
     if (mean < 30000 && most < 1.35 * mean - 15 * chain + 600) return true;
-    // A step over very little takes longer on the device (replays: 6 of 128 x 384 with 8 of 128 x 128 94.5 us in one launch, 74.0 without),
-    // but the caller waits for his own 14 launches less: steps of a model of 14 such matrices, one behind the other, 149 us and 199 (matrices
-    // of those sizes run in a workgroup each since; the rule is for sets of slightly larger ones).  A
-    // step that is being recorded has no such launches when it is replayed.
+    // A step over very little takes longer on the device, but the caller waits for his own 14 launches less.  Sets of 2 to 24 matrices of 129 x
+    // 129 to 256 x 768, steps one behind the other, one launch | a launch per product: with gradient clipping and an AdamW group around them, where
+    // the host sets the pace, 126 to 148 us | 156 to 177; alone, where the device does, 98 to 119 | 84 to 105.  The former are training
+    // iterations.  A step that is being recorded has no such launches when it is replayed.
     return !recorded && l.e[0].p_ptrs && l.p_dtype != GEMM_UPD_RESULT && 0.032 * most + 0.64 * chain + 55 < 120;
 }
 

@@ -9,7 +9,9 @@ from lmms_engine_amd import _abi
 from tests.test_gpu_parity import env  # noqa: F401
 
 MIXED = [(512, 512, 16), (256, 512, 16), (1408, 512, 16), (512, 1408, 8)]
-TINY = [(384, 128, 4), (128, 128, 4), (64, 128, 4), (128, 384, 2)]  # the 64-row matrices run in a workgroup each
+# the 64-row matrices run in a workgroup each; those of 128 rows would, were they alone
+TINY = [(384, 256, 2), (128, 128, 4), (64, 128, 4), (256, 384, 2)]
+ALONE = [(384, 128, 4), (128, 128, 4), (64, 128, 4), (128, 384, 2)]
 
 
 def _check_order(shapes, steps, update, xcds):
@@ -60,6 +62,10 @@ def test_calls_that_stay_with_a_launch_per_product():
     assert not _abi.flow_tiles([(896, 4864, 72), (896, 896, 48)], 5, True)  # large
     assert not _abi.flow_tiles([(256, 1024, 48)], 0, False)
     assert not _abi.flow_tiles([(16, 2048, 48)], 5, True)  # a workgroup per matrix
+    assert not _abi.flow_tiles(ALONE, 5, True) and not _abi.flow_tiles([(128, 512, 48)], 5, False)
+    for kind in ("syrk", "sympoly", "bx_axpy", "bx_axpy_update"):
+        assert [launch for _, _, launch in _abi.routes(ALONE, kind)] == [-1] * 4
+        assert [launch >= 0 for _, _, launch in _abi.routes(TINY, kind)] == [True, True, False, True]
     assert _abi.flow_tiles([(256, 1024, 48)], 5, False)
     for cfg in (_abi.CFG_STAGED, _abi.CFG_128_PINGPONG):
         _abi.check(_abi.lib().muon_hip_set_gemm_config(cfg))
