@@ -179,12 +179,13 @@ int muon_hip_step_multi(const muon_hip_bucket* buckets, int n, int p_dtype, int 
 
 /* Which kernels the products of such a call take on a device of `cus` compute units where they are launched one by one, one entry per
  * bucket, for the product named by its MUON_HIP_K_ id (syrk, sympoly, bx, bx_update), or for the last one of muon_hip_ns_result over
- * one bucket, on 128-tiles where it writes `out`; touches no device.  For tests and measurements. */
+ * one bucket, on 128-tiles where it writes `out`; for MUON_HIP_K_SMALL_CHAIN the launches of the matrices that a workgroup each takes (height: the rows
+ * that the kernel is built for).  Touches no device.  For tests and measurements. */
 #define MUON_HIP_ROUTE_RESULT 0x100
 typedef struct {
     int cfg;    /* MUON_HIP_CFG_256_PERSIST: the persistent kernel; otherwise the configuration of the one-tile kernel */
     int height; /* rows of a tile */
-    int launch; /* which launch of the stage it goes with; -1: no product, the whole chain runs in one workgroup per matrix */
+    int launch; /* which launch of the stage it goes with; -1: no product, the whole chain runs in one workgroup per matrix (MUON_HIP_K_SMALL_CHAIN: it does not) */
 } muon_hip_route;
 int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cus, muon_hip_route* out);
 

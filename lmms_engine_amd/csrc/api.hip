@@ -563,8 +563,8 @@ int ns_chain(const Work& all, int steps, double a, double b, double c, const Upd
 // What a description of a call stands on in place of a workspace: plans hold addresses, nothing is read through them.
 alignas(256) char g_nowhere[256];
 
-// The buckets of a call whose products are tiled, as ns_chain parts them, and where they stand in the call.
-int tiled_buckets(const muon_hip_bucket* buckets, int n, Work& w, int* from) {
+// The buckets of a call whose products are tiled, as ns_chain parts them, and where they stand in the call; or the others.
+int tiled_buckets(const muon_hip_bucket* buckets, int n, Work& w, int* from, bool others = false) {
     Work all;
     all.n = n;
     for (int i = 0; i < n; ++i) {
@@ -572,7 +572,7 @@ int tiled_buckets(const muon_hip_bucket* buckets, int n, Work& w, int* from) {
         all.b[i].p_ptrs = (const void* const*)g_nowhere;
     }
     for (int i = 0; i < n; ++i)
-        if (!in_workgroups(all, i)) {
+        if (in_workgroups(all, i) == others) {
             from[w.n] = i;
             w.b[w.n++] = all.b[i];
         }
@@ -732,12 +732,22 @@ int muon_hip_routes(const muon_hip_bucket* buckets, int n, int kernel_id, int cu
     const int epi = kernel_id == MUON_HIP_K_SYRK ? EPI_SYRK : kernel_id == MUON_HIP_K_SYMPOLY ? EPI_SYMPOLY : EPI_BX;
     const bool result = kernel_id == MUON_HIP_ROUTE_RESULT;
     if (result && n != 1) return fail(MUON_HIP_EINVAL, "a result is that of one bucket");
-    if (epi == EPI_BX && !result && kernel_id != MUON_HIP_K_BX && kernel_id != MUON_HIP_K_BX_UPDATE) return fail(MUON_HIP_EINVAL, "not a product");
+    const bool chain = kernel_id == MUON_HIP_K_SMALL_CHAIN;
+    if (epi == EPI_BX && !result && !chain && kernel_id != MUON_HIP_K_BX && kernel_id != MUON_HIP_K_BX_UPDATE) return fail(MUON_HIP_EINVAL, "not a product");
     Work w;
     int from[MUON_HIP_MAX_BUCKETS];
     for (int i = 0; i < n; ++i) out[i] = muon_hip_route{MUON_HIP_CFG_AUTO, 0, -1};
-    if (int rc = tiled_buckets(buckets, n, w, from)) return rc;
+    if (int rc = tiled_buckets(buckets, n, w, from, chain)) return rc;
     if (!w.n) return 0;
+    if (chain) {
+        ChainBucket small[MUON_HIP_MAX_BUCKETS] = {};
+        ChainRoute r[MUON_HIP_MAX_BUCKETS];
+        int order[MUON_HIP_MAX_BUCKETS];
+        for (int i = 0; i < w.n; ++i) small[i].rows = w.b[i].p.rows, small[i].cols = w.b[i].p.cols, small[i].batch = w.b[i].p.batch;
+        if (plan_ns_chain(small, w.n, cus, r, order) < 0) return fail(MUON_HIP_EINVAL, "no workgroup holds these matrices");
+        for (int i = 0; i < w.n; ++i) out[from[i]] = muon_hip_route{MUON_HIP_CFG_AUTO, 16 * r[i].blocks, r[i].launch};
+        return 0;
+    }
     GemmItem items[MUON_HIP_MAX_BUCKETS];
     GemmRoute route[MUON_HIP_MAX_BUCKETS];
     const bool adapt = stage_items(w, epi, 0, 1.0, 1.0, 1.0, ppx_counters(w), items);

@@ -32,5 +32,11 @@ struct ChainMath {
 bool chain_fits(int M, int K);
 // Whether a bucket's result is better written to `out` by the chain than copied there from X, on a device of `cus` compute units.
 bool chain_writes(int rows, int cols, int batch, const void* out, int cus);
+// The launches of a list on a device of `cus` compute units: for each bucket the kernel (blocks of 16 rows, fragments of X per lane) and the
+// launch that takes it, and the order in which the buckets start.  Returns how many launches there are, or -1 where a bucket does not fit.
+struct ChainRoute {
+    int blocks, frags, launch;
+};
+int plan_ns_chain(const ChainBucket* buckets, int n, int cus, ChainRoute* route, int* order);
 // Every bucket must fit; steps >= 1.  cus: compute units of the device.
 hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, int cus, hipStream_t stream);

@@ -755,41 +755,62 @@ bool chain_writes(int rows, int cols, int batch, const void* out, int cus) {
 // narrow ones lose a place: two workgroups of 8 fragments share a compute unit on their own kernel, on a wider one each has its own.
 // Steps (us, apart | together): 308 narrow with 84 of 16 x 5632 and 5632 x 16 178 | 140, a quarter of them 134 | 100; 12 of 24 x
 // 1024 to 2624 in three widths 164 | 82; 504 narrow of 24 x 1024 with 168 of 24 x 2200 189 | 199; 616 with 168 of rank 16 272 | 262.
+// With eight row blocks a workgroup has a compute unit of its own on either kernel (LDS, and registers), so there is nothing to lose: 400 of
+// 128 x 128 with 20 of 128 x 512 171 | 102, 1000 with 100 294 | 243, 400 of 128 x 256 with 300 of 128 x 400 347 | 269.
 //
 // Matrices of fewer row blocks go along, as if their rows were padded, while every workgroup of the launch has a compute unit of its own and
 // their waves have no more columns than those of the launch have: then they end before those do.
-hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, int cus, hipStream_t stream) {
-    if (n < 1 || n > CHAIN_MAX_LIST || cm.steps < 1) return hipErrorInvalidValue;
-    int order[CHAIN_MAX_LIST], per[CHAIN_MAX_LIST], blocks[CHAIN_MAX_LIST];
-    bool done[CHAIN_MAX_LIST] = {};
+int plan_ns_chain(const ChainBucket* buckets, int n, int cus, ChainRoute* route, int* order) {
+    if (n < 1 || n > CHAIN_MAX_LIST) return -1;
+    int per[CHAIN_MAX_LIST], blocks[CHAIN_MAX_LIST];
     for (int i = 0; i < n; ++i) {
         const ChainBucket& k = buckets[i];
         const int M = std::min(k.rows, k.cols), K = std::max(k.rows, k.cols);
-        if (!chain_fits(M, K)) return hipErrorInvalidValue;
+        if (!chain_fits(M, K)) return -1;
         blocks[i] = chain_blocks(M);
         per[i] = chain_per_wave(K);
         order[i] = i;
+        route[i].launch = -1;
     }
     std::stable_sort(order, order + n, [&](int x, int y) { return blocks[x] != blocks[y] ? blocks[x] > blocks[y] : per[x] > per[y]; });
+    int launches = 0;
     for (int at = 0; at < n; ++at) {
         const int head = order[at], mt = blocks[head], frags = chain_class(per[head] * mt);
-        if (done[head]) continue;
-        long narrow = 0;
+        if (route[head].launch >= 0) continue;
+        long narrow = 0, used = 0;
         for (int i = 0; i < n; ++i)
-            if (!done[i] && blocks[i] == mt && chain_class(per[i] * mt) == 8) narrow += buckets[i].batch;
-        const bool together = 2 * narrow <= 3L * cus;
+            if (route[i].launch < 0 && blocks[i] == mt && chain_class(per[i] * mt) == 8) narrow += buckets[i].batch;
+        const bool together = mt == 8 || 2 * narrow <= 3L * cus;
+        for (int k = at; k < n; ++k) {
+            const int i = order[k];
+            if (route[i].launch >= 0) continue;
+            if (blocks[i] == mt ? !together && chain_class(per[i] * mt) != frags : per[i] > per[head] || used + buckets[i].batch > cus) continue;
+            route[i] = ChainRoute{mt, frags, launches};
+            used += buckets[i].batch;
+        }
+        ++launches;
+    }
+    return launches;
+}
+
+hipError_t launch_ns_chain(const ChainBucket* buckets, int n, const ChainMath& cm, int cus, hipStream_t stream) {
+    ChainRoute route[CHAIN_MAX_LIST];
+    int order[CHAIN_MAX_LIST];
+    const int launches = plan_ns_chain(buckets, n, cus, route, order);
+    if (launches < 0 || cm.steps < 1) return hipErrorInvalidValue;
+    for (int k = 0; k < launches; ++k) {
         ChainList l;
         l.n = 0;
         l.start[0] = 0;
-        for (int k = at; k < n; ++k) {
-            const int i = order[k];
-            if (done[i]) continue;
-            const bool own = blocks[i] == mt ? together || chain_class(per[i] * mt) == frags : per[i] <= per[head] && (long)l.start[l.n] + buckets[i].batch <= cus;
-            if (!own) continue;
+        int mt = 0, frags = 0;
+        for (int j = 0; j < n; ++j) {
+            const int i = order[j];
+            if (route[i].launch != k) continue;
+            mt = route[i].blocks;
+            frags = route[i].frags;
             l.b[l.n] = buckets[i];
             l.start[l.n + 1] = l.start[l.n] + buckets[i].batch;
             ++l.n;
-            done[i] = true;
         }
         if (hipError_t e = mt == 8 ? launch_as<8>(frags, l, cm, stream) : mt == 4 ? launch_as<4>(frags, l, cm, stream)
                            : mt == 2 ? launch_as<2>(frags, l, cm, stream) : launch_as<1>(frags, l, cm, stream);

@@ -59,7 +59,7 @@ def test_infinities_zeros_and_nan(env, rows, cols):
 # compute units has at once
 @pytest.mark.parametrize("shapes", [
     [(s, 1) for s in SHAPES] + [((64, 128), 2), ((16, 96), 1), ((24, 500), 1), ((16, 2048), 1)], [((128, 384), 4), ((64, 128), 4), ((256, 512), 8)],
-    [((128, 128), 200), ((48, 100), 56)], [((128, 128), 200), ((48, 100), 57)],
+    [((128, 128), 200), ((48, 100), 56)], [((128, 128), 200), ((48, 100), 57)], [((128, 128), 385), ((100, 400), 3)],
 ])
 @pytest.mark.parametrize("dtype,offset", [(torch.float32, 0), (torch.bfloat16, 0), (torch.bfloat16, 3)])
 def test_steps_are_bitwise_the_tiled_products(env, shapes, dtype, offset):

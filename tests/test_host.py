@@ -327,6 +327,16 @@ def test_the_last_product_writes_the_result_where_that_costs_less_than_the_copy(
     assert direct or result == plain
 
 
+@pytest.mark.parametrize("shapes,launches", [
+    ([(128, 128, 385), (128, 512, 1)], [0, 0]), ([(512, 128, 20), (100, 100, 3000)], [0, 0]),  # one workgroup per compute unit on either kernel
+    ([(16, 96, 384), (16, 5000, 5)], [0, 0]), ([(16, 96, 385), (16, 5000, 5)], [1, 0]),  # the narrow ones share compute units on their own kernel
+    ([(128, 512, 200), (64, 128, 56), (64, 129, 1)], [0, 0, 1]), ([(128, 384, 4), (64, 513, 4), (64, 512, 4), (16, 128, 4)], [0, 1, 0, 0]),
+])
+def test_launches_of_matrices_in_workgroups(shapes, launches):
+    assert [launch for _, _, launch in _abi.routes(shapes, "small_chain")] == launches
+    assert [launch for _, _, launch in _abi.routes(shapes, "syrk")] == [-1] * len(shapes)
+
+
 def test_clip_grad_norm_host_behaviour():
     """What clip_grad_norm_ decides before any kernel runs: the empty cases return what torch's
     _get_total_norm returns, a NaN order and CPU gradients are refused (no fallback path)."""
