@@ -80,6 +80,44 @@ __device__ __forceinline__ FourOf<PT> update_four(const FourOf<PT>& p, uint32_t 
 __device__ __forceinline__ bool whole_rows(const void* p, int cols, bool turn) { return !turn && cols % 8 == 0 && (((uintptr_t)p) & 15) == 0; }
 __device__ __forceinline__ bool turned_pieces(const void* p, int M, bool turn, int elem) { return turn && M % 4 == 0 && ((uintptr_t)p & (4 * elem - 1)) == 0; }
 
+// The first `left` of W elements from any address on (whole pieces where they are all there, four together and single ones where they are not),
+// and back.
+template <int W, typename PT, typename V>
+__device__ __forceinline__ void load_cut(V& o, const PT* a, int left) {
+    typedef PT __attribute__((ext_vector_type(W), aligned(sizeof(PT)))) whole_any;
+    typedef FourOf<PT> __attribute__((aligned(sizeof(PT)))) four_any;
+    if (left >= W) {
+        o = *(const whole_any*)a;
+        return;
+    }
+    if (W == 8 && left >= 4) {
+        const FourOf<PT> f = *(const four_any*)a;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = f[e];
+    }
+#pragma unroll
+    for (int e = 0; e < W - 1; ++e)
+        if (e < left && (W == 4 || e >= 4 || left < 4) && e != 3) o[e] = a[e];
+}
+template <int W, typename PT, typename V>
+__device__ __forceinline__ void store_cut(PT* a, const V& o, int left) {
+    typedef PT __attribute__((ext_vector_type(W), aligned(sizeof(PT)))) whole_any;
+    typedef FourOf<PT> __attribute__((aligned(sizeof(PT)))) four_any;
+    if (left >= W) {
+        *(whole_any*)a = o;
+        return;
+    }
+    if (W == 8 && left >= 4) {
+        FourOf<PT> f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = o[e];
+        *(four_any*)a = f;
+    }
+#pragma unroll
+    for (int e = 0; e < W - 1; ++e)
+        if (e < left && (W == 4 || e >= 4 || left < 4) && e != 3) a[e] = o[e];
+}
+
 // Elsewhere in pieces from any address, or element by element, eight columns of a row of X at a time.  In two halves, so that the loads of several pieces are in flight
 // before the first store (the compiler cannot know that the pieces are apart: one after the other they cost a trip to memory each, eight for
 // a turned piece; see kBatch).
@@ -284,19 +322,44 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
                     }
             }
     }
+    // eight row blocks, elsewhere: the same pieces at the address of any element, and those that the matrix ends in element by element
+    const bool cut = MT == 8 && !vec && !tvec;
+    if constexpr (MT == 8)
+        if (cut) {
+#pragma unroll
+            for (int j = 0; j < NCH; ++j)
+#pragma unroll
+                for (int t = 0; t < MT; ++t) {
+                    if (j >= per) continue;
+                    if (turn) {
+                        const int row = chain_row<MT>(t, 4 * (lane & 3)), col = (first + j) * 32 + (lane >> 2);
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            bf16x4 p = {zero8[0], zero8[1], zero8[2], zero8[3]};
+                            load_cut<4>(p, u + (long)(col + 16 * h) * M + row, col + 16 * h < K ? M - row : 0);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) x[j][t][4 * h + e] = p[e];
+                        }
+                    } else {
+                        const int row = chain_row<MT>(t, i), col = col0 + j * 32;
+                        load_cut<8>(x[j][t], u + (long)row * K + col, row < M ? K - col : 0);
+                    }
+                }
+        }
     // d = bf(bf(sqrt(sum)) + 1e-7), in the order of the normalisation kernel: both halves of the workgroup add the same sums
     for (int t = (tid & 255) + 256; t < k.nparts; t += 256) s += k.partials[(long)b * k.nparts + t];
     s = wave_sum(s);
     if (lane == 0 && wave < 4) red[wave] = s;
     __syncthreads();
     const DivideBf16 div(rbf(rbf(sqrtf((red[0] + red[1]) + (red[2] + red[3]))) + 1e-7f));
-    bool exact = (vec || tvec) && div.fast;
+    const bool turned_in = tvec || (cut && turn);
+    bool exact = (vec || tvec || cut) && div.fast;
     if (exact) {
 #pragma unroll
         for (int j = 0; j < NCH; ++j)
             if (j < per) {
 #pragma unroll
-                for (int t = 0; t < MT; ++t) exact &= div.quick(x[j][t], tvec ? turn_in(tl, x[j][t], lane) : x[j][t]);
+                for (int t = 0; t < MT; ++t) exact &= div.quick(x[j][t], turned_in ? turn_in(tl, x[j][t], lane) : x[j][t]);
             }
     }
     if (!__all(exact)) {
@@ -623,6 +686,63 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
             }
         }
     };
+    // Eight row blocks, elsewhere: pieces of eight bf16 or four fp32 columns (turned: of four rows) at the address of any element, straight from the
+    // registers.  Element by element and through the work area, as below, such steps were slower than on the tiles: us, tiles | that | this,
+    // bf16: 300 of 511 x 127 249 | 289 | 233, 16 of 399 x 127 100 | 105 | 94, 300 of 101 x 511 236 | 260 | 227, one 512 x 128 behind a boundary 98 | 106 | 99.
+    // What is left is the unit that takes apart pieces behind a 4-byte boundary, lane by lane.
+    auto cut_update = [&](auto* pp) {
+        using PT = std::remove_pointer_t<decltype(pp)>;
+        auto run = [&](auto turned_c) {
+            constexpr bool TURNED = decltype(turned_c)::value;
+            constexpr int W = !TURNED && sizeof(PT) == 2 ? 8 : 4, H = 8 / W;  // elements of a piece, pieces of a fragment
+            constexpr int G = NCH * MT == 8 ? 4 : 8;
+            typedef PT __attribute__((ext_vector_type(W))) piece_t;
+            // piece h of fragment (j, t): where it lies, and how many elements from there on are the matrix's
+            auto place = [&](int j, int t, int h, long& at) {
+                const int row = chain_row<MT>(t, TURNED ? 4 * q : i), col = TURNED ? (first + j) * 32 + i + 16 * h : col0 + j * 32 + W * h;
+                at = TURNED ? (long)col * M + row : (long)row * K + col;
+                return j >= per ? 0 : TURNED ? (col < K ? M - row : 0) : row < M ? K - col : 0;
+            };
+#pragma unroll
+            for (int f0 = 0; f0 < NCH * MT; f0 += G) {
+                if (f0 / MT >= per) break;
+                piece_t o[G][H];
+#pragma unroll
+                for (int g = 0; g < G; ++g)
+#pragma unroll
+                    for (int h = 0; h < H; ++h) {
+                        long at;
+                        const int left = place((f0 + g) / MT, (f0 + g) % MT, h, at);
+                        load_cut<W>(o[g][h], pp + at, left);
+                    }
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const int j = (f0 + g) / MT, t = (f0 + g) % MT;
+                    if (j >= per) continue;
+                    const u32x4 v = __builtin_bit_cast(u32x4, TURNED ? turn_out(tl, x[j][t], lane) : x[j][t]);
+#pragma unroll
+                    for (int h = 0; h < H; ++h) {
+                        long at;
+                        const int left = place(j, t, h, at);
+                        if (left <= 0) continue;
+                        piece_t n;
+#pragma unroll
+                        for (int w = 0; w < W / 4; ++w) {
+                            FourOf<PT> f;
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) f[e] = o[g][h][4 * w + e];
+                            f = update_four<PT>(f, v[2 * (h + w)], v[2 * (h + w) + 1], k.scale, cm.decay, cm.alpha);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) n[4 * w + e] = f[e];
+                        }
+                        store_cut<W>(pp + at, n, left);
+                    }
+                }
+            }
+        };
+        if (turn) run(std::true_type{});
+        else run(std::false_type{});
+    };
     auto try_pieces = [&](auto* pp) {
         if (turned_pieces(p, M, turn, sizeof(*pp))) piece_update(pp, std::true_type{});
         else if (whole_rows(p, k.cols, turn)) piece_update(pp, std::false_type{});
@@ -630,6 +750,13 @@ __device__ __forceinline__ void chain_matrix(const ChainBucket& k, int b, const 
         return true;
     };
     if (k.p_ptrs && (cm.p_dtype == MUON_HIP_BF16 ? try_pieces((bf16_t*)p) : try_pieces((float*)p))) return;
+    if constexpr (MT == 8) {
+        if (k.p_ptrs) {
+            if (cm.p_dtype == MUON_HIP_BF16) cut_update((bf16_t*)p);
+            else cut_update((float*)p);
+            return;
+        }
+    }
 #pragma unroll
     for (int j = 0; j < NCH; ++j)
 #pragma unroll

@@ -86,6 +86,40 @@ def test_steps_are_bitwise_the_tiled_products(env, shapes, dtype, offset):
         assert torch.equal(p, q), s
 
 
+# every number of elements that a row's last piece of eight, or a column's last piece of four, can have, in a wave's first and second chunk
+@pytest.mark.parametrize("dtype,offsets", [(torch.float32, (0, 1)), (torch.bfloat16, (0, 1, 4))])
+def test_parameters_that_end_inside_a_piece(env, dtype, offsets):
+    lib, dev, code = env["lib"], env["dev"], _abi.dtype_code(dtype)
+    shapes = [(66, 472 + k) for k in range(1, 8)] + [(66, 240 + k) for k in range(1, 8)] + [(479 - k, 124 + k) for k in range(1, 4)] + [(130 + k, 68 - k) for k in range(1, 4)]
+    for rows, cols in shapes:
+        print(f"cut pieces {rows}x{cols} {dtype}", flush=True)
+        gen = torch.Generator().manual_seed(rows + cols)
+        n = rows * cols
+        w, g = (torch.randn(2, rows, cols, generator=gen).to(dtype) for _ in range(2))
+        ws = torch.empty(lib.muon_hip_workspace_bytes(rows, cols, 2), dtype=torch.uint8, device=dev)
+        assert _abi.routes([(rows, cols, 2)], "small_chain")[0][1] == 128
+        for by in offsets:
+            out = []
+            for folded in (True, False):
+                place = torch.full((2, -(-n // 8) * 8 + 16), 7.0, dtype=dtype, device=dev)
+                p = place[:, by:by + n]
+                p.copy_(w.view(2, n))
+                gd, m = g.to(dev), torch.zeros(2, rows, cols, dtype=dtype, device=dev)
+                table = torch.tensor([t.data_ptr() for x in (p, gd, m) for t in x], dtype=torch.int64, device=dev)
+                tp, tg, tm = (table.data_ptr() + 16 * i for i in range(3))
+                ns = (3.4445, -4.775, 2.0315)
+                if folded:
+                    _abi.check(lib.muon_hip_step_grouped(tp, tg, tm, code, code, code, ws.data_ptr(), rows, cols, 2, 0.02, 0.01, 0.95, 1, 5, 0.7, *ns, 0, 0))
+                else:
+                    _abi.check(lib.muon_hip_momentum_norm(tg, tm, code, code, ws.data_ptr(), rows, cols, 2, 0.95, 1, 0, 0))
+                    _abi.check(lib.muon_hip_ns_grouped(ws.data_ptr(), rows, cols, 2, 5, *ns, 0))
+                    _abi.check(lib.muon_hip_apply_update(tp, code, ws.data_ptr(), rows, cols, 2, 5, 0.7, 0.02, 0.01, 0))
+                torch.cuda.synchronize()
+                assert bool((place[:, :by] == 7).all()) and bool((place[:, by + n:] == 7).all())
+                out.append(p.clone())
+            assert torch.equal(*out) and not torch.equal(out[0].cpu(), w.view(2, n)), (rows, cols, by)
+
+
 @pytest.mark.parametrize("rows,cols,batch", [(100, 333, 3), (333, 100, 3), (333, 101, 2), (128, 256, 260), (511, 128, 2)])
 def test_results_and_stages_bitwise(env, rows, cols, batch):
     """muon_hip_ns_result against muon_hip_ns_grouped and muon_hip_ns_output, on aligned outputs and on others, and nothing around them."""
