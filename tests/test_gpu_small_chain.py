@@ -1,6 +1,6 @@
 """Matrices with a short side of at most 64, whose whole Newton-Schulz chain runs in one workgroup each (small_chain.hip): edges
 of the 16-row blocks and 32-column chunks, one chunk per wave and less, the longest long side of every kernel and one past it
-(which the tiled products take), both orientations, ragged sizes."""
+(which the tiled products take), one row past it, both orientations, ragged sizes."""
 import pytest
 import torch
 
@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 1), (1, 9), (3, 33), (15, 16), (16, 31), (16, 256), (16, 257), (13, 2048), (16, 2049), (16, 4097), (16, 8192), (7, 8185),
           (17, 17), (32, 96), (24, 1024), (32, 1025), (31, 4095), (33, 64), (64, 64), (64, 512), (48, 513), (50, 1025), (64, 2048),
-          (16, 8193), (32, 4097), (64, 2049), (65, 128)]
+          (16, 8193), (32, 4097), (64, 2049), (65, 128), (65, 513)]
 
 
 @pytest.mark.parametrize("rows,cols", SHAPES)

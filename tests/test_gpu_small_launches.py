@@ -133,12 +133,18 @@ def test_named_configurations_agree_bitwise(env, rows, cols, batch):
         assert torch.equal(o, out[0]), i
 
 
-# 32 workgroups of the normalisation per 128 x 512 matrix: 512 matrices are the most whose workgroups add the norm's partial sums
-# themselves, one more takes the launch that adds them; turned matrices have no such limit
-@pytest.mark.parametrize("rows,cols,batch", [(128, 512, 512), (128, 512, 513), (512, 128, 1100)])
+# 64 workgroups of the normalisation per 200 x 512 matrix: 256 matrices are the most whose workgroups add the norm's partial sums
+# themselves, one more takes the launch that adds them; turned matrices have no such limit, up to 256 partial sums of 4096 elements each
+@pytest.mark.parametrize("rows,cols,batch", [(200, 512, 256), (200, 512, 257), (512, 200, 600), (1025, 1024, 3), (1024, 1025, 3), (1024, 1024, 3)])
 def test_norms_of_large_and_small_batches_agree_bitwise(env, rows, cols, batch):
     print(f"norms {batch} x {rows} x {cols}", flush=True)
+    assert env["abi"].routes([(rows, cols, batch)], "syrk")[0][2] >= 0  # (matrices that a workgroup holds do not come that way)
     g = torch.randn(batch, rows, cols, generator=torch.Generator().manual_seed(batch)).bfloat16().to(env["dev"])
     got = env["mu"].fast_newtonschulz(g, 1)
     for lo in (0, batch // 2, batch - 3):
         assert torch.equal(got[lo:lo + 3], env["mu"].fast_newtonschulz(g[lo:lo + 3], 1)), lo
+    d = (g.double().square().sum((1, 2), keepdim=True).sqrt().bfloat16().float() + 1e-7).bfloat16()
+    x = env["mu"].fast_newtonschulz(g, 0)
+    want = (g.float() / d.float()).bfloat16()
+    # the norm itself is a bf16 value, whose neighbour it may come out as: at most 2^-7 away, and both quotients are rounded by up to 2^-9
+    assert bool(((x.float() - want.float()).abs() <= 3 * 2.0**-8 * want.float().abs()).all())
