@@ -69,10 +69,6 @@ __device__ __forceinline__ uint32_t axpy_bf16x2(float a, uint32_t x, uint32_t v)
     const uint32_t p = pack_bf16x2(a * low_bf16(x), a * high_bf16(x));
     return pack_bf16x2(low_bf16(p) + low_bf16(v), high_bf16(p) + high_bf16(v));
 }
-__device__ __forceinline__ bf16x8 axpy_bf16x8(float a, const bf16x8& x, const bf16x8& v) {
-    const u32x4 xw = __builtin_bit_cast(u32x4, x), vw = __builtin_bit_cast(u32x4, v);
-    return __builtin_bit_cast(bf16x8, u32x4{axpy_bf16x2(a, xw[0], vw[0]), axpy_bf16x2(a, xw[1], vw[1]), axpy_bf16x2(a, xw[2], vw[2]), axpy_bf16x2(a, xw[3], vw[3])});
-}
 
 // bf(u / d) with IEEE division, for bf16 values u and one bf16 value d.  u times the reciprocal of d rounds to the same value: a quotient of
 // two 8-bit significands is never halfway between two bf16 values (u = m d with an odd 9-bit m needs more than 8 bits) and at least 2^-17 of
