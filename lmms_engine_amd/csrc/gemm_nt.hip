@@ -426,7 +426,8 @@ __device__ __forceinline__ void epilogue_nn(const GemmArgs& g, const TileCoord& 
         }
     }
     // FOLD: the parameter, and this thread's piece u of the tile in it
-    const bool result = FOLD && g.upd_dtype == GEMM_UPD_RESULT;
+    // (launch_gemm_nt: no other kernel is given a result to write)
+    const bool result = FOLD && BM == 128 && NT == 512 && g.upd_dtype == GEMM_UPD_RESULT;
     void* pbase = !FOLD ? nullptr : result ? (bf16_t*)g.upd_ptrs + (long)tc.bidx * g.upd_rows * g.upd_cols : const_cast<void*>(g.upd_ptrs[tc.bidx]);
     const bool pbf = g.upd_dtype == MUON_HIP_BF16;
     constexpr int NSTRIP = BM / 128, NWV = NT / 64;
@@ -2278,6 +2279,7 @@ hipError_t launch_gemm_nt(const GemmItem* items, int n, bool adapt, hipStream_t 
             const long t = count_tiles(items[i], width, height);
             GemmArgs& g = l.g[l.n];
             g = items[i].g;
+            if (g.upd_dtype == GEMM_UPD_RESULT && cfg != GEMM_CFG_128_PINGPONG) return hipErrorInvalidValue;
             g.tiles_m = (g.rows + height - 1) / height;
             g.tiles_n = (g.cols + width - 1) / width;
             g.tiles_per_mat = (int)(t / g.batch);
