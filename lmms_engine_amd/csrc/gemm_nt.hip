@@ -2169,7 +2169,7 @@ int plan_gemm_nt(const GemmItem* items, int n, bool adapt, int cus, GemmRoute* r
     }
     // Large matrices and those that were to go along need not end in one launch (the persistent symmetric products take reductions of up to
     // PPX_SYRK_MAXK columns): what has too few large ones beside it in its own launch goes back to its 128-tiles.  A step over 100 of 1024 x
-    // 2048 with 4 of 256 x 12288, whose four tiles of X.Xt were left alone like that: 5265 us, so 4994.
+    // 2048 with 4 of 256 x 12288, whose four tiles of X.Xt were left alone like that: 5314 us, so 4977.
     for (;;) {
         const int launches = place_launches(items, n, adapt, cus, cfg, route);
         bool alone = false;

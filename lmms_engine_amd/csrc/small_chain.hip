@@ -24,7 +24,8 @@
 // Eight waves share the columns of X in chunks of 32, a run of consecutive chunks each.  Lane (i = l%16, q = l/16) of a wave holds
 // X[r][8q .. 8q+7] of a chunk for one row r of every block of 16 rows (chain_row): an operand fragment of
 // v_mfma_f32_16x16x32_bf16 as it stands, so
-//   A = X Xt      contracts such fragments with one another; the sum of a 16x16 block goes from wave to wave through LDS;
+//   A = X Xt      contracts such fragments with one another; the sum of a 16x16 block goes from wave to wave through LDS (beyond 64 rows all of X
+//                 does, and a wave sums whole blocks);
 //   B = bA + cAA  is a handful of MFMAs on A in LDS;
 //   X' = aX + BX  contracts rows, for which a chunk is turned on its way through 1 KB of LDS: a transposing read gives four rows of
 //                 one column, and the rows are dealt to the lanes so that two blocks make eight consecutive rows, the fragment
@@ -246,6 +247,7 @@ struct ChainShared<8> {
     float red[4];
     int left[1];
 };
+static_assert(sizeof(ChainShared<8>) <= 139 * 1024 && sizeof(ChainShared<8>) > 80 * 1024, "one workgroup of eight row blocks per compute unit, of 160 KB");
 
 // Matrix b of bucket k.  MT blocks of 16 rows (1, 2, 4 or 8), up to NCH chunks of 32 columns per wave.
 template <int MT, int NCH>
