@@ -65,7 +65,7 @@ def test_widths_together_and_apart_are_bitwise_the_tiled_products(env, narrow, w
     assert all(torch.equal(p, q) for p, q in zip(*out))
 
 
-@pytest.mark.parametrize("rows,cols", [(16, 96), (64, 128), (20, 61), (128, 256)])
+@pytest.mark.parametrize("rows,cols", [(16, 96), (64, 128), (20, 61), (128, 256), (101, 259)])
 def test_quotients_among_the_subnormal_numbers(env, rows, cols):
     """Elements so far below the norm that X = u / d is no normal number, beside ordinary ones: the quotient itself, of IEEE division, in X
     after no iteration, and the same bits on the chain and on the tiled kernels after one."""
